@@ -381,6 +381,17 @@ int lq_adam8_latent_w4_step(const void *grad, void *codes, int32_t *residual, co
                             int dk3, int qk1, float qb1, int qk2, float qb2, int qk3, double beta1, double beta2,
                             double eps, double step_size, void *stream);
 
+/* The same step for an A16W4 layer in stochastic-rounding mode (lbit = 0): lq_adam8_update's direction
+ * bf16(m / d) fed straight into lq_requant_sr with lr = step_size, without ever being stored. Moments, block parameters
+ * and codes are those of the two calls bit for bit (Philox mode; the call consumes N*K/8 counters). codes_in / codes_out:
+ * N*K/2 bytes, native layout, 4-byte aligned, may alias each other; scales, zeros: bf16[N*K/128]; the rest as
+ * lq_adam8_update with n = N*K. Replaces the Adam chain and the requantise step of MyAdam.update_step
+ * (utils/quant.py:1081-1144). */
+int lq_adam8_sr_step(const void *grad, const void *codes_in, void *codes_out, const void *scales, const void *zeros,
+                     uint8_t *state1, uint8_t *state2, float *scale1, float *max1, float *scale2, float *max2, int64_t N,
+                     int64_t K, int group, int block_elems, double beta1, double beta2, double eps, double step_size,
+                     uint64_t philox_seed, uint64_t philox_offset, void *stream);
+
 /* The same for an 8-bit-weight layer (QLinearA8W8 with lbit = 4): the parameter is rebuilt from the int8 codes, the
  * per-row bf16 scales and the residual words exactly as lq_latent_w8_reconstruct does
  * (ResidualTensor.add((p.data * p.qparam).to(dtype)), utils/quant.py:826-837, 1069-1070), updated, and re-quantised

@@ -21,9 +21,9 @@ __device__ __forceinline__ u32x2_t act_quant8(const u32x4_t v, float c, float r)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const float f = (j & 1) ? lq_bf16_hi(v[j >> 1]) : lq_bf16_lo(v[j >> 1]);
-        const float a = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(f * 127.0f));
+        const float a = lq_bf16r(f * 127.0f);
         if (kFast) {
-            const float q = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(a * r)) + 128.0f;
+            const float q = lq_bf16r(a * r) + 128.0f;
             switch (j & 3) {
                 case 0: w[j >> 2] = act_cvt_pk_u8<0>(q, w[j >> 2]); break;
                 case 1: w[j >> 2] = act_cvt_pk_u8<1>(q, w[j >> 2]); break;
@@ -31,7 +31,7 @@ __device__ __forceinline__ u32x2_t act_quant8(const u32x4_t v, float c, float r)
                 default: w[j >> 2] = act_cvt_pk_u8<3>(q, w[j >> 2]); break;
             }
         } else {
-            const float q = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(a / c));
+            const float q = lq_bf16r(a / c);
             const float rr = q == q ? __builtin_amdgcn_fmed3f(rintf(q), -128.0f, 127.0f) : 0.0f;
             w[j >> 2] |= ((unsigned)(int)rr & 0xFFu) << (8 * (j & 3));
         }
@@ -58,8 +58,8 @@ __device__ __forceinline__ void act_quant_piece(const unsigned short *__restrict
     } else {
         for (long long i = base; i < n && i < base + 8; ++i) {
             float f = lq_bf16_bits_to_f32(x[i]);
-            float a = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(f * 127.0f));
-            float q = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(a / c));
+            float a = lq_bf16r(f * 127.0f);
+            float q = lq_bf16r(a / c);
             float rr = q == q ? __builtin_amdgcn_fmed3f(rintf(q), -128.0f, 127.0f) : 0.0f;
             x8[i] = (signed char)(int)rr;
         }
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void act_quant_dyn_kernel(const unsigned short
     k = wg_max_u32(k, red);
     const float c = max_key_value(k);
     float alpha = c * (1.0f / 127.0f);
-    if (alpha_bf16) alpha = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(alpha));
+    if (alpha_bf16) alpha = lq_bf16r(alpha);
     const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
     if (gid == 0) {
         work[0] = c;
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void act_dequant_kernel(const u32x4_t *__restr
                                                           int per_token) {
     const long long L = (long long)blockIdx.x * 256 + threadIdx.x;
     if (L >= n_chunks) return;
-    const float s = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(scale[per_token ? L / chunks_per_row : 0]));
+    const float s = lq_bf16r(scale[per_token ? L / chunks_per_row : 0]);
     const u32x4_t c = x8[L];
     u32x4_t o[2];
 #pragma unroll
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void act_fake_quant_kernel(const unsigned shor
     const long long base = ((long long)blockIdx.x * 256 + threadIdx.x) * 8;
     if (base >= n) return;
     auto one = [&](float f) {
-        const float a = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(f * s));
+        const float a = lq_bf16r(f * s);
         const float q = a != a ? a : __builtin_amdgcn_fmed3f(rintf(a), -128.0f, 127.0f);
         return fast ? q * r : q / s;
     };

@@ -15,130 +15,124 @@
 // Every tensor operation computes in fp32 and rounds its result to the tensor's type; an
 // operation of the form a + alpha * b is a fused multiply-add inside the tensor library's
 // kernels. This kernel is that chain in one pass with the same rounding points, so its results
-// equal the chain's bit for bit: 8 elements per thread (16 bytes of gradient and parameter, 8
-// bytes of each moment), the block's minimum and maximum found by a reduction over the BS/8
-// threads of the block, 6 bytes read and 4 written per element instead of ~120.
+// equal the chain's bit for bit.
 //
-// In its latent mode the kernel also takes over the two passes around the step in the exact
-// 4-bit-residual mode of the A16W4 layer: the parameter is rebuilt from codes and residual words
-// (as lq_latent_w4_reconstruct does) and the updated value goes straight back to codes and
-// residual words (as lq_latent_w4_requant does); a thread's 8 elements are one code word and one
-// residual word. The whole optimizer step of a layer is then one pass over 4 + 4 bytes of codes
-// and residual, 16 of gradient and 16 of moments per 8 elements.
+// What becomes of the direction is the kernel's mode: it updates a bf16 parameter, is stored, is fed straight into the
+// stochastic-rounding requantizer (lq_requant_math.h: the codes are rewritten and the direction never stored), or
+// updates a latent weight kept as codes + residual words, rebuilt and re-quantised on the spot with the arithmetic of
+// lq_latent_w4_* / lq_latent_w8_*.
+//
+// The kernel is bound by vector-ALU issue (the bytes alone would take half its time), so the split and the sequences
+// below are chosen for instructions per element: a block of 2048 is 128 threads of two 8-element chunks (4 M elements
+// still give 16 waves per compute unit, and the block reduction costs 16 elements instead of 8), rounding to bf16 is one
+// conversion whose other half is zero, and the operands on which a short sequence would not be exact are looked for with
+// the minima and maxima that the block reduction needs anyway, one branch per chunk. Measured on 8192 x 2048 with
+// operands from HBM (bytes at the 5.05 TB/s of a large copy in brackets), against the form with 8 elements per thread,
+// two rounding instructions, two barriers and the exact square root computed beside the short one:
+//   parameter 42.5 -> 37.6 us (33.3), direction 39.3 -> 30.7 (26.6), direction + requantizer 48.2 -> 33.7 in one pass
+//   (23.3), int4 + residual 63.0 -> 50.6 (26.7), int8 + residual 60.4 -> 48.5 (29.9).
 #include "lq_latent_math.h"
+#include "lq_requant_math.h"
 
 namespace {
 
-__device__ __forceinline__ float bf16r(float v) { return lq_bf16r(v); }
-
 struct Adam8Params {
     const u32x4_t *grad;     // bf16
-    u32x4_t *param;          // bf16, updated in place, or null
-    u32x4_t *direction;      // bf16 m / d, or null
+    u32x4_t *param;          // bf16, updated in place
+    u32x4_t *direction;      // bf16 m / d (or |m / d|)
     u32x2_t *state1, *state2;  // uint8 moments, updated in place
     float *scale1, *max1, *scale2, *max2;  // per block, updated in place
-    long long n_threads;     // elements / 8
+    long long n_blocks;
     float beta1, one_minus_beta1, beta2, one_minus_beta2, eps, neg_step;
-    // latent mode: the parameter lives as codes + residual words (one of each per thread)
+    // latent and stochastic-rounding modes of a 4-bit layer: one code word per 8 elements, group scales and zeros
+    const unsigned *codes_in;
     unsigned *codes, *residual;
     const unsigned short *wscales, *wzeros;  // per group of 128 elements
     CodecParams dequant_curve, quant_curve;
     // latent mode of an 8-bit-weight layer: int8 codes (8 per thread), one bf16 scale per row of K elements
     u32x2_t *codes8;
     const unsigned short *qscales;
-    long long threads_per_row;  // K / 8
+    long long chunks_per_row;  // K / 8
+    unsigned long long seed, offset;  // stochastic rounding: one Philox block per chunk
 };
 
-enum { LATENT_NONE = 0, LATENT_W4 = 1, LATENT_W8 = 2 };
+// What the step does with m / d
+enum {
+    ADAM_PARAM = 0,   // bf16 parameter in place
+    ADAM_DIR = 1,     // bf16(m / d) stored
+    ADAM_SR = 2,      // stochastic-rounding requantizer on 4-bit codes
+    ADAM_W4 = 3,      // 4-bit codes + residual words
+    ADAM_W8 = 4,      // int8 codes + residual words
+    ADAM_RATIO = 5,   // bf16(|m| / d) stored and nothing updated
+};
 
-// minimum and maximum over the W threads that share a block (W = 16: one 16-lane row of the
-// wave, by cross-lane shuffles; W = 256: the whole workgroup, through LDS)
-template <int W>
-__device__ __forceinline__ void block_minmax(float &lo, float &hi, float (*red)[2]) {
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-        lo = fminf(lo, __shfl_xor(lo, off, 64));
-        hi = fmaxf(hi, __shfl_xor(hi, off, 64));
-    }
-    if constexpr (W == 256) {
-#pragma unroll
-        for (int off = 16; off < 64; off <<= 1) {
-            lo = fminf(lo, __shfl_xor(lo, off, 64));
-            hi = fmaxf(hi, __shfl_xor(hi, off, 64));
-        }
-        const int wave = threadIdx.x >> 6;
-        __syncthreads();  // the previous use of red has been read
-        if ((threadIdx.x & 63) == 0) { red[wave][0] = lo; red[wave][1] = hi; }
-        __syncthreads();
-        lo = fminf(fminf(red[0][0], red[1][0]), fminf(red[2][0], red[3][0]));
-        hi = fmaxf(fmaxf(red[0][1], red[1][1]), fmaxf(red[2][1], red[3][1]));
-    }
+__device__ __forceinline__ float min3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
 }
-
-// byte SEL of `old` replaced by sat_u8(rne(v)) (v_cvt_pk_u8_f32)
-template <int SEL>
-__device__ __forceinline__ unsigned cvt_pk_u8(float v, unsigned old) {
-    unsigned r;
-    asm("v_cvt_pk_u8_f32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "n"(SEL), "v"(old));
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float min2(float a, float b) {  // (fminf would first quiet operands of unknown origin)
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float max2(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float min3_abs(float a, float b, float c) {  // of |a|, |b| and c
+    float r;
+    asm("v_min3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
 
-// m / d, correctly rounded, for two bf16 numbers. The quotient of two 8-bit significands keeps a relative
-// distance of at least 2^-33 from every midpoint of two fp32 numbers (m = d * mid has no solution: mid has 25
-// significant bits), and q0 = m r with the hardware reciprocal r (one ulp), corrected once by the exact residual
-// (q0 + (m - q0 d) r, one rounding), is within 2^-45 of the quotient: it rounds to the same fp32 number as the
-// IEEE division (every significand pair and every one-ulp variant of r is checked on the CPU). Quotients or
-// divisors outside [2^-40, 2^40] (residual underflow, overflow, zero, NaN) take the division (div_bf16_operands
-// names this sequence in the comments below; it is written out in the kernel).
+// byte I (0..7) of a pair of words as a float
+template <int I>
+__device__ __forceinline__ float byte_f32(const u32x2_t &w) {
+    return (float)((w[I >> 2] >> (8 * (I & 3))) & 0xFFu);
+}
 
 // x[8] -> uint8 codes with the block's (scale, max); returns them packed, 8 bytes.
-// The quotient (hi - x) / scale must be the correctly rounded one (a quotient one ulp off can fall
-// on the other side of a rounding tie). The divisor is shared by the whole block, so the division
-// is done with its correctly rounded reciprocal r = RN(1 / scale) and two residual corrections:
-// q0 = t*r; q1 = q0 + (t - q0*scale)*r is within one ulp of t/scale, and one more correction of a
-// quotient within one ulp returns RN(t / scale) exactly (Markstein's theorem; the residuals are
-// exact as long as they do not underflow, and a numerator below 2^-100 gives code 0 either way
-// because scale >= 1e-10). Half the instructions of an IEEE division. A scale above 2^60 (or NaN)
-// takes the plain division.
-__device__ __forceinline__ u32x2_t quantize8(const float x[8], float scale, float hi) {
+// The quotient (hi - x) / scale must be the correctly rounded one (a quotient one ulp off can fall on the other side of
+// a rounding tie). The divisor is shared by the whole block: with its correctly rounded reciprocal r = RN(1 / scale) and
+// what that leaves out, rl = (1 - r scale) r, q = t r + t rl is within one ulp of t / scale, and one residual correction
+// of a quotient within one ulp returns RN(t / scale) exactly (Markstein's theorem; the residual is exact as long as it
+// does not underflow, and a numerator below 2^-100 gives code 0 either way because scale >= 1e-10). A scale above 2^60
+// (or NaN) takes the plain division.
+__device__ __forceinline__ u32x2_t quantize8(const float (&x)[8], float scale, float hi, float r, float rl) {
     unsigned w[2] = {0u, 0u};
-    const bool fast = scale <= 0x1p60f;
-    const float r = 1.0f / scale;
+    float q[8];
+    if (scale <= 0x1p60f) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const float t = hi - x[k];
-        float q;
-        if (fast) {
-            const float q0 = t * r;
-            const float q1 = fmaf(fmaf(-q0, scale, t), r, q0);
-            q = fmaf(fmaf(-q1, scale, t), r, q1);
-        } else {
-            q = t / scale;
+        for (int k = 0; k < 8; ++k) {
+            const float t = hi - x[k];
+            const float q0 = fmaf(t, r, t * rl);
+            q[k] = fmaf(fmaf(-q0, scale, t), r, q0);
         }
-        // clamp(rint(q), 0, 255) and the byte insertion in one instruction (round to nearest even, saturating,
-        // NaN -> 0 like fmaxf(NaN, 0))
-        switch (k & 3) {
-            case 0: w[k >> 2] = cvt_pk_u8<0>(q, w[k >> 2]); break;
-            case 1: w[k >> 2] = cvt_pk_u8<1>(q, w[k >> 2]); break;
-            case 2: w[k >> 2] = cvt_pk_u8<2>(q, w[k >> 2]); break;
-            default: w[k >> 2] = cvt_pk_u8<3>(q, w[k >> 2]); break;
-        }
+    } else {
+        asm volatile("; plain division");  // (keeps this side from being computed along with the other one)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) q[k] = (hi - x[k]) / scale;
+    }
+    // clamp(rint(q), 0, 255) and the byte insertion in one instruction (round to nearest even, saturating,
+    // NaN -> 0 like fmaxf(NaN, 0))
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        w[h] = act_cvt_pk_u8<0>(q[4 * h], w[h]);
+        w[h] = act_cvt_pk_u8<1>(q[4 * h + 1], w[h]);
+        w[h] = act_cvt_pk_u8<2>(q[4 * h + 2], w[h]);
+        w[h] = act_cvt_pk_u8<3>(q[4 * h + 3], w[h]);
     }
     return u32x2_t{w[0], w[1]};
 }
 
-// bf16(sqrt(v)) for a bf16 value v. The square root of a number with 8 significant bits never
-// comes closer than 2^-19 (relative) to the midpoint of two bf16 values, so any fp32 square root
-// within two ulps rounds to the same bf16 value as the correctly rounded one (checked for every
-// bf16 input by the CPU tests); the hardware's v_sqrt_f32 (one ulp) replaces the ~12-instruction
-// correctly rounded sequence. Inputs below 2^-100 (the instruction does not take denormals) go
-// through the exact one.
-__device__ __forceinline__ float sqrt_bf16_to_bf16(float v) {
-    if (v >= 0x1p-100f) return bf16r(__builtin_amdgcn_sqrtf(v));
-    return bf16r(__builtin_sqrtf(v));
-}
-
-// A thread's 8 updated latent values back to one code word and one residual word (codec parameters by value)
+// A chunk's 8 updated latent values back to one code word and one residual word (codec parameters by value)
 template <bool kFast>
 __device__ __forceinline__ void requant8(const float (&out)[8], float ws, float wz, float wr, const CodecParams pq,
                                          unsigned &cnew, unsigned &rnew) {
@@ -151,7 +145,7 @@ __device__ __forceinline__ void requant8(const float (&out)[8], float ws, float 
     }
 }
 
-// The same for an 8-bit-weight layer: 8 code bytes and one residual word per thread
+// The same for an 8-bit-weight layer: 8 code bytes and one residual word per chunk
 template <bool kFast>
 __device__ __forceinline__ void requant8_w8(const float (&out)[8], float ws, float wr, const CodecParams pq, u32x2_t &cnew,
                                             unsigned &rnew) {
@@ -166,160 +160,226 @@ __device__ __forceinline__ void requant8_w8(const float (&out)[8], float ws, flo
     cnew = u32x2_t{cw[0], cw[1]};
 }
 
-template <int BS, int LATENT>
-__global__ __launch_bounds__(256) void adam8_update_kernel(Adam8Params a) {
-    constexpr int W = BS / 8;  // threads per block of the moments
-    __shared__ float red[4][2];
-    __shared__ float vtab[16];  // latent mode: dequantised values of the 16 residual nibbles
-    if constexpr (LATENT != LATENT_NONE) {
+// BS elements share one (scale, max) pair per moment: TPB threads of CH chunks of 8 elements, chunk c of thread t being
+// elements 8 (c TPB + t) .. + 7 of the block, so that every access of a wave is contiguous.
+template <int BS, int MODE>
+__global__ __launch_bounds__(256) void adam8_kernel(Adam8Params a) {
+    constexpr int CH = BS == 2048 ? 2 : 1, TPB = BS / 8 / CH, BPW = 256 / TPB;
+    __shared__ float red[4][4];
+    __shared__ float vtab[16];  // latent modes: dequantised values of the 16 residual nibbles
+    if constexpr (MODE == ADAM_W4 || MODE == ADAM_W8) {
         lq_latent_fill_value_table(vtab, a.dequant_curve);
         __syncthreads();
     }
-    const long long T = (long long)blockIdx.x * 256 + threadIdx.x;
-    const bool live = T < a.n_threads;  // n is a multiple of BS: a block is all-live or all-dead
-    const long long Tc = live ? T : 0;
-    const long long blk = Tc / W;
-    const u32x4_t g4 = a.grad[Tc];
-    const u32x2_t q1 = a.state1[Tc], q2 = a.state2[Tc];
+    const int t = threadIdx.x % TPB;
+    long long blk = (long long)blockIdx.x * BPW + threadIdx.x / TPB;
+    const bool live = blk < a.n_blocks;
+    if (!live) blk = 0;
+    const long long first = blk * (BS / 8) + t;  // the thread's first chunk; the next ones are TPB further
+    u32x4_t g4[CH], p4[CH];
+    u32x2_t q1[CH], q2[CH], c8[CH];
+    unsigned cword[CH], rword[CH];
+    unsigned short wsb[CH], wzb[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const long long T = first + c * TPB;
+        g4[c] = a.grad[T];
+        q1[c] = a.state1[T];
+        q2[c] = a.state2[T];
+        if constexpr (MODE == ADAM_PARAM) p4[c] = a.param[T];
+        if constexpr (MODE == ADAM_W4 || MODE == ADAM_SR) {
+            cword[c] = a.codes_in[T];
+            wsb[c] = a.wscales[T >> 4];
+            wzb[c] = a.wzeros[T >> 4];
+        }
+        if constexpr (MODE == ADAM_W8) {
+            c8[c] = a.codes8[T];
+            wsb[c] = a.qscales[T / a.chunks_per_row];
+        }
+        if constexpr (MODE == ADAM_W4 || MODE == ADAM_W8) rword[c] = a.residual[T];
+    }
     const float sc1 = a.scale1[blk], mx1 = a.max1[blk], sc2 = a.scale2[blk], mx2 = a.max2[blk];
-    u32x4_t p4 = {0u, 0u, 0u, 0u};
-    unsigned cword = 0, rword = 0;
-    float ws = 0.0f, wz = 0.0f;
-    u32x2_t c8 = {0u, 0u};
-    if constexpr (LATENT == LATENT_W4) {
-        cword = a.codes[Tc];
-        rword = a.residual[Tc];
-        ws = lq_bf16_bits_to_f32(a.wscales[Tc >> 4]);
-        wz = lq_bf16_bits_to_f32(a.wzeros[Tc >> 4]);
-    } else if constexpr (LATENT == LATENT_W8) {
-        c8 = a.codes8[Tc];
-        rword = a.residual[Tc];
-        ws = lq_bf16_bits_to_f32(a.qscales[Tc / a.threads_per_row]);
-    } else if (a.param) {
-        p4 = a.param[Tc];
-    }
 
-    // Phase 1: the moments. The square root and the quotient use short sequences that are exact on all but
-    // extreme operands; whether any of a thread's 8 elements is such an operand is collected in one flag per
-    // sequence, and the (cold) exact sequences then redo all 8: one branch per thread instead of one per element.
-    float m[8], d[8], v[8], out[8];
-    bool odd_sqrt = false;
+    float m[CH][8], d[CH][8];
+    float lo1, hi1, lo2, hi2;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const float g = (k & 1) ? lq_bf16_hi(g4[k >> 1]) : lq_bf16_lo(g4[k >> 1]);
-        const float c1 = (float)((q1[k >> 2] >> (8 * (k & 3))) & 0xFFu);
-        const float c2 = (float)((q2[k >> 2] >> (8 * (k & 3))) & 0xFFu);
-        float mk = bf16r(mx1 - c1 * sc1);
-        const float s2 = mx2 - c2 * sc2;
-        float vk = bf16r(s2 * s2);
-        mk = bf16r(mk * a.beta1);
-        mk = bf16r(fmaf(a.one_minus_beta1, g, mk));
-        vk = bf16r(vk * a.beta2);
-        vk = bf16r(fmaf(a.one_minus_beta2 * g, g, vk));
-        m[k] = mk;
-        v[k] = vk;
-        // bf16(sqrt(v)) from the hardware's one-ulp square root (see sqrt_bf16_to_bf16); it does not take
-        // denormals, so nonzero inputs below 2^-100 go through the exact one (zero, negative and NaN inputs give
-        // the same result either way)
-        d[k] = bf16r(__builtin_amdgcn_sqrtf(vk));
-        odd_sqrt |= vk < 0x1p-100f && vk > 0.0f;
-    }
-    if (odd_sqrt) {
+    for (int c = 0; c < CH; ++c) {
+        const long long T = first + c * TPB;
+        float v[8], ratio[8];
+        float g[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) d[k] = sqrt_bf16_to_bf16(v[k]);
-    }
-    float ratio[8];
-    bool odd_div = false;
+        for (int k = 0; k < 8; ++k) g[k] = (k & 1) ? lq_bf16_hi(g4[c][k >> 1]) : lq_bf16_lo(g4[c][k >> 1]);
+        const float c1[8] = {byte_f32<0>(q1[c]), byte_f32<1>(q1[c]), byte_f32<2>(q1[c]), byte_f32<3>(q1[c]),
+                             byte_f32<4>(q1[c]), byte_f32<5>(q1[c]), byte_f32<6>(q1[c]), byte_f32<7>(q1[c])};
+        const float c2[8] = {byte_f32<0>(q2[c]), byte_f32<1>(q2[c]), byte_f32<2>(q2[c]), byte_f32<3>(q2[c]),
+                             byte_f32<4>(q2[c]), byte_f32<5>(q2[c]), byte_f32<6>(q2[c]), byte_f32<7>(q2[c])};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        d[k] = bf16r(d[k] + a.eps);
-        const float r = __builtin_amdgcn_rcpf(d[k]);
-        const float q0 = m[k] * r;
-        if (LATENT == LATENT_NONE && !a.param) {
-            // Only bf16(m / d) is stored here, and the quotient of two bf16 numbers never comes closer
-            // than 2^-17 (relative) to the midpoint of two bf16 values (256 m_a = (2j+1) m_b has no
-            // solution with 8-bit significands), so any fp32 quotient within a few ulps rounds to the
-            // same bf16 value as the correctly rounded one (every significand pair is checked by the
-            // CPU tests): reciprocal and product instead of the division sequence. Results outside
-            // [2^-100, 2^100] (bf16 subnormals, overflow, NaN; zero numerators excepted) take the division.
-            ratio[k] = q0;
-            const float ar = fabsf(q0);
-            odd_div |= !(ar <= 0x1p100f && (ar >= 0x1p-100f || m[k] == 0.0f));
-        } else {
-            // The fp32 quotient itself enters the update: one residual correction of q0 gives the IEEE
-            // quotient of two bf16 numbers (div_bf16_operands) unless quotient or divisor leave [2^-40, 2^40].
-            ratio[k] = fmaf(fmaf(-q0, d[k], m[k]), r, q0);
-            const float aq = fabsf(ratio[k]), ad = fabsf(d[k]);
-            odd_div |= !(aq >= 0x1p-40f && aq <= 0x1p40f && ad >= 0x1p-40f && ad <= 0x1p40f);
+        for (int k = 0; k < 8; ++k) {
+            float mk = lq_bf16r(mx1 - c1[k] * sc1);
+            const float s2 = mx2 - c2[k] * sc2;
+            float vk = lq_bf16r(s2 * s2);
+            mk = lq_bf16r(mk * a.beta1);
+            m[c][k] = lq_bf16r(fmaf(a.one_minus_beta1, g[k], mk));
+            vk = lq_bf16r(vk * a.beta2);
+            v[k] = lq_bf16r(fmaf(a.one_minus_beta2 * g[k], g[k], vk));
+            // bf16(sqrt(v)) of a bf16 v: the square root of a number with 8 significant bits never comes closer than
+            // 2^-19 (relative) to the midpoint of two bf16 values, so the hardware's one-ulp square root rounds to the
+            // same bf16 value as the correctly rounded one (checked for every bf16 input by the CPU tests)
+            d[c][k] = lq_bf16r(lq_bf16r_trans(__builtin_amdgcn_sqrtf(v[k])) + a.eps);
+            // m / d of two bf16 numbers: reciprocal and product. Where the fp32 quotient itself enters an update, one
+            // residual correction makes it the IEEE one: the quotient of two 8-bit significands keeps a relative
+            // distance of at least 2^-33 from every midpoint of two fp32 numbers, and the corrected value is within
+            // 2^-45 of it (every significand pair and every one-ulp variant of the reciprocal is checked on the CPU).
+            // Where only bf16(m / d) is used the product does: the quotient never comes closer than 2^-17 to the
+            // midpoint of two bf16 values.
+            const float r = __builtin_amdgcn_rcpf(d[c][k]);
+            ratio[k] = m[c][k] * r;
+            if constexpr (MODE == ADAM_PARAM || MODE == ADAM_W4 || MODE == ADAM_W8)
+                ratio[k] = fmaf(fmaf(-ratio[k], d[c][k], m[c][k]), r, ratio[k]);
         }
-    }
-    if (odd_div) {
+        float clo1 = m[c][0], chi1 = m[c][0], clo2 = d[c][0], chi2 = d[c][0], mmin = fabsf(m[c][0]), vmin = v[0];
+        if (c) { clo1 = lo1; chi1 = hi1; clo2 = lo2; chi2 = hi2; }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) ratio[k] = m[k] / d[k];
-    }
+        for (int k = 0; k < 8; k += 2) {
+            clo1 = min3(m[c][k], m[c][k + 1], clo1); chi1 = max3(m[c][k], m[c][k + 1], chi1);
+            clo2 = min3(d[c][k], d[c][k + 1], clo2); chi2 = max3(d[c][k], d[c][k + 1], chi2);
+            mmin = min3_abs(m[c][k], m[c][k + 1], mmin);
+            vmin = min3(v[k], v[k + 1], vmin);
+        }
+        // The short sequences hold for v >= 2^-100 and 2^-80 <= |m| <= 2^80, 2^-40 <= d <= 2^40 (no subnormal, no
+        // underflowing residual, no overflow; NaN and infinity pass through them as through the plain ones). Chunks
+        // with anything else, zeros among them, take the plain operations.
+        const bool plain = !(vmin >= 0x1p-100f && mmin >= 0x1p-80f && fmaxf(fabsf(clo1), fabsf(chi1)) <= 0x1p80f &&
+                             clo2 >= 0x1p-40f && chi2 <= 0x1p40f);
+        if (plain) {
+            asm volatile("; plain square roots and divisions");
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if constexpr (LATENT == LATENT_W4) {
-            const float p = bf16r(lq_latent_value(lq_code(cword, k), vtab[(rword >> (28 - 4 * k)) & 0xFu], ws, wz));
-            out[k] = bf16r(fmaf(a.neg_step, ratio[k], p));
-        } else if constexpr (LATENT == LATENT_W8) {
-            const float p = bf16r(lq_latent_w8_value(c8[k >> 2] >> (8 * (k & 3)), vtab[(rword >> (28 - 4 * k)) & 0xFu], ws));
-            out[k] = bf16r(fmaf(a.neg_step, ratio[k], p));
-        } else if (a.param) {
-            const float p = (k & 1) ? lq_bf16_hi(p4[k >> 1]) : lq_bf16_lo(p4[k >> 1]);
-            out[k] = fmaf(a.neg_step, ratio[k], p);
-        } else {
-            out[k] = ratio[k];
+            for (int k = 0; k < 8; ++k) {
+                d[c][k] = lq_bf16r(lq_bf16r_trans(__builtin_sqrtf(v[k])) + a.eps);
+                ratio[k] = m[c][k] / d[c][k];
+                clo2 = fminf(clo2, d[c][k]);
+                chi2 = fmaxf(chi2, d[c][k]);
+            }
         }
-    }
-    if constexpr (LATENT == LATENT_W4) {
-        const bool fast = (ws >= 0x1p-40f) && (ws <= 0x1p40f);
-        const float wr = 1.0f / ws;
-        unsigned cnew = 0, rnew = 0;
-        if (fast) requant8<true>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
-        else requant8<false>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
-        if (live) {
-            a.codes[T] = cnew;
-            a.residual[T] = rnew;
-        }
-    } else if constexpr (LATENT == LATENT_W8) {
-        const bool fast = (fabsf(ws) >= 0x1p-40f) && (fabsf(ws) <= 0x1p40f);
-        const float wr = 1.0f / ws;
-        u32x2_t cnew;
-        unsigned rnew = 0;
-        if (fast) requant8_w8<true>(out, ws, wr, a.quant_curve, cnew, rnew);
-        else requant8_w8<false>(out, ws, wr, a.quant_curve, cnew, rnew);
-        if (live) {
-            a.codes8[T] = cnew;
-            a.residual[T] = rnew;
-        }
-    } else if (live) {
-        const u32x4_t o = {lq_pack_bf16(out[0], out[1]), lq_pack_bf16(out[2], out[3]), lq_pack_bf16(out[4], out[5]),
-                           lq_pack_bf16(out[6], out[7])};
-        if (a.param) a.param[T] = o;
-        else a.direction[T] = o;
-    }
+        lo1 = clo1; hi1 = chi1; lo2 = clo2; hi2 = chi2;
 
-    // the moments back to uint8 with the block's new (scale, max)
-    float lo1 = m[0], hi1 = m[0], lo2 = d[0], hi2 = d[0];
+        if constexpr (MODE == ADAM_W4) {
+            const float ws = lq_bf16_bits_to_f32(wsb[c]), wz = lq_bf16_bits_to_f32(wzb[c]);
+            float out[8];
 #pragma unroll
-    for (int k = 1; k < 8; ++k) {
-        lo1 = fminf(lo1, m[k]); hi1 = fmaxf(hi1, m[k]);
-        lo2 = fminf(lo2, d[k]); hi2 = fmaxf(hi2, d[k]);
+            for (int k = 0; k < 8; ++k) {
+                const float p = lq_bf16r(lq_latent_value(lq_code(cword[c], k), vtab[(rword[c] >> (28 - 4 * k)) & 0xFu], ws, wz));
+                out[k] = lq_bf16r(fmaf(a.neg_step, ratio[k], p));
+            }
+            const float wr = 1.0f / ws;
+            unsigned cnew = 0, rnew = 0;
+            if ((ws >= 0x1p-40f) && (ws <= 0x1p40f)) requant8<true>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
+            else requant8<false>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
+            if (live) {
+                a.codes[T] = cnew;
+                a.residual[T] = rnew;
+            }
+        } else if constexpr (MODE == ADAM_W8) {
+            const float ws = lq_bf16_bits_to_f32(wsb[c]);
+            float out[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float p = lq_bf16r(lq_latent_w8_value(c8[c][k >> 2] >> (8 * (k & 3)), vtab[(rword[c] >> (28 - 4 * k)) & 0xFu], ws));
+                out[k] = lq_bf16r(fmaf(a.neg_step, ratio[k], p));
+            }
+            const float wr = 1.0f / ws;
+            u32x2_t cnew;
+            unsigned rnew = 0;
+            if ((fabsf(ws) >= 0x1p-40f) && (fabsf(ws) <= 0x1p40f)) requant8_w8<true>(out, ws, wr, a.quant_curve, cnew, rnew);
+            else requant8_w8<false>(out, ws, wr, a.quant_curve, cnew, rnew);
+            if (live) {
+                a.codes8[T] = cnew;
+                a.residual[T] = rnew;
+            }
+        } else if constexpr (MODE == ADAM_SR) {
+            const float ws = lq_bf16_bits_to_f32(wsb[c]), wz = lq_bf16_bits_to_f32(wzb[c]);
+            const unsigned long long ctr = a.offset + (unsigned long long)T;
+            const lq_u4 A = lq_philox4x32_10((unsigned)ctr, (unsigned)(ctr >> 32), 0u, 0u, (unsigned)a.seed, (unsigned)(a.seed >> 32));
+            const unsigned aw[4] = {A.x, A.y, A.z, A.w};
+            float dir[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) dir[k] = lq_bf16r(ratio[k]);
+            const RequantGroup rg = requant_group(ws, wz);
+            unsigned cnew = requant_word(cword[c], dir, aw, -a.neg_step, rg);
+            if (!rg.fast) {
+                asm volatile("; one operation at a time");
+                cnew = 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    cnew |= requant_elem(lq_code(cword[c], k), ws, wz, dir[k], -a.neg_step, (aw[k >> 1] >> (16 * (k & 1))) & 0xFFFFu)
+                            << (4 * (k ^ 1));
+            }
+            if (live) a.codes[T] = cnew;
+        } else {
+            float out[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if constexpr (MODE == ADAM_PARAM) {
+                    const float p = (k & 1) ? lq_bf16_hi(p4[c][k >> 1]) : lq_bf16_lo(p4[c][k >> 1]);
+                    out[k] = fmaf(a.neg_step, ratio[k], p);
+                } else {
+                    out[k] = MODE == ADAM_RATIO ? fabsf(ratio[k]) : ratio[k];
+                }
+            }
+            const u32x4_t o = {lq_pack_bf16(out[0], out[1]), lq_pack_bf16(out[2], out[3]), lq_pack_bf16(out[4], out[5]),
+                               lq_pack_bf16(out[6], out[7])};
+            if (live) {
+                if constexpr (MODE == ADAM_PARAM) a.param[T] = o;
+                else a.direction[T] = o;
+            }
+        }
     }
-    block_minmax<W>(lo1, hi1, red);
-    block_minmax<W>(lo2, hi2, red);
+    if constexpr (MODE == ADAM_RATIO) return;
+
+    // the moments back to uint8 with the block's new (scale, max): minima and maxima over the block's threads (a
+    // 16-lane row of the wave, or two waves, through LDS)
+#pragma unroll
+    for (int off = 1; off < (TPB < 64 ? TPB : 64); off <<= 1) {
+        lo1 = min2(lo1, __shfl_xor(lo1, off, 64));
+        hi1 = max2(hi1, __shfl_xor(hi1, off, 64));
+        lo2 = min2(lo2, __shfl_xor(lo2, off, 64));
+        hi2 = max2(hi2, __shfl_xor(hi2, off, 64));
+    }
+    if constexpr (TPB == 128) {
+        const int wave = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) == 0) *reinterpret_cast<f32x4_t *>(red[wave]) = f32x4_t{lo1, hi1, lo2, hi2};
+        __syncthreads();
+        const f32x4_t other = *reinterpret_cast<const f32x4_t *>(red[wave ^ 1]);
+        lo1 = min2(lo1, other[0]); hi1 = max2(hi1, other[1]);
+        lo2 = min2(lo2, other[2]); hi2 = max2(hi2, other[3]);
+    }
     const float inv255 = 1.0f / 255.0f;  // the tensor library divides by a scalar as a multiplication by its reciprocal
     const float ns1 = (hi1 - lo1) * inv255 + 1e-10f;
     const float ns2 = (hi2 - lo2) * inv255 + 1e-10f;
-    if (live) {
-        a.state1[T] = quantize8(m, ns1, hi1);
-        a.state2[T] = quantize8(d, ns2, hi2);
-        if (T % W == 0) {
-            a.scale1[blk] = ns1; a.max1[blk] = hi1;
-            a.scale2[blk] = ns2; a.max2[blk] = hi2;
+    const float r1 = 1.0f / ns1, r2 = 1.0f / ns2;
+    const float rl1 = fmaf(-r1, ns1, 1.0f) * r1, rl2 = fmaf(-r2, ns2, 1.0f) * r2;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const u32x2_t n1 = quantize8(m[c], ns1, hi1, r1, rl1), n2 = quantize8(d[c], ns2, hi2, r2, rl2);
+        if (live) {
+            a.state1[first + c * TPB] = n1;
+            a.state2[first + c * TPB] = n2;
         }
     }
+    if (live && t == 0) {
+        a.scale1[blk] = ns1; a.max1[blk] = hi1;
+        a.scale2[blk] = ns2; a.max2[blk] = hi2;
+    }
+}
+
+template <int MODE>
+int adam8_launch(const char *who, Adam8Params &a, int64_t n, int block_elems, void *stream) {
+    a.n_blocks = n / block_elems;
+    const int per_wg = block_elems == 2048 ? 2 : 16;
+    const unsigned wgs = (unsigned)((a.n_blocks + per_wg - 1) / per_wg);
+    if (block_elems == 2048) hipLaunchKernelGGL((adam8_kernel<2048, MODE>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL((adam8_kernel<128, MODE>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, a);
+    return lq_check_launch(who);
 }
 
 }  // namespace
@@ -359,14 +419,9 @@ extern "C" int lq_adam8_update(const void *grad, void *param_or_null, void *dire
     a.direction = (u32x4_t *)direction_or_null;
     a.state1 = (u32x2_t *)state1; a.state2 = (u32x2_t *)state2;
     a.scale1 = scale1; a.max1 = max1; a.scale2 = scale2; a.max2 = max2;
-    a.n_threads = n / 8;
     adam8_scalars(a, beta1, beta2, eps, step_size);
-    const unsigned blocks = (unsigned)((a.n_threads + 255) / 256);
-    if (block_elems == 2048)
-        hipLaunchKernelGGL((adam8_update_kernel<2048, LATENT_NONE>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL((adam8_update_kernel<128, LATENT_NONE>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, a);
-    return lq_check_launch("lq_adam8_update");
+    if (param_or_null) return adam8_launch<ADAM_PARAM>("lq_adam8_update", a, n, block_elems, stream);
+    return adam8_launch<ADAM_DIR>("lq_adam8_update", a, n, block_elems, stream);
 }
 
 extern "C" int lq_adam8_latent_w4_step(const void *grad, void *codes, int32_t *residual, const void *scales,
@@ -390,18 +445,12 @@ extern "C" int lq_adam8_latent_w4_step(const void *grad, void *codes, int32_t *r
     a.grad = (const u32x4_t *)grad;
     a.state1 = (u32x2_t *)state1; a.state2 = (u32x2_t *)state2;
     a.scale1 = scale1; a.max1 = max1; a.scale2 = scale2; a.max2 = max2;
-    a.n_threads = n / 8;
-    a.codes = (unsigned *)codes; a.residual = (unsigned *)residual;
+    a.codes_in = a.codes = (unsigned *)codes; a.residual = (unsigned *)residual;
     a.wscales = (const unsigned short *)scales; a.wzeros = (const unsigned short *)zeros;
     a.dequant_curve = lq_codec_dequant_params(dk1, db1, dk2, db2, dk3);
     a.quant_curve = lq_codec_quant_params(qk1, qb1, qk2, qb2, qk3);
     adam8_scalars(a, beta1, beta2, eps, step_size);
-    const unsigned blocks = (unsigned)((a.n_threads + 255) / 256);
-    if (block_elems == 2048)
-        hipLaunchKernelGGL((adam8_update_kernel<2048, LATENT_W4>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL((adam8_update_kernel<128, LATENT_W4>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, a);
-    return lq_check_launch("lq_adam8_latent_w4_step");
+    return adam8_launch<ADAM_W4>("lq_adam8_latent_w4_step", a, n, block_elems, stream);
 }
 
 extern "C" int lq_adam8_latent_w8_step(const void *grad, int8_t *codes, int32_t *residual, const void *qscales, uint8_t *state1,
@@ -423,17 +472,34 @@ extern "C" int lq_adam8_latent_w8_step(const void *grad, int8_t *codes, int32_t 
     a.grad = (const u32x4_t *)grad;
     a.state1 = (u32x2_t *)state1; a.state2 = (u32x2_t *)state2;
     a.scale1 = scale1; a.max1 = max1; a.scale2 = scale2; a.max2 = max2;
-    a.n_threads = n / 8;
     a.codes8 = (u32x2_t *)codes; a.residual = (unsigned *)residual;
     a.qscales = (const unsigned short *)qscales;
-    a.threads_per_row = K / 8;
+    a.chunks_per_row = K / 8;
     a.dequant_curve = lq_codec_dequant_params(dk1, db1, dk2, db2, dk3);
     a.quant_curve = lq_codec_quant_params(qk1, qb1, qk2, qb2, qk3);
     adam8_scalars(a, beta1, beta2, eps, step_size);
-    const unsigned blocks = (unsigned)((a.n_threads + 255) / 256);
-    if (block_elems == 2048)
-        hipLaunchKernelGGL((adam8_update_kernel<2048, LATENT_W8>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL((adam8_update_kernel<128, LATENT_W8>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, a);
-    return lq_check_launch("lq_adam8_latent_w8_step");
+    return adam8_launch<ADAM_W8>("lq_adam8_latent_w8_step", a, n, block_elems, stream);
+}
+
+extern "C" int lq_adam8_sr_step(const void *grad, const void *codes_in, void *codes_out, const void *scales, const void *zeros,
+                                uint8_t *state1, uint8_t *state2, float *scale1, float *max1, float *scale2, float *max2,
+                                int64_t N, int64_t K, int group, int block_elems, double beta1, double beta2, double eps,
+                                double step_size, uint64_t philox_seed, uint64_t philox_offset, void *stream) {
+    LQ_REQUIRE(N > 0 && K > 0 && K % LQ_GROUP == 0, "lq_adam8_sr_step: need N > 0, K a positive multiple of %d", LQ_GROUP);
+    LQ_REQUIRE(group == LQ_GROUP, "lq_adam8_sr_step: group must be %d", LQ_GROUP);
+    const int64_t n = N * K;
+    int rc = adam8_check("lq_adam8_sr_step", grad, state1, state2, scale1, max1, scale2, max2, n, block_elems);
+    if (rc) return rc;
+    LQ_REQUIRE(codes_in && codes_out && scales && zeros, "lq_adam8_sr_step: null pointer argument");
+    LQ_REQUIRE(lq_aligned(codes_in, 4) && lq_aligned(codes_out, 4) && lq_aligned(scales, 2) && lq_aligned(zeros, 2),
+               "lq_adam8_sr_step: codes must be 4-byte, scales and zeros 2-byte aligned");
+    Adam8Params a = {};
+    a.grad = (const u32x4_t *)grad;
+    a.state1 = (u32x2_t *)state1; a.state2 = (u32x2_t *)state2;
+    a.scale1 = scale1; a.max1 = max1; a.scale2 = scale2; a.max2 = max2;
+    a.codes_in = (const unsigned *)codes_in; a.codes = (unsigned *)codes_out;
+    a.wscales = (const unsigned short *)scales; a.wzeros = (const unsigned short *)zeros;
+    a.seed = philox_seed; a.offset = philox_offset;
+    adam8_scalars(a, beta1, beta2, eps, step_size);
+    return adam8_launch<ADAM_SR>("lq_adam8_sr_step", a, n, block_elems, stream);
 }

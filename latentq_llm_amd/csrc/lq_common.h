@@ -38,6 +38,20 @@ __device__ __forceinline__ unsigned lq_pack_bf16(float a, float b) {
     r[1] = (__bf16)b;
     return __builtin_bit_cast(unsigned, r);
 }
+// Rounded to bf16, as a float: the high half of a packed conversion whose low half is zero (one instruction; written
+// with the vector type the compiler converts and then moves the halves about).
+// v must not come straight from a transcendental instruction (v_sqrt, v_rcp): the hardware wants a wait state in between,
+// which the compiler does not put before inline assembly; lq_bf16r_trans brings its own.
+__device__ __forceinline__ float lq_bf16r(float v) {
+    float r;
+    asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+__device__ __forceinline__ float lq_bf16r_trans(float v) {
+    float r;
+    asm("s_nop 0\n\tv_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
 __device__ __forceinline__ unsigned short lq_f32_to_bf16_bits(float a) {
     __bf16 r = (__bf16)a;
     return __builtin_bit_cast(unsigned short, r);

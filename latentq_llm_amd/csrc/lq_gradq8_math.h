@@ -5,7 +5,7 @@
 
 namespace {
 
-__device__ __forceinline__ float bf16r(float v) { return lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(v)); }
+__device__ __forceinline__ float bf16r(float v) { return lq_bf16r(v); }
 
 __device__ __forceinline__ float bf16_of(const u32x4_t v, int j) { return (j & 1) ? lq_bf16_hi(v[j >> 1]) : lq_bf16_lo(v[j >> 1]); }
 

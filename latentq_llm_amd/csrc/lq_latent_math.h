@@ -5,8 +5,6 @@
 #include "lq_common.h"
 #include "lq_residual_codec.h"
 
-__device__ __forceinline__ float lq_bf16r(float v) { return lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(v)); }
-
 // The dequantised value of a residual nibble depends on nothing but the nibble, so a workgroup keeps
 // the 16 values bf16(value(n - 8)) in LDS and an element costs one LDS read instead of the curve's
 // dozen selects and operations. Threads 0..15 fill the table; the caller synchronises before use.

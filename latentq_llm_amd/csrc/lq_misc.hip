@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void w8_requant_kernel(const u32x4_t *__restri
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const float t = (j & 1) ? lq_bf16_hi(v[j >> 1]) : lq_bf16_lo(v[j >> 1]);
-            const float q = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(t * r)) + 128.0f;
+            const float q = lq_bf16r(t * r) + 128.0f;
             switch (j & 3) {
                 case 0: w[j >> 2] = act_cvt_pk_u8<0>(q, w[j >> 2]); break;
                 case 1: w[j >> 2] = act_cvt_pk_u8<1>(q, w[j >> 2]); break;
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void w8_requant_kernel(const u32x4_t *__restri
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const float t = (j & 1) ? lq_bf16_hi(v[j >> 1]) : lq_bf16_lo(v[j >> 1]);
-            const float q = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(t / c));
+            const float q = lq_bf16r(t / c);
             const float rr = q == q ? __builtin_amdgcn_fmed3f(rintf(q), -128.0f, 127.0f) : 0.0f;
             w[j >> 2] |= ((unsigned)(int)rr & 0xFFu) << (8 * (j & 3));
         }

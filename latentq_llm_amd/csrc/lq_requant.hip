@@ -26,39 +26,12 @@
 //
 // This translation unit is compiled with -ffp-contract=off: every rounding below is written out
 // explicitly (fmaf where a fused operation is meant).
-#include "lq_common.h"
+#include "lq_requant_math.h"
 
 namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWordsPerThread = 4;  // 4 consecutive words = 32 elements of one quantisation group
-
-// float -> uint32, truncating, saturating: NaN and negatives give 0, values >= 2^32 give 2^32 - 1
-__device__ __forceinline__ unsigned cvt_u32_sat(float x) {
-    unsigned r;
-    asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
-    return r;
-}
-// acc + (low or high 16 bits of word), saturating at 2^32 - 1
-template <int HI>
-__device__ __forceinline__ unsigned add_half_sat(unsigned word, unsigned acc) {
-    unsigned r;
-    if (HI) asm("v_mad_u32_u16 %0, %1, 1, %2 op_sel:[1,0,0,0] clamp" : "=v"(r) : "v"(word), "v"(acc));
-    else asm("v_mad_u32_u16 %0, %1, 1, %2 clamp" : "=v"(r) : "v"(word), "v"(acc));
-    return r;
-}
-
-// The definition, one operation per line (any inputs). a < 65536.
-__device__ __forceinline__ unsigned requant_elem(unsigned q, float s, float z, float g, float lr, unsigned a) {
-    const float d = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits((float)q - z));
-    const float w = lq_bf16_bits_to_f32(lq_f32_to_bf16_bits(d * s));
-    const float t = fmaf(-lr, g, w);
-    const float r16 = (1.0f / s) * 65536.0f;
-    const float c16 = fmaf(z, 65536.0f, 0.5f);
-    const unsigned S = add_half_sat<0>(a, cvt_u32_sat(fmaf(t, r16, c16)));
-    const unsigned c = S >> 16;
-    return c > 15u ? 15u : c;
-}
 
 // 16-bit draw from an injected uniform: floor(u * 2^16), NaN and negatives -> 0, u >= 1 -> 65535
 __device__ __forceinline__ unsigned draw_of_uniform(float u) {
@@ -129,12 +102,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
         asm volatile("" : "+v"(sbits), "+v"(zbits));
     }
     const float s = __uint_as_float(sbits << 16), z = __uint_as_float(zbits << 16);
-    // One-fma dequantisation: z*s and q*s are exact in fp32 (8-bit significands) and for an integer zero
-    // with |q - z| <= 255 the difference q - z is exact in bf16, so fma(q/512, 512*s, -(z*s)) is the
-    // exact (q - z) * s and one rounding to bf16 gives what the two roundings of the definition give.
-    const bool fast = (z == floorf(z)) && (fabsf(z) <= 240.0f) && (s >= 0x1p-100f) && (s <= 0x1p100f);
-    const float r16 = (1.0f / s) * 65536.0f;
-    const float nzs = -(z * s), s512 = s * 512.0f, c16 = fmaf(z, 65536.0f, 0.5f);
+    const RequantGroup rg = requant_group(s, z);
 
     u32x4_t out;
 #pragma unroll
@@ -151,31 +119,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
             aw[i][2] = draw_of_uniform(ub[0]) | (draw_of_uniform(ub[1]) << 16);
             aw[i][3] = draw_of_uniform(ub[2]) | (draw_of_uniform(ub[3]) << 16);
         }
-        const unsigned cw = codes[i];
-        const unsigned lo4 = cw & 0x0F0F0F0Fu;         // odd elements
-        const unsigned hi4 = (cw >> 4) & 0x0F0F0F0Fu;  // even elements
-        // the codes as q/512, two per conversion
-        const lq_f32x2_t e0 = lq_nibbles_lo(hi4), e1 = lq_nibbles_hi(hi4), o0 = lq_nibbles_lo(lo4), o1 = lq_nibbles_hi(lo4);
-        const float qf[8] = {e0[0], o0[0], e0[1], o0[1], e1[0], o1[0], e1[1], o1[1]};
-        unsigned S[8];
+        float gv[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const unsigned gw = g[i][j >> 1];
-            const float gv = (j & 1) ? lq_bf16_hi(gw) : lq_bf16_lo(gw);
-            // bf16-rounded weight as a float: the high half of a packed pair whose low half is zero
-            const float w = __uint_as_float(lq_pack_bf16(0.0f, fmaf(qf[j], s512, nzs)));
-            const float t = fmaf(-lr, gv, w);
-            const unsigned X = cvt_u32_sat(fmaf(t, r16, c16));
-            const unsigned Sj = (j & 1) ? add_half_sat<1>(aw[i][j >> 1], X) : add_half_sat<0>(aw[i][j >> 1], X);
-            S[j] = Sj < 0xFFFFFu ? Sj : 0xFFFFFu;  // code <= 15
-        }
-        // code of element j = byte 2 of S[j]; even elements go to the high nibbles, odd ones to the low
-        const unsigned sel = 0x0C0C0602u;  // bytes (S1.b2, S0.b2, 0, 0) of v_perm_b32(S0, S1)
-        const unsigned ev = (__builtin_amdgcn_perm(S[6], S[4], sel) << 16) | __builtin_amdgcn_perm(S[2], S[0], sel);
-        const unsigned od = (__builtin_amdgcn_perm(S[7], S[5], sel) << 16) | __builtin_amdgcn_perm(S[3], S[1], sel);
-        out[i] = (ev << 4) | od;
+        for (int j = 0; j < 8; ++j) gv[j] = (j & 1) ? lq_bf16_hi(g[i][j >> 1]) : lq_bf16_lo(g[i][j >> 1]);
+        out[i] = requant_word(codes[i], gv, aw[i], lr, rg);
     }
-    if (fast) *reinterpret_cast<u32x4_t *>(codes_out + L * kWordsPerThread) = out;
+    if (rg.fast) *reinterpret_cast<u32x4_t *>(codes_out + L * kWordsPerThread) = out;
     else requant_thread_general<kPhilox>(codes_in, codes_out, (const unsigned short *)grad, (const float *)u, s, z, lr, L, cbase, k0, k1);
 }
 

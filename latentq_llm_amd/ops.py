@@ -448,9 +448,11 @@ def act_dequant_i8(x8, scale, per_token: bool):
 
 
 def adam8_update(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size, param=None,
-                 direction=None):
-    """One Adam step on uint8 block-wise moments (all updated in place). Either ``param`` (bf16, updated in
-    place: param -= step_size * m / d) or ``direction`` (bf16, receives m / d) is given."""
+                 direction=None, requant=None):
+    """One Adam step on uint8 block-wise moments (all updated in place). One of ``param`` (bf16, updated in
+    place: param -= step_size * m / d), ``direction`` (bf16, receives m / d) and ``requant`` is given: the last is
+    (codes, scales, zeros, shape, seed, offset) of a stochastic-rounding layer, whose new codes are returned, those of
+    ``requant_sr`` on the direction with lr = step_size (lq_adam8_sr_step)."""
     _chk(grad, torch.bfloat16, "grad")
     n = grad.numel()
     for t, name in ((state1, "state1"), (state2, "state2")):
@@ -464,8 +466,21 @@ def adam8_update(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2,
         _chk(t, torch.float32, name)
         if t.numel() != nblk:
             raise ValueError(f"{name} must hold one value per block")
-    if (param is None) == (direction is None):
-        raise ValueError("give exactly one of param and direction")
+    if (param is not None) + (direction is not None) + (requant is not None) != 1:
+        raise ValueError("give exactly one of param, direction and requant")
+    if requant is not None:
+        codes, scales, zeros, (N, K), seed, offset = requant
+        _codes_ok(codes, N, K)
+        _qparam_ok(scales, zeros, N, K)
+        if n != N * K:
+            raise ValueError("grad must hold N*K elements")
+        out = torch.empty_like(codes)
+        with torch.cuda.device(grad.device):
+            _C.call("lq_adam8_sr_step", grad.data_ptr(), codes.data_ptr(), out.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
+                    state1.data_ptr(), state2.data_ptr(), scale1.data_ptr(), max1.data_ptr(), scale2.data_ptr(), max2.data_ptr(),
+                    N, K, GROUP, n // nblk, float(beta1), float(beta2), float(eps), float(step_size),
+                    seed & (2**64 - 1), offset & (2**64 - 1), _stream(grad))
+        return out
     out = param if param is not None else direction
     _chk(out, torch.bfloat16, "param" if param is not None else "direction")
     if out.numel() != n:

@@ -1145,11 +1145,19 @@ class MyAdam(torch.optim.Adam):
             bias_correction1 = 1 - beta1 ** state["step"]
             bias_correction2 = 1 - beta2 ** state["step"]
             step_size = config["lr"] * math.sqrt(bias_correction2) / bias_correction1
-            direction = torch.empty_like(grad) if sr_mode else None
-            ops.adam8_update(grad, state["state1"], state["state2"], state["qmap1"], state["absmax1"], state["qmap2"],
-                             state["absmax2"], beta1, beta2, group["eps"], step_size,
-                             param=None if sr_mode else pdata, direction=direction)
-            self._requantise(p, pdata, direction if sr_mode else None, step_size, is_q, sr_mode)
+            requant = None
+            if sr_mode:  # the direction goes straight into the requantizer
+                scales, zeros, shape = _flat_qparam(p.qparam)
+                requant = (p.data, scales, zeros, shape, self.sr_seed, self.sr_offset)
+            new = ops.adam8_update(grad, state["state1"], state["state2"], state["qmap1"], state["absmax1"], state["qmap2"],
+                                   state["absmax2"], beta1, beta2, group["eps"], step_size,
+                                   param=None if sr_mode else pdata, requant=requant)
+            if sr_mode:
+                p.data = new
+                self.sr_offset += (p.numel() + 7) // 8
+                self._release_grad(p)
+            else:
+                self._requantise(p, pdata, None, step_size, is_q, sr_mode)
             return
         if q8:
             exp_avg = DeQfunc_8bit_opt(state["state1"].to(grad.device), [state["qmap1"], state["absmax1"]]).to(grad.dtype)
@@ -1223,10 +1231,7 @@ class MyAdam(torch.optim.Adam):
                                      group["eps"], step_size)
             r.weight_scale = qs
             r.lock_mu = r.mu
-            if isinstance(p.grad, GradientQTensor):
-                p.grad.zero()
-            else:
-                p.grad = None
+            self._release_grad(p)
             return True
         scales, zeros, shape = _flat_qparam(p.qparam)
         if not (scales.dtype == torch.bfloat16 and zeros.dtype == torch.bfloat16 and scales.is_contiguous()
@@ -1243,10 +1248,7 @@ class MyAdam(torch.optim.Adam):
                                  group["eps"], step_size)
         r.weight_scale = scales.contiguous().reshape(-1, 1)
         r.lock_mu = r.mu
-        if isinstance(p.grad, GradientQTensor):
-            p.grad.zero()
-        else:
-            p.grad = None
+        self._release_grad(p)
         return True
 
     def _requantise(self, p, pdata, direction, step_size, is_q, sr_mode):
@@ -1262,6 +1264,10 @@ class MyAdam(torch.optim.Adam):
                 p.data = Qfunc_8bit_res(pdata, p.residual, qscales=p.qparam)
             elif p.wbit == 4:
                 p.data = Qfunc_4bit_g_res(pdata, p.residual, qparam=p.qparam)
+        self._release_grad(p)
+
+    @staticmethod
+    def _release_grad(p):
         if isinstance(p.grad, GradientQTensor):
             p.grad.zero()
         else:
