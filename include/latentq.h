@@ -392,6 +392,13 @@ int lq_adam8_sr_step(const void *grad, const void *codes_in, void *codes_out, co
                      int64_t K, int group, int block_elems, double beta1, double beta2, double eps, double step_size,
                      uint64_t philox_seed, uint64_t philox_offset, void *stream);
 
+/* What the periodic choice of the residual codec's curve looks at (MyAdam.update_step, utils/quant.py:1117-1122):
+ * ratio_out = bf16(|m| / d) of the step that lq_adam8_update would take, with nothing updated. ratio_out: bf16[n],
+ * 16-byte aligned; the rest as lq_adam8_update. */
+int lq_adam8_ratio(const void *grad, const uint8_t *state1, const uint8_t *state2, const float *scale1, const float *max1,
+                   const float *scale2, const float *max2, void *ratio_out, int64_t n, int block_elems, double beta1,
+                   double beta2, double eps, void *stream);
+
 /* The same for an 8-bit-weight layer (QLinearA8W8 with lbit = 4): the parameter is rebuilt from the int8 codes, the
  * per-row bf16 scales and the residual words exactly as lq_latent_w8_reconstruct does
  * (ResidualTensor.add((p.data * p.qparam).to(dtype)), utils/quant.py:826-837, 1069-1070), updated, and re-quantised

@@ -503,3 +503,18 @@ extern "C" int lq_adam8_sr_step(const void *grad, const void *codes_in, void *co
     adam8_scalars(a, beta1, beta2, eps, step_size);
     return adam8_launch<ADAM_SR>("lq_adam8_sr_step", a, n, block_elems, stream);
 }
+
+extern "C" int lq_adam8_ratio(const void *grad, const uint8_t *state1, const uint8_t *state2, const float *scale1,
+                              const float *max1, const float *scale2, const float *max2, void *ratio_out, int64_t n,
+                              int block_elems, double beta1, double beta2, double eps, void *stream) {
+    int rc = adam8_check("lq_adam8_ratio", grad, state1, state2, scale1, max1, scale2, max2, n, block_elems);
+    if (rc) return rc;
+    LQ_REQUIRE(ratio_out && lq_aligned(ratio_out, 16), "lq_adam8_ratio: ratio_out must be given and 16-byte aligned");
+    Adam8Params a = {};
+    a.grad = (const u32x4_t *)grad;
+    a.direction = (u32x4_t *)ratio_out;
+    a.state1 = (u32x2_t *)state1; a.state2 = (u32x2_t *)state2;  // (read only in this mode)
+    a.scale1 = (float *)scale1; a.max1 = (float *)max1; a.scale2 = (float *)scale2; a.max2 = (float *)max2;
+    adam8_scalars(a, beta1, beta2, eps, 0.0);
+    return adam8_launch<ADAM_RATIO>("lq_adam8_ratio", a, n, block_elems, stream);
+}

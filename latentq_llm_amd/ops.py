@@ -493,6 +493,29 @@ def adam8_update(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2,
     return out
 
 
+def adam8_ratio(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps):
+    """bf16(|m| / d) of the step ``adam8_update`` would take with these operands, nothing updated (lq_adam8_ratio)."""
+    _chk(grad, torch.bfloat16, "grad")
+    n = grad.numel()
+    for t, name in ((state1, "state1"), (state2, "state2")):
+        _chk(t, torch.uint8, name)
+        if t.numel() != n:
+            raise ValueError(f"{name} must hold as many elements as grad")
+    nblk = scale1.numel()
+    if nblk == 0 or n % nblk:
+        raise ValueError("the number of blocks must divide the number of elements")
+    for t, name in ((scale1, "scale1"), (max1, "max1"), (scale2, "scale2"), (max2, "max2")):
+        _chk(t, torch.float32, name)
+        if t.numel() != nblk:
+            raise ValueError(f"{name} must hold one value per block")
+    out = torch.empty_like(grad)
+    with torch.cuda.device(grad.device):
+        _C.call("lq_adam8_ratio", grad.data_ptr(), state1.data_ptr(), state2.data_ptr(), scale1.data_ptr(), max1.data_ptr(),
+                scale2.data_ptr(), max2.data_ptr(), out.data_ptr(), n, n // nblk, float(beta1), float(beta2), float(eps),
+                _stream(grad))
+    return out
+
+
 def adam8_latent_w4_step(grad, codes, residual_int, scales, zeros, shape, state1, state2, scale1, max1, scale2, max2,
                          dequant_curve, quant_curve, beta1, beta2, eps, step_size):
     """The Adam step of an lbit = 4 layer in one pass: codes (packed, N*K/2 bytes), residual_int

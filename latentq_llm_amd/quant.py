@@ -848,7 +848,13 @@ class ResidualTensor(object):
     def update_mu(self, optmizer_std):
         """Pick the companding curve from the ratio scale / typical update (utils/quant.py:813-824);
         as in the reference the `> 75.8` test is overwritten by the chain below it."""
-        mu = (self.weight_scale / (optmizer_std + 1e-8)).mean().item()
+        self.pick_mu(self.mean_ratio(optmizer_std).item())
+
+    def mean_ratio(self, optmizer_std):
+        """The ratio update_mu looks at, as a 0-dim tensor."""
+        return (self.weight_scale / (optmizer_std + 1e-8)).mean()
+
+    def pick_mu(self, mu):
         self.mu = 2 if mu > 36.5 else (1 if mu > 16.2 else 0)
         if self.mu != self.lock_mu:
             print(f'{self.name} now mu level is {mu}({self.mu}), pre is {self.lock_mu}')
@@ -1011,6 +1017,7 @@ class MyAdam(torch.optim.Adam):
         self.statedevice = 'cpu' if cpu else 'cuda'
         self.sr_seed = sr_seed
         self.sr_offset = 0
+        self._chosen = frozenset()  # ids of the parameters whose curve the current step has chosen already
 
     def add_param_group(self, param_group):
         """Accepts QuantTensor / FPTensor objects next to tensors (utils/quant.py:934-959)."""
@@ -1038,6 +1045,7 @@ class MyAdam(torch.optim.Adam):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
+        self._chosen = self._choose_curves()
         for gindex, group in enumerate(self.param_groups):
             for pindex, p in enumerate(group["params"]):
                 if p.grad is None:
@@ -1045,6 +1053,7 @@ class MyAdam(torch.optim.Adam):
                 if len(self.state[p]) == 0:
                     self.init_state(group, p, gindex, pindex)
                 self.update_step(group, p, gindex, pindex)
+        self._chosen = frozenset()
         return loss
 
     def to_gpu(self):
@@ -1114,6 +1123,49 @@ class MyAdam(torch.optim.Adam):
             raise AssertionError("wbit must be 4 or 8")
         return p.residual.data.to(dtype)
 
+    def _is_mu_step(self, p, state):
+        """Whether this step chooses the residual codec's curve anew (utils/quant.py:1117)."""
+        return (state["step"] + 1 > 250 and (state["step"] + 1) % self.mu_updata_f == (self.mu_updata_f - 1)
+                and isinstance(getattr(p, 'residual', None), ResidualTensor))
+
+    @staticmethod
+    def _adam8_ok(p, state, config, grad):
+        """Whether the fused Adam kernels take this parameter's moments and gradient."""
+        return (FUSED_ADAM8 and state["state1"].dtype == torch.uint8 and config["weight_decay"] == 0 and grad.is_cuda
+                and grad.dtype == torch.bfloat16 and grad.is_contiguous()
+                and all(state[k].device == grad.device and state[k].is_contiguous()
+                        for k in ("state1", "state2", "qmap1", "absmax1", "qmap2", "absmax2"))
+                and p.numel() // len(state["absmax1"]) in (2048, 128))
+
+    @torch.no_grad()
+    def _choose_curves(self):
+        """The curve choice of every parameter whose turn it is (every mu_updata_f steps after step 250), ahead of the
+        updates: the ratio of each is formed on the device from the moments the step is about to have (lq_adam8_ratio and
+        the tensor operations of the chain), and the host waits once for all of them. A parameter chosen here (their ids are
+        returned) takes the fused step like any other; one that the kernels do not take is left to update_step's chain."""
+        chosen = []
+        for gindex, group in enumerate(self.param_groups):
+            for pindex, p in enumerate(group["params"]):
+                state = self.state.get(p)
+                if p.grad is None or not state or not isinstance(p, QuantTensor) or not self._is_mu_step(p, state):
+                    continue
+                config = self.get_config(gindex, pindex, group)
+                grad = p.grad.get_value() if isinstance(p.grad, GradientQTensor) else p.grad
+                if p.residual.init or p.residual.weight_scale is None or not FUSED_LATENT or not self._adam8_ok(p, state, config, grad):
+                    continue
+                beta1, beta2 = config["betas"]
+                step = state["step"] + 1
+                step_size = config["lr"] * math.sqrt(1 - beta2 ** step) / (1 - beta1 ** step)
+                ratio = ops.adam8_ratio(grad, state["state1"], state["state2"], state["qmap1"], state["absmax1"],
+                                        state["qmap2"], state["absmax2"], beta1, beta2, group["eps"])
+                std = torch.mean(ratio.view(p.residual.qshape), dim=1, keepdim=True) * step_size
+                chosen.append((p, p.residual.mean_ratio(std)))
+        if chosen:
+            dev = chosen[0][1].device
+            for (p, _), mu in zip(chosen, torch.stack([m.to(dev) for _, m in chosen]).tolist()):
+                p.residual.pick_mu(mu)
+        return frozenset(id(p) for p, _ in chosen)
+
     @torch.no_grad()
     def update_step(self, group, p, gindex, pindex):
         state = self.state[p]
@@ -1124,13 +1176,8 @@ class MyAdam(torch.optim.Adam):
         if is_q and isinstance(grad, GradientQTensor):
             grad = grad.get_value()
         q8 = state["state1"].dtype == torch.uint8
-        mu_step = (state["step"] + 1 > 250 and (state["step"] + 1) % self.mu_updata_f == (self.mu_updata_f - 1)
-                   and isinstance(getattr(p, 'residual', None), ResidualTensor))
-        adam8_ok = (FUSED_ADAM8 and q8 and config["weight_decay"] == 0 and not mu_step and grad.is_cuda
-                    and grad.dtype == torch.bfloat16 and grad.is_contiguous()
-                    and all(state[k].device == grad.device and state[k].is_contiguous()
-                            for k in ("state1", "state2", "qmap1", "absmax1", "qmap2", "absmax2"))
-                    and p.numel() // len(state["absmax1"]) in (2048, 128))
+        mu_step = self._is_mu_step(p, state) and id(p) not in self._chosen
+        adam8_ok = not mu_step and self._adam8_ok(p, state, config, grad)
         if adam8_ok and FUSED_LATENT and is_q and not sr_mode and self._fused_latent_step(group, p, state, config, grad):
             return
         if is_q:
@@ -1186,8 +1233,7 @@ class MyAdam(torch.optim.Adam):
         else:
             pdata.addcdiv_(exp_avg, denom, value=-step_size)
 
-        if (state["step"] > 250 and state["step"] % self.mu_updata_f == (self.mu_updata_f - 1)
-                and isinstance(getattr(p, 'residual', None), ResidualTensor)):
+        if mu_step:
             std = torch.mean((abs(exp_avg) / denom).view(p.residual.qshape), dim=1, keepdim=True) * step_size
             p.residual.update_mu(std)
 

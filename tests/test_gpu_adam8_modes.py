@@ -85,3 +85,56 @@ def test_step_on_operands_outside_the_short_sequences(hip_lib, block):
         assert torch.equal(p, want_p) and torch.equal(direction, want_dir)
         for x, y, w in zip(st, other, (q1, w1, h1, q2, w2, h2)):
             assert torch.equal(x, w) and torch.equal(y, w)
+
+
+@pytest.mark.parametrize("wbit,lr", [(4, 2e-5), (4, 1e-3), (8, 2e-6)])
+def test_step_that_chooses_the_residual_curve_fused_equals_the_chain(hip_lib, monkeypatch, wbit, lr):
+    """Every mu_updata_f steps after step 250 the residual codec's curve is chosen from the step itself: chosen curve,
+    codes, residual words and moments equal the chain of tensor operations, and the fused kernels ran."""
+    from latentq_llm_amd import ops
+    from latentq_llm_amd import quant as Q
+    from tests.util import make_w4
+    N, K = 256, 512
+
+    def run(fused):
+        monkeypatch.setattr(Q, "FUSED_ADAM8", fused)
+        g = torch.Generator().manual_seed(4)
+        weights = []
+        for i in range(2):
+            if wbit == 4:
+                layer = Q.QLinearA16W4(K, N, bias=False, lbit=4, gbit=16)
+                _, packed, s, z = make_w4(N, K, 5 + i)
+                layer.scales.data, layer.zeros.data = s.cuda(), z.cuda()
+                layer.weight.set_value(packed.cuda(), [layer.scales, layer.zeros, layer.wshape])
+            else:
+                layer = Q.QLinearA8W8(K, N, bias=False, lbit=4, gbit=16)
+                layer.qscales.data = ((torch.randn(N, 1, generator=g) * 3e-4).abs() + 1e-5).to(torch.bfloat16).cuda()
+                layer.weight.set_value(torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).cuda(), layer.qscales)
+            weights.append(layer.weight)
+        opt = Q.MyAdam([{"params": weights}], lr=lr, betas=(0.9, 0.95), obit=8, mu_updata_f=20)
+        torch.manual_seed(9)
+        for step in range(5):
+            for w in weights:
+                w.grad = (torch.randn(N, K, generator=g) * 1e-3).to(torch.bfloat16).cuda()
+                if step == 2:
+                    opt.state[w]["step"] = 257  # the next but one step is number 259
+            opt.step()
+        out = []
+        for w in weights:
+            s = opt.state[w]
+            assert s["step"] == 260
+            out += [torch.tensor(w.residual.mu), torch.tensor(w.residual.lock_mu), w.data, w.residual.residual_int] + [
+                s[k] for k in ("state1", "qmap1", "absmax1", "state2", "qmap2", "absmax2")]
+        return out
+
+    calls = []
+    real = ops.adam8_ratio
+    monkeypatch.setattr(ops, "adam8_ratio", lambda *a: (calls.append(1), real(*a))[1])
+    fused = run(True)
+    assert len(calls) == 2
+    plain = run(False)
+    assert len(calls) == 2
+    for x, y in zip(fused, plain):
+        assert torch.equal(x.cpu(), y.cpu())
+    if lr < 1e-4:
+        assert int(fused[0]) == 2  # the curve did change
