@@ -30,7 +30,7 @@
 // operands from HBM (bytes at the 5.05 TB/s of a large copy in brackets), against the form with 8 elements per thread,
 // two rounding instructions, two barriers and the exact square root computed beside the short one:
 //   parameter 42.5 -> 37.6 us (33.3), direction 39.3 -> 30.7 (26.6), direction + requantizer 48.2 -> 33.7 in one pass
-//   (23.3), int4 + residual 63.0 -> 50.6 (26.7), int8 + residual 60.4 -> 48.5 (29.9).
+//   (23.3), int4 + residual 63.0 -> 46.8 (26.7), int8 + residual 60.4 -> 46.6 (29.9).
 #include "lq_latent_math.h"
 #include "lq_requant_math.h"
 
@@ -265,10 +265,11 @@ __global__ __launch_bounds__(256) void adam8_kernel(Adam8Params a) {
 
         if constexpr (MODE == ADAM_W4) {
             const float ws = lq_bf16_bits_to_f32(wsb[c]), wz = lq_bf16_bits_to_f32(wzb[c]);
-            float out[8];
+            float out[8], wq[8];
+            lq_latent_weights(cword[c], ws, wz, lq_latent_one_fma(ws, wz), wq);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                const float p = lq_bf16r(lq_latent_value(lq_code(cword[c], k), vtab[(rword[c] >> (28 - 4 * k)) & 0xFu], ws, wz));
+                const float p = lq_bf16r(lq_latent_value(wq[k], vtab[(rword[c] >> (28 - 4 * k)) & 0xFu], ws));
                 out[k] = lq_bf16r(fmaf(a.neg_step, ratio[k], p));
             }
             const float wr = 1.0f / ws;

@@ -9,6 +9,7 @@ struct CodecParams {
     float c1, c2, c3;  // forward slopes (quant) or inverse slopes (dequant)
     float b1, b2;
     int t1, t2;
+    float t1f, t2f;  // the same as floats
 };
 
 // roundf (halves away from zero) as trunc(x + copysign(pred(0.5), x)): the sum cannot reach the next integer
@@ -31,8 +32,9 @@ __device__ __forceinline__ float level_3fold(float x, const CodecParams &p) {
     const float arg = in1 ? x : (S - (in2 ? p.b1 : p.b2));
     const float slope = in1 ? p.c1 : (in2 ? p.c2 : p.c3);
     const float lv = lq_round_half_away(fmaf(arg, slope, v));
-    const float r = lv + (float)(in2 ? p.t1 : p.t2);
-    return in1 ? lv : (x < 0.0f ? -r : r);
+    // r >= 0: the level of a positive argument is at least -1 (an exact half rounds away from zero) and t1 at least 1
+    const float r = lv + (in2 ? p.t1f : p.t2f);
+    return in1 ? lv : __builtin_copysignf(r, x);
 }
 
 __device__ __forceinline__ float level_uniform(float x) {
@@ -50,6 +52,15 @@ __device__ __forceinline__ unsigned nibble_of(float lv, bool &carry) {
     unsigned t;
     asm("v_cvt_u32_f32 %0, %1" : "=v"(t) : "v"(lv + 8.0f));
     return carry ? 1u : (t & 0xFu);
+}
+
+// The same for a level of level_3fold of an |x| <= 1/2, which is no wild input: without a carry it is at most 7, and the
+// conversion's saturation is all that a level below -8 needs
+__device__ __forceinline__ unsigned nibble_of_half(float lv, bool &carry) {
+    carry = lv > 7.5f;
+    unsigned t;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(t) : "v"(lv + 8.0f));
+    return carry ? 1u : t;
 }
 
 // nibble - 8 -> value of the three-segment curve (inverse slopes in p), branch-free
@@ -71,6 +82,7 @@ inline CodecParams lq_codec_quant_params(int k1, float b1, int k2, float b2, int
     p.c2 = (float)k2 / (b2 - b1);
     p.c3 = (float)((double)k3 / (0.5 - (double)b2));
     p.b1 = b1; p.b2 = b2; p.t1 = k1; p.t2 = k1 + k2;
+    p.t1f = (float)p.t1; p.t2f = (float)p.t2;
     return p;
 }
 
@@ -80,6 +92,7 @@ inline CodecParams lq_codec_dequant_params(int k1, float b1, int k2, float b2, i
     p.c2 = (b2 - b1) / (float)k2;
     p.c3 = (float)((0.5 - (double)b2) / (double)k3);
     p.b1 = b1; p.b2 = b2; p.t1 = k1; p.t2 = k1 + k2;
+    p.t1f = (float)p.t1; p.t2f = (float)p.t2;
     return p;
 }
 
