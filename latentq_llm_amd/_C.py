@@ -100,6 +100,25 @@ def load():
     return lib
 
 
+_native = None
+
+
+def native():
+    """The native binding (csrc/lq_bind.cpp), loaded once. Built with the library and as mandatory as it."""
+    global _native
+    if _native is None:
+        import torch  # noqa: F401  (its libraries first)
+        load()
+        try:
+            from . import _lqbind
+        except ImportError as e:
+            raise LatentQError(f"the binding _lqbind.so is missing or does not load ({e}): build it with "
+                               "`python -m latentq_llm_amd.build`") from e
+        _lqbind.set_error(LatentQError)
+        _native = _lqbind
+    return _native
+
+
 def call(name: str, *args) -> None:
     lib = load()
     rc = getattr(lib, name)(*args)

@@ -1,7 +1,8 @@
-"""Build liblatentq_hip.so (gfx950) in-tree with hipcc.
+"""Build liblatentq_hip.so (gfx950) and the Python binding _lqbind.so in-tree.
 
-`python -m latentq_llm_amd.build` compiles every translation unit under
-``csrc/`` and links the C-ABI shared library next to this file. hipcc
+`python -m latentq_llm_amd.build` compiles every HIP translation unit under
+``csrc/`` with hipcc, links the C-ABI shared library next to this file, and
+compiles ``csrc/lq_bind.cpp`` (host code) against it and torch's headers. hipcc
 cross-compiles without a GPU, so this runs anywhere ROCm is installed.
 """
 from __future__ import annotations
@@ -16,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "obj")
 LIB = os.path.join(HERE, "liblatentq_hip.so")
+BIND = os.path.join(HERE, "_lqbind.so")
 
 ARCH = "gfx950"
 # Packed-FP32 VALU instructions are disabled for every device translation unit.
@@ -49,10 +51,39 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_binding(out: str) -> str:
+    """lq_bind.cpp to an object: plain host C++ that sees HIP's and torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{d}" for d in include_paths("cuda")), f"-I{sysconfig.get_paths()['include']}",
+           "-c", os.path.join(CSRC, "lq_bind.cpp"), "-o", out]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on lq_bind.cpp:\n{r.stdout}\n{r.stderr}")
+    return out
+
+
+def _link_binding(obj: str) -> None:
+    import torch
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = BIND + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, obj, f"-L{HERE}", f"-l:{os.path.basename(LIB)}", f"-L{libs}", "-ltorch_python", "-ltorch",
+           "-lc10", "-ltorch_hip", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"linking _lqbind.so failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, BIND)
+
+
 def build_library(verbose: bool = True, jobs: int = 8) -> str:
     os.makedirs(OBJ, exist_ok=True)
     srcs = sources()
-    with ThreadPoolExecutor(max_workers=min(jobs, len(srcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + 1)) as ex:
+        bind = ex.submit(_compile_binding, os.path.join(OBJ, "lq_bind.o"))
         objs = list(ex.map(_compile, srcs))
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-fno-gpu-rdc", "-o", tmp, *objs]
@@ -60,8 +91,9 @@ def build_library(verbose: bool = True, jobs: int = 8) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
+    _link_binding(bind.result())
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources", file=sys.stderr)
+        print(f"built {LIB} from {len(srcs)} sources, and {BIND}", file=sys.stderr)
     return LIB
 
 

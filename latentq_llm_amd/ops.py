@@ -1,5 +1,9 @@
 """Tensor-level wrappers over the C ABI: validate, allocate outputs with torch, pass raw pointers
-and the current HIP stream. PyTorch is used for device memory and streams only."""
+and the current HIP stream. PyTorch is used for device memory and streams only.
+
+The wrappers a training or decoding loop calls hand their operands to the native binding first (csrc/lq_bind.cpp), which
+does the same checks, allocation and call in a tenth of the host time and returns None for anything that is not in the
+plain form; the Python below then runs its own checks and raises what is wrong."""
 from __future__ import annotations
 
 import torch
@@ -9,8 +13,20 @@ from . import _C
 GROUP = 128
 
 
+_native = None
+
+
+def _fast():
+    """The native binding, loaded at first use."""
+    global _native
+    if _native is None:
+        _native = _C.native()
+    return _native
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    index = t.device.index
+    return _fast().current_stream(torch.cuda.current_device() if index is None else index)
 
 
 def _chk(t: torch.Tensor, dtype, name: str):
@@ -102,9 +118,22 @@ def _workspace(t, rows, cols):
     return buf, buf.data_ptr(), buf.numel()
 
 
+def linear4(x, codes, scales, zeros, shape, bias=None):
+    """a16w4_forward for x of any number of dimensions; None if an operand is not in the plain form the native binding
+    takes (the caller then brings it into form, or lets a16w4_forward say what is wrong)."""
+    N, K = shape
+    rows = x.numel() // K if K else 0
+    ws = _workspace(x, rows, N)[0] if 16 < rows <= 2048 and x.is_cuda else None
+    return (_native or _fast()).linear4(x, codes, scales, zeros, N, K, bias, ws)
+
+
 def a16w4_forward(x, codes, scales, zeros, shape, bias=None, out=None):
     """Y[M,N] = X[M,K] . deq(W)[N,K]^T (+ bias) in bf16 with fp32 accumulation."""
     N, K = shape
+    if out is None and x.dim() == 2:
+        y = linear4(x, codes, scales, zeros, shape, bias)
+        if y is not None:
+            return y
     _chk(x, torch.bfloat16, "x")
     if x.dim() != 2 or x.shape[1] != K:
         raise ValueError(f"x must be [M,{K}], got {tuple(x.shape)}")
@@ -165,6 +194,10 @@ def a16w4_gate_up_silu(x, gate, up, shape, out=None, save=False):
     (codes, scales, zeros) triples of two [N, K] matrices. Needs K % 256 == 0 above 16 tokens.
     save=True (lq_a16w4_gate_up_silu_save) also stores the two products and returns (h, g, u)."""
     N, K = shape
+    if out is None and x.dim() == 2:
+        r = (_native or _fast()).gate_up(x, *gate, *up, N, K, save)
+        if r is not None:
+            return r
     _chk(x, torch.bfloat16, "x")
     if x.dim() != 2 or x.shape[1] != K:
         raise ValueError(f"x must be [M,{K}], got {tuple(x.shape)}")
@@ -196,6 +229,10 @@ def a16w4_dx_silu_bwd(dy, codes, scales, zeros, shape, g, u):
     """The backward of a gated MLP's down projection with the backward of h = silu(g) * u as its epilogue
     (lq_a16w4_dx_silu_bwd): returns (dg, du), bf16 [M, K] each, for dy [M, N] and the saved products g, u [M, K]."""
     N, K = shape
+    if dy.dim() == 2:
+        r = (_native or _fast()).dx_silu(dy, codes, scales, zeros, N, K, g, u)
+        if r is not None:
+            return r
     _chk(dy, torch.bfloat16, "dy")
     if dy.dim() != 2 or dy.shape[1] != N:
         raise ValueError(f"dy must be [M,{N}], got {tuple(dy.shape)}")
@@ -218,6 +255,10 @@ def a16w4_dx_silu_bwd(dy, codes, scales, zeros, shape, g, u):
 def a16w4_dx(dy, codes, scales, zeros, shape, out=None, accumulate=False):
     """dX[M,K] = dY[M,N] . deq(W)[N,K]; accumulate=True: out = bf16(out + bf16(dY . deq(W))) (lq_a16w4_dx_acc)."""
     N, K = shape
+    if out is None and not accumulate and dy.dim() == 2 and dy.is_cuda and dy.shape[0]:
+        r = (_native or _fast()).dx4(dy, codes, scales, zeros, N, K, _workspace(dy, dy.shape[0], K)[0])
+        if r is not None:
+            return r
     _chk(dy, torch.bfloat16, "dy")
     if dy.dim() != 2 or dy.shape[1] != N:
         raise ValueError(f"dy must be [M,{N}], got {tuple(dy.shape)}")
@@ -252,6 +293,10 @@ def a16w4_dx_pair(dy1, w1, dy2, w2, shape, out=None):
     """dX[M,K] = bf16(dY1 . deq(W1) + dY2 . deq(W2)) in one launch (lq_a16w4_dx_pair); w1, w2 = (codes, scales, zeros)
     of two [N, K] matrices."""
     N, K = shape
+    if out is None and dy1.dim() == 2:
+        r = (_native or _fast()).dx_pair(dy1, *w1, dy2, *w2, N, K)
+        if r is not None:
+            return r
     for name, dy, w in (("dy1", dy1, w1), ("dy2", dy2, w2)):
         _chk(dy, torch.bfloat16, name)
         if dy.dim() != 2 or dy.shape[1] != N:
@@ -315,9 +360,20 @@ def w8_requant(latent, qscales):
     return out
 
 
+def infer8(x, w8, qscales, bias=None, per_token: bool = False):
+    """The forward of an 8-bit layer in inference for x of any number of dimensions: the activation quantiser and the int8
+    product (act_quant_i8_dynamic or _per_token, a8w8_forward). None if an operand is not in the plain form the native
+    binding takes."""
+    return (_native or _fast()).infer8(x, w8, qscales, bias, per_token)
+
+
 def a8w8_forward(x8, w8, sx, sw, bias=None, want_acc: bool = False):
     """bf16 Y = ((int32 X8.W8^T) * sx[m]) * sw[n] (+ bias); optionally also the int32 accumulators.
     sw is fp32 [N], or the bf16 per-channel scales as the modules store them (lq_a8w8_fwd_qs)."""
+    if not want_acc and x8.dim() == 2:
+        y = (_native or _fast()).linear8(x8, w8, sx, sw, bias)
+        if y is not None:
+            return y
     _chk(x8, torch.int8, "x8")
     _chk(w8, torch.int8, "w8")
     _chk(sx, torch.float32, "sx")
@@ -355,6 +411,10 @@ def a8w8_dx_ok(dy, w8, qscales):
 
 def a8w8_dx(dy, w8, qscales):
     """dX[M,K] = dY[M,N] . bf16(W8 * qscales)[N,K] from the int8 codes (lq_a8w8_dx)."""
+    if dy.dim() == 2:
+        dx = (_native or _fast()).dx8(dy, w8, qscales)
+        if dx is not None:
+            return dx
     if not a8w8_dx_ok(dy, w8, qscales):
         raise ValueError("a8w8_dx needs contiguous GPU operands: dy bf16 [M,N], w8 int8 [N,K], qscales bf16 [N], N % 64 == 0, K % 128 == 0")
     M, N = dy.shape
@@ -383,6 +443,9 @@ def act_quant_i8_dynamic(x, alpha_bf16: bool = False):
     """The dynamic layers' activation quantiser with clampv = x.max() found on the device
     (lq_act_quant_i8_dynamic): returns (x8 int8 [M,K], sx fp32 [M] filled with alpha = clampv/127, work) where
     work[0:1] is the clamp value and work[1:2] alpha, both fp32 device tensors. x: bf16 [M, K], M*K > 0."""
+    r = (_native or _fast()).quant8(x, bool(alpha_bf16))
+    if r is not None:
+        return r
     _chk(x, torch.bfloat16, "x")
     if x.dim() != 2 or x.numel() == 0:
         raise ValueError("x must be a non-empty [M, K] matrix")
@@ -398,6 +461,9 @@ def act_quant_i8_dynamic(x, alpha_bf16: bool = False):
 
 def act_quant_i8_per_token(x):
     """Per-token activation quantiser (lq_act_quant_i8_per_token): (x8 int8 [M,K], sx fp32 [M] = rowmax|x| / 127)."""
+    r = (_native or _fast()).quant8_token(x)
+    if r is not None:
+        return r
     _chk(x, torch.bfloat16, "x")
     if x.dim() != 2 or x.numel() == 0 or x.shape[1] % 8:
         raise ValueError("x must be a non-empty [M, K] matrix with K a multiple of 8")
@@ -434,6 +500,9 @@ def act_dequant_ok(x8, scale, per_token: bool) -> bool:
 def act_dequant_i8(x8, scale, per_token: bool):
     """bf16(x8 * bf16(scale)) (lq_act_dequant_i8): scale fp32 [M] (per token) or one element; the values of
     ``x8.to(torch.bfloat16) * scale.to(torch.bfloat16)``."""
+    r = (_native or _fast()).dequant8(x8, scale, bool(per_token))
+    if r is not None:
+        return r
     _chk(x8, torch.int8, "x8")
     _chk(scale, torch.float32, "scale")
     if x8.dim() != 2 or x8.numel() == 0 or x8.shape[1] % 16:
@@ -453,6 +522,15 @@ def adam8_update(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2,
     place: param -= step_size * m / d), ``direction`` (bf16, receives m / d) and ``requant`` is given: the last is
     (codes, scales, zeros, shape, seed, offset) of a stochastic-rounding layer, whose new codes are returned, those of
     ``requant_sr`` on the direction with lr = step_size (lq_adam8_sr_step)."""
+    r = None
+    if direction is None and (param is None) != (requant is None):
+        moments = (grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size)
+        if requant is None:
+            r = (_native or _fast()).adam8_param(*moments, param)
+        else:
+            r = (_native or _fast()).adam8_sr(*moments, *requant[:3], *requant[3], *requant[4:])
+    if r is not None:
+        return r
     _chk(grad, torch.bfloat16, "grad")
     n = grad.numel()
     for t, name in ((state1, "state1"), (state2, "state2")):
@@ -523,6 +601,10 @@ def adam8_latent_w4_step(grad, codes, residual_int, scales, zeros, shape, state1
     The curves are (k1, b1, k2, b2, k3) tuples: the one the residual was stored with and the
     current one."""
     N, K = shape
+    r = (_native or _fast()).adam8_w4(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size, codes, scales,
+                                      zeros, N, K, residual_int, dequant_curve, quant_curve)
+    if r is not None:
+        return r
     _chk(grad, torch.bfloat16, "grad")
     if grad.numel() != N * K:
         raise ValueError("grad must hold N*K elements")
@@ -559,6 +641,10 @@ def adam8_latent_w8_step(grad, codes, residual_int, qscales, state1, state2, sca
     """The Adam step of an 8-bit-weight layer in lbit = 4 mode in one pass: codes (int8 [N, K]), residual_int
     (int32[N*K/8]) and the uint8 moments with their block parameters are all updated in place; qscales bf16 [N].
     The curves are (k1, b1, k2, b2, k3) tuples: the one the residual was stored with and the current one."""
+    r = (_native or _fast()).adam8_w8(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size, codes, qscales,
+                                      residual_int, dequant_curve, quant_curve)
+    if r is not None:
+        return r
     _chk(grad, torch.bfloat16, "grad")
     _chk(codes, torch.int8, "codes")
     if codes.dim() != 2 or codes.shape[1] % 8:
@@ -599,6 +685,10 @@ def gradq8_quant(dw, q, scale, accumulate: bool, noise=None, seed: int = 0, offs
     """The 8-bit gradient accumulator in one pass (lq_gradq8_quant): dw bf16 [N, K]; q int8 [N, K] and
     scale bf16 [N, 1] are updated in place (scale only when ``accumulate`` is False). ``noise`` is an
     optional bf16 [N, K] tensor of rounding noise; without it the Philox stream (seed, offset) is used."""
+    if noise is None:
+        r = (_native or _fast()).gradq8(dw, q, scale, bool(accumulate), seed, offset)
+        if r is not None:
+            return r
     _chk(dw, torch.bfloat16, "dw")
     _chk(q, torch.int8, "q")
     _chk(scale, torch.bfloat16, "scale")
@@ -638,6 +728,9 @@ def _weight_grad_native_ok(dy, x, k_mult=8):
 def weight_grad(dy, x):
     """dW = dY^T X for 2-D operands: the library's own GEMM (lq_weight_grad: both operands read as they lie in
     memory) for bf16 GPU operands with a multiple of 64 tokens, the tensor library's product otherwise."""
+    dw = (_native or _fast()).weight_grad(dy, x)
+    if dw is not None:
+        return dw
     if _weight_grad_native_ok(dy, x):
         N, K = dy.shape[1], x.shape[1]
         dw = torch.empty((N, K), dtype=torch.bfloat16, device=dy.device)
@@ -660,6 +753,8 @@ def weight_grad_acc_ok(dy, x, g) -> bool:
 def weight_grad_acc(dy, x, g):
     """g = bf16(g + bf16(dY^T X)) in place (lq_weight_grad_acc): the weight-gradient GEMM with the bf16 ``add_`` of the
     gradient accumulation as its epilogue; the same bits as ``g.add_(weight_grad(dy, x))``."""
+    if (_native or _fast()).weight_grad_acc(dy, x, g) is not None:
+        return g
     if not weight_grad_acc_ok(dy, x, g):
         raise ValueError("weight_grad_acc needs contiguous bf16 GPU operands, M % 64 == 0, N % 8 == 0, K % 8 == 0 and g [N, K]")
     N, K = dy.shape[1], x.shape[1]
@@ -671,6 +766,8 @@ def weight_grad_acc(dy, x, g):
 def weight_grad_acc8(dy, x, q, scale, noise=None, seed: int = 0, offset: int = 0):
     """q = quant(dequant(q) + dY^T X) in place (lq_weight_grad_acc8): the weight-gradient GEMM with the add_ form of
     the 8-bit gradient accumulator as its epilogue. dy bf16 [M,N], x bf16 [M,K], q int8 [N,K], scale bf16 [N,1]."""
+    if noise is None and (_native or _fast()).weight_grad_acc8(dy, x, q, scale, seed, offset) is not None:
+        return q
     if not _weight_grad_native_ok(dy, x, 16):
         raise ValueError("weight_grad_acc8 needs contiguous bf16 GPU operands, M % 64 == 0, N % 8 == 0, K % 16 == 0")
     N, K = dy.shape[1], x.shape[1]

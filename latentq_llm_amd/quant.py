@@ -207,6 +207,9 @@ def _as_bf16_2d(x):
 
 
 def _w4_linear(input, weight_d, qparamw4, bias):
+    y = ops.linear4(input, weight_d, *qparamw4, bias)
+    if y is not None:
+        return y
     scales, zeros, shape = _flat_qparam(qparamw4)
     b = None if bias is None else bias.detach().to(torch.bfloat16).contiguous()
     y = ops.a16w4_forward(_as_bf16_2d(input), weight_d, scales, zeros, shape, b)
@@ -218,15 +221,12 @@ class QLinearFunctionW4(torch.autograd.Function):
     packed codes (never a materialised W): dX on the HIP dequant-GEMM, dW = dY^T X pushed to
     dict_temp for the backward hook, dB = sum dY."""
 
+    # (ctx in forward, no setup_context: with one, every call binds its arguments to forward's signature, 10 us)
     @staticmethod
-    def forward(input, weight_d, qparamw4, bias):
-        return _w4_linear(input, weight_d, qparamw4, bias)
-
-    @staticmethod
-    def setup_context(ctx, inputs, output):
-        input, weight_d, qparamw4, bias = inputs
+    def forward(ctx, input, weight_d, qparamw4, bias):
         ctx.save_for_backward(input, weight_d.data, bias)
         ctx.save_qparamw4 = qparamw4
+        return _w4_linear(input, weight_d, qparamw4, bias)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -248,12 +248,8 @@ class QLinearFunctionW4_eval(torch.autograd.Function):
     """Inference A16W4 linear (utils/quant.py:149-169): no state saved, no gradients."""
 
     @staticmethod
-    def forward(input, weight_d, qparamw4, bias):
+    def forward(ctx, input, weight_d, qparamw4, bias):
         return _w4_linear(input, weight_d, qparamw4, bias)
-
-    @staticmethod
-    def setup_context(ctx, inputs, output):
-        pass
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -354,15 +350,11 @@ class QLinearFunctionA8W8_static(torch.autograd.Function):
     """Static activation clamp (utils/quant.py:172-211)."""
 
     @staticmethod
-    def forward(input, weight_d, qparamaw, bias):
+    def forward(ctx, input, weight_d, qparamaw, bias):
         clampv, qscales = qparamaw
-        return _a8w8_linear(input, weight_d, qscales, bias, clampv, alpha_in_bf16=False)[0]
-
-    @staticmethod
-    def setup_context(ctx, inputs, output):
-        input, weight_d, qparamaw, bias = inputs
         ctx.save_for_backward(input, weight_d.data, bias)
         ctx.save_qparamaw = qparamaw
+        return _a8w8_linear(input, weight_d, qscales, bias, clampv, alpha_in_bf16=False)[0]
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -540,10 +532,22 @@ class _QLinearBase(nn.Module):
         out = fn.apply(x.reshape(-1, x.shape[-1]), self.weight.data, self._qparam(), self.bias)
         return out.reshape(x.shape[:-1] + (self.output_features,))
 
+    def _infer(self, x):
+        """The layer's result where nothing is differentiated and every operand is in the form the kernels take; None
+        otherwise. The same kernels as the autograd Functions run, without the Function around them: in decoding that
+        costs the host as much as the kernel takes."""
+        return None
+
     def forward(self, x):
-        return self._apply_fn(self._fn_eval if self.hook_handle is None else self._fn_train, x)
+        if self.hook_handle is None:
+            return self.forward_eval(x)
+        return self._apply_fn(self._fn_train, x)
 
     def forward_eval(self, x):
+        if not torch.is_grad_enabled():
+            y = self._infer(x)
+            if y is not None:
+                return y
         return self._apply_fn(self._fn_eval, x)
 
     def before_save(self):
@@ -570,6 +574,10 @@ class QLinearA16W4(_QLinearBase):
 
     def _qparam(self):
         return self.weight.qparam
+
+    def _infer(self, x):
+        w = self.weight
+        return ops.linear4(x, w.data, *w.qparam, self._parameters["bias"])
 
     def to(self, device: Optional[Union[int, torch.device]]):
         """Moves the QuantTensor and re-binds its qparam to the moved buffers; returns None like
@@ -601,6 +609,9 @@ class QLinearA8W8(_QLinearBase):
         if self.act_quant == "per_token":
             return (self.clampv, self.qscales.data, "per_token")
         return (self.clampv, self.qscales.data)
+
+    def _infer(self, x):
+        return ops.infer8(x, self.weight.data, self._buffers["qscales"], self._parameters["bias"], self.act_quant == "per_token")
 
     def to(self, device: Optional[Union[int, torch.device]]):
         self.weight = self.weight.to(device=device)
