@@ -196,6 +196,14 @@ def _pending_dw(grad_output, input):
     return ops.weight_grad(grad_output, input)
 
 
+def _hand_over(layer, dw):
+    """The weight gradient of one backward to its layer: through dict_temp and backward_hook_fn, as the reference's
+    full-backward hook collects it, or left in dict_temp where no layer is known (a Function applied by itself)."""
+    dict_temp.append(dw)
+    if layer is not None:
+        backward_hook_fn(layer, None, None)
+
+
 # ------------------------------------------------------------------------ autograd: A16W4 --
 # The reference gates the bias gradient on needs_input_grad[2] (utils/quant.py:143, 208, 249, 290,
 # 371), which is the flag of the non-tensor qparam argument and therefore always False: QLinear
@@ -223,9 +231,10 @@ class QLinearFunctionW4(torch.autograd.Function):
 
     # (ctx in forward, no setup_context: with one, every call binds its arguments to forward's signature, 10 us)
     @staticmethod
-    def forward(ctx, input, weight_d, qparamw4, bias):
+    def forward(ctx, input, weight_d, qparamw4, bias, layer=None):
         ctx.save_for_backward(input, weight_d.data, bias)
         ctx.save_qparamw4 = qparamw4
+        ctx.layer = layer
         return _w4_linear(input, weight_d, qparamw4, bias)
 
     @staticmethod
@@ -238,10 +247,10 @@ class QLinearFunctionW4(torch.autograd.Function):
             grad_input = ops.a16w4_dx(dy, weight_d, scales, zeros, shape)
             if grad_input.dtype != input.dtype:
                 grad_input = grad_input.to(input.dtype)
-        dict_temp.append(_pending_dw(dy, _as_bf16_2d(input)))  # dW = dY^T X (utils/quant.py:141-142)
+        _hand_over(ctx.layer, _pending_dw(dy, _as_bf16_2d(input)))  # dW = dY^T X (utils/quant.py:141-142)
         if bias is not None and ctx.needs_input_grad[_BIAS_FLAG]:
             grad_bias = grad_output.sum(0)
-        return grad_input, None, None, grad_bias
+        return grad_input, None, None, grad_bias, None
 
 
 class QLinearFunctionW4_eval(torch.autograd.Function):
@@ -340,17 +349,18 @@ def _a8w8_backward_common(ctx, grad_output, input_f, weight_f, bias, detach_dw=F
                 grad_input = grad_output.mm((w8.to(grad_output.dtype) * qscales).to(grad_output.dtype))
         else:
             grad_input = grad_output.mm(weight_f)
-    dict_temp.append(_pending_dw(grad_output, input_f))
+    _hand_over(ctx.layer, _pending_dw(grad_output, input_f))
     if bias is not None and ctx.needs_input_grad[_BIAS_FLAG]:
         grad_bias = grad_output.sum(0)
-    return grad_input, None, None, grad_bias
+    return grad_input, None, None, grad_bias, None
 
 
 class QLinearFunctionA8W8_static(torch.autograd.Function):
     """Static activation clamp (utils/quant.py:172-211)."""
 
     @staticmethod
-    def forward(ctx, input, weight_d, qparamaw, bias):
+    def forward(ctx, input, weight_d, qparamaw, bias, layer=None):
+        ctx.layer = layer
         clampv, qscales = qparamaw
         ctx.save_for_backward(input, weight_d.data, bias)
         ctx.save_qparamaw = qparamaw
@@ -368,7 +378,8 @@ class QLinearFunctionA8W8_dynamic0(torch.autograd.Function):
     """Dynamic clamp = input.max(), saves the bf16 input (utils/quant.py:214-252)."""
 
     @staticmethod
-    def forward(ctx, input, weight_d, qparamaw, bias):
+    def forward(ctx, input, weight_d, qparamaw, bias, layer=None):
+        ctx.layer = layer
         qscales = qparamaw[1]
         out, _, work = _a8w8_linear_dynamic(input, weight_d, qscales, bias, alpha_in_bf16=False)
         ctx.save_for_backward(input, weight_d.data, bias)
@@ -388,7 +399,8 @@ class QLinearFunctionA8W8_dynamic(torch.autograd.Function):
     QLinearA8W8 dispatches to when training."""
 
     @staticmethod
-    def forward(ctx, input, weight_d, qparamaw, bias):
+    def forward(ctx, input, weight_d, qparamaw, bias, layer=None):
+        ctx.layer = layer
         qscales = qparamaw[1]
         per_token = _per_token(qparamaw)
         out, x8, scale = _a8w8_linear_dynamic(input, weight_d, qscales, bias, alpha_in_bf16=True, per_token=per_token)
@@ -450,7 +462,8 @@ class QLinearFunctionQAT_dynamic(torch.autograd.Function):
     """bf16 latent weight, quantised to int8 on the fly (utils/quant.py:334-374)."""
 
     @staticmethod
-    def forward(ctx, input, weight_f, qparamaw, bias):
+    def forward(ctx, input, weight_f, qparamaw, bias, layer=None):
+        ctx.layer = layer
         qscales = qparamaw[1]
         out, _, work = _a8w8_linear_dynamic(input, _qat_weight_i8(weight_f, qscales), qscales, bias, alpha_in_bf16=False)
         ctx.save_for_backward(input, weight_f.data, bias)
@@ -510,6 +523,17 @@ def backward_hook_fn(module, grad_out, grad_in):
 
 
 # -------------------------------------------------------------------------------- modules --
+class _HookHandle(object):
+    """What add_hook leaves in hook_handle: remove() ends the delivery of weight gradients (they then stay in dict_temp,
+    as with the reference's hook removed)."""
+
+    def __init__(self):
+        self.active = True
+
+    def remove(self):
+        self.active = False
+
+
 class _QLinearBase(nn.Module):
     _repr_name = "QLinear"
 
@@ -526,11 +550,14 @@ class _QLinearBase(nn.Module):
         self.hook_handle = None
 
     def add_hook(self):
-        self.hook_handle = self.register_full_backward_hook(backward_hook_fn)
+        """The layer's weight gradients are delivered to weight.grad from now on (until hook_handle.remove()). The
+        reference registers backward_hook_fn as a full-backward hook; here the Functions call it themselves, since such a
+        hook wraps a layer's inputs and outputs in autograd nodes of their own (47 us of host time per step and layer)."""
+        self.hook_handle = _HookHandle()
 
-    def _apply_fn(self, fn, x):
-        out = fn.apply(x.reshape(-1, x.shape[-1]), self.weight.data, self._qparam(), self.bias)
-        return out.reshape(x.shape[:-1] + (self.output_features,))
+    def _apply_fn(self, fn, x, *layer):
+        out = fn.apply(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), self.weight.data, self._qparam(), self.bias, *layer)
+        return out if x.dim() == 2 else out.reshape(x.shape[:-1] + (self.output_features,))
 
     def _infer(self, x):
         """The layer's result where nothing is differentiated and every operand is in the form the kernels take; None
@@ -541,7 +568,7 @@ class _QLinearBase(nn.Module):
     def forward(self, x):
         if self.hook_handle is None:
             return self.forward_eval(x)
-        return self._apply_fn(self._fn_train, x)
+        return self._apply_fn(self._fn_train, x, self if getattr(self.hook_handle, "active", False) else None)
 
     def forward_eval(self, x):
         if not torch.is_grad_enabled():
