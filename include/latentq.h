@@ -430,7 +430,7 @@ int lq_gradq8_quant(const void *dw, int8_t *q_inout, void *scale_inout, int accu
  * Weight gradient of a quantised linear layer, dW[N,K] = dY[M,N]^T . X[M,K] (bf16, fp32 accumulation):
  * `grad_output.t().mm(input)` of QLinearFunctionW4.backward and its A8W8 / QAT siblings (reference
  * utils/quant.py:141-142, 207, 248, 289, 370). Both operands are read as they lie in memory (no transposed
- * copy). dy: bf16 [M,N]; x: bf16 [M,K]; M % 64 == 0, N % 8 == 0; dy, x and the output 16-byte aligned.
+ * copy). dy: bf16 [M,N]; x: bf16 [M,K]; any M > 0, N % 8 == 0; dy, x and the output 16-byte aligned.
  *   lq_weight_grad:      dw_out = bf16(dW), bf16 [N,K], K % 8 == 0.
  *   lq_weight_grad_acc:  dw_inout = bf16(dw_inout + bf16(dW)): the `module.weight.grad.add_(dW)` of backward_hook_fn
  *     (utils/quant.py:398-411) on every micro-batch after the first when the gradient is kept in bf16 (gbit = 16),

@@ -320,7 +320,7 @@ bool dw_operands(PyObject *const *a, const at::Tensor **dy, const at::Tensor **x
     *dy = bf16(a[0]);
     *x = bf16(a[1]);
     return *dy && *x && (*dy)->dim() == 2 && (*x)->dim() == 2 && (*dy)->size(0) == (*x)->size(0) && (*dy)->size(0) > 0 &&
-           (*dy)->size(0) % 64 == 0 && (*dy)->size(1) > 0 && (*dy)->size(1) % 8 == 0 && (*x)->size(1) > 0 && (*x)->size(1) % k_mult == 0 &&
+           (*dy)->size(1) > 0 && (*dy)->size(1) % 8 == 0 && (*x)->size(1) > 0 && (*x)->size(1) % k_mult == 0 &&
            aligned16(*dy) && aligned16(*x) && same_device(*dy, *x);
 }
 

@@ -7,19 +7,28 @@
 // 16-lane block, lane i receives the four elements of column i of the 4 x 16 block the 16 lanes address. No
 // transposed copy of dY is made anywhere.
 //
-// Workgroup: 256 (n) x 256 (k) outputs, 512 threads = 8 waves in a 2 (n) x 4 (k) grid; a wave owns 128 x 64
-// outputs (4 x 2 MFMA 32x32x16 tiles, 128 accumulator registers). Two LDS stages of 64 KB (64 rows of dY and 64
-// rows of X, 512 bytes each); one workgroup per CU.
+// Two tile sizes (dw_takes_small_tiles below chooses):
+//   256 (n) x 256 (k) outputs, 512 threads = 8 waves in a 2 (n) x 4 (k) grid; a wave owns 128 x 64 outputs (4 x 2 MFMA
+//     32x32x16 tiles, 128 accumulator registers). Steps of 64 tokens, two LDS stages of 64 KB (64 rows of dY and 64 rows
+//     of X, 512 bytes each); one workgroup per CU.
+//   128 x 128 outputs, 256 threads = 2 x 2 waves of 64 x 64. Steps of 32 tokens, four stages of 16 KB, two workgroups
+//     per CU: for outputs whose large tiles leave most of the device idle. There a workgroup has nothing but its own
+//     prefetch distance to cover its waits, which is what the four stages are for (2048 x 2048 outputs, 2048 tokens:
+//     20.4 us against 26.4 with two stages of 64 tokens). Deeper stages gain the large tile nothing (159 against 157 us
+//     on 11008 x 4096: it is bound by power, 79 % of the matrix pipe's cycles when few CUs run it).
 //
-// Reduction step = 64 tokens in four slices of 16. Lane l: r = l % 32, h = l / 32; in slice t the lane's operand
-// for column r of a 32-column fragment is tokens 16 t + 8 h .. + 7: two transposing reads (tokens .. + 3 and
-// + 4 .. + 7). In each read block lane i (of 16) addresses row i / 4 of the block's 4 token rows at columns
-// 4 (i % 4) .. + 3 of its 16 columns. A row's 512 bytes are sixteen 32-byte segments; segment s of token row m
-// sits at position s ^ 2 (m & 3), which spreads the 4 rows x 2 column blocks that 32 lanes read over all 64 banks;
-// the swizzle is free, since an LDS-direct load lets a lane choose the global 16 bytes that land in its slot.
+// A slice is 16 tokens. Lane l: r = l % 32, h = l / 32; in slice t the lane's operand for column r of a 32-column
+// fragment is tokens 16 t + 8 h .. + 7: two transposing reads (tokens .. + 3 and + 4 .. + 7). In each read block lane i
+// (of 16) addresses row i / 4 of the block's 4 token rows at columns 4 (i % 4) .. + 3 of its 16 columns. A row is a
+// number of 32-byte segments; segment s of token row m sits at position s ^ 2 (m & 3), which spreads the 4 rows x 2
+// column blocks that 32 lanes read over all 64 banks; the swizzle is free, since an LDS-direct load lets a lane choose
+// the global 16 bytes that land in its slot.
 //
-// Pipeline as in the int8 tile kernel: one s_barrier per step before its last slice, the loads of the step after
-// next go into the stage that barrier releases, loads as inline assembly with explicit waits.
+// Any number of tokens: see `first` below. Against the tensor library's product, which took the token counts that are
+// no multiple of 64 before: 500 tokens, 5504 x 2048 outputs 18.4 against 24.7 us, 1000 tokens, 11008 x 4096 87 against 116.
+//
+// Pipeline as in the int8 tile kernel: one s_barrier per step before its last slice, loads as inline assembly with
+// explicit waits.
 //
 // D = Xfrag x dYfrag^T: a lane owns 4 consecutive k of one n. Epilogues (through LDS, 16-byte pieces of rows):
 //   store  dW rounded to bf16;
@@ -53,23 +62,24 @@ typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 template <int I>
 using ic = std::integral_constant<int, I>;
 
-constexpr int TILE = 256;            // outputs per workgroup along n and along k
-constexpr int ROWB = TILE * 2;       // bytes per staged token row of one operand
-constexpr int STEP_M = 64;           // tokens per reduction step
-constexpr int OP_STAGE = STEP_M * ROWB;  // 32 KB per operand and stage
-constexpr int STAGE = 2 * OP_STAGE;
-constexpr int NT = 512;
-constexpr int LOADS = OP_STAGE / 16 / NT;  // 16-byte loads per thread, operand and stage: 4
-
-template <bool ACC8>
-__global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
-    constexpr int WM = 2, WN = 4;           // waves along n, along k
-    constexpr int TM = TILE / WM, TN = TILE / WN;  // wave tile: 128 n x 64 k
+// TILE: outputs per workgroup along n and along k. 256: 8 waves of 128 x 64, one workgroup per CU. 128: 4 waves of
+// 64 x 64, two workgroups per CU. STEP_M: tokens per reduction step; NST: LDS stages of one step.
+template <int TILE, int STEP_M, int NST, bool ACC8>
+__global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwParams p) {
+    constexpr int NT = TILE == 256 ? 512 : 256;
+    constexpr int ROWB = TILE * 2;           // bytes per staged token row of one operand
+    constexpr int OP_STAGE = STEP_M * ROWB;  // bytes per operand and stage
+    constexpr int STAGE = 2 * OP_STAGE;
+    constexpr int LOADS = OP_STAGE / 16 / NT;  // 16-byte loads per thread, operand and stage
+    constexpr int SL = STEP_M / 16;            // slices of a step (an even number)
+    constexpr int WM = 2, WN = NT / 64 / WM;       // waves along n, along k
+    constexpr int TM = TILE / WM, TN = TILE / WN;  // wave tile: 128 n x 64 k, or 64 x 64
     constexpr int FM = TM / 32, FN = TN / 32;
-    // two stages; the accumulate epilogue stages every wave's whole 128 x 64 block (144-byte rows) instead
-    constexpr int LDS_BYTES = ACC8 && 8 * TM * (TN * 2 + 16) > 2 * STAGE ? 8 * TM * (TN * 2 + 16) : 2 * STAGE;
+    // the stages; the accumulate epilogue stages every wave's whole block (144-byte rows) instead
+    constexpr int EP_ALL = WM * WN * TM * (TN * 2 + 16);
+    constexpr int LDS_BYTES = ACC8 && EP_ALL > NST * STAGE ? EP_ALL : NST * STAGE;
     __shared__ __attribute__((aligned(16))) unsigned char lds_all[LDS_BYTES];
-    auto stage = [&](auto i) -> unsigned char * { return lds_all + decltype(i)::value * STAGE; };
+    auto stage = [&](int i) -> unsigned char * { return lds_all + (i % NST) * STAGE; };
 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -92,16 +102,20 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     const int bw = rest < GN ? rest : GN;
     const int tile_n = within / bw, tile_k = band * GN + within % bw;
     const int n0 = tile_n * TILE, k0 = tile_k * TILE;
-    const int nk = p.M / STEP_M;
+    // A number of tokens that is no multiple of the step leaves the FIRST step short: it covers tokens 0 .. first - 1 (its
+    // other rows re-read the last of them and are masked out of both operands), and every later step starts on a full
+    // stride. The steps after it are then those of a multiple of 64.
+    const int nk = (p.M + STEP_M - 1) / STEP_M;
+    const int first = p.M - (nk - 1) * STEP_M;
 
-    // ---- staging: slot s = i * 512 + thread of an operand's stage is token row s / 32, 16-byte position s % 32;
-    // it receives the 16 bytes of segment (pos / 2) ^ 2 (row & 3), half pos & 1. Columns past the end of a matrix
+    // ---- staging: slot s = i * NT + thread of an operand's stage is token row s / (TILE / 8), 16-byte position
+    // s % (TILE / 8); it receives the 16 bytes of segment (pos / 2) ^ 2 (row & 3), half pos & 1. Columns past the end of a matrix
     // re-read its last 8 columns (their results are dropped).
     unsigned a_off[LOADS], b_off[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
         const int s = i * NT + (int)threadIdx.x;
-        const int row = s >> 5, pos = s & 31;
+        const int row = s / (TILE / 8), pos = s % (TILE / 8);
         const int c16 = ((((pos >> 1) ^ (2 * (row & 3))) << 1) | (pos & 1));
         int ca = n0 / 8 + c16, cb = k0 / 8 + c16;
         ca = ca < p.N / 8 ? ca : p.N / 8 - 1;
@@ -110,14 +124,23 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
         b_off[i] = (unsigned)((long long)row * p.K * 2 + (long long)cb * 16);
     }
     // load i of a step: 0 .. LOADS-1 fill the dY rows of the stage, LOADS .. 2 LOADS-1 its X rows
-    auto issue_one = [&](int kt, unsigned char *st, int i) {
+    auto issue_off = [&](long long row0, unsigned char *st, int i, unsigned off) {
         const bool is_b = i >= LOADS;
         const int ii = is_b ? i - LOADS : i;
-        const unsigned char *src = is_b ? p.x + (long long)kt * STEP_M * p.K * 2 : p.dy + (long long)kt * STEP_M * p.N * 2;
+        const unsigned char *src = is_b ? p.x + row0 * p.K * 2 : p.dy + row0 * p.N * 2;
         const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>(
             (lds_void *)(st + (is_b ? OP_STAGE : 0) + (ii * NT + wave * 64) * 16));
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :: "s"(lds_addr), "v"(is_b ? b_off[ii < LOADS ? ii : 0] : a_off[ii < LOADS ? ii : 0]), "s"(src) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds_addr), "v"(off), "s"(src) : "memory");
+    };
+    auto issue_one = [&](int kt, unsigned char *st, int i) {  // kt >= 1, or a full first step
+        const int ii = i >= LOADS ? i - LOADS : i;
+        issue_off((long long)kt * STEP_M - (STEP_M - first), st, i, i >= LOADS ? b_off[ii < LOADS ? ii : 0] : a_off[ii < LOADS ? ii : 0]);
+    };
+    auto issue_first = [&](unsigned char *st, int i) {  // step 0: rows past `first` re-read the last one
+        const int ii = i >= LOADS ? i - LOADS : i;
+        const int over = (ii * NT + (int)threadIdx.x) / (TILE / 8) - (first - 1);
+        const unsigned back = over > 0 ? (unsigned)over : 0u;
+        issue_off(0, st, i, i >= LOADS ? b_off[ii < LOADS ? ii : 0] - back * (unsigned)(p.K * 2) : a_off[ii < LOADS ? ii : 0] - back * (unsigned)(p.N * 2));
     };
 
     // ---- fragments. Read block = lane / 16: column block (lane / 16) & 1 of the fragment's 32 columns, token half
@@ -134,6 +157,15 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
 #pragma unroll
     for (int i = 0; i < FN; ++i) b_col[i] = OP_STAGE + col_off(wn * TN + 32 * i);
     const int row_lane = (8 * h + (i16 >> 2)) * ROWB;  // + 16 t rows for slice t, + 4 rows for the second read
+    // a short first step: the lane's tokens 16 t + 8 h + e of slice t with 16 t + 8 h + e >= first become zero
+    auto mask_frag = [&](u32x4_t &f, int t) {
+        const int valid = first - (16 * t + 8 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const unsigned keep = valid >= 2 * e + 2 ? 0xFFFFFFFFu : valid == 2 * e + 1 ? 0x0000FFFFu : 0u;
+            f[e] &= keep;
+        }
+    };
     auto read_frags = [&](const unsigned char *st, int t, u32x4_t *af, u32x4_t *bf) {
         const unsigned char *base = st + row_lane + t * 16 * ROWB;
 #pragma unroll
@@ -161,53 +193,80 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
             for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
 
     u32x4_t af[2][FM], bf[2][FN];
-    // Step kt on stage S = kt % 2: the operands of its first slice are already in af[0] / bf[0]. The barrier of a
-    // step releases its stage, into which the last slice issues the dY half of step kt + 2 and the next step's
-    // first slice the X half.
-    auto step = [&](int kt, auto si) {
-        constexpr int S = decltype(si)::value;
-        unsigned char *cur = stage(ic<S>()), *nxt = stage(ic<S ^ 1>());
-        const int kt_b = kt + 1 < nk ? kt + 1 : nk - 1, kt_a = kt + 2 < nk ? kt + 2 : nk - 1;
+    auto mfma_slice = [&](const u32x4_t *a, const u32x4_t *b) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            if (t == 3) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (t < 3) read_frags(cur, t + 1, af[(t + 1) & 1], bf[(t + 1) & 1]);
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+            for (int j = 0; j < FM; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, b[i]),
+                                                                   __builtin_bit_cast(bf16x8_t, a[j]), acc[i][j], 0, 0, 0);
+    };
+    // Step kt: the operands of its first slice are already in af[0] / bf[0]. The barrier stands before the last slice: it
+    // finds step kt + 1 landed (all but the loads of the steps after it), every wave's reads of this step returned, and
+    // releases this step's stage. The last slice then reads the first operands of step kt + 1 and issues the dY half of
+    // step kt + NST into the stage just released; the next step's first slice issues the X half.
+    auto step = [&](int kt, auto si, auto masked) {
+        constexpr int S = decltype(si)::value;                 // the step's stage
+        constexpr bool MASKED = decltype(masked)::value != 0;  // the short first step
+        unsigned char *cur = stage(S), *nxt = stage(S + 1), *left = stage(S + NST - 1);
+        // (the last steps re-load the last step's rows)
+        const int kt_x = kt + NST - 1 < nk ? kt + NST - 1 : nk - 1, kt_dy = kt + NST < nk ? kt + NST : nk - 1;
+        auto load = [&](int k, unsigned char *st, int i) {
+            if (MASKED && k == 0) issue_first(st, i);
+            else issue_one(k, st, i);
+        };
+#pragma unroll
+        for (int t = 0; t < SL; ++t) {
+            if (t == SL - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * 2 * LOADS) : "memory");
+            if (t < SL - 1) read_frags(cur, t + 1, af[(t + 1) & 1], bf[(t + 1) & 1]);
             else read_frags(nxt, 0, af[0], bf[0]);
             if (t == 0) {
-                // X half of the loads of step kt + 1 (its stage was released by the previous barrier)
 #pragma unroll
-                for (int i = LOADS; i < 2 * LOADS; ++i) issue_one(kt_b, nxt, i);
+                for (int i = LOADS; i < 2 * LOADS; ++i) load(kt_x, left, i);
             }
-            if (t == 3) {
-                // dY half of the loads of step kt + 2, into the stage just released
+            if (t == SL - 1) {
 #pragma unroll
-                for (int i = 0; i < LOADS; ++i) issue_one(kt_a, cur, i);
+                for (int i = 0; i < LOADS; ++i) load(kt_dy, cur, i);
             }
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (MASKED) {
 #pragma unroll
-            for (int i = 0; i < FN; ++i)
+                for (int j = 0; j < FM; ++j) mask_frag(af[t & 1][j], t);
 #pragma unroll
-                for (int j = 0; j < FM; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, bf[t & 1][i]),
-                                                                       __builtin_bit_cast(bf16x8_t, af[t & 1][j]), acc[i][j], 0, 0, 0);
+                for (int i = 0; i < FN; ++i) mask_frag(bf[t & 1][i], t);
+            }
+            mfma_slice(af[t & 1], bf[t & 1]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
 
-    // prologue: step 0 entirely, the dY half of step 1; wait for step 0
+    // prologue: steps 0 .. NST - 2 and the dY half of step NST - 1; wait for step 0. A short first step takes the last
+    // stage, so that the loop below starts on stage 0 either way.
+    const int shift = first < STEP_M ? NST - 1 : 0;
 #pragma unroll
-    for (int i = 0; i < 2 * LOADS; ++i) issue_one(0, stage(ic<0>()), i);
+    for (int s = 0; s < NST; ++s)
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) issue_one(nk > 1 ? 1 : 0, stage(ic<1>()), i);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS) : "memory");
-    read_frags(lds_all, 0, af[0], bf[0]);
+        for (int i = 0; i < (s == NST - 1 ? LOADS : 2 * LOADS); ++i) {
+            const int k = s < nk ? s : nk - 1;
+            if (k == 0) issue_first(stage(s + shift), i);
+            else issue_one(k, stage(s + shift), i);
+        }
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * 2 * LOADS + LOADS) : "memory");
+    read_frags(stage(shift), 0, af[0], bf[0]);
     __builtin_amdgcn_sched_barrier(0);
     int kt = 0;
-    for (; kt + 2 <= nk; kt += 2) {
-        step(kt, ic<0>());
-        step(kt + 1, ic<1>());
+    if (first < STEP_M) step(kt++, ic<NST - 1>(), ic<1>());
+    for (; kt + NST <= nk; kt += NST) {
+        step(kt, ic<0>(), ic<0>());
+        step(kt + 1, ic<1>(), ic<0>());
+        if constexpr (NST > 2) step(kt + 2, ic<2 % NST>(), ic<0>());
+        if constexpr (NST > 3) step(kt + 3, ic<3 % NST>(), ic<0>());
     }
-    if (kt < nk) step(kt, ic<0>());
+    static_assert(NST <= 4, "the loop above has up to four steps");
+    const int rem = nk - kt;
+    if (rem > 0) step(kt, ic<0>(), ic<0>());
+    if constexpr (NST > 2) if (rem > 1) step(kt + 1, ic<1>(), ic<0>());
+    if constexpr (NST > 3) if (rem > 2) step(kt + 2, ic<2 % NST>(), ic<0>());
     // the clamped prefetches of the last steps are still writing LDS: drain them
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
@@ -310,22 +369,47 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     }
 }
 
-static int launch_dw(DwParams p, bool acc8, hipStream_t st, const char *who) {
+template <int TILE, int STEP_M, int NST>
+static int launch_dw_tile(DwParams p, bool acc8, hipStream_t st, const char *who) {
     p.tiles_n = (p.N + TILE - 1) / TILE;
     p.tiles_k = (p.K + TILE - 1) / TILE;
     const long long nwg = (long long)p.tiles_n * p.tiles_k;
     if (nwg > 0x7FFFFFFFll) return lq_fail(LQ_ERR_BAD_ARG, "%s: problem too large", who);
-    // the 32-bit lane offsets of the loads span 64 token rows
+    // the 32-bit lane offsets of the loads span a step's token rows
     if (64ll * 2 * (p.N > p.K ? p.N : p.K) >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: rows too long", who);
-    if (acc8) hipLaunchKernelGGL(gemm_dw_kernel<true>, dim3((unsigned)nwg), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(gemm_dw_kernel<false>, dim3((unsigned)nwg), dim3(NT), 0, st, p);
+    const dim3 grid((unsigned)nwg), block(TILE == 256 ? 512 : 256);
+    if (acc8) hipLaunchKernelGGL((gemm_dw_kernel<TILE, STEP_M, NST, true>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((gemm_dw_kernel<TILE, STEP_M, NST, false>), grid, block, 0, st, p);
     return lq_check_launch(who);
+}
+
+// Which tile a product takes: the smaller of two estimates in microseconds, both of the form (time per 64-token step,
+// summed over the rounds of workgroups) x steps + fixed, fitted to 30 shapes from 64 to 4096 tokens and 768^2 to
+// 11008 x 4096 outputs. A round of 256 x 256 tiles steps in 1.13 us while it leaves two fifths of the CUs idle and in 1.55
+// with all of them busy (power); 128 x 128 tiles step in 0.40 to 0.48 us alone on a CU, in 0.62 to 0.85 as the second
+// workgroup of a CU joins. Both sides, small and large: 2048 tokens, 2048^2 20.4 / 39.8 us; 2048 x 4096 36.2 / 43.9;
+// 3072^2 47.6 / 44.1; 11008 x 4096 176 / 157; 1024 tokens, 3072 x 768 12.0 / 23.1; 300 tokens, 2048 x 4096 16.0 / 13.3.
+static bool dw_takes_small_tiles(long long M, long long N, long long K, long long cus) {
+    const double steps = (double)M / 64.0;
+    const long long t256 = ((N + 255) / 256) * ((K + 255) / 256), t128 = ((N + 127) / 128) * ((K + 127) / 128);
+    const double r256 = (double)(t256 % cus) / (double)cus;          // the last round's share of the CUs
+    const double r128 = (double)(t128 % (2 * cus)) / (double)cus;    // 0 .. 2 workgroups per CU
+    const double last256 = r256 == 0 ? 0 : r256 <= 0.56 ? 1.13 : 1.13 + 0.42 * (r256 - 0.56) / 0.44;
+    const double last128 = r128 == 0 ? 0 : r128 <= 1 ? 0.40 + 0.08 * r128 : 0.62 + 0.23 * (r128 - 1);
+    const double rounds256 = (double)(t256 / cus), rounds128 = (double)(t128 / (2 * cus));
+    const double est256 = (1.55 * rounds256 + last256) * steps + 8 + 4 * rounds256;
+    const double est128 = (0.85 * rounds128 + last128) * steps + (t128 <= cus ? 5 : 9) + 4 * rounds128;
+    return est128 < est256;
+}
+
+static int launch_dw(const DwParams &p, bool acc8, hipStream_t st, const char *who) {
+    return dw_takes_small_tiles(p.M, p.N, p.K, lq_device_cu_count()) ? launch_dw_tile<128, 32, 4>(p, acc8, st, who)
+                                                                       : launch_dw_tile<256, 64, 2>(p, acc8, st, who);
 }
 
 static int check_dw(const char *who, const void *dy, const void *x, int64_t M, int64_t N, int64_t K, int k_mult) {
     LQ_REQUIRE(dy && x, "%s: null pointer argument", who);
     LQ_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "%s: M, N, K must be positive", who);
-    LQ_REQUIRE(M % 64 == 0, "%s: M=%lld (tokens) must be a multiple of 64", who, (long long)M);
     LQ_REQUIRE(N % 8 == 0 && K % k_mult == 0, "%s: N=%lld must be a multiple of 8 and K=%lld of %d", who, (long long)N, (long long)K, k_mult);
     LQ_REQUIRE(lq_aligned(dy, 16) && lq_aligned(x, 16), "%s: dy and x must be 16-byte aligned", who);
     return LQ_OK;

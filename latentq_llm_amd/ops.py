@@ -721,13 +721,13 @@ def transpose_bf16(x):
 def _weight_grad_native_ok(dy, x, k_mult=8):
     return (dy.is_cuda and x.is_cuda and dy.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and dy.dim() == 2
             and x.dim() == 2 and dy.is_contiguous() and x.is_contiguous() and dy.shape[0] == x.shape[0]
-            and dy.shape[0] > 0 and dy.shape[0] % 64 == 0 and dy.shape[1] % 8 == 0 and x.shape[1] % k_mult == 0
+            and dy.shape[0] > 0 and dy.shape[1] % 8 == 0 and x.shape[1] % k_mult == 0
             and dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
 
 
 def weight_grad(dy, x):
     """dW = dY^T X for 2-D operands: the library's own GEMM (lq_weight_grad: both operands read as they lie in
-    memory) for bf16 GPU operands with a multiple of 64 tokens, the tensor library's product otherwise."""
+    memory) for contiguous bf16 GPU operands whose rows are whole 16-byte pieces, the tensor library's product otherwise."""
     dw = (_native or _fast()).weight_grad(dy, x)
     if dw is not None:
         return dw
@@ -756,7 +756,7 @@ def weight_grad_acc(dy, x, g):
     if (_native or _fast()).weight_grad_acc(dy, x, g) is not None:
         return g
     if not weight_grad_acc_ok(dy, x, g):
-        raise ValueError("weight_grad_acc needs contiguous bf16 GPU operands, M % 64 == 0, N % 8 == 0, K % 8 == 0 and g [N, K]")
+        raise ValueError("weight_grad_acc needs contiguous bf16 GPU operands, N % 8 == 0, K % 8 == 0 and g [N, K]")
     N, K = dy.shape[1], x.shape[1]
     with torch.cuda.device(dy.device):
         _C.call("lq_weight_grad_acc", dy.data_ptr(), x.data_ptr(), g.data_ptr(), dy.shape[0], N, K, _stream(dy))
@@ -769,7 +769,7 @@ def weight_grad_acc8(dy, x, q, scale, noise=None, seed: int = 0, offset: int = 0
     if noise is None and (_native or _fast()).weight_grad_acc8(dy, x, q, scale, seed, offset) is not None:
         return q
     if not _weight_grad_native_ok(dy, x, 16):
-        raise ValueError("weight_grad_acc8 needs contiguous bf16 GPU operands, M % 64 == 0, N % 8 == 0, K % 16 == 0")
+        raise ValueError("weight_grad_acc8 needs contiguous bf16 GPU operands, N % 8 == 0, K % 16 == 0")
     N, K = dy.shape[1], x.shape[1]
     _chk(q, torch.int8, "q")
     _chk(scale, torch.bfloat16, "scale")

@@ -190,7 +190,7 @@ class _PendingWeightGrad(object):
 
 def _pending_dw(grad_output, input):
     """What a Function's backward appends to dict_temp: the pending product where the library's own GEMM can form it
-    (contiguous bf16 GPU operands, a multiple of 64 tokens), the product itself otherwise."""
+    (contiguous bf16 GPU operands), the product itself otherwise."""
     if FUSED_GRADQ and ops._weight_grad_native_ok(grad_output, input):
         return _PendingWeightGrad(grad_output, input)
     return ops.weight_grad(grad_output, input)
