@@ -106,7 +106,7 @@ int lq_a16w4_dx(const void *dy, const void *codes, const void *scales, const voi
                 void *dx, int64_t M, int64_t N, int64_t K, int group, void *stream);
 
 /* The same two products with a scratch buffer the library may use (it allocates nothing itself):
- * when the output has so few 128 x 128 tiles that they would occupy less than half of the device,
+ * when the output has so few 128 x 128 tiles that they would occupy at most half of the device,
  * the reduction is cut into up to 8 slices, each workgroup writes an fp32 partial tile into the
  * workspace and a second kernel adds the slices in a fixed order (results are deterministic), adds
  * the bias and rounds to bf16. workspace: 16-byte aligned device memory of workspace_bytes bytes,
@@ -188,9 +188,9 @@ int lq_a16w4_dx_pair(const void *dy1, const void *codes1, const void *scales1, c
  * rough cost model of measured per-step times (see lq_gemm.hip); it is exposed so that callers and
  * tests can see it. No counterpart in the reference. */
 #define LQ_PLAN_GEMV 0         /* M <= 16: one GEMV launch */
-#define LQ_PLAN_GEMV_CHUNKS 1  /* 17..128 tokens: GEMV launches of 16 tokens each */
+#define LQ_PLAN_GEMV_CHUNKS 1  /* 17..32 tokens: GEMV launches of 16 tokens each */
 #define LQ_PLAN_DIRECT 2       /* weights-direct forward kernel, 128 x 256 tiles */
-#define LQ_PLAN_STAGED_128 3   /* staged kernel, 128 x 128 tiles */
+#define LQ_PLAN_STAGED_128 3   /* staged kernel, 128 x 128 tiles (forward: 32, 64 or 128 rows) */
 #define LQ_PLAN_STAGED_256 4   /* staged kernel, 256 x 128 tiles */
 #define LQ_PLAN_DIRECT_128 5   /* weights-direct forward kernel, 128 x 128 tiles */
 int lq_a16w4_plan(int backward, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int compute_units,

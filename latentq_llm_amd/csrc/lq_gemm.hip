@@ -4,8 +4,9 @@
 //   MODE_W4_DX  : dX[M,K] = dY[M,N] . deq(W)[N,K]       (same, W tile transposed on the way out of LDS)
 //   MODE_W8_DX  : dX[M,K] = dY[M,N] . (W8 * qs)[N,K]    (MODE_W4_DX with int8 codes and one bf16 scale per row n)
 //
-// (The forward pass of large grids runs the weights-direct kernel of lq_gemm_fwd.hip instead; the int8 GEMM of the
-// A8W8 layers is lq_gemm_i8.hip, dispatched from this file.)
+// (MODE_W4_FWD serves large grids whose K has an odd number of groups only. The other large grids run the
+// weights-direct kernels of lq_gemm_fwd.hip, grids of up to one workgroup per compute unit the kernel of
+// lq_gemm_staged.hip; the int8 GEMM of the A8W8 layers is lq_gemm_i8.hip, dispatched from this file.)
 //
 // Common structure. "A" is the activation-side operand, row-major with the reduction
 // dimension contiguous. "B" is the weight-side operand, presented in LDS as
@@ -661,6 +662,12 @@ long long lq_gemm_i8_256_workgroups(int M, int N);
 int lq_gemm_i8_tile_launch(const void *x8, const void *w8, const float *sx, const void *sw, bool sw_bf16, const void *bias, void *y,
                            int *acc_or_null, int M, int N, int K, int tile, int stages, hipStream_t st);
 
+// both operands staged, for few workgroups (lq_gemm_staged.hip)
+double lq_gemm_staged_plan(long long M, long long N, int groups, size_t ws_bytes, long long cus, int *rows, int *splits, int *per_split);
+int lq_gemm_staged_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y,
+                          float *partial, int M, int N, int K, int rows, int splits, int per_split, hipStream_t st,
+                          unsigned long long *clk, const char *who);
+
 // GEMV path (lq_gemv.hip)
 int lq_gemv_a16w4_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias,
                          void *y, int M, int N, int K, hipStream_t st);
@@ -682,7 +689,7 @@ static int check_w4_common(const char *who, const void *a, const void *codes, co
     return LQ_OK;
 }
 
-// Split reduction for grids that fill less than half of the compute units: the reduction is cut
+// Split reduction of the dX kernels for grids that fill less than half of the compute units: the reduction is cut
 // into up to 8 slices of an even number of steps (at least 8) so that every unit gets at most one
 // workgroup, fp32 partial tiles go to the caller's workspace, then a reduce kernel adds them. Both
 // staged tile heights are tried (128 x 128 at ~0.56 us per step, 256 x 128 at pace_big); the plan
@@ -726,68 +733,62 @@ static SplitPlan plan_split(long long M, long long C, int total_steps, size_t ws
 struct W4Plan {
     int kernel = LQ_PLAN_STAGED_128;
     int splits = 1, steps_per_split = 0;
+    int rows = 128;  // forward LQ_PLAN_STAGED_128: rows of the tile (32, 64 or 128), 128 columns
 };
 
-// Forward pass, M > 16. Rough time per 64-deep step of the three kernels without a split
-// (microseconds, measured): the weights-direct kernel (128 x 256 tiles) takes ~0.86 with one
-// workgroup on a compute unit and ~1.45 for two sharing it; the staged kernel ~0.56 per round of
-// 128 x 128 tiles and ~0.88 per round of 256 x 128 tiles (one workgroup per unit and round). The
-// weights-direct kernel with 128 x 128 tiles fits three workgroups on a unit: ~0.55-0.61 alone (the
-// more units are busy, the lower the clock: 0.55 up to three quarters of them, 0.61 with all), ~0.74
-// as soon as a few units hold two, ~1.23 for two everywhere, ~1.38 for three; a full round of the
-// staged 128 x 128 tiles likewise takes ~0.66 instead of ~0.56. The weights-direct kernels load scales and zeros four groups at a time: rows
-// must be 4-byte aligned, i.e. the number of groups per row even.
+// Forward pass, M > 16, by the number of 128 x 128 output tiles T:
+//   T <= half of the units             the staged kernel, which plans its row tile and its slices of K itself
+//                                      (1.2 to 1.6 times the speed of the weights-direct kernels there: 11.5 against
+//                                      15.0 us on 1024 x 1536 x 1536, 23.6 against 34 on 384 x 4096 x 4096; level at
+//                                      T = 144)
+//   odd number of groups per row       rules the weights-direct kernels out (they load scales and zeros four groups at
+//                                      a time, rows must be 4-byte aligned): the staged kernel up to one tile per unit,
+//                                      beyond that the kernel with weight waves and 256 x 128 tiles (4224 x 4096:
+//                                      40 against 48 us at T = 256, 70 against 66 at 384)
+//   T <= units, K >= 8192              the staged kernel's 128-row tiles, whole (4096 x 11008: 79.0 against 86.9 us at
+//                                      T = 192, 95.6 against 98.5 at 256); for shorter K the difference is small (0 to
+//                                      4 us) and the weights-direct kernel keeps them
+//   else                               one of the two weights-direct kernels, by rough time per 64-deep step
+//                                      (microseconds, measured): 128 x 256 tiles take ~0.86 with one workgroup on a
+//                                      compute unit and ~1.45 for two sharing it. The kernel with 128 x 128 tiles fits
+//                                      three workgroups on a unit: ~0.55-0.61 alone (the more units are busy, the lower
+//                                      the clock: 0.55 up to three quarters of them, 0.61 with all), ~0.74 as soon as a
+//                                      few units hold two, ~1.23 for two everywhere, ~1.38 for three.
+// Up to 32 tokens two GEMV launches of 16 are a little faster where a launch does not wait for the matrix' bytes
+// (4096 x 4096: 10.0 / 10.8 us at 17 / 32 tokens against 10.5 / 11.1; 2048 x 2048: 7.1 / 7.8 against 7.4 / 8.0); at
+// 11008 x 4096 they take 23.3 us against 15.7. One token beyond a GEMV launch keeps the GEMV (the second launch then
+// is the one-token kernel) below K = 8192, although 11008 x 4096 takes 20.0 us so against 15.7.
 static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     W4Plan out;
+    if ((M == 17 && K < 8192) || (M <= 32 && N * K <= 4096ll * 4096)) {
+        out.kernel = LQ_PLAN_GEMV_CHUNKS;
+        return out;
+    }
+    const int groups = (int)(K / LQ_GROUP);
+    const long long tiles = (M + 127) / 128 * ((N + 127) / 128);
+    if (tiles * 2 <= cus) {
+        int per = 0;
+        lq_gemm_staged_plan(M, N, groups, ws_bytes, cus, &out.rows, &out.splits, &per);
+        if (out.splits > 1) out.steps_per_split = 2 * per;
+        return out;
+    }
+    if (tiles <= cus && (groups % 2 != 0 || K >= 8192)) return out;  // whole, 128 rows
+    if (groups % 2 != 0) {
+        out.kernel = LQ_PLAN_STAGED_256;
+        return out;
+    }
     const long long wg_direct = lq_gemm_fwd_direct_workgroups((int)M, (int)N);
     const long long rem = wg_direct % (2 * cus);
-    const double est_direct = (K / LQ_GROUP) % 2 != 0 ? 1e30
-                              : 1.45 * (double)(wg_direct / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.86 : 1.45);
-    const long long cols = (N + 127) / 128;
-    const long long tiles_small = ((M + 127) / 128) * cols;
-    const double est_small = tiles_small <= cus && 4 * tiles_small > 3 * cus ? 0.66 : 0.56 * (double)((tiles_small + cus - 1) / cus);
-    const double est_big = 0.88 * (double)((((M + 255) / 256) * cols + cus - 1) / cus);
-    double est_direct128 = 1e30;
-    if ((K / LQ_GROUP) % 2 == 0) {
-        const long long wg = lq_gemm_fwd_direct128_workgroups((int)M, (int)N);
-        const long long rem128 = wg % (3 * cus);
-        const double tail = rem128 == 0 ? 0.0
-                            : 4 * rem128 <= 3 * cus ? 0.55
-                            : rem128 <= cus ? 0.61
-                            : rem128 <= 2 * cus ? 0.74 + 0.49 * (double)(rem128 - cus) / (double)cus
-                                                : 1.38;
-        est_direct128 = 1.38 * (double)(wg / (3 * cus)) + tail;
-    }
-    double step_us = est_direct;
-    out.kernel = LQ_PLAN_DIRECT;
-    if (est_direct128 < step_us) { step_us = est_direct128; out.kernel = LQ_PLAN_DIRECT_128; }
-    if (est_small < step_us) { step_us = est_small; out.kernel = LQ_PLAN_STAGED_128; }
-    if (est_big < step_us) { step_us = est_big; out.kernel = LQ_PLAN_STAGED_256; }
-    double est_gemm = step_us * (double)(K / 64 + 3) + 4.0;
-    const SplitPlan sp = plan_split(M, N, (int)(K / 64), ws_bytes, 0.88, cus);
-    if (sp.splits >= 2 && sp.est_us < est_gemm) {
-        out.kernel = sp.big ? LQ_PLAN_STAGED_256 : LQ_PLAN_STAGED_128;
-        out.splits = sp.splits;
-        out.steps_per_split = sp.steps_per_split;
-        est_gemm = sp.est_us;
-    }
-    if (M <= 128) {
-        // A few more tokens than one GEMV takes: the GEMM's 128-row tiles would be mostly padding and
-        // its grid (N/128 workgroups, each walking all of K) fills a fraction of the device, so
-        // chunks of 16 tokens through the GEMV can be faster: the first streams the weights from
-        // HBM at near memory speed, the others find them in the last-level cache. Rough costs in
-        // microseconds: a GEMV chunk takes its bytes at ~1.8 TB/s the first time (at least 6) and
-        // ~2.3 TB/s after (at least 5; measured).
-        const long long chunks = (M + 15) / 16;
-        const double bytes = (double)(N * K / 2 + N * (K / LQ_GROUP) * 4);
-        const double first_us = bytes / 1.8e6 > 6.0 ? bytes / 1.8e6 : 6.0;
-        const double next_us = bytes / 2.3e6 > 5.0 ? bytes / 2.3e6 : 5.0;
-        if (first_us + (chunks - 1) * next_us < est_gemm) {
-            out.kernel = LQ_PLAN_GEMV_CHUNKS;
-            out.splits = 1;
-            out.steps_per_split = 0;
-        }
-    }
+    const double est_direct = 1.45 * (double)(wg_direct / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.86 : 1.45);
+    const long long wg = lq_gemm_fwd_direct128_workgroups((int)M, (int)N);
+    const long long rem128 = wg % (3 * cus);
+    const double tail = rem128 == 0 ? 0.0
+                        : 4 * rem128 <= 3 * cus ? 0.55
+                        : rem128 <= cus ? 0.61
+                        : rem128 <= 2 * cus ? 0.74 + 0.49 * (double)(rem128 - cus) / (double)cus
+                                            : 1.38;
+    const double est_direct128 = 1.38 * (double)(wg / (3 * cus)) + tail;
+    out.kernel = est_direct128 < est_direct ? LQ_PLAN_DIRECT_128 : LQ_PLAN_DIRECT;
     return out;
 }
 
@@ -809,10 +810,11 @@ static W4Plan plan_dx(long long M, long long N, long long K, size_t ws_bytes, lo
     return out;
 }
 
-static int launch_split_reduce(const GemmParams &p, int splits, hipStream_t st, const char *who) {
-    const long long MC = (long long)p.M * p.C;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((MC / 8 + 255) / 256)), dim3(256), 0, st, p.partial, p.bias,
-                       (unsigned short *)p.c, MC, p.C, splits);
+static int launch_split_reduce(const float *partial, const void *bias_or_null, void *out, int64_t M, int64_t C, int splits,
+                               hipStream_t st, const char *who) {
+    const long long MC = (long long)M * C;
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((MC / 8 + 255) / 256)), dim3(256), 0, st, partial,
+                       (const unsigned short *)bias_or_null, (unsigned short *)out, MC, (int)C, splits);
     return lq_check_launch(who);
 }
 
@@ -839,19 +841,18 @@ static int a16w4_fwd_impl(const char *who, const void *x, const void *codes, con
     if (plan.kernel == LQ_PLAN_DIRECT || plan.kernel == LQ_PLAN_DIRECT_128)
         return lq_gemm_fwd_direct_launch(x, codes, scales, zeros, bias_or_null, y, (int)M, (int)N, (int)K, (hipStream_t)stream, clk,
                                          plan.kernel == LQ_PLAN_DIRECT_128);
+    if (plan.kernel == LQ_PLAN_STAGED_128) {
+        rc = lq_gemm_staged_launch(x, codes, scales, zeros, bias_or_null, y, (float *)workspace, (int)M, (int)N, (int)K, plan.rows,
+                                   plan.splits, plan.steps_per_split / 2, (hipStream_t)stream, clk, who);
+        if (rc || plan.splits < 2) return rc;
+        return launch_split_reduce((const float *)workspace, bias_or_null, y, M, N, plan.splits, (hipStream_t)stream, who);
+    }
     GemmParams p = {};
     p.clk = clk;
     p.a = x; p.b = codes; p.scales = (const unsigned short *)scales; p.zeros = (const unsigned short *)zeros;
     p.bias = (const unsigned short *)bias_or_null; p.c = y;
     p.M = (int)M; p.C = (int)N; p.R = (int)K; p.Kw = (int)K;
-    if (plan.splits >= 2) {
-        p.partial = (float *)workspace;
-        p.steps_per_split = plan.steps_per_split;
-    }
-    rc = plan.kernel == LQ_PLAN_STAGED_256 ? launch_gemm<MODE_W4_FWD, 256, 128, 2, 2>(p, (hipStream_t)stream, who)
-                                           : launch_gemm<MODE_W4_FWD, 128, 128, 2, 2>(p, (hipStream_t)stream, who);
-    if (rc || plan.splits < 2) return rc;
-    return launch_split_reduce(p, plan.splits, (hipStream_t)stream, who);
+    return launch_gemm<MODE_W4_FWD, 256, 128, 2, 2>(p, (hipStream_t)stream, who);
 }
 
 static int gate_up_impl(const char *who, const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
@@ -938,7 +939,7 @@ static int a16w4_dx_impl(const char *who, const void *dy, const void *codes, con
     rc = plan.kernel == LQ_PLAN_STAGED_256 ? launch_gemm<MODE_W4_DX, 256, 128, 2, 2>(p, (hipStream_t)stream, who)
                                            : launch_gemm<MODE_W4_DX, 128, 128, 2, 2>(p, (hipStream_t)stream, who);
     if (rc || plan.splits < 2) return rc;
-    return launch_split_reduce(p, plan.splits, (hipStream_t)stream, who);
+    return launch_split_reduce(p.partial, nullptr, dx, M, K, plan.splits, (hipStream_t)stream, who);
 }
 
 // Scratch of the entry point that allocates nothing: one array per device, part of the code object,
@@ -999,7 +1000,7 @@ extern "C" int lq_calib_gemm_clocks(int backward, const void *a, const void *cod
     const long long wg = plan.kernel == LQ_PLAN_DIRECT ? lq_gemm_fwd_direct_workgroups((int)M, (int)N)
                          : plan.kernel == LQ_PLAN_DIRECT_128 ? lq_gemm_fwd_direct128_workgroups((int)M, (int)N)
                          : plan.kernel == LQ_PLAN_STAGED_256 ? ((M + 255) / 256) * ((cols + 127) / 128)
-                                                             : ((M + 127) / 128) * ((cols + 127) / 128);
+                                                             : ((M + plan.rows - 1) / plan.rows) * ((cols + 127) / 128);
     LQ_REQUIRE(4 * wg <= clocks_capacity, "lq_calib_gemm_clocks: clocks must hold %lld values, holds %lld", 4 * wg,
                (long long)clocks_capacity);
     *workgroups = wg;
