@@ -168,6 +168,8 @@ int lq_a16w4_gate_up_silu(const void *x, const void *codes_gate, const void *sca
  *   lq_a16w4_dx_pair: dx = bf16(dY1 . deq(W1) + dY2 . deq(W2)) for two layers of one shape [N,K] fed by the same
  *     input (gate and up): one launch whose reduction runs through both products, the sum kept in fp32 (one rounding
  *     where lq_a16w4_dx followed by lq_a16w4_dx_acc has two). dy1, dy2: bf16 [M,N]; dx: bf16 [M,K]; N % 64 == 0.
+ *   lq_a16w4_dx_pair_ws: the same with a scratch buffer (16-byte aligned, used and left behind as by lq_a16w4_dx_ws), with
+ *     which the reduction of outputs of few tiles is cut into slices.
  * Shapes and alignment as lq_a16w4_dx / lq_a16w4_gate_up_silu; all outputs 16-byte aligned. */
 int lq_a16w4_gate_up_silu_save(const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
                                const void *codes_up, const void *scales_up, const void *zeros_up, void *h, void *g_out,
@@ -180,6 +182,9 @@ int lq_a16w4_dx_acc(const void *dy, const void *codes, const void *scales, const
 int lq_a16w4_dx_pair(const void *dy1, const void *codes1, const void *scales1, const void *zeros1, const void *dy2,
                      const void *codes2, const void *scales2, const void *zeros2, void *dx, int64_t M, int64_t N,
                      int64_t K, int group, void *stream);
+int lq_a16w4_dx_pair_ws(const void *dy1, const void *codes1, const void *scales1, const void *zeros1, const void *dy2,
+                        const void *codes2, const void *scales2, const void *zeros2, void *dx, int64_t M, int64_t N,
+                        int64_t K, int group, void *workspace, int64_t workspace_bytes, void *stream);
 
 /* Which kernel lq_a16w4_fwd(_ws) (backward = 0) or lq_a16w4_dx(_ws) (backward = 1) would run for a
  * shape and a workspace size, and how it would cut the reduction; launches nothing. *kernel is
@@ -230,9 +235,12 @@ int lq_a8w8_fwd_qs(const void *x, const void *w, const float *sx, const void *qs
  * (`weight_d.to(dtype) * qscales`, utils/quant.py:200-206, 239-245, 281-288) and multiplies with
  * `grad_output.mm(weight_forward)`; here it is formed tile by tile inside the GEMM and never stored.
  * dy: bf16 [M,N]; w: int8 [N,K]; qscales_bf16: bf16 [N]; dx: bf16 [M,K]; N % 64 == 0, K % 128 == 0; dy, w, dx
- * 16-byte aligned. fp32 accumulation, one bf16 rounding of the result. */
+ * 16-byte aligned. fp32 accumulation, one bf16 rounding of the result. lq_a8w8_dx_ws: with a scratch buffer, as
+ * lq_a16w4_dx_ws. */
 int lq_a8w8_dx(const void *dy, const void *w, const void *qscales_bf16, void *dx, int64_t M, int64_t N, int64_t K,
                void *stream);
+int lq_a8w8_dx_ws(const void *dy, const void *w, const void *qscales_bf16, void *dx, int64_t M, int64_t N, int64_t K,
+                  void *workspace, int64_t workspace_bytes, void *stream);
 
 /* Per-tensor symmetric activation quantizer used in front of lq_a8w8_fwd:
  *   x8 = clamp(round_half_even(x * (127/clampv)), -128, 127)

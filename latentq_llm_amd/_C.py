@@ -29,6 +29,7 @@ SIGNATURES = {
     "lq_a16w4_dequant": [_vp, _vp, _vp, _vp, _i64, _i64, _i32, _vp],
     "lq_a8w8_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "lq_a8w8_dx": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "lq_a8w8_dx_ws": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp],
     "lq_act_quant_i8": [_vp, _vp, _vp, _i64, _vp],
     "lq_act_quant_i8_dynamic": [_vp, _vp, _vp, _vp, _i64, _i64, _i32, _vp],
     "lq_act_quant_i8_per_token": [_vp, _vp, _vp, _i64, _i64, _vp],
@@ -42,6 +43,7 @@ SIGNATURES = {
     "lq_a16w4_dx_silu_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "lq_a16w4_dx_acc": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "lq_a16w4_dx_pair": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
+    "lq_a16w4_dx_pair_ws": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp],
     "lq_w8_requant": [_vp, _vp, _vp, _i64, _i64, _vp],
     "lq_residual_quant_s": [_vp, _vp, _i64, _i32, _vp],
     "lq_gradq8_quant": [_vp, _vp, _vp, _i32, _i64, _i64, _vp, _u64, _u64, _vp],

@@ -200,20 +200,23 @@ PyObject *dx_silu(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     return Py_BuildValue("NN", wrap(std::move(dg)), wrap(std::move(du)));
 }
 
-// dy1, w1 (3), dy2, w2 (3), N, K -> dx
+// dy1, w1 (3), dy2, w2 (3), N, K, workspace -> dx
 PyObject *dx_pair(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    LQ_ARGS(10)
+    LQ_ARGS(11)
     const int64_t N = integer(a[8]), K = integer(a[9]);
     const at::Tensor *d1 = bf16(a[0]), *d2 = bf16(a[4]);
     const int64_t M = rows_of(d1, N);
     W4 w1, w2;
+    void *ws;
+    int64_t ws_bytes;
     if (M <= 0 || rows_of(d2, N) != M || !w1.load(a + 1, N, K) || !w2.load(a + 5, N, K) || !same_device(d1, w1.codes) ||
-        !same_device(d1, d2) || !same_device(d1, w2.codes))
+        !same_device(d1, d2) || !same_device(d1, w2.codes) || !workspace(a[10], d1, &ws, &ws_bytes))
         return none();
     On on(*d1);
     at::Tensor dx = make_rows(*d1, K, at::kBFloat16);
-    LQ_CALL(lq_a16w4_dx_pair, d1->data_ptr(), w1.codes->data_ptr(), w1.scales->data_ptr(), w1.zeros->data_ptr(), d2->data_ptr(),
-            w2.codes->data_ptr(), w2.scales->data_ptr(), w2.zeros->data_ptr(), dx.data_ptr(), M, N, K, LQ_GROUP, on.stream);
+    LQ_CALL(lq_a16w4_dx_pair_ws, d1->data_ptr(), w1.codes->data_ptr(), w1.scales->data_ptr(), w1.zeros->data_ptr(), d2->data_ptr(),
+            w2.codes->data_ptr(), w2.scales->data_ptr(), w2.zeros->data_ptr(), dx.data_ptr(), M, N, K, LQ_GROUP, ws,
+            ws_bytes, on.stream);
     return wrap(std::move(dx));
 }
 
@@ -262,17 +265,20 @@ PyObject *infer8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     return wrap(std::move(y));
 }
 
-// dy, w8, qscales -> dx
+// dy, w8, qscales, workspace -> dx
 PyObject *dx8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    LQ_ARGS(3)
+    LQ_ARGS(4)
     const at::Tensor *dy = bf16(a[0]), *w = plain(a[1], at::kChar), *qs = bf16(a[2]);
     if (!dy || !w || !qs || w->dim() != 2 || w->numel() == 0) return none();
     const int64_t N = w->size(0), K = w->size(1), M = rows_of(dy, N);
-    if (M <= 0 || qs->numel() != N || N % 64 || K % 128 || !aligned16(dy) || !aligned16(w) || !same_device(dy, w) || !same_device(dy, qs))
+    void *ws;
+    int64_t ws_bytes;
+    if (M <= 0 || qs->numel() != N || N % 64 || K % 128 || !aligned16(dy) || !aligned16(w) || !same_device(dy, w) || !same_device(dy, qs) ||
+        !workspace(a[3], dy, &ws, &ws_bytes))
         return none();
     On on(*dy);
     at::Tensor dx = make_rows(*dy, K, at::kBFloat16);
-    LQ_CALL(lq_a8w8_dx, dy->data_ptr(), w->data_ptr(), qs->data_ptr(), dx.data_ptr(), M, N, K, on.stream);
+    LQ_CALL(lq_a8w8_dx_ws, dy->data_ptr(), w->data_ptr(), qs->data_ptr(), dx.data_ptr(), M, N, K, ws, ws_bytes, on.stream);
     return wrap(std::move(dx));
 }
 

@@ -79,7 +79,8 @@ struct GemmParams {
     const unsigned short *ep_g, *ep_u;
     unsigned short *c2;
     // MODE_W4_DX, two products into one output: c = a * deq(b) + a2 * deq(b2), both pairs of the shape (M, R) x (R, C).
-    // The reduction runs over the first pair's R / 64 steps and then over the second's; a2 = null: one product.
+    // The reduction runs over the first pair's R / 64 steps and then over the second's (a split reduction cuts the whole
+    // of it); a2 = null: one product.
     const void *a2, *b2;
     const unsigned short *scales2, *zeros2;
 };
@@ -178,9 +179,11 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
     const int m0 = tile_m * BM, c0 = tile_n * BN;
     // reduction steps of this workgroup: all of them, or one slice of a split reduction
     const int k0 = p.partial ? (int)blockIdx.y * p.steps_per_split : 0;
-    const bool pair = MODE == MODE_W4_DX && p.a2 != nullptr;  // never together with a split reduction
+    const bool pair = MODE == MODE_W4_DX && p.a2 != nullptr;
     const int n1 = p.R / RT;                                  // steps of the first (or only) product
-    const int nk = p.partial ? (n1 - k0 < p.steps_per_split ? n1 - k0 : p.steps_per_split) : pair ? 2 * n1 : n1;
+    const int n_all = pair ? 2 * n1 : n1;
+    const int nk = p.partial && n_all - k0 < p.steps_per_split ? n_all - k0 : p.partial ? p.steps_per_split : n_all;
+    const int n_first = n1 - k0;  // pair: from this step of the workgroup on it is the second product
     const int groups_per_row = p.Kw / LQ_GROUP;
 
     if (is_weight_wave) {
@@ -225,9 +228,9 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
             s_src[0] = p.scales + ((long long)k0 * 64 + b_row) * groups_per_row + g;
             z_src[0] = p.zeros + ((long long)k0 * 64 + b_row) * groups_per_row + g;
             if (pair) {
-                b_src2 = (const unsigned char *)p.b2 + (long long)b_row * (p.Kw / 2) + c0 / 2 + b_w0 * 16;
-                s_src2 = p.scales2 + (long long)b_row * groups_per_row + g;
-                z_src2 = p.zeros2 + (long long)b_row * groups_per_row + g;
+                b_src2 = (const unsigned char *)p.b2 + ((long long)k0 * 64 + b_row) * (p.Kw / 2) + c0 / 2 + b_w0 * 16;
+                s_src2 = p.scales2 + ((long long)k0 * 64 + b_row) * groups_per_row + g;
+                z_src2 = p.zeros2 + ((long long)k0 * 64 + b_row) * groups_per_row + g;
             }
         }
 
@@ -262,7 +265,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
                 for (int i = 0; i < 4; ++i) { S.w[i] = v0[i]; S.w[4 + i] = v1[i]; }
                 S.s[0] = s_src[0][row_off];
             } else {
-                const bool second = kt >= n1 && pair;
+                const bool second = kt >= n_first && pair;
                 const long long row_off = (long long)(second ? kt - n1 : kt) * 64;
                 u32x4_t v = *reinterpret_cast<const u32x4_t *>((second ? b_src2 : b_src[0]) + row_off * (p.Kw / 2));
 #pragma unroll
@@ -353,7 +356,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
         a_off[i] = (unsigned)((gr - m0) * lda + ch * 16);
     }
     const unsigned char *a_base = (const unsigned char *)p.a + m0 * lda + (long long)k0 * ROWB;
-    const unsigned char *a_base2 = pair ? (const unsigned char *)p.a2 + m0 * lda : a_base;
+    const unsigned char *a_base2 = pair ? (const unsigned char *)p.a2 + m0 * lda + (long long)k0 * ROWB : a_base;
     // LDS-direct load: lane l of the wave writes 16 bytes at (wave-uniform base) + 16*l. Written as
     // inline assembly (M0 = LDS base, one wait state, then the load with a scalar base and a 32-bit
     // lane offset) so that the compiler's wait-count insertion does not see an LDS write it cannot
@@ -362,7 +365,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
     static_assert(APT % 4 == 0, "A loads are issued in four parts per tile");
     // part q (0..3) of a tile's loads: APT/4 of them
     auto issue_a_part = [&](int kt, unsigned char *la, int q) {
-        const bool second = kt >= n1 && pair;
+        const bool second = kt >= n_first && pair;
         const unsigned long long addr = (unsigned long long)((second ? a_base2 : a_base) + (long long)(second ? kt - n1 : kt) * ROWB);
         // the load takes its base from scalar registers
         const unsigned char *src = (const unsigned char *)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(addr >> 32)) << 32) |
@@ -618,7 +621,7 @@ int launch_gemm(GemmParams p, hipStream_t st, const char *who) {
     auto kern = gemm_kernel<MODE, BM, BN, WM, WN>;
     const long long nwg = (long long)p.tiles_m * p.tiles_n;
     if (nwg > 0x7FFFFFFFll) return lq_fail(LQ_ERR_BAD_ARG, "%s: problem too large", who);
-    const int total_steps = p.R / 64;
+    const int total_steps = p.R / 64 * (p.a2 ? 2 : 1);
     const unsigned splits = p.partial ? (unsigned)((total_steps + p.steps_per_split - 1) / p.steps_per_split) : 1u;
     hipLaunchKernelGGL(kern, dim3((unsigned)nwg, splits), dim3(128 * WM * WN), 0, st, p);
     return lq_check_launch(who);
@@ -792,12 +795,18 @@ static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, l
     return out;
 }
 
-// dX: rounds of one workgroup per compute unit at ~0.54 us per 64-deep step for 128 x 128 tiles,
-// ~0.75 for 256 x 128 (a second small-tile workgroup on the same unit adds its full time), or a split reduction.
+// dX: rounds of one workgroup per compute unit at ~0.54 us per 64-deep step for 128 x 128 tiles (0.62 in a last round that
+// fills more than three quarters of the units: 1024 x 4096 x 4096 takes 44.5 us), ~0.75 for 256 x 128 (a second small-tile
+// workgroup on the same unit adds its full time), or a split reduction. Two products into one output (lq_a16w4_dx_pair_ws)
+// are planned as one over twice the rows of W. Unsplit -> this plan, weights from HBM, us (M x N x K, output M x K):
+//   pair of 5504 x 2048   100 tokens 94 -> 21, 500: 98 -> 38, 1000: 100 -> 56
+//   pair of 11008 x 4096  256 tokens 193 -> 57, 512: 194 -> 94, 1024: 212 -> 172; 2048 stays whole (316 against 338)
+//   int8 8192 x 2048      64 tokens 68 -> 17, 512: 79 -> 32, 1024: 84 -> 45, 2048: 91 -> 74
 static W4Plan plan_dx(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     W4Plan out;
-    const long long cols = (K + 127) / 128;
-    const double est_small = 0.54 * (double)((((M + 127) / 128) * cols + cus - 1) / cus);
+    const long long cols = (K + 127) / 128, small = (M + 127) / 128 * cols, last = small % cus;
+    const double pace_last = last == 0 || 4 * last > 3 * cus ? 0.62 : 0.54;
+    const double est_small = 0.54 * (double)((small + cus - 1) / cus - 1) + pace_last;
     const double est_big = 0.75 * (double)((((M + 255) / 256) * cols + cus - 1) / cus);
     out.kernel = est_small < est_big ? LQ_PLAN_STAGED_128 : LQ_PLAN_STAGED_256;
     const double est_gemm = (est_small < est_big ? est_small : est_big) * (double)(N / 64 + 3) + 4.0;
@@ -909,6 +918,18 @@ extern "C" int lq_a16w4_fwd_ws(const void *x, const void *codes, const void *sca
                           workspace && workspace_bytes > 0 ? (size_t)workspace_bytes : 0, stream);
 }
 
+// A planned dX product: the GEMM, and the sum of its slices if the reduction is cut
+template <int MODE>
+static int launch_dx(GemmParams p, const W4Plan &plan, void *workspace, hipStream_t st, const char *who) {
+    if (plan.splits >= 2) {
+        p.partial = (float *)workspace;
+        p.steps_per_split = plan.steps_per_split;
+    }
+    const int rc = plan.kernel == LQ_PLAN_STAGED_256 ? launch_gemm<MODE, 256, 128, 2, 2>(p, st, who) : launch_gemm<MODE, 128, 128, 2, 2>(p, st, who);
+    if (rc || plan.splits < 2) return rc;
+    return launch_split_reduce(p.partial, nullptr, p.c, p.M, p.C, plan.splits, st, who);
+}
+
 struct DxEpilogue {
     int mode = EP_STORE;
     const void *g = nullptr, *u = nullptr;
@@ -932,14 +953,7 @@ static int a16w4_dx_impl(const char *who, const void *dy, const void *codes, con
     p.c = dx;
     p.M = (int)M; p.C = (int)K; p.R = (int)N; p.Kw = (int)K;
     const W4Plan plan = plan_dx(M, N, K, workspace ? ws_bytes : 0, lq_device_cu_count());
-    if (plan.splits >= 2) {
-        p.partial = (float *)workspace;
-        p.steps_per_split = plan.steps_per_split;
-    }
-    rc = plan.kernel == LQ_PLAN_STAGED_256 ? launch_gemm<MODE_W4_DX, 256, 128, 2, 2>(p, (hipStream_t)stream, who)
-                                           : launch_gemm<MODE_W4_DX, 128, 128, 2, 2>(p, (hipStream_t)stream, who);
-    if (rc || plan.splits < 2) return rc;
-    return launch_split_reduce(p.partial, nullptr, dx, M, K, plan.splits, (hipStream_t)stream, who);
+    return launch_dx<MODE_W4_DX>(p, plan, workspace, (hipStream_t)stream, who);
 }
 
 // Scratch of the entry point that allocates nothing: one array per device, part of the code object,
@@ -1043,23 +1057,36 @@ extern "C" int lq_a16w4_dx_acc(const void *dy, const void *codes, const void *sc
 // dx = dy1 * deq(W1) + dy2 * deq(W2) for two layers of the same shape that share their input (gate and up of an MLP
 // block): one launch whose reduction runs through the first product and on into the second, the sum kept in the fp32
 // accumulators (one rounding to bf16 where lq_a16w4_dx followed by lq_a16w4_dx_acc has two).
-extern "C" int lq_a16w4_dx_pair(const void *dy1, const void *codes1, const void *scales1, const void *zeros1, const void *dy2,
-                                const void *codes2, const void *scales2, const void *zeros2, void *dx, int64_t M, int64_t N,
-                                int64_t K, int group, void *stream) {
-    const char *who = "lq_a16w4_dx_pair";
+static int dx_pair_impl(const char *who, const void *dy1, const void *codes1, const void *scales1, const void *zeros1, const void *dy2,
+                        const void *codes2, const void *scales2, const void *zeros2, void *dx, int64_t M, int64_t N, int64_t K,
+                        int group, void *workspace, size_t ws_bytes, void *stream) {
     int rc = check_w4_common(who, dy1, codes1, scales1, zeros1, dx, M, N, K, group);
     if (rc) return rc;
     rc = check_w4_common(who, dy2, codes2, scales2, zeros2, dx, M, N, K, group);
     if (rc) return rc;
     LQ_REQUIRE(N % 64 == 0, "%s: N=%lld must be a multiple of 64", who, (long long)N);
+    LQ_REQUIRE(!workspace || lq_aligned(workspace, 16), "%s: the workspace must be 16-byte aligned", who);
     GemmParams p = {};
     p.a = dy1; p.b = codes1; p.scales = (const unsigned short *)scales1; p.zeros = (const unsigned short *)zeros1;
     p.a2 = dy2; p.b2 = codes2; p.scales2 = (const unsigned short *)scales2; p.zeros2 = (const unsigned short *)zeros2;
     p.c = dx;
     p.M = (int)M; p.C = (int)K; p.R = (int)N; p.Kw = (int)K;
-    const W4Plan plan = plan_dx(M, N, K, 0, lq_device_cu_count());
-    return plan.kernel == LQ_PLAN_STAGED_256 ? launch_gemm<MODE_W4_DX, 256, 128, 2, 2>(p, (hipStream_t)stream, who)
-                                             : launch_gemm<MODE_W4_DX, 128, 128, 2, 2>(p, (hipStream_t)stream, who);
+    // planned as one product over 2 N
+    return launch_dx<MODE_W4_DX>(p, plan_dx(M, 2 * N, K, workspace ? ws_bytes : 0, lq_device_cu_count()), workspace, (hipStream_t)stream, who);
+}
+
+extern "C" int lq_a16w4_dx_pair(const void *dy1, const void *codes1, const void *scales1, const void *zeros1, const void *dy2,
+                                const void *codes2, const void *scales2, const void *zeros2, void *dx, int64_t M, int64_t N,
+                                int64_t K, int group, void *stream) {
+    return dx_pair_impl("lq_a16w4_dx_pair", dy1, codes1, scales1, zeros1, dy2, codes2, scales2, zeros2, dx, M, N, K, group, nullptr, 0,
+                        stream);
+}
+
+extern "C" int lq_a16w4_dx_pair_ws(const void *dy1, const void *codes1, const void *scales1, const void *zeros1, const void *dy2,
+                                   const void *codes2, const void *scales2, const void *zeros2, void *dx, int64_t M, int64_t N,
+                                   int64_t K, int group, void *workspace, int64_t workspace_bytes, void *stream) {
+    return dx_pair_impl("lq_a16w4_dx_pair_ws", dy1, codes1, scales1, zeros1, dy2, codes2, scales2, zeros2, dx, M, N, K, group, workspace,
+                        workspace && workspace_bytes > 0 ? (size_t)workspace_bytes : 0, stream);
 }
 
 extern "C" int lq_a16w4_dx_silu_bwd(const void *dh_dy, const void *codes, const void *scales, const void *zeros, const void *g,
@@ -1082,8 +1109,8 @@ extern "C" int lq_a16w4_dx_ws(const void *dy, const void *codes, const void *sca
 
 // dX of an 8-bit-weight layer straight from the int8 codes: the staged dX kernel with the weight waves forming
 // bf16(w8 * qs[n]) instead of dequantising int4 groups.
-extern "C" int lq_a8w8_dx(const void *dy, const void *w, const void *qscales_bf16, void *dx, int64_t M, int64_t N, int64_t K,
-                          void *stream) {
+extern "C" int lq_a8w8_dx_ws(const void *dy, const void *w, const void *qscales_bf16, void *dx, int64_t M, int64_t N, int64_t K,
+                             void *workspace, int64_t workspace_bytes, void *stream) {
     LQ_REQUIRE(dy && w && qscales_bf16 && dx, "lq_a8w8_dx: null pointer argument");
     LQ_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) && N * K < (1ll << 40),
                "lq_a8w8_dx: M, N, K must be positive (M=%lld N=%lld K=%lld)", (long long)M, (long long)N, (long long)K);
@@ -1093,9 +1120,14 @@ extern "C" int lq_a8w8_dx(const void *dy, const void *w, const void *qscales_bf1
     GemmParams p = {};
     p.a = dy; p.b = w; p.scales = (const unsigned short *)qscales_bf16; p.c = dx;
     p.M = (int)M; p.C = (int)K; p.R = (int)N; p.Kw = (int)K;
-    const W4Plan plan = plan_dx(M, N, K, 0, lq_device_cu_count());
-    return plan.kernel == LQ_PLAN_STAGED_256 ? launch_gemm<MODE_W8_DX, 256, 128, 2, 2>(p, (hipStream_t)stream, "lq_a8w8_dx")
-                                             : launch_gemm<MODE_W8_DX, 128, 128, 2, 2>(p, (hipStream_t)stream, "lq_a8w8_dx");
+    LQ_REQUIRE(!workspace || lq_aligned(workspace, 16), "lq_a8w8_dx: the workspace must be 16-byte aligned");
+    const size_t ws_bytes = workspace && workspace_bytes > 0 ? (size_t)workspace_bytes : 0;
+    return launch_dx<MODE_W8_DX>(p, plan_dx(M, N, K, ws_bytes, lq_device_cu_count()), workspace, (hipStream_t)stream, "lq_a8w8_dx");
+}
+
+extern "C" int lq_a8w8_dx(const void *dy, const void *w, const void *qscales_bf16, void *dx, int64_t M, int64_t N, int64_t K,
+                          void *stream) {
+    return lq_a8w8_dx_ws(dy, w, qscales_bf16, dx, M, N, K, nullptr, 0, stream);
 }
 
 static int a8w8_fwd_impl(const void *x, const void *w, const float *sx, const void *sw, bool sw_bf16, const void *bias_or_null,

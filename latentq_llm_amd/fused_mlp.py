@@ -57,7 +57,7 @@ class _FusedMLPTrain(torch.autograd.Function):
         dg, du = ops.a16w4_dx_silu_bwd(dy, *_w4(down), (mlp.outfeatures, inter), g, u)
         dx = None
         if ctx.needs_input_grad[0]:
-            dx = ops.a16w4_dx_pair(dg, _w4(gate), du, _w4(up), (inter, K))
+            dx = ops.a16w4_dx_pair(dg, _w4(gate), du, _w4(up), (inter, K), split=True)
         for layer, dyl, xin in ((down, dy, h), (up, du, x2), (gate, dg, x2)):
             if layer.hook_handle is not None:
                 dict_temp.append(_pending_dw(dyl, xin))

@@ -289,12 +289,13 @@ def a16w4_dx(dy, codes, scales, zeros, shape, out=None, accumulate=False):
     return dx
 
 
-def a16w4_dx_pair(dy1, w1, dy2, w2, shape, out=None):
+def a16w4_dx_pair(dy1, w1, dy2, w2, shape, out=None, split: bool = False):
     """dX[M,K] = bf16(dY1 . deq(W1) + dY2 . deq(W2)) in one launch (lq_a16w4_dx_pair); w1, w2 = (codes, scales, zeros)
-    of two [N, K] matrices."""
+    of two [N, K] matrices. split: outputs of few tiles may cut the reduction into slices (lq_a16w4_dx_pair_ws)."""
     N, K = shape
+    split = split and out is None and dy1.is_cuda and dy1.dim() == 2
     if out is None and dy1.dim() == 2:
-        r = (_native or _fast()).dx_pair(dy1, *w1, dy2, *w2, N, K)
+        r = (_native or _fast()).dx_pair(dy1, *w1, dy2, *w2, N, K, _workspace(dy1, dy1.shape[0], K)[0] if split else None)
         if r is not None:
             return r
     for name, dy, w in (("dy1", dy1, w1), ("dy2", dy2, w2)):
@@ -412,7 +413,8 @@ def a8w8_dx_ok(dy, w8, qscales):
 def a8w8_dx(dy, w8, qscales):
     """dX[M,K] = dY[M,N] . bf16(W8 * qscales)[N,K] from the int8 codes (lq_a8w8_dx)."""
     if dy.dim() == 2:
-        dx = (_native or _fast()).dx8(dy, w8, qscales)
+        ws = _workspace(dy, dy.shape[0], w8.shape[1])[0] if dy.is_cuda and w8.dim() == 2 else None
+        dx = (_native or _fast()).dx8(dy, w8, qscales, ws)
         if dx is not None:
             return dx
     if not a8w8_dx_ok(dy, w8, qscales):
