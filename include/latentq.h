@@ -271,6 +271,15 @@ int lq_act_quant_i8_dynamic(const void *x, int8_t *x8, float *sx, float *work, i
  * x: bf16[M,K], 16-byte aligned, K % 8 == 0; x8: int8[M,K]; sx: fp32[M]. */
 int lq_act_quant_i8_per_token(const void *x, int8_t *x8, float *sx, int64_t M, int64_t K, void *stream);
 
+/* The forward of an 8-bit layer on a few tokens as one launch, the activation quantiser included:
+ *   per_token == 0: lq_act_quant_i8_dynamic (alpha_bf16 = 0) followed by lq_a8w8_fwd_qs, the same bits;
+ *   per_token != 0: lq_act_quant_i8_per_token followed by lq_a8w8_fwd_qs, the same bits.
+ * x: bf16[M,K]; w: int8[N,K]; qscales: bf16[N]; y: bf16[M,N]; x, w, y 16-byte aligned. It takes up to 16 tokens whose int8
+ * form fits the kernel's LDS: lq_a8w8_infer_takes says whether (1) or not (0); other sizes are refused. */
+int lq_a8w8_infer_takes(int64_t M, int64_t N, int64_t K);
+int lq_a8w8_infer(const void *x, const void *w, const void *qscales_bf16, const void *bias_or_null, void *y, int per_token,
+                  int64_t M, int64_t N, int64_t K, void *stream);
+
 /* The quantised activations back as bf16 for the backward pass: out[m,k] = bf16(x8[m,k] * bf16(s)), s = scale[m]
  * (per_token != 0) or scale[0]: the values of `x8.to(dtype) * scale.to(dtype)` that the training Function's backward
  * multiplies dY^T with (utils/quant.py:277-280) as one pass instead of two tensor operations. x8: int8 [M,K], 16-byte

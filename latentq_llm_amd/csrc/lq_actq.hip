@@ -4,41 +4,9 @@
 //   lq_act_quant_i8_per_token one scale per token row from the row's absolute maximum (one pass over HBM)
 // and, for the backward passes, lq_act_dequant_i8 (int8 -> bf16) and lq_act_fake_quant (bf16 -> bf16 on the int8 grid)
 #include "lq_common.h"
+#include "lq_actq_math.h"
 
 namespace {
-
-// x8 = clamp(rne(bf16(bf16(x * 127) / clampv)), -128, 127); 8 elements per thread.
-// The clamp value is the maximum of a bf16 tensor in every use the reference makes of it, i.e. a bf16 number;
-// the quotient of two bf16 numbers keeps 2^-17 (relative) from every bf16 rounding tie, so bf16(a / c) is
-// bf16(a * RN(1/c)) (kFast: c has no bits below bf16's and 2^-40 <= |c| <= 2^40; decided once per launch's
-// uniform value, any other clamp value takes the division). clamp(rint(q), -128, 127) is sat_u8(rne(q + 128)) - 128:
-// q is a bf16 number, so the sum is exact wherever it matters. A NaN becomes 0 (what the tensor library's
-// float -> int8 conversion makes of it); the byte conversion would make it -128, so 8 inputs with a NaN among
-// them take the slow form.
-template <bool kFast>
-__device__ __forceinline__ u32x2_t act_quant8(const u32x4_t v, float c, float r) {
-    unsigned w[2] = {0u, 0u};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float f = (j & 1) ? lq_bf16_hi(v[j >> 1]) : lq_bf16_lo(v[j >> 1]);
-        const float a = lq_bf16r(f * 127.0f);
-        if (kFast) {
-            const float q = lq_bf16r(a * r) + 128.0f;
-            switch (j & 3) {
-                case 0: w[j >> 2] = act_cvt_pk_u8<0>(q, w[j >> 2]); break;
-                case 1: w[j >> 2] = act_cvt_pk_u8<1>(q, w[j >> 2]); break;
-                case 2: w[j >> 2] = act_cvt_pk_u8<2>(q, w[j >> 2]); break;
-                default: w[j >> 2] = act_cvt_pk_u8<3>(q, w[j >> 2]); break;
-            }
-        } else {
-            const float q = lq_bf16r(a / c);
-            const float rr = q == q ? __builtin_amdgcn_fmed3f(rintf(q), -128.0f, 127.0f) : 0.0f;
-            w[j >> 2] |= ((unsigned)(int)rr & 0xFFu) << (8 * (j & 3));
-        }
-    }
-    if (kFast) return u32x2_t{w[0] ^ 0x80808080u, w[1] ^ 0x80808080u};
-    return u32x2_t{w[0], w[1]};
-}
 
 // The 8 elements from `base` on, for the clamp value c (uniform over the launch).
 __device__ __forceinline__ void act_quant_piece(const unsigned short *__restrict__ x, signed char *__restrict__ x8, long long base,
@@ -46,15 +14,7 @@ __device__ __forceinline__ void act_quant_piece(const unsigned short *__restrict
     if (base >= n) return;
     if (base + 8 <= n && (((uintptr_t)(x + base)) & 15) == 0 && (((uintptr_t)(x8 + base)) & 7) == 0) {
         const u32x4_t v = *reinterpret_cast<const u32x4_t *>(x + base);
-        const bool c_is_bf16 = (__float_as_uint(c) & 0xFFFFu) == 0u && fabsf(c) >= 0x1p-40f && fabsf(c) <= 0x1p40f;
-        // a NaN among the 8 inputs: the two forms differ on it (see above)
-        bool any_nan = false;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) any_nan |= (v[j] & 0x7FFFu) > 0x7F80u || (v[j] & 0x7FFF0000u) > 0x7F800000u;
-        u32x2_t o;
-        if (c_is_bf16 && !any_nan) o = act_quant8<true>(v, c, 1.0f / c);
-        else o = act_quant8<false>(v, c, 0.0f);
-        *reinterpret_cast<u32x2_t *>(x8 + base) = o;
+        *reinterpret_cast<u32x2_t *>(x8 + base) = act_quant8_any(v, c);
     } else {
         for (long long i = base; i < n && i < base + 8; ++i) {
             float f = lq_bf16_bits_to_f32(x[i]);
@@ -73,28 +33,6 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const unsigned short *__
 }
 
 // ---- the tensor's own maximum as clamp value ---------------------------------------------------
-// Order-preserving 16-bit key of a bf16 pattern: a larger value has a larger key, -0 < +0, and every NaN has the
-// largest key of all, so that an integer maximum over the keys is the tensor library's max(), which returns NaN as
-// soon as one element is NaN.
-__device__ __forceinline__ unsigned max_key(unsigned b) {
-    const unsigned a = b & 0x7FFFu;
-    const unsigned k = (b & 0x8000u) ? 0x7FFFu - a : 0x8000u | a;
-    return a > 0x7F80u ? 0xFFFFu : k;
-}
-__device__ __forceinline__ float max_key_value(unsigned k) {
-    const unsigned b = k == 0xFFFFu ? 0x7FC0u : (k & 0x8000u) ? (k & 0x7FFFu) : 0x8000u | (0x7FFFu - k);
-    return __uint_as_float(b << 16);
-}
-
-__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        const unsigned other = (unsigned)__shfl_xor((int)v, o, 64);
-        v = v > other ? v : other;
-    }
-    return v;
-}
-
 // Maximum over a workgroup of 256 threads, returned to every thread.
 __device__ __forceinline__ unsigned wg_max_u32(unsigned v, unsigned *red) {
     v = wave_max_u32(v);
@@ -115,12 +53,7 @@ __global__ __launch_bounds__(256) void tensor_max_kernel(const unsigned short *_
     const u32x4_t *x16 = reinterpret_cast<const u32x4_t *>(x);
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
         const u32x4_t v = x16[i];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const unsigned lo = max_key(v[j] & 0xFFFFu), hi = max_key(v[j] >> 16);
-            k = k > lo ? k : lo;
-            k = k > hi ? k : hi;
-        }
+        k = max_key8(v, k);
     }
     if (blockIdx.x == 0 && (long long)threadIdx.x < n - n8 * 8) {
         const unsigned t = max_key(x[n8 * 8 + threadIdx.x]);
@@ -171,15 +104,7 @@ __global__ __launch_bounds__(256) void act_quant_token_kernel(const unsigned sho
     const int n16 = K / 8, T = (n16 + 63) / 64;
     u32x4_t v[PT];
     unsigned amax = 0u;
-    auto take = [&](const u32x4_t &w) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const unsigned a = w[j] & 0x7FFF7FFFu;
-            const unsigned lo = a & 0xFFFFu, hi = a >> 16;
-            amax = amax > lo ? amax : lo;
-            amax = amax > hi ? amax : hi;
-        }
-    };
+    auto take = [&](const u32x4_t &w) { amax = act_amax8(w, amax); };
 #pragma unroll
     for (int t = 0; t < PT; ++t) {
         const int i = lane + 64 * t;
@@ -196,17 +121,7 @@ __global__ __launch_bounds__(256) void act_quant_token_kernel(const unsigned sho
     const float am = __uint_as_float(amax << 16);
     const float inv = am == 0.0f ? 0.0f : 127.0f / am;
     if (lane == 0) sx[m] = am / 127.0f;
-    auto quant = [&](const u32x4_t &w) {
-        unsigned o[2] = {0u, 0u};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float f = (j & 1) ? lq_bf16_hi(w[j >> 1]) : lq_bf16_lo(w[j >> 1]);
-            const float r = rintf(f * inv);
-            const float rr = r == r ? __builtin_amdgcn_fmed3f(r, -128.0f, 127.0f) : 0.0f;
-            o[j >> 2] |= ((unsigned)(int)rr & 0xFFu) << (8 * (j & 3));
-        }
-        return u32x2_t{o[0], o[1]};
-    };
+    auto quant = [&](const u32x4_t &w) { return act_quant8_token(w, inv); };
 #pragma unroll
     for (int t = 0; t < PT; ++t) {
         const int i = lane + 64 * t;

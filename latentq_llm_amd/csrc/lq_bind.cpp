@@ -252,7 +252,12 @@ PyObject *infer8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     const void *bias;
     if (M <= 0 || K % 8 || qs->numel() != N || !bias_of(a[3], N, &bias) || !same_device(x, w) || !same_device(x, qs)) return none();
     On on(*x);
-    at::Tensor x8 = make(x->sizes(), at::kChar, *x), sx = make({M}, at::kFloat, *x), y = make_rows(*x, N, at::kBFloat16);
+    at::Tensor y = make_rows(*x, N, at::kBFloat16);
+    if (aligned16(x) && aligned16(w) && lq_a8w8_infer_takes(M, N, K)) {
+        LQ_CALL(lq_a8w8_infer, x->data_ptr(), w->data_ptr(), qs->data_ptr(), bias, y.data_ptr(), a[4] == Py_True, M, N, K, on.stream);
+        return wrap(std::move(y));
+    }
+    at::Tensor x8 = make(x->sizes(), at::kChar, *x), sx = make({M}, at::kFloat, *x);
     if (a[4] == Py_True) {
         LQ_CALL(lq_act_quant_i8_per_token, x->data_ptr(), (int8_t *)x8.data_ptr(), (float *)sx.data_ptr(), M, K, on.stream);
     } else {

@@ -665,6 +665,10 @@ long long lq_gemm_i8_256_workgroups(int M, int N);
 int lq_gemm_i8_tile_launch(const void *x8, const void *w8, const float *sx, const void *sw, bool sw_bf16, const void *bias, void *y,
                            int *acc_or_null, int M, int N, int K, int tile, int stages, hipStream_t st);
 
+// int8 product of up to 32 tokens (lq_gemv_i8.hip)
+int lq_gemv_i8_launch(const void *x8, const void *w8, const float *sx, const void *sw, bool sw_bf16, const void *bias, void *y,
+                      int *acc_or_null, int M, int N, int K, hipStream_t st);
+
 // both operands staged, for few workgroups (lq_gemm_staged.hip)
 double lq_gemm_staged_plan(long long M, long long N, int groups, size_t ws_bytes, long long cus, int *rows, int *splits, int *per_split);
 int lq_gemm_staged_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y,
@@ -1140,14 +1144,25 @@ static int a8w8_fwd_impl(const void *x, const void *w, const float *sx, const vo
     LQ_REQUIRE(lq_aligned(x, 16) && lq_aligned(w, 16) && lq_aligned(y, 16) && lq_aligned(sx, 4) && lq_aligned(sw, sw_bf16 ? 2 : 4) &&
                    (!acc_or_null || lq_aligned(acc_or_null, 16)),
                "lq_a8w8_fwd: x, w, y, acc must be 16-byte aligned");
+    const long long cus = lq_device_cu_count();
+    // Few tokens: 16 columns per workgroup, K shared by its waves. us against 64 x 64 and 128 x 128 tiles: 2048^2 at 17 / 32 tokens
+    // 4.7 / 5.2, 7.3 / 7.4, 10.2; 2048 x 8192 10.4 / 13.0, 13.8 / 14.2, 23.6; level with 64 x 64 tiles at 8192 x 2048 and 32
+    // tokens (two workgroups per unit, each reading all tokens), behind them from 48 tokens on (12.1 against 7.8 there).
+    if (M <= 16 || (M <= 32 && N <= 32 * cus))
+        return lq_gemv_i8_launch(x, w, sx, sw, sw_bf16, bias_or_null, y, acc_or_null, (int)M, (int)N, (int)K, (hipStream_t)stream);
+    // 64 x 64 tiles while no unit gets more than two of them: a step of a 128 x 128 tile fetches 32 KB, which takes a unit
+    // twice as long as the 16 KB of this tile, and few tiles leave units idle. us against 128 x 128 tiles: 2048^2 at 64 / 512 / 1024
+    // tokens 7.6 / 8.3 / 11.5 against 10.7 / 11.5 / 12.4, 2048 x 8192 at 128 / 512 15.5 / 17.1 against 25.3 / 26.6; with three
+    // (2048^2 at 1500) 17.1 against 12.9.
+    if (((M + 63) / 64) * ((N + 63) / 64) <= 2 * cus)
+        return lq_gemm_i8_tile_launch(x, w, sx, sw, sw_bf16, bias_or_null, y, acc_or_null, (int)M, (int)N, (int)K, 64, 4, (hipStream_t)stream);
     // 256 x 256 tiles, both operands through LDS, when they occupy more than half of the compute
     // units; below that the staged kernel's smaller tiles fill the device better
-    if (lq_gemm_i8_256_workgroups((int)M, (int)N) * 2 > (long long)lq_device_cu_count())
+    if (lq_gemm_i8_256_workgroups((int)M, (int)N) * 2 > cus)
         return lq_gemm_i8_tile_launch(x, w, sx, sw, sw_bf16, bias_or_null, y, acc_or_null, (int)M, (int)N, (int)K, 256, 2, (hipStream_t)stream);
     // the same kernel with 128 x 128 tiles (two workgroups per CU) when there are more of them than
     // compute units; measured 40.6 -> 37.0 us on 2048 x 4096 x 4096
     const long long tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
-    const long long cus = lq_device_cu_count();
     if (tiles128 > cus)
         return lq_gemm_i8_tile_launch(x, w, sx, sw, sw_bf16, bias_or_null, y, acc_or_null, (int)M, (int)N, (int)K, 128, 2, (hipStream_t)stream);
     // A workgroup with a CU to itself: four 32 KB stages (loads three steps ahead). Nothing covers such a workgroup's

@@ -280,7 +280,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) 
 long long lq_gemm_i8_256_workgroups(int M, int N) { return (long long)((M + 255) / 256) * ((N + 255) / 256); }
 
 // Called by lq_a8w8_fwd (lq_gemm.hip) after argument validation: K % 128 == 0, N % 16 == 0.
-// tile = 256 or 128 (square tiles, 8 waves each); stages = 2, or 4 with the 128 tile.
+// tile = 256 or 128 (square tiles, 8 waves each) or 64 (4 waves); stages = 2, or 4 with the 128 tile (64: always 4).
 int lq_gemm_i8_tile_launch(const void *x8, const void *w8, const float *sx, const void *sw, bool sw_bf16, const void *bias, void *y,
                            int *acc_or_null, int M, int N, int K, int tile, int stages, hipStream_t st) {
     I8Params p = {};
@@ -294,6 +294,7 @@ int lq_gemm_i8_tile_launch(const void *x8, const void *w8, const float *sx, cons
     // the 32-bit lane offsets of the loads span up to 256 rows
     if (256ll * K >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "lq_a8w8_fwd: K too large");
     if (tile == 256) hipLaunchKernelGGL((gemm_i8_tile_kernel<256, 256, 2, 4, 2>), dim3((unsigned)nwg), dim3(512), 0, st, p);
+    else if (tile == 64) hipLaunchKernelGGL((gemm_i8_tile_kernel<64, 64, 2, 2, 4>), dim3((unsigned)nwg), dim3(256), 0, st, p);
     else if (stages == 4) hipLaunchKernelGGL((gemm_i8_tile_kernel<128, 128, 2, 4, 4>), dim3((unsigned)nwg), dim3(512), 0, st, p);
     else hipLaunchKernelGGL((gemm_i8_tile_kernel<128, 128, 2, 4, 2>), dim3((unsigned)nwg), dim3(512), 0, st, p);
     return lq_check_launch("lq_a8w8_fwd");
