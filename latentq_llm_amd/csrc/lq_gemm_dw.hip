@@ -7,10 +7,20 @@
 // 16-lane block, lane i receives the four elements of column i of the 4 x 16 block the 16 lanes address. No
 // transposed copy of dY is made anywhere.
 //
-// Two tile sizes (dw_takes_small_tiles below chooses):
+// Two tile sizes (dw_takes_small_tiles below chooses) and two ways through the large one:
 //   256 (n) x 256 (k) outputs, 512 threads = 8 waves in a 2 (n) x 4 (k) grid; a wave owns 128 x 64 outputs (4 x 2 MFMA
 //     32x32x16 tiles, 128 accumulator registers). Steps of 64 tokens, two LDS stages of 64 KB (64 rows of dY and 64 rows
 //     of X, 512 bytes each); one workgroup per CU.
+//   the same tile and steps, 256 threads = 2 x 2 waves of 128 x 128 (256 accumulators, one wave per SIMD): 128 instead of
+//     192 KB of fragment reads per 64 tokens, which is power the matrix cores get. A lone wave has to issue everything
+//     between its own MFMAs, so the reads of the next slice and the loads are dealt out one or two per MFMA, the reads
+//     over the first half of a slice, and the whole old gradient is requested before the accumulating epilogue starts. us
+//     at 2048 tokens, 8 waves -> 4 (store / accumulate in bf16): 11008 x 4096 172 / 191 -> 157 / 181, 3072^2 49 / 60 -> 45 / 56;
+//     4096 tokens, 11008 x 4096 310 / 327 -> 296 / 315. The int8 accumulator's epilogue is vector work that wants two
+//     waves (196 -> 211), and with few steps a lone wave's prologue and epilogue show (300 tokens 41 / 64 -> 45 / 71, level
+//     at 1024 to 1500): those keep the 8 waves. The sums are taken in the same order, so a gradient stored and then
+//     added to an int8 accumulator still has the bits of the fused epilogue. (Steps of 32 tokens in four stages are as
+//     fast, but cut a number of tokens that is no multiple of 64 into other slices.)
 //   128 x 128 outputs, 256 threads = 2 x 2 waves of 64 x 64. Steps of 32 tokens, four stages of 16 KB, two workgroups
 //     per CU: for outputs whose large tiles leave most of the device idle. There a workgroup has nothing but its own
 //     prefetch distance to cover its waits, which is what the four stages are for (2048 x 2048 outputs, 2048 tokens:
@@ -62,11 +72,10 @@ typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 template <int I>
 using ic = std::integral_constant<int, I>;
 
-// TILE: outputs per workgroup along n and along k. 256: 8 waves of 128 x 64, one workgroup per CU. 128: 4 waves of
-// 64 x 64, two workgroups per CU. STEP_M: tokens per reduction step; NST: LDS stages of one step.
-template <int TILE, int STEP_M, int NST, bool ACC8>
-__global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwParams p) {
-    constexpr int NT = TILE == 256 ? 512 : 256;
+// TILE: outputs per workgroup along n and along k, NT: its threads. STEP_M: tokens per reduction step; NST: LDS stages of
+// one step.
+template <int TILE, int NT, int STEP_M, int NST, bool ACC8>
+__global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     constexpr int ROWB = TILE * 2;           // bytes per staged token row of one operand
     constexpr int OP_STAGE = STEP_M * ROWB;  // bytes per operand and stage
     constexpr int STAGE = 2 * OP_STAGE;
@@ -75,6 +84,8 @@ __global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwPara
     constexpr int WM = 2, WN = NT / 64 / WM;       // waves along n, along k
     constexpr int TM = TILE / WM, TN = TILE / WN;  // wave tile: 128 n x 64 k, or 64 x 64
     constexpr int FM = TM / 32, FN = TN / 32;
+    constexpr bool kLone = FM * FN == 16;  // 256 accumulators: one wave per SIMD
+    static_assert(!kLone || !ACC8, "the int8 epilogue wants two waves per SIMD");
     // the stages; the accumulate epilogue stages every wave's whole block (144-byte rows) instead
     constexpr int EP_ALL = WM * WN * TM * (TN * 2 + 16);
     constexpr int LDS_BYTES = ACC8 && EP_ALL > NST * STAGE ? EP_ALL : NST * STAGE;
@@ -166,21 +177,19 @@ __global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwPara
             f[e] &= keep;
         }
     };
+    // half e (tokens .. + 3, .. + 7) of fragment f of slice t: dY fragments 0 .. FM - 1, then X fragments
+    auto read_half = [&](const unsigned char *st, int t, u32x4_t *af, u32x4_t *bf, int f, int e) {
+        const unsigned char *base = st + row_lane + (t * 16 + 4 * e) * ROWB;
+        const u32x2_t v = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(base + (f < FM ? a_col[f < FM ? f : 0] : b_col[f >= FM ? f - FM : 0]))));
+        u32x4_t &d = f < FM ? af[f < FM ? f : 0] : bf[f >= FM ? f - FM : 0];
+        d[2 * e] = v[0];
+        d[2 * e + 1] = v[1];
+    };
     auto read_frags = [&](const unsigned char *st, int t, u32x4_t *af, u32x4_t *bf) {
-        const unsigned char *base = st + row_lane + t * 16 * ROWB;
 #pragma unroll
-        for (int j = 0; j < FM; ++j) {
-            const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(base + a_col[j]));
-            const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(base + a_col[j] + 4 * ROWB));
-            const u32x2_t l2 = __builtin_bit_cast(u32x2_t, lo), h2 = __builtin_bit_cast(u32x2_t, hi);
-            af[j] = u32x4_t{l2[0], l2[1], h2[0], h2[1]};
-        }
-#pragma unroll
-        for (int i = 0; i < FN; ++i) {
-            const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(base + b_col[i]));
-            const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(base + b_col[i] + 4 * ROWB));
-            const u32x2_t l2 = __builtin_bit_cast(u32x2_t, lo), h2 = __builtin_bit_cast(u32x2_t, hi);
-            bf[i] = u32x4_t{l2[0], l2[1], h2[0], h2[1]};
+        for (int f = 0; f < FM + FN; ++f) {
+            read_half(st, t, af, bf, f, 0);
+            read_half(st, t, af, bf, f, 1);
         }
     };
 
@@ -218,8 +227,32 @@ __global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwPara
 #pragma unroll
         for (int t = 0; t < SL; ++t) {
             if (t == SL - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * 2 * LOADS) : "memory");
-            if (t < SL - 1) read_frags(cur, t + 1, af[(t + 1) & 1], bf[(t + 1) & 1]);
-            else read_frags(nxt, 0, af[0], bf[0]);
+            const unsigned char *src = t < SL - 1 ? cur : nxt;
+            const int tn = t < SL - 1 ? t + 1 : 0;
+            if constexpr (kLone && !MASKED) {
+                // one wave per SIMD: everything else is dealt out between the MFMAs, the reads of the next slice (in the
+                // order in which it uses them) over the first half of them, so that they are back when it starts
+                static_assert(FM == FN && LOADS <= FM * FN, "one load per MFMA at most");
+#pragma unroll
+                for (int m = 0; m < FM * FN; ++m) {
+                    constexpr int kReads = 2 * (FM + FN), kPer = kReads / (FM * FN / 2);
+#pragma unroll
+                    for (int q = 0; q < kPer; ++q) {
+                        const int n = m * kPer + q;  // halves: dY 0, X 0, dY 1, X 1, ...
+                        if (n < kReads) read_half(src, tn, af[tn & 1], bf[tn & 1], (n >> 1) % 2 == 0 ? (n >> 2) : FM + (n >> 2), n & 1);
+                    }
+                    if (m % 2 == 1 && m / 2 < LOADS) {
+                        if (t == 0) load(kt_x, left, LOADS + m / 2);
+                        if (t == SL - 1) load(kt_dy, cur, m / 2);
+                    }
+                    const int i = m / FM, j = m % FM;
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, bf[t & 1][i]),
+                                                                       __builtin_bit_cast(bf16x8_t, af[t & 1][j]), acc[i][j], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                continue;
+            }
+            read_frags(src, tn, af[tn & 1], bf[tn & 1]);
             if (t == 0) {
 #pragma unroll
                 for (int i = LOADS; i < 2 * LOADS; ++i) load(kt_x, left, i);
@@ -276,43 +309,60 @@ __global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwPara
     constexpr int EP = TN * 2 + 16;  // row pitch of the staging area
     const int kw0 = k0 + wn * TN;
     if constexpr (!ACC8) {
-        // 32 rows (one j) at a time; 16 bytes per lane, 8 lanes on the 128 contiguous bytes of a row
+        // 32 rows (one j) at a time; 16 bytes per lane, TN / 8 lanes on the contiguous bytes of a row
         unsigned char *ep = lds_all + wave * (32 * EP);
-        const int ep_row = lane >> 3, ep_chunk = lane & 7;
+        constexpr int LPR = TN / 8, RPI = 64 / LPR;
+        const int ep_row = lane / LPR, ep_chunk = lane % LPR;
         const int kc = kw0 + ep_chunk * 8;
+        constexpr int IT = 32 / RPI;
+        unsigned short *const out = p.dw + (long long)(n0 + wm * TM + ep_row) * p.K + kc;
+        auto live = [&](int j, int it) { return n0 + wm * TM + j * 32 + it * RPI + ep_row < p.N && kc < p.K; };
+        auto piece = [&](int j, int it) { return reinterpret_cast<u32x4_t *>(out + (long long)(j * 32 + it * RPI) * p.K); };
+        auto emit = [&](auto accumulate) {
+            constexpr bool ACC = decltype(accumulate)::value != 0;
+            // The old gradient of the rows ahead: a lone wave has no other to cover the latency, and its fragments' registers
+            // are free by now, so it asks for the whole block at once; two waves per SIMD take 32 rows at a time.
+            constexpr int AHEAD = kLone ? FM : 1;
+            u32x4_t old[ACC ? AHEAD : 1][IT];
+            auto fetch = [&](int j) {
 #pragma unroll
-        for (int j = 0; j < FM; ++j) {
-            const int nrow0 = n0 + wm * TM + j * 32;
-#pragma unroll
-            for (int i = 0; i < FN; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const u32x2_t o = {lq_pack_bf16(acc[i][j][4 * q], acc[i][j][4 * q + 1]), lq_pack_bf16(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3])};
-                    *reinterpret_cast<u32x2_t *>(ep + r * EP + (i * 32 + 8 * q + 4 * h) * 2) = o;
+                for (int it = 0; it < IT; ++it) {
+                    old[ACC ? j % AHEAD : 0][it] = u32x4_t{0u, 0u, 0u, 0u};
+                    if (live(j, it)) old[ACC ? j % AHEAD : 0][it] = *piece(j, it);
                 }
+            };
+            if constexpr (ACC && AHEAD > 1) {
 #pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                const int row = it * 8 + ep_row;
-                const u32x4_t o = *reinterpret_cast<const u32x4_t *>(ep + row * EP + ep_chunk * 16);
-                const int nn = nrow0 + row;
-                if (nn < p.N && kc < p.K) {
-                    unsigned short *dst = p.dw + (long long)nn * p.K + kc;
-                    if (p.accumulate) {
+                for (int j = 0; j < FM; ++j) fetch(j);
+            }
+#pragma unroll
+            for (int j = 0; j < FM; ++j) {
+                if constexpr (ACC && AHEAD == 1) fetch(j);
+#pragma unroll
+                for (int i = 0; i < FN; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const u32x2_t o = {lq_pack_bf16(acc[i][j][4 * q], acc[i][j][4 * q + 1]), lq_pack_bf16(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3])};
+                        *reinterpret_cast<u32x2_t *>(ep + r * EP + (i * 32 + 8 * q + 4 * h) * 2) = o;
+                    }
+#pragma unroll
+                for (int it = 0; it < IT; ++it) {
+                    u32x4_t o = *reinterpret_cast<const u32x4_t *>(ep + (it * RPI + ep_row) * EP + ep_chunk * 16);
+                    if constexpr (ACC) {
                         // the bf16 addition a tensor `add_` of the stored product would make
-                        const u32x4_t old = *reinterpret_cast<const u32x4_t *>(dst);
-                        u32x4_t sum;
+                        const u32x4_t g = old[j % AHEAD][it];
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            sum[e] = lq_pack_bf16(lq_bf16_lo(old[e]) + lq_bf16_lo(o[e]), lq_bf16_hi(old[e]) + lq_bf16_hi(o[e]));
-                        *reinterpret_cast<u32x4_t *>(dst) = sum;
-                    } else {
-                        *reinterpret_cast<u32x4_t *>(dst) = o;
+                            o[e] = lq_pack_bf16(lq_bf16_lo(g[e]) + lq_bf16_lo(o[e]), lq_bf16_hi(g[e]) + lq_bf16_hi(o[e]));
                     }
+                    if (live(j, it)) *piece(j, it) = o;
                 }
             }
-        }
+        };
+        if (p.accumulate) emit(ic<1>());
+        else emit(ic<0>());
     } else {
-        // The whole 128 x 64 block of the wave goes to LDS as bf16 first (straight-line code), then a rolled loop of
+        // The whole block of the wave goes to LDS as bf16 first (straight-line code), then a rolled loop of
         // 8 passes of 16 rows does the accumulator arithmetic: unrolled over the accumulator registers that
         // arithmetic would be some 50 KB of code, more than the instruction cache holds. 16 consecutive k per lane
         // (one Philox block), 4 lanes per row.
@@ -326,11 +376,12 @@ __global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwPara
                     const u32x2_t o = {lq_pack_bf16(acc[i][j][4 * q], acc[i][j][4 * q + 1]), lq_pack_bf16(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3])};
                     *reinterpret_cast<u32x2_t *>(ep + (j * 32 + r) * EP + (i * 32 + 8 * q + 4 * h) * 2) = o;
                 }
-        const int q_row = lane >> 2, q_piece = lane & 3;
+        constexpr int PPR = TN / 16, RPP = 64 / PPR;  // pieces per row, rows per pass
+        const int q_row = lane / PPR, q_piece = lane % PPR;
         const int kq = kw0 + q_piece * 16;
         const int nw0 = n0 + wm * TM;
         auto fetch = [&](int pass, u32x4_t &oldq, float &sc) {
-            const int nn = nw0 + pass * 16 + q_row;
+            const int nn = nw0 + pass * RPP + q_row;
             const bool live = nn < p.N && kq < p.K;
             oldq = *reinterpret_cast<const u32x4_t *>(p.q + (live ? (long long)nn * p.K + kq : 0));
             sc = lq_bf16_bits_to_f32(p.scale[live ? nn : 0]);
@@ -339,11 +390,11 @@ __global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwPara
         float s_next;
         fetch(0, old_next, s_next);
 #pragma unroll 1
-        for (int pass = 0; pass < TM / 16; ++pass) {
+        for (int pass = 0; pass < TM / RPP; ++pass) {
             const u32x4_t oldq = old_next;
             const float sc = s_next;
-            if (pass + 1 < TM / 16) fetch(pass + 1, old_next, s_next);
-            const int row = pass * 16 + q_row;
+            if (pass + 1 < TM / RPP) fetch(pass + 1, old_next, s_next);
+            const int row = pass * RPP + q_row;
             const int nn = nw0 + row;
             const bool live = nn < p.N && kq < p.K;
             const u32x4_t v0 = *reinterpret_cast<const u32x4_t *>(ep + row * EP + q_piece * 32);
@@ -369,17 +420,16 @@ __global__ __launch_bounds__(TILE == 256 ? 512 : 256) void gemm_dw_kernel(DwPara
     }
 }
 
-template <int TILE, int STEP_M, int NST>
-static int launch_dw_tile(DwParams p, bool acc8, hipStream_t st, const char *who) {
+template <int TILE, int NT, int STEP_M, int NST, bool ACC8>
+static int launch_dw_tile(DwParams p, hipStream_t st, const char *who) {
     p.tiles_n = (p.N + TILE - 1) / TILE;
     p.tiles_k = (p.K + TILE - 1) / TILE;
     const long long nwg = (long long)p.tiles_n * p.tiles_k;
     if (nwg > 0x7FFFFFFFll) return lq_fail(LQ_ERR_BAD_ARG, "%s: problem too large", who);
     // the 32-bit lane offsets of the loads span a step's token rows
     if (64ll * 2 * (p.N > p.K ? p.N : p.K) >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: rows too long", who);
-    const dim3 grid((unsigned)nwg), block(TILE == 256 ? 512 : 256);
-    if (acc8) hipLaunchKernelGGL((gemm_dw_kernel<TILE, STEP_M, NST, true>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((gemm_dw_kernel<TILE, STEP_M, NST, false>), grid, block, 0, st, p);
+    const dim3 grid((unsigned)nwg), block(NT);
+    hipLaunchKernelGGL((gemm_dw_kernel<TILE, NT, STEP_M, NST, ACC8>), grid, block, 0, st, p);
     return lq_check_launch(who);
 }
 
@@ -403,8 +453,11 @@ static bool dw_takes_small_tiles(long long M, long long N, long long K, long lon
 }
 
 static int launch_dw(const DwParams &p, bool acc8, hipStream_t st, const char *who) {
-    return dw_takes_small_tiles(p.M, p.N, p.K, lq_device_cu_count()) ? launch_dw_tile<128, 32, 4>(p, acc8, st, who)
-                                                                       : launch_dw_tile<256, 64, 2>(p, acc8, st, who);
+    if (dw_takes_small_tiles(p.M, p.N, p.K, lq_device_cu_count()))
+        return acc8 ? launch_dw_tile<128, 256, 32, 4, true>(p, st, who) : launch_dw_tile<128, 256, 32, 4, false>(p, st, who);
+    if (acc8) return launch_dw_tile<256, 512, 64, 2, true>(p, st, who);
+    // 4 waves of 128 x 128 from where their faster steps outweigh the longer way in and out (see the top of the file)
+    return p.M >= 1536 ? launch_dw_tile<256, 256, 64, 2, false>(p, st, who) : launch_dw_tile<256, 512, 64, 2, false>(p, st, who);
 }
 
 static int check_dw(const char *who, const void *dy, const void *x, int64_t M, int64_t N, int64_t K, int k_mult) {

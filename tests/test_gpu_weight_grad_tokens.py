@@ -62,3 +62,27 @@ def test_rows_past_the_last_token_do_not_count(ops):
     buf_dy[M - 1, 3] = float("inf")
     dw = ops.weight_grad(buf_dy.cuda()[:M], buf_x.cuda()[:M])
     assert torch.isinf(dw[3]).all() and torch.equal(dw[4:], torch.full_like(dw[4:], 42.0))
+
+
+# 1536 tokens and more on 256 x 256 tiles: 4 waves of 128 x 128 where the int8 epilogue has 8 of 128 x 64; tokens of every
+# kind of first step, outputs that end inside a tile
+@pytest.mark.parametrize("M,N,K", [(1536, 2048, 4096), (1537, 2056, 4112), (1586, 3080, 3088), (1599, 4096, 2064)])
+def test_four_waves_per_tile(ops, M, N, K):
+    dy, x = randn_bf16((M, N), M).cuda(), randn_bf16((M, K), M + 1).cuda()
+    dw = ops.weight_grad(dy, x)
+    assert rel_l2(dw, dy.double().t() @ x.double()) < 2.5e-3  # as above
+    gen = torch.Generator().manual_seed(M)
+    # few enough terms that every sum is an integer bf16 holds
+    dyi = (torch.randint(-1, 2, (M, N), generator=gen) * (torch.rand((M, 1), generator=gen) < 0.1)).to(torch.bfloat16).cuda()
+    xi = torch.randint(-1, 2, (M, K), generator=gen).to(torch.bfloat16).cuda()
+    want = dyi.double().t() @ xi.double()
+    assert float(want.abs().max()) <= 256 and torch.equal(ops.weight_grad(dyi, xi).double(), want)
+    g = randn_bf16((N, K), 7).cuda()
+    want = g.clone().add_(dw)
+    assert torch.equal(ops.weight_grad_acc(dy, x, g), want)
+    q, s = torch.empty((N, K), dtype=torch.int8, device="cuda"), torch.empty((N, 1), dtype=torch.bfloat16, device="cuda")
+    ops.gradq8_quant(dw, q, s, False, seed=3, offset=0)
+    want_q = q.clone()
+    ops.gradq8_quant(dw, want_q, s, True, seed=3, offset=99)
+    ops.weight_grad_acc8(dy, x, q, s, seed=3, offset=99)
+    assert torch.equal(q, want_q)
