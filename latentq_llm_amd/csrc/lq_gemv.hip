@@ -66,8 +66,10 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
                                                           const unsigned short *__restrict__ zeros2 = nullptr) {
     static_assert(!GU || (NT == 2 && !QS), "gate / up mode: two tiles, scales and zeros straight from memory");
     constexpr int RT = GU ? 1 : NT;  // 16-row tiles of output rows per workgroup
-    __shared__ float red[WAVES][NT][4][64];
+    static_assert(MP * kXRow >= NT * 4 * 64 * 4, "a wave's partial sums fit where its activations were");
     __shared__ __attribute__((aligned(16))) unsigned char xs[WAVES][MP][kXRow];
+    // a wave's partial sums [tile][4][lane] take the place of the token rows it staged (its reads of them have returned)
+    auto red = [&](int w, int j, int r) -> float & { return reinterpret_cast<float *>(&xs[w][0][0])[(j * 4 + r) * 64 + (threadIdx.x & 63)]; };
     extern __shared__ __attribute__((aligned(16))) unsigned char sq[];  // QS: scales then zeros of the workgroup's rows
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // scalar: uniform control flow
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red[wave][j][r][lane] = acc[j][r];
+        for (int r = 0; r < 4; ++r) red(wave, j, r) = acc[j][r];
     __syncthreads();
     if constexpr (GU) {
         if (wave == 0) {
@@ -260,8 +262,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
                 float g = 0.f, u = 0.f;
 #pragma unroll
                 for (int w = 0; w < WAVES; ++w) {
-                    g += red[w][0][r][lane];
-                    u += red[w][1][r][lane];
+                    g += red(w, 0, r);
+                    u += red(w, NT - 1, r);
                 }
                 const int m = 4 * kq + r;
                 if (m < M) y[(long long)m * N + row] = lq_f32_to_bf16_bits(g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u);
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
         for (int r = 0; r < 4; ++r) {
             float v = 0.f;
 #pragma unroll
-            for (int w = 0; w < WAVES; ++w) v += red[w][wave][r][lane];
+            for (int w = 0; w < WAVES; ++w) v += red(w, wave, r);
             const int m = 4 * kq + r;
             if (m < M) y[(long long)m * N + orow] = lq_f32_to_bf16_bits(v + b);
         }
@@ -306,6 +308,39 @@ void launch_gu(const GemvGuArgs &a) {
                        (const unsigned char *)a.codes, (const unsigned short *)a.scales, (const unsigned short *)a.zeros,
                        (const unsigned short *)nullptr, (unsigned short *)a.y, a.M, a.N, a.K, (const unsigned char *)a.codes2,
                        (const unsigned short *)a.scales2, (const unsigned short *)a.zeros2);
+}
+
+// Waves per workgroup of the gate / up pass, MP staged rows. A grid of c workgroups per CU should be resident at once: the
+// staged rows (1040 MP bytes a wave) of c of them have to fit the CU's 160 KB and their waves its registers (16 of this
+// kernel). Within that the fewest rounds of batches, and the fewest waves for that number of rounds. us, 8 waves (what
+// every size took before) -> this rule, both matrices:
+//   11008 x 4096 (c = 3)  1 token 15.9 -> 14.1 (4 waves), 8: 22.7 -> 15.2 (4), 12: 23.4 -> 16.0 (4), 16: 24.0 -> 18.5 (3)
+//   8192 x 2560 (c = 2)   8: 13.0 -> 9.3 (5), 12: 13.2 -> 11.0 (3), 16: 13.5 -> 11.3 (3)
+//   6144 x 3072 (c = 2)   8: 12.4 -> 9.5 (6), 12: 12.6 -> 10.4 (3), 16: 12.8 -> 10.8 (3)
+// (12 rows and more on 5 or 6 waves are slower although two such workgroups fit: 6144 x 3072 at 12 tokens 11.7 on 6.)
+int gu_waves(int MP, int N, int batches, int cus) {
+    const int c = (N / 16 + cus - 1) / cus;
+    int most = (160 << 10) / c / (MP * kXRow);
+    if (c > 1 && most > 16 / c) most = 16 / c;
+    if (c > 1 && MP >= 12 && most > 4) most = 4;
+    if (most > (MP == 4 ? 16 : 8)) most = MP == 4 ? 16 : 8;
+    if (most < 2) most = 2;
+    const int rounds = (batches + most - 1) / most;
+    const int w = (batches + rounds - 1) / rounds;
+    return w < 2 ? 2 : w <= 6 ? w : w <= 8 ? (most >= 8 ? 8 : 6) : 16;
+}
+
+template <int MP>
+void launch_gu_waves(int w, const GemvGuArgs &a) {
+    switch (w) {
+        case 2: launch_gu<2, MP>(a); break;
+        case 3: launch_gu<3, MP>(a); break;
+        case 4: launch_gu<4, MP>(a); break;
+        case 5: launch_gu<5, MP>(a); break;
+        case 6: launch_gu<6, MP>(a); break;
+        case 8: launch_gu<8, MP>(a); break;
+        default: if constexpr (MP == 4) launch_gu<16, MP>(a); else launch_gu<8, MP>(a);
+    }
 }
 
 template <int W, int MP, int NT>
@@ -366,6 +401,9 @@ int lq_gemv_a16w4_launch(const void *x, const void *codes, const void *scales, c
         // many tokens and enough rows for one 32-row workgroup per CU: half the activation traffic;
         // 4 waves = 65 KB of staged activations: two workgroups per CU, all of them resident at once
         launch_waves<16, 2, 4>(pick_waves(batches, 4), a);
+    } else if (M <= 12 && batches > 8) {
+        // (11.4 -> 10.8 us on 4096 x 11008 at 12 tokens, 8.6 -> 7.8 on 2560 x 8192: the loads of four dead rows)
+        launch_waves<12, 1, 8>(8, a);
     } else {
         // 16 staged token rows cost a wave 16.25 KB of LDS, which caps the workgroup at 8 waves
         launch_waves<16, 1, 8>(pick_waves(batches, 8), a);
@@ -379,21 +417,12 @@ int lq_gemv_a16w4_gate_up_launch(const void *x, const void *codes_g, const void 
                                  const void *codes_u, const void *scales_u, const void *zeros_u, void *h, int M, int N, int K,
                                  hipStream_t st) {
     const GemvGuArgs a = {x, codes_g, scales_g, zeros_g, codes_u, scales_u, zeros_u, h, M, N, K, st};
-    const int batches = (K / LQ_GROUP + 3) / 4;
-    if (M <= 4) {
-        switch (pick_waves(batches, 16)) {
-            case 2: launch_gu<2, 4>(a); break;
-            case 4: launch_gu<4, 4>(a); break;
-            case 8: launch_gu<8, 4>(a); break;
-            default: launch_gu<16, 4>(a); break;
-        }
-    } else {
-        // 16 staged token rows cost a wave 16.25 KB of LDS: at most 8 waves
-        switch (pick_waves(batches, 8)) {
-            case 2: launch_gu<2, 16>(a); break;
-            case 4: launch_gu<4, 16>(a); break;
-            default: launch_gu<8, 16>(a); break;
-        }
-    }
+    const int batches = (K / LQ_GROUP + 3) / 4, cus = lq_device_cu_count();
+    const int mp = (M + 3) / 4 * 4;
+    const int w = gu_waves(mp, N, batches, cus);
+    if (mp == 4) launch_gu_waves<4>(w, a);
+    else if (mp == 8) launch_gu_waves<8>(w, a);
+    else if (mp == 12) launch_gu_waves<12>(w, a);
+    else launch_gu_waves<16>(w, a);
     return lq_check_launch("lq_a16w4_gate_up_silu(gemv)");
 }
