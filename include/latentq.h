@@ -150,6 +150,14 @@ int lq_a16w4_gate_up_silu(const void *x, const void *codes_gate, const void *sca
                           const void *codes_up, const void *scales_up, const void *zeros_up, void *h, int64_t M,
                           int64_t N, int64_t K, int group, void *stream);
 
+/* Both forms (g_out and u_out null: lq_a16w4_gate_up_silu; given: lq_a16w4_gate_up_silu_save below) with a scratch buffer as
+ * lq_a16w4_fwd_ws: with 8 M N bytes and more of it, some 17 to 200 tokens run as one launch of small row tiles whose fp32
+ * partial products a second launch combines. */
+int lq_a16w4_gate_up_silu_ws(const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
+                             const void *codes_up, const void *scales_up, const void *zeros_up, void *h, void *g_out_or_null,
+                             void *u_out_or_null, int64_t M, int64_t N, int64_t K, int group, void *workspace,
+                             int64_t workspace_bytes, void *stream);
+
 /* The gated MLP block in training, three entry points that take the tensor-library glue between the six
  * products of `down(silu(gate(x)) * up(x))` and its backward into the GEMM epilogues. In the reference that
  * block is transformers' LlamaMLP with its three nn.Linear replaced by QLinearA16W4 (main0.py:300-343), i.e.

@@ -160,26 +160,26 @@ PyObject *dx4(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     return wrap(std::move(dx));
 }
 
-// x, gate (codes, scales, zeros), up (codes, scales, zeros), N, K, save -> h, or (h, g, u)
+// x, gate (codes, scales, zeros), up (codes, scales, zeros), N, K, save, workspace -> h, or (h, g, u)
 PyObject *gate_up(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    LQ_ARGS(10)
+    LQ_ARGS(11)
     const int64_t N = integer(a[7]), K = integer(a[8]);
     const bool save = a[9] == Py_True;
     const at::Tensor *x = bf16(a[0]);
     const int64_t M = rows_of(x, K);
     W4 g, u;
-    if (M <= 0 || !g.load(a + 1, N, K) || !u.load(a + 4, N, K) || !same_device(x, g.codes) || !same_device(x, u.codes)) return none();
+    void *ws;
+    int64_t ws_bytes;
+    if (M <= 0 || !g.load(a + 1, N, K) || !u.load(a + 4, N, K) || !same_device(x, g.codes) || !same_device(x, u.codes) ||
+        !workspace(a[10], x, &ws, &ws_bytes))
+        return none();
     On on(*x);
-    at::Tensor h = make_rows(*x, N, at::kBFloat16);
-    if (!save) {
-        LQ_CALL(lq_a16w4_gate_up_silu, x->data_ptr(), g.codes->data_ptr(), g.scales->data_ptr(), g.zeros->data_ptr(),
-                u.codes->data_ptr(), u.scales->data_ptr(), u.zeros->data_ptr(), h.data_ptr(), M, N, K, LQ_GROUP, on.stream);
-        return wrap(std::move(h));
-    }
-    at::Tensor go = make_rows(*x, N, at::kBFloat16), uo = make_rows(*x, N, at::kBFloat16);
-    LQ_CALL(lq_a16w4_gate_up_silu_save, x->data_ptr(), g.codes->data_ptr(), g.scales->data_ptr(), g.zeros->data_ptr(),
-            u.codes->data_ptr(), u.scales->data_ptr(), u.zeros->data_ptr(), h.data_ptr(), go.data_ptr(), uo.data_ptr(), M, N, K,
-            LQ_GROUP, on.stream);
+    at::Tensor h = make_rows(*x, N, at::kBFloat16), go, uo;
+    if (save) go = make_rows(*x, N, at::kBFloat16), uo = make_rows(*x, N, at::kBFloat16);
+    LQ_CALL(lq_a16w4_gate_up_silu_ws, x->data_ptr(), g.codes->data_ptr(), g.scales->data_ptr(), g.zeros->data_ptr(),
+            u.codes->data_ptr(), u.scales->data_ptr(), u.zeros->data_ptr(), h.data_ptr(), save ? go.data_ptr() : nullptr,
+            save ? uo.data_ptr() : nullptr, M, N, K, LQ_GROUP, ws, ws_bytes, on.stream);
+    if (!save) return wrap(std::move(h));
     return Py_BuildValue("NNN", wrap(std::move(h)), wrap(std::move(go)), wrap(std::move(uo)));
 }
 

@@ -649,6 +649,38 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
                                                     lq_pack_bf16(v[4], v[5]), lq_pack_bf16(v[6], v[7])};
 }
 
+// h = bf16(silu(g) * u) for the fp32 sums g and u of the slices of two products, partial[2][splits][M N]; the two products
+// themselves as well when their buffers are given. 8 elements per thread.
+__global__ __launch_bounds__(256) void gate_up_reduce_kernel(const float *__restrict__ partial, unsigned short *__restrict__ h,
+                                                            unsigned short *__restrict__ g_out, unsigned short *__restrict__ u_out,
+                                                            long long MN, int splits) {
+    const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (e >= MN) return;
+    float v[2][8];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[w][k] = 0.f;
+        for (int s = 0; s < splits; ++s) {
+            const float *src = partial + (long long)(w * splits + s) * MN + e;
+            const f32x4_t a = *reinterpret_cast<const f32x4_t *>(src), b = *reinterpret_cast<const f32x4_t *>(src + 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { v[w][k] += a[k]; v[w][4 + k] += b[k]; }
+        }
+    }
+    auto store = [&](unsigned short *dst, const float *f) {
+        *reinterpret_cast<u32x4_t *>(dst + e) = u32x4_t{lq_pack_bf16(f[0], f[1]), lq_pack_bf16(f[2], f[3]), lq_pack_bf16(f[4], f[5]), lq_pack_bf16(f[6], f[7])};
+    };
+    float o[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k] = v[0][k] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[0][k])) * v[1][k];
+    store(h, o);
+    if (g_out) {
+        store(g_out, v[0]);
+        store(u_out, v[1]);
+    }
+}
+
 }  // namespace
 
 // weights-direct forward GEMM (lq_gemm_fwd.hip)
@@ -674,6 +706,10 @@ double lq_gemm_staged_plan(long long M, long long N, int groups, size_t ws_bytes
 int lq_gemm_staged_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y,
                           float *partial, int M, int N, int K, int rows, int splits, int per_split, hipStream_t st,
                           unsigned long long *clk, const char *who);
+
+int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *scales_g, const void *zeros_g, const void *codes_u,
+                               const void *scales_u, const void *zeros_u, float *partial, int M, int N, int K, int rows, int splits,
+                               int per_split, hipStream_t st, const char *who);
 
 // GEMV path (lq_gemv.hip)
 int lq_gemv_a16w4_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias,
@@ -870,7 +906,7 @@ static int a16w4_fwd_impl(const char *who, const void *x, const void *codes, con
 
 static int gate_up_impl(const char *who, const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
                         const void *codes_up, const void *scales_up, const void *zeros_up, void *h, void *g_out, void *u_out,
-                        int64_t M, int64_t N, int64_t K, int group, void *stream) {
+                        int64_t M, int64_t N, int64_t K, int group, void *workspace, size_t ws_bytes, void *stream) {
     int rc = check_w4_common(who, x, codes_gate, scales_gate, zeros_gate, h, M, N, K, group);
     if (rc) return rc;
     rc = check_w4_common(who, x, codes_up, scales_up, zeros_up, h, M, N, K, group);
@@ -890,6 +926,33 @@ static int gate_up_impl(const char *who, const void *x, const void *codes_gate, 
                                             (int)K, (hipStream_t)stream);
     }
     LQ_REQUIRE(K % 256 == 0, "%s: K=%lld must be a multiple of 256 for more than 16 tokens", who, (long long)K);
+    LQ_REQUIRE(!workspace || lq_aligned(workspace, 16), "%s: the workspace must be 16-byte aligned", who);
+    // Few tokens leave most of a 128-row tile empty and most units idle: the staged kernel then runs both products as one
+    // launch of 32, 64 or 128 rows, planned as one product of 2 N columns, and a second launch adds its slices and forms h.
+    // Both sides estimated: the weights-direct kernel by its pace per 64-deep step (0.58 to 0.68 us for a workgroup with a
+    // unit to itself, 1.3 for two) plus 7 us, the staged one by its own plan plus, where that is not in it, the partial
+    // products' way through the cache. us against the weights-direct kernel and the two plain products with tensor glue:
+    //   11008 x 4096  17 / 45 / 128 tokens  25.7 / 27.7 / 37.3 against 51.1 / 50.4 / 50.5 and 45.5 / 43.9 / 55.7; behind from
+    //                 160 on (64.5 against 52.1)
+    //   6144 x 3072   17 / 64 / 256         13.4 / 20.2 / 30.9 against 35.8 / 35.9 / 36.4; level at 300
+    //   3072 x 1024   17 / 128 / 300        10.3 / 11.7 / 15.3 against 15.0 / 15.1 / 15.5; 19.2 against 15.6 at 400
+    if (ws_bytes >= (size_t)8 * M * N) {
+        const long long cus = lq_device_cu_count();
+        const long long wg = ((M + 127) / 128) * ((N + 127) / 128), rem = wg % (2 * cus);
+        const double est_direct = (1.3 * (double)(wg / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.66 : 1.3)) * (double)(K / 64) + 7.0;
+        int rows = 128, splits = 1, per = (int)(K / LQ_GROUP);
+        double est = lq_gemm_staged_plan(M, 2 * N, (int)(K / LQ_GROUP), ws_bytes, cus, &rows, &splits, &per);
+        if (splits == 1) est += 1.7 + 0.53e-6 * 8.0 * (double)M * (double)N;
+        if (est < est_direct) {
+            rc = lq_gemm_staged_pair_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, (float *)workspace, (int)M,
+                                            (int)N, (int)K, rows, splits, per, (hipStream_t)stream, who);
+            if (rc) return rc;
+            const long long MN = (long long)M * N;
+            hipLaunchKernelGGL(gate_up_reduce_kernel, dim3((unsigned)((MN / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                               (const float *)workspace, (unsigned short *)h, (unsigned short *)g_out, (unsigned short *)u_out, MN, splits);
+            return lq_check_launch(who);
+        }
+    }
     return lq_gemm_fwd_gate_up_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h, g_out, u_out, (int)M,
                                       (int)N, (int)K, (hipStream_t)stream);
 }
@@ -898,7 +961,7 @@ extern "C" int lq_a16w4_gate_up_silu(const void *x, const void *codes_gate, cons
                                      const void *codes_up, const void *scales_up, const void *zeros_up, void *h, int64_t M,
                                      int64_t N, int64_t K, int group, void *stream) {
     return gate_up_impl("lq_a16w4_gate_up_silu", x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h, nullptr,
-                        nullptr, M, N, K, group, stream);
+                        nullptr, M, N, K, group, nullptr, 0, stream);
 }
 
 extern "C" int lq_a16w4_gate_up_silu_save(const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
@@ -906,7 +969,16 @@ extern "C" int lq_a16w4_gate_up_silu_save(const void *x, const void *codes_gate,
                                           void *u_out, int64_t M, int64_t N, int64_t K, int group, void *stream) {
     LQ_REQUIRE(g_out && u_out, "lq_a16w4_gate_up_silu_save: null pointer argument");
     return gate_up_impl("lq_a16w4_gate_up_silu_save", x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h, g_out,
-                        u_out, M, N, K, group, stream);
+                        u_out, M, N, K, group, nullptr, 0, stream);
+}
+
+extern "C" int lq_a16w4_gate_up_silu_ws(const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
+                                        const void *codes_up, const void *scales_up, const void *zeros_up, void *h,
+                                        void *g_out_or_null, void *u_out_or_null, int64_t M, int64_t N, int64_t K, int group,
+                                        void *workspace, int64_t workspace_bytes, void *stream) {
+    return gate_up_impl("lq_a16w4_gate_up_silu_ws", x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h,
+                        g_out_or_null, u_out_or_null, M, N, K, group, workspace,
+                        workspace && workspace_bytes > 0 ? (size_t)workspace_bytes : 0, stream);
 }
 
 extern "C" int lq_a16w4_fwd(const void *x, const void *codes, const void *scales, const void *zeros,

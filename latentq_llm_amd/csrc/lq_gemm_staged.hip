@@ -28,8 +28,11 @@ struct StagedParams {
     const unsigned char *x;  // bf16 [M, K]
     const unsigned char *w;  // packed codes
     const unsigned short *scales, *zeros, *bias;
+    // a second matrix of the same shape on the same activations (blockIdx.z = 1), or null: both give partial products
+    const unsigned char *w2;
+    const unsigned short *scales2, *zeros2;
     unsigned short *y;       // bf16 [M, N]
-    float *partial;          // split reduction: fp32 [splits][M][N], or null
+    float *partial;          // partial products: fp32 [matrices][splits][M][N], or null
     int M, N, K;
     int tiles_m, tiles_n;
     int groups_per_split;    // groups of 128 k per slice (blockIdx.y)
@@ -106,8 +109,10 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
         q_off = (unsigned)(gr - c0) * (unsigned)G * 2u;
     }
     const unsigned char *a_base = p.x + (long long)m0 * lda;
-    const unsigned char *c_base = p.w + (long long)c0 * ldw;
-    const unsigned char *q_base = (const unsigned char *)((wave < 2 ? p.scales : p.zeros) + (long long)c0 * G);
+    const bool second = blockIdx.z != 0;
+    const unsigned char *c_base = (second ? p.w2 : p.w) + (long long)c0 * ldw;
+    const unsigned short *q_mat = wave < 2 ? (second ? p.scales2 : p.scales) : second ? p.zeros2 : p.zeros;
+    const unsigned char *q_base = (const unsigned char *)(q_mat + (long long)c0 * G);
     auto to_lds16 = [&](unsigned char *dst, unsigned off, const unsigned char *src) {
         const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)dst);
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(src) : "memory");
@@ -206,7 +211,7 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
 
     // ---- epilogue: acc[j][q]: row m0 + 32 j + r, column c0 + 32 wave + 8 (q / 4) + 4 h + q % 4
     if (p.partial) {
-        float *part = p.partial + (long long)blockIdx.y * p.M * p.N;
+        float *part = p.partial + (long long)(blockIdx.z * gridDim.y + blockIdx.y) * p.M * p.N;
 #pragma unroll
         for (int j = 0; j < FM; ++j) {
             const int m = m0 + 32 * j + r;
@@ -260,7 +265,7 @@ template <int FM>
 int launch_staged(StagedParams p, int splits, hipStream_t st, const char *who) {
     p.tiles_m = (p.M + 32 * FM - 1) / (32 * FM);
     p.tiles_n = (p.N + kCols - 1) / kCols;
-    hipLaunchKernelGGL(gemm_staged_kernel<FM>, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(gemm_staged_kernel<FM>, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits, p.w2 ? 2u : 1u), dim3(256), 0, st, p);
     return lq_check_launch(who);
 }
 
@@ -303,6 +308,22 @@ double lq_gemm_staged_plan(long long M, long long N, int groups, size_t ws_bytes
         }
     }
     return best;
+}
+
+// Gate and up product of few tokens as one launch of twice the tiles: fp32 partial products [2][splits][M][N] to `partial`,
+// to be added and combined by the caller. Shapes as below; splits >= 1.
+int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *scales_g, const void *zeros_g, const void *codes_u,
+                               const void *scales_u, const void *zeros_u, float *partial, int M, int N, int K, int rows, int splits,
+                               int per_split, hipStream_t st, const char *who) {
+    StagedParams p = {};
+    p.x = (const unsigned char *)x;
+    p.w = (const unsigned char *)codes_g; p.scales = (const unsigned short *)scales_g; p.zeros = (const unsigned short *)zeros_g;
+    p.w2 = (const unsigned char *)codes_u; p.scales2 = (const unsigned short *)scales_u; p.zeros2 = (const unsigned short *)zeros_u;
+    p.M = M; p.N = N; p.K = K;
+    p.partial = partial; p.groups_per_split = per_split;
+    if (rows == 32) return launch_staged<1>(p, splits, st, who);
+    if (rows == 64) return launch_staged<2>(p, splits, st, who);
+    return launch_staged<4>(p, splits, st, who);
 }
 
 // splits > 1: fp32 partial products [splits][M][N] to `partial`, to be added by the caller; else bf16 (x W^T + bias) to y.

@@ -195,7 +195,8 @@ def a16w4_gate_up_silu(x, gate, up, shape, out=None, save=False):
     save=True (lq_a16w4_gate_up_silu_save) also stores the two products and returns (h, g, u)."""
     N, K = shape
     if out is None and x.dim() == 2:
-        r = (_native or _fast()).gate_up(x, *gate, *up, N, K, save)
+        ws = _workspace(x, x.shape[0], 2 * N)[0] if 16 < x.shape[0] <= 2048 and x.is_cuda else None
+        r = (_native or _fast()).gate_up(x, *gate, *up, N, K, save, ws)
         if r is not None:
             return r
     _chk(x, torch.bfloat16, "x")
@@ -215,13 +216,11 @@ def a16w4_gate_up_silu(x, gate, up, shape, out=None, save=False):
     u = torch.empty_like(out) if save else None
     if M:
         with torch.cuda.device(x.device):
-            if save:
-                _C.call("lq_a16w4_gate_up_silu_save", x.data_ptr(), gate[0].data_ptr(), gate[1].data_ptr(), gate[2].data_ptr(),
-                        up[0].data_ptr(), up[1].data_ptr(), up[2].data_ptr(), out.data_ptr(), g.data_ptr(), u.data_ptr(),
-                        M, N, K, GROUP, _stream(x))
-            else:
-                _C.call("lq_a16w4_gate_up_silu", x.data_ptr(), gate[0].data_ptr(), gate[1].data_ptr(), gate[2].data_ptr(),
-                        up[0].data_ptr(), up[1].data_ptr(), up[2].data_ptr(), out.data_ptr(), M, N, K, GROUP, _stream(x))
+            keep, ws, ws_bytes = _workspace(x, M, 2 * N) if M > 16 else (None, None, 0)
+            _C.call("lq_a16w4_gate_up_silu_ws", x.data_ptr(), gate[0].data_ptr(), gate[1].data_ptr(), gate[2].data_ptr(),
+                    up[0].data_ptr(), up[1].data_ptr(), up[2].data_ptr(), out.data_ptr(), g.data_ptr() if save else None,
+                    u.data_ptr() if save else None, M, N, K, GROUP, ws, ws_bytes, _stream(x))
+            del keep
     return (out, g, u) if save else out
 
 

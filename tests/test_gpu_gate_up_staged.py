@@ -1,0 +1,29 @@
+"""The gate / up product of 17 tokens and more with a workspace: small row tiles of both matrices and the launch that combines
+their partial products, at the edges of the row tiles and of the columns, cut into slices and whole; against float64 and
+against the two plain products, alone, stored (training form) and into a caller's buffer."""
+import pytest
+import torch
+
+from tests.util import make_w4, randn_bf16, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 16, 256), (31, 144, 512), (32, 128, 1280), (33, 2048, 1024), (64, 4112, 768), (65, 528, 2048),
+                                   (96, 11008, 512), (127, 256, 4096), (129, 5504, 2048), (200, 1040, 256), (257, 64, 2304)])
+def test_gate_up(M, N, K):
+    from latentq_llm_amd import ops
+    mats, dense = [], []
+    for seed in (1, 2):
+        _, p, s, z = make_w4(N, K, seed)
+        mats.append((p.cuda(), s.cuda(), z.cuda()))
+        dense.append(ops.a16w4_dequant(*mats[-1], (N, K)).double())
+    x = randn_bf16((M, K), 3).cuda()
+    g, u = (x.double() @ w.t() for w in dense)
+    want = g * torch.sigmoid(g) * u
+    h = ops.a16w4_gate_up_silu(x, *mats, (N, K))
+    assert rel_l2(h, want) < 2.5e-3  # one bf16 rounding (2^-9) of fp32 sums
+    hs, gs, us = ops.a16w4_gate_up_silu(x, *mats, (N, K), save=True)
+    assert torch.equal(hs, h) and rel_l2(gs, g) < 2.5e-3 and rel_l2(us, u) < 2.5e-3
+    out = torch.full_like(h, float("nan"))
+    assert ops.a16w4_gate_up_silu(x, *mats, (N, K), out=out) is out and torch.equal(out, h)
