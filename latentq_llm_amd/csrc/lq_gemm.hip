@@ -711,6 +711,10 @@ int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *s
                                const void *scales_u, const void *zeros_u, float *partial, int M, int N, int K, int rows, int splits,
                                int per_split, hipStream_t st, const char *who);
 
+// 17 to 64 tokens, one launch with 16 columns per compute unit (lq_gemm_few.hip)
+int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
+                       int K, hipStream_t st, const char *who);
+
 // GEMV path (lq_gemv.hip)
 int lq_gemv_a16w4_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias,
                          void *y, int M, int N, int K, hipStream_t st);
@@ -779,7 +783,10 @@ struct W4Plan {
     int rows = 128;  // forward LQ_PLAN_STAGED_128: rows of the tile (32, 64 or 128), 128 columns
 };
 
-// Forward pass, M > 16, by the number of 128 x 128 output tiles T:
+// Forward pass, M > 16. Up to 64 tokens, with 16 columns for each of more than half of the units and at most all of them:
+// the kernel of lq_gemm_few.hip where its time, which grows with the tokens' bytes each unit takes in (2 us + 0.5 us per 1000 k
+// + 0.42 per 16 tokens and 1000 k, less with fewer units asking; 12 % rms over 64 timings), is under the staged kernel's
+// estimate. Otherwise by the number of 128 x 128 output tiles T:
 //   T <= half of the units             the staged kernel, which plans its row tile and its slices of K itself
 //                                      (1.2 to 1.6 times the speed of the weights-direct kernels there: 11.5 against
 //                                      15.0 us on 1024 x 1536 x 1536, 23.6 against 34 on 384 x 4096 x 4096; level at
@@ -803,6 +810,15 @@ struct W4Plan {
 // is the one-token kernel) below K = 8192, although 11008 x 4096 takes 20.0 us so against 15.7.
 static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     W4Plan out;
+    if (M <= 64 && N <= 16 * cus && 2 * N > 16 * cus) {
+        int rows = 0, splits = 0, per = 0;
+        const double units = 0.4 + 0.6 * (double)N / (double)(16 * cus);
+        const double est = 2.0 + 1e-3 * (double)K * (0.5 + 0.42 * (double)((M + 15) / 16)) * units;
+        if (est < lq_gemm_staged_plan(M, N, (int)(K / LQ_GROUP), ws_bytes, cus, &rows, &splits, &per)) {
+            out.kernel = LQ_PLAN_FEW;
+            return out;
+        }
+    }
     if ((M == 17 && K < 8192) || (M <= 32 && N * K <= 4096ll * 4096)) {
         out.kernel = LQ_PLAN_GEMV_CHUNKS;
         return out;
@@ -887,6 +903,8 @@ static int a16w4_fwd_impl(const char *who, const void *x, const void *codes, con
         }
         return LQ_OK;
     }
+    if (plan.kernel == LQ_PLAN_FEW)
+        return lq_gemm_few_launch(x, codes, scales, zeros, bias_or_null, y, (int)M, (int)N, (int)K, (hipStream_t)stream, who);
     if (plan.kernel == LQ_PLAN_DIRECT || plan.kernel == LQ_PLAN_DIRECT_128)
         return lq_gemm_fwd_direct_launch(x, codes, scales, zeros, bias_or_null, y, (int)M, (int)N, (int)K, (hipStream_t)stream, clk,
                                          plan.kernel == LQ_PLAN_DIRECT_128);

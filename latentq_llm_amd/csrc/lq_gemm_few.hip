@@ -1,0 +1,185 @@
+// Forward of the A16W4 layers for 17 to 64 tokens and up to 16 columns per compute unit, in one launch:
+//   Y[M,N] = X[M,K] . deq(W)[N,K]^T (+ bias)
+//
+// Bound: latency, and what a compute unit takes in from L2 (64 bytes a clock). The staged kernel (lq_gemm_staged.hip) has to cut K
+// into slices to fill the device with such an output, and the launch that adds the slices costs as much as the product's
+// own loop. Here a workgroup owns 16 columns and all of K, shared among its four waves: every compute unit reads all of X (0.5
+// MB at 64 tokens and K = 4096: 3.9 us at that rate, the price of having no second launch).
+//
+// A wave takes every fourth group of 128 k and works on its own: its part of X, its codes, scales and zeros come by LDS-direct
+// loads into stages that no other wave touches, D of them deep, with a wait and no barrier. The four partial sums meet in
+// LDS at the end.
+//
+// us against the staged kernel with its second launch (and 16-token GEMV launches up to 32 tokens), weights from HBM:
+//     N x K          17 tokens       32              48              64
+//     4096 x 4096    10.3 -> 7.2     11.4 -> 7.6     13.6 -> 8.8     12.3 -> 9.9
+//     2560 x 2560    9.9 -> 6.3      9.8 -> 6.3      10.0 -> 6.8     10.3 -> 7.4
+//     4096 x 1024    9.9 -> 6.0      9.7 -> 6.2      8.0 -> 6.0      8.0 -> 6.1
+//     2560 x 8192    12.1 -> 9.7     12.9 -> 10.8    14.3 -> 13.2    15.0 / 15.6
+//     4096 x 11008   15.8 -> 14.9    15.7 / 17.2     17.5 / 21.7     18.2 / 25.6   (the last three stay with the staged kernel)
+// X arrives at 30 bytes a clock and unit, half of what L2 gives a unit reading alone; letting the units start at different
+// groups changes nothing.
+//
+// MFMA 16x16x32, weights first: lane l holds columns 4 (l / 16) .. + 3 of token l % 16. With r = l % 16, h = l / 16 slice w = 0..3 of
+// a group has the lane's operands at k = 32 h + 8 w .. + 7: word w of the 16 bytes of codes of row r, and a 16-byte piece of X.
+#include "lq_common.h"
+
+#include <type_traits>
+
+namespace {
+
+struct FewParams {
+    const unsigned char *x;  // bf16 [M, K]
+    const unsigned char *w;  // packed codes
+    const unsigned short *scales, *zeros, *bias;
+    unsigned short *y;       // bf16 [M, N]
+    int M, N, K;
+};
+
+typedef __attribute__((address_space(3))) void lds_void;
+
+template <int I>
+using ic = std::integral_constant<int, I>;
+
+constexpr int kWaves = 4;
+
+// LDS layout of a wave's stage (16-byte pieces, swizzled so that 16 lanes reading one piece of 16 rows cover all banks):
+//   activations  16 MT rows of 256 bytes, piece c of row i at c ^ (i & 15)
+//   codes        16 rows of 64 bytes, piece c of row i at c ^ ((i >> 2) & 3)
+//   scales, zeros  a dword per row each, the bf16 value in its lower half (and 32 dwords of copies)
+// MT: groups of 16 tokens, D: stages
+template <int MT, int D>
+__global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(FewParams p) {
+    constexpr int A_BYTES = MT * 4096, STAGE = A_BYTES + 1024 + 256;
+    constexpr int LOADS = 4 * MT + 2;
+    static_assert((D - 1) * LOADS < 64, "the wait counts loads in six bits");
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves * D * STAGE];
+
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, h = lane >> 4;
+    const int c0 = blockIdx.x * 16;
+    const int G = p.K / LQ_GROUP;
+    unsigned char *const mine = lds + wave * (D * STAGE);
+
+    // ---- loads: instruction i < 4 MT brings rows 4 i .. 4 i + 3 of the wave's group of X
+    const unsigned lda = (unsigned)p.K * 2u;
+    unsigned a_off[4 * MT];
+#pragma unroll
+    for (int i = 0; i < 4 * MT; ++i) {
+        const int row = 4 * i + (lane >> 4);
+        a_off[i] = (unsigned)(row < p.M ? row : p.M - 1) * lda + ((lane & 15) ^ (row & 15)) * 16;
+    }
+    const int crow = lane >> 2;
+    const unsigned c_off = (unsigned)crow * (unsigned)(p.K / 2) + ((lane & 3) ^ ((crow >> 2) & 3)) * 16;
+    const unsigned q_off = (unsigned)r * (unsigned)G * 2u;
+    const unsigned char *c_base = p.w + (long long)c0 * (p.K / 2);
+    const unsigned char *s_base = (const unsigned char *)(p.scales + (long long)c0 * G);
+    const unsigned char *z_base = (const unsigned char *)(p.zeros + (long long)c0 * G);
+    // scales on lanes 0..15 (and 32..47), zeros on 16..31 (and 48..63): one instruction, 64-bit addresses
+    const unsigned char *q_lane = (h & 1 ? z_base : s_base) + q_off;
+    auto to_lds = [&](unsigned char *dst, unsigned off, const unsigned char *src) {
+        const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)dst);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(src) : "memory");
+    };
+    // group g into stage st, the codes (from HBM) first
+    auto issue = [&](int g, unsigned char *st) {
+        to_lds(st + A_BYTES, c_off, c_base + (long long)g * 64);
+        const unsigned q_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(st + A_BYTES + 1024));
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off" ::"s"(q_addr), "v"(q_lane + (long long)g * 2) : "memory");
+#pragma unroll
+        for (int i = 0; i < 4 * MT; ++i) to_lds(st + i * 1024, a_off[i], p.x + (long long)g * 256);
+    };
+
+    f32x4_t acc[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    const int ng = wave < G ? (G - wave + kWaves - 1) / kWaves : 0;  // the wave's groups: wave, wave + 4, ...
+    auto group = [&](int i, auto si) {
+        constexpr int S = decltype(si)::value;
+        unsigned char *st = mine + S * STAGE;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * LOADS) : "memory");
+        const u32x4_t c = *reinterpret_cast<const u32x4_t *>(st + A_BYTES + r * 64 + ((h ^ ((r >> 2) & 3)) << 4));
+        const unsigned *q = reinterpret_cast<const unsigned *>(st + A_BYTES + 1024);
+        const float sc = __uint_as_float(q[r] << 16);
+        const float nzs = -(__uint_as_float(q[16 + r] << 16) * sc), s512 = sc * 512.0f;
+        u32x4_t x[4][MT];
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) x[w][j] = *reinterpret_cast<const u32x4_t *>(st + (16 * j + r) * 256 + (((4 * h + w) ^ r) << 4));
+        // the stage is free once these reads have returned; past the wave's last group: re-read it (nothing uses it)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        issue(wave + kWaves * (i + D < ng ? i + D : ng - 1), st);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            float f[8];
+            lq_dequant_word_f32(c[w], s512, nzs, f);
+            const u32x4_t b = {lq_pack_bf16(f[0], f[1]), lq_pack_bf16(f[2], f[3]), lq_pack_bf16(f[4], f[5]), lq_pack_bf16(f[6], f[7])};
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, x[w][j]), acc[j], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (ng > 0) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) issue(wave + kWaves * (d < ng ? d : ng - 1), mine + d * STAGE);
+        int i = 0;
+        for (; i + D <= ng; i += D) {
+            group(i, ic<0>());
+            group(i + 1, ic<1>());
+            if constexpr (D > 2) group(i + 2, ic<2 % D>());
+            if constexpr (D > 3) group(i + 3, ic<3 % D>());
+        }
+        static_assert(D >= 2 && D <= 4, "the loop above names up to four stages");
+        if (i < ng) group(i, ic<0>());
+        if constexpr (D > 2) if (i + 1 < ng) group(i + 1, ic<1>());
+        if constexpr (D > 3) if (i + 2 < ng) group(i + 2, ic<2 % D>());
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped loads of the last groups
+    __syncthreads();
+
+    // ---- partial sums [wave][token][16 columns]
+    float *part = reinterpret_cast<float *>(lds);
+#pragma unroll
+    for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4_t *>(part + ((wave * MT + j) * 16 + r) * 16 + 4 * h) = acc[j];
+    __syncthreads();
+    for (int q = threadIdx.x; q < MT * 64; q += 64 * kWaves) {
+        const int m = q >> 2, c = c0 + 4 * (q & 3);
+        if (m >= p.M) continue;
+        f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const f32x4_t a = *reinterpret_cast<const f32x4_t *>(part + w * (MT * 256) + q * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += a[e];
+        }
+        if (p.bias) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += lq_bf16_bits_to_f32(p.bias[c + e]);
+        }
+        *reinterpret_cast<u32x2_t *>(p.y + (long long)m * p.N + c) = u32x2_t{lq_pack_bf16(v[0], v[1]), lq_pack_bf16(v[2], v[3])};
+    }
+}
+
+}  // namespace
+
+// 16 < M <= 64, N % 16 == 0, K % 128 == 0 are guaranteed by the caller.
+int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
+                       int K, hipStream_t st, const char *who) {
+    FewParams p = {};
+    p.x = (const unsigned char *)x; p.w = (const unsigned char *)codes;
+    p.scales = (const unsigned short *)scales; p.zeros = (const unsigned short *)zeros;
+    p.bias = (const unsigned short *)bias; p.y = (unsigned short *)y;
+    p.M = M; p.N = N; p.K = K;
+    // the 32-bit lane offsets of the loads span the tokens' rows and 16 rows of codes
+    if (128ll * K >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: K too large", who);
+    const dim3 grid((unsigned)(N / 16)), block(64 * kWaves);
+    if (M <= 32) hipLaunchKernelGGL((gemm_few_kernel<2, 4>), grid, block, 0, st, p);
+    else if (M <= 48) hipLaunchKernelGGL((gemm_few_kernel<3, 3>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((gemm_few_kernel<4, 2>), grid, block, 0, st, p);
+    return lq_check_launch(who);
+}
