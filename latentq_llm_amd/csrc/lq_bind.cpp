@@ -20,10 +20,15 @@ namespace {
 
 PyObject *g_error = nullptr;  // LatentQError
 
-// A plain tensor (Tensor or Parameter, no other subclass) on a GPU, contiguous, of the given type
+// A plain tensor (Tensor or Parameter, no other subclass) on a GPU, contiguous, of the given type. The wrappers of function
+// transforms (vmap, functional gradients, functionalisation) have the Python type of a plain tensor and no memory of their own.
 const at::Tensor *plain(PyObject *o, at::ScalarType type) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
+    constexpr c10::DispatchKeySet kWrapped({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                            c10::DispatchKey::Batched, c10::DispatchKey::Functionalize, c10::DispatchKey::Python,
+                                            c10::DispatchKey::ZeroTensor, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
+    if (t.key_set().has_any(kWrapped) || !t.has_storage()) return nullptr;
     return t.is_cuda() && t.scalar_type() == type && t.is_contiguous() ? &t : nullptr;
 }
 
