@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import ops, quant
 
 
 def _w4(layer):
@@ -96,7 +96,8 @@ class QuantLlamaMLP(nn.Module):
         out_shape = x.shape[:-1] + (self.intermediate_size,)
         x2 = x.reshape(-1, x.shape[-1])
         M, K = x2.shape
-        if x2.dtype == torch.bfloat16 and M > 0 and (M <= 16 or K % 256 == 0):
+        # (where a trace or a transform watches, 17 to 63 tokens go through the layers' Functions, which it sees)
+        if x2.dtype == torch.bfloat16 and M > 0 and (M <= 16 or (K % 256 == 0 and (M >= 64 or quant._unwatched()))):
             if not x2.is_contiguous():
                 x2 = x2.contiguous()
             h = ops.a16w4_gate_up_silu(x2, _w4(self.gate_proj), _w4(self.up_proj), (self.intermediate_size, K))

@@ -28,6 +28,7 @@ from functools import reduce
 from typing import Optional, Union
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn as nn
 
 from . import ops
@@ -204,6 +205,19 @@ def _hand_over(layer, dw):
         backward_hook_fn(layer, None, None)
 
 
+def _unwatched():
+    """Whether nothing but autograd's own switch decides if a call has to go through its Function: no trace is recorded (it
+    would hold a direct call's result as a constant), no forward-mode level is open (a direct call would drop the tangent)
+    and no function transform is active."""
+    return torch._C._get_tracing_state() is None and fwAD._current_level < 0 and not torch._C._are_functorch_transforms_active()
+
+
+def _ctx_form(fn, forward):
+    """The same Function with ctx in forward: torch binds the arguments of one with setup_context to forward's signature on
+    every call (10 us), which only function transforms need."""
+    return type(torch.autograd.Function)(fn.__name__, (torch.autograd.Function,), {"forward": staticmethod(forward), "backward": staticmethod(fn.backward)})
+
+
 # ------------------------------------------------------------------------ autograd: A16W4 --
 # The reference gates the bias gradient on needs_input_grad[2] (utils/quant.py:143, 208, 249, 290,
 # 371), which is the flag of the non-tensor qparam argument and therefore always False: QLinear
@@ -229,13 +243,16 @@ class QLinearFunctionW4(torch.autograd.Function):
     packed codes (never a materialised W): dX on the HIP dequant-GEMM, dW = dY^T X pushed to
     dict_temp for the backward hook, dB = sum dY."""
 
-    # (ctx in forward, no setup_context: with one, every call binds its arguments to forward's signature, 10 us)
     @staticmethod
-    def forward(ctx, input, weight_d, qparamw4, bias, layer=None):
+    def forward(input, weight_d, qparamw4, bias, layer=None):
+        return _w4_linear(input, weight_d, qparamw4, bias)
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        input, weight_d, qparamw4, bias = inputs[:4]
         ctx.save_for_backward(input, weight_d.data, bias)
         ctx.save_qparamw4 = qparamw4
-        ctx.layer = layer
-        return _w4_linear(input, weight_d, qparamw4, bias)
+        ctx.layer = inputs[4] if len(inputs) > 4 else None
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -257,8 +274,12 @@ class QLinearFunctionW4_eval(torch.autograd.Function):
     """Inference A16W4 linear (utils/quant.py:149-169): no state saved, no gradients."""
 
     @staticmethod
-    def forward(ctx, input, weight_d, qparamw4, bias):
+    def forward(input, weight_d, qparamw4, bias):
         return _w4_linear(input, weight_d, qparamw4, bias)
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        pass
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -359,12 +380,16 @@ class QLinearFunctionA8W8_static(torch.autograd.Function):
     """Static activation clamp (utils/quant.py:172-211)."""
 
     @staticmethod
-    def forward(ctx, input, weight_d, qparamaw, bias, layer=None):
-        ctx.layer = layer
+    def forward(input, weight_d, qparamaw, bias, layer=None):
         clampv, qscales = qparamaw
+        return _a8w8_linear(input, weight_d, qscales, bias, clampv, alpha_in_bf16=False)[0]
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        input, weight_d, qparamaw, bias = inputs[:4]
         ctx.save_for_backward(input, weight_d.data, bias)
         ctx.save_qparamaw = qparamaw
-        return _a8w8_linear(input, weight_d, qscales, bias, clampv, alpha_in_bf16=False)[0]
+        ctx.layer = inputs[4] if len(inputs) > 4 else None
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -523,6 +548,19 @@ def backward_hook_fn(module, grad_out, grad_in):
 
 
 # -------------------------------------------------------------------------------- modules --
+def _w4_forward_ctx(ctx, input, weight_d, qparamw4, bias, layer=None):
+    ctx.save_for_backward(input, weight_d.data, bias)
+    ctx.save_qparamw4 = qparamw4
+    ctx.layer = layer
+    return _w4_linear(input, weight_d, qparamw4, bias)
+
+
+_CTX_FORMS = {
+    QLinearFunctionW4: _ctx_form(QLinearFunctionW4, _w4_forward_ctx),
+    QLinearFunctionW4_eval: _ctx_form(QLinearFunctionW4_eval, lambda ctx, *args: _w4_linear(*args)),
+}
+
+
 class _HookHandle(object):
     """What add_hook leaves in hook_handle: remove() ends the delivery of weight gradients (they then stay in dict_temp,
     as with the reference's hook removed)."""
@@ -556,6 +594,8 @@ class _QLinearBase(nn.Module):
         self.hook_handle = _HookHandle()
 
     def _apply_fn(self, fn, x, *layer):
+        if not torch._C._are_functorch_transforms_active():
+            fn = _CTX_FORMS.get(fn, fn)
         out = fn.apply(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), self.weight.data, self._qparam(), self.bias, *layer)
         return out if x.dim() == 2 else out.reshape(x.shape[:-1] + (self.output_features,))
 
@@ -571,7 +611,7 @@ class _QLinearBase(nn.Module):
         return self._apply_fn(self._fn_train, x, self if getattr(self.hook_handle, "active", False) else None)
 
     def forward_eval(self, x):
-        if not torch.is_grad_enabled():
+        if not torch.is_grad_enabled() and _unwatched():
             y = self._infer(x)
             if y is not None:
                 return y
