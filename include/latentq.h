@@ -418,6 +418,28 @@ int lq_adam8_sr_step(const void *grad, const void *codes_in, void *codes_out, co
                      int64_t K, int group, int block_elems, double beta1, double beta2, double eps, double step_size,
                      uint64_t philox_seed, uint64_t philox_offset, void *stream);
 
+/* The three steps above for several parameters with one launch per eight of them: the _queued forms check their arguments and
+ * append the step to a queue (null: they run it, as the plain forms do); lq_adam8_queue_run launches and empties it. Every
+ * buffer has to stay allocated, and untouched by other work, until then; the stream given to a _queued form is not used. The
+ * steps of a queue must not share a buffer that one of them writes. A queue belongs to the caller and to one thread at a time. */
+int lq_adam8_queue_new(void **queue_out);
+int lq_adam8_queue_free(void *queue);
+int lq_adam8_queue_run(void *queue, void *stream);
+int lq_adam8_latent_w4_step_queued(const void *grad, void *codes, int32_t *residual, const void *scales, const void *zeros,
+                                   uint8_t *state1, uint8_t *state2, float *scale1, float *max1, float *scale2, float *max2,
+                                   int64_t N, int64_t K, int group, int block_elems, int dk1, float db1, int dk2, float db2,
+                                   int dk3, int qk1, float qb1, int qk2, float qb2, int qk3, double beta1, double beta2,
+                                   double eps, double step_size, void *stream, void *queue_or_null);
+int lq_adam8_latent_w8_step_queued(const void *grad, int8_t *codes, int32_t *residual, const void *qscales, uint8_t *state1,
+                                   uint8_t *state2, float *scale1, float *max1, float *scale2, float *max2, int64_t N, int64_t K,
+                                   int block_elems, int dk1, float db1, int dk2, float db2, int dk3, int qk1, float qb1, int qk2,
+                                   float qb2, int qk3, double beta1, double beta2, double eps, double step_size, void *stream,
+                                   void *queue_or_null);
+int lq_adam8_sr_step_queued(const void *grad, const void *codes_in, void *codes_out, const void *scales, const void *zeros,
+                            uint8_t *state1, uint8_t *state2, float *scale1, float *max1, float *scale2, float *max2, int64_t N,
+                            int64_t K, int group, int block_elems, double beta1, double beta2, double eps, double step_size,
+                            uint64_t philox_seed, uint64_t philox_offset, void *stream, void *queue_or_null);
+
 /* What the periodic choice of the residual codec's curve looks at (MyAdam.update_step, utils/quant.py:1117-1122):
  * ratio_out = bf16(|m| / d) of the step that lq_adam8_update would take, with nothing updated. ratio_out: bf16[n],
  * 16-byte aligned; the rest as lq_adam8_update. */

@@ -69,6 +69,15 @@ SIGNATURES = {
     "lq_adam8_ratio": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _f64, _f64, _f64, _vp],
     "lq_adam8_sr_step": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _f64, _f64, _f64, _f64,
                          _u64, _u64, _vp],
+    "lq_adam8_queue_new": [_vp],
+    "lq_adam8_queue_free": [_vp],
+    "lq_adam8_queue_run": [_vp, _vp],
+    "lq_adam8_sr_step_queued": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _f64, _f64, _f64, _f64,
+                                _u64, _u64, _vp, _vp],
+    "lq_adam8_latent_w4_step_queued": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32,
+                                       _i32, _f32, _i32, _f32, _i32, _i32, _f32, _i32, _f32, _i32, _f64, _f64, _f64, _f64, _vp, _vp],
+    "lq_adam8_latent_w8_step_queued": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32,
+                                       _i32, _f32, _i32, _f32, _i32, _i32, _f32, _i32, _f32, _i32, _f64, _f64, _f64, _f64, _vp, _vp],
     "lq_adam8_latent_w4_step": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32,
                                 _i32, _f32, _i32, _f32, _i32, _i32, _f32, _i32, _f32, _i32, _f64, _f64, _f64, _f64, _vp],
     "lq_adam8_latent_w8_step": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32,

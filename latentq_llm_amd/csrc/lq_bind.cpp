@@ -398,7 +398,7 @@ PyObject *gradq8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
 
 // The operands every form of the optimizer step shares: grad, state1, state2, scale1, max1, scale2, max2
 struct Adam {
-    const at::Tensor *grad, *s1, *s2;
+    const at::Tensor *grad, *s1, *s2, *blocks[4];
     float *f[4];
     int64_t n, block;
     bool load(PyObject *const *o) {
@@ -412,6 +412,7 @@ struct Adam {
         for (int i = 0; i < 4; ++i) {
             const at::Tensor *t = plain(o[3 + i], at::kFloat);
             if (!t || !same_device(grad, t) || (i ? t->numel() != nblk : (nblk = t->numel()) == 0)) return false;
+            blocks[i] = t;
             f[i] = (float *)t->data_ptr();
         }
         block = n / nblk;
@@ -446,9 +447,60 @@ PyObject *adam8_param(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     return a[11];
 }
 
-// grad ... max2, beta1, beta2, eps, step_size, codes, scales, zeros, N, K, seed, offset -> new codes
+// Steps of several parameters that one launch will run: what is queued, on which stream, and the tensors it works on
+#define ADAM_STATE(s) (s).s1, (s).s2, (s).blocks[0], (s).blocks[1], (s).blocks[2], (s).blocks[3]
+struct AdamQueue {
+    void *items = nullptr;
+    void *stream = nullptr;
+    c10::Device device{c10::kCPU};
+    std::vector<at::Tensor> keep;
+    ~AdamQueue() { lq_adam8_queue_free(items); }
+    static constexpr const char *kName = "adam8_queue";
+
+    // The queue to append to, or null to run the step now: no queue given, or one of another stream or device. The tensors
+    // stay referenced until the queue is run.
+    static void *take(PyObject *o, const On &on, const at::Tensor &like, std::initializer_list<const at::Tensor *> used) {
+        if (!PyCapsule_IsValid(o, kName)) return nullptr;
+        AdamQueue *q = static_cast<AdamQueue *>(PyCapsule_GetPointer(o, kName));
+        if (q->keep.empty()) {
+            q->stream = on.stream;
+            q->device = like.device();
+        }
+        if (q->stream != on.stream || q->device != like.device()) return nullptr;
+        for (const at::Tensor *t : used) q->keep.push_back(*t);
+        return q->items;
+    }
+};
+
+// -> a queue
+PyObject *adam8_queue(PyObject *, PyObject *const *, Py_ssize_t nargs) {
+    LQ_ARGS(0)
+    AdamQueue *q = new AdamQueue;
+    if (lq_adam8_queue_new(&q->items) != LQ_OK) {
+        delete q;
+        return PyErr_NoMemory();
+    }
+    PyObject *o = PyCapsule_New(q, AdamQueue::kName, [](PyObject *c) { delete static_cast<AdamQueue *>(PyCapsule_GetPointer(c, AdamQueue::kName)); });
+    if (!o) delete q;
+    return o;
+}
+
+// queue ->: runs what is in it
+PyObject *adam8_run(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
+    LQ_ARGS(1)
+    AdamQueue *q = static_cast<AdamQueue *>(PyCapsule_GetPointer(a[0], AdamQueue::kName));
+    if (!q) return nullptr;
+    if (q->keep.empty()) return none();
+    c10::OptionalDeviceGuard guard(q->device);
+    std::vector<at::Tensor> keep;  // until the launches are out
+    keep.swap(q->keep);
+    LQ_CALL(lq_adam8_queue_run, q->items, q->stream);
+    return none();
+}
+
+// grad ... max2, beta1, beta2, eps, step_size, codes, scales, zeros, N, K, seed, offset, queue -> new codes
 PyObject *adam8_sr(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    LQ_ARGS(18)
+    LQ_ARGS(19)
     Adam s;
     double v[4];
     const int64_t N = integer(a[14]), K = integer(a[15]);
@@ -457,8 +509,9 @@ PyObject *adam8_sr(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     const uint64_t seed = PyLong_AsUnsignedLongLongMask(a[16]), offset = PyLong_AsUnsignedLongLongMask(a[17]);
     On on(*s.grad);
     at::Tensor out = at::empty_like(*w.codes);
-    LQ_CALL(lq_adam8_sr_step, s.grad->data_ptr(), w.codes->data_ptr(), out.data_ptr(), w.scales->data_ptr(), w.zeros->data_ptr(), s.p1(),
-            s.p2(), s.f[0], s.f[1], s.f[2], s.f[3], N, K, LQ_GROUP, (int)s.block, v[0], v[1], v[2], v[3], seed, offset, on.stream);
+    void *queue = AdamQueue::take(a[18], on, *s.grad, {s.grad, w.codes, &out, w.scales, w.zeros, ADAM_STATE(s)});
+    LQ_CALL(lq_adam8_sr_step_queued, s.grad->data_ptr(), w.codes->data_ptr(), out.data_ptr(), w.scales->data_ptr(), w.zeros->data_ptr(), s.p1(),
+            s.p2(), s.f[0], s.f[1], s.f[2], s.f[3], N, K, LQ_GROUP, (int)s.block, v[0], v[1], v[2], v[3], seed, offset, on.stream, queue);
     return wrap(std::move(out));
 }
 
@@ -479,9 +532,9 @@ struct Curve {
     }
 };
 
-// grad ... max2, beta1, beta2, eps, step_size, codes, scales, zeros, N, K, residual, dequant curve, quant curve -> codes
+// grad ... max2, beta1, beta2, eps, step_size, codes, scales, zeros, N, K, residual, dequant curve, quant curve, queue -> codes
 PyObject *adam8_w4(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    LQ_ARGS(19)
+    LQ_ARGS(20)
     Adam s;
     double v[4];
     const int64_t N = integer(a[14]), K = integer(a[15]);
@@ -492,16 +545,17 @@ PyObject *adam8_w4(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
         !q.load(a[18]) || !same_device(s.grad, w.codes) || !same_device(s.grad, r))
         return none();
     On on(*s.grad);
-    LQ_CALL(lq_adam8_latent_w4_step, s.grad->data_ptr(), w.codes->data_ptr(), (int32_t *)r->data_ptr(), w.scales->data_ptr(),
+    void *queue = AdamQueue::take(a[19], on, *s.grad, {s.grad, w.codes, r, w.scales, w.zeros, ADAM_STATE(s)});
+    LQ_CALL(lq_adam8_latent_w4_step_queued, s.grad->data_ptr(), w.codes->data_ptr(), (int32_t *)r->data_ptr(), w.scales->data_ptr(),
             w.zeros->data_ptr(), s.p1(), s.p2(), s.f[0], s.f[1], s.f[2], s.f[3], N, K, LQ_GROUP, (int)s.block, d.k1, d.b1, d.k2, d.b2,
-            d.k3, q.k1, q.b1, q.k2, q.b2, q.k3, v[0], v[1], v[2], v[3], on.stream);
+            d.k3, q.k1, q.b1, q.k2, q.b2, q.k3, v[0], v[1], v[2], v[3], on.stream, queue);
     Py_INCREF(a[11]);
     return a[11];
 }
 
-// grad ... max2, beta1, beta2, eps, step_size, codes, qscales, residual, dequant curve, quant curve -> codes
+// grad ... max2, beta1, beta2, eps, step_size, codes, qscales, residual, dequant curve, quant curve, queue -> codes
 PyObject *adam8_w8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    LQ_ARGS(16)
+    LQ_ARGS(17)
     Adam s;
     double v[4];
     Curve d, q;
@@ -510,9 +564,10 @@ PyObject *adam8_w8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
         !sized(r, s.n / 8) || !d.load(a[14]) || !q.load(a[15]) || !same_device(s.grad, c) || !same_device(s.grad, qs) || !same_device(s.grad, r))
         return none();
     On on(*s.grad);
-    LQ_CALL(lq_adam8_latent_w8_step, s.grad->data_ptr(), (int8_t *)c->data_ptr(), (int32_t *)r->data_ptr(), qs->data_ptr(), s.p1(), s.p2(),
+    void *queue = AdamQueue::take(a[16], on, *s.grad, {s.grad, c, r, qs, ADAM_STATE(s)});
+    LQ_CALL(lq_adam8_latent_w8_step_queued, s.grad->data_ptr(), (int8_t *)c->data_ptr(), (int32_t *)r->data_ptr(), qs->data_ptr(), s.p1(), s.p2(),
             s.f[0], s.f[1], s.f[2], s.f[3], c->size(0), c->size(1), (int)s.block, d.k1, d.b1, d.k2, d.b2, d.k3, q.k1, q.b1, q.k2, q.b2,
-            q.k3, v[0], v[1], v[2], v[3], on.stream);
+            q.k3, v[0], v[1], v[2], v[3], on.stream, queue);
     Py_INCREF(a[11]);
     return a[11];
 }
@@ -548,7 +603,7 @@ PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     LQ_METHOD(linear4), LQ_METHOD(dx4), LQ_METHOD(gate_up), LQ_METHOD(dx_silu), LQ_METHOD(dx_pair), LQ_METHOD(linear8), LQ_METHOD(infer8),
     LQ_METHOD(dx8), LQ_METHOD(quant8), LQ_METHOD(quant8_token), LQ_METHOD(dequant8), LQ_METHOD(weight_grad),
-    LQ_METHOD(weight_grad_acc), LQ_METHOD(weight_grad_acc8), LQ_METHOD(gradq8), LQ_METHOD(adam8_param), LQ_METHOD(adam8_sr),
+    LQ_METHOD(weight_grad_acc), LQ_METHOD(weight_grad_acc8), LQ_METHOD(gradq8), LQ_METHOD(adam8_param), LQ_METHOD(adam8_sr), LQ_METHOD(adam8_queue), LQ_METHOD(adam8_run),
     LQ_METHOD(adam8_w4), LQ_METHOD(adam8_w8), LQ_METHOD(current_stream), LQ_METHOD(set_error), {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_lqbind", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

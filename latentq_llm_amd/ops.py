@@ -518,18 +518,19 @@ def act_dequant_i8(x8, scale, per_token: bool):
 
 
 def adam8_update(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size, param=None,
-                 direction=None, requant=None):
+                 direction=None, requant=None, queue=None):
     """One Adam step on uint8 block-wise moments (all updated in place). One of ``param`` (bf16, updated in
     place: param -= step_size * m / d), ``direction`` (bf16, receives m / d) and ``requant`` is given: the last is
     (codes, scales, zeros, shape, seed, offset) of a stochastic-rounding layer, whose new codes are returned, those of
-    ``requant_sr`` on the direction with lr = step_size (lq_adam8_sr_step)."""
+    ``requant_sr`` on the direction with lr = step_size (lq_adam8_sr_step); with a queue (adam8_queue) they are written when
+    it is run."""
     r = None
     if direction is None and (param is None) != (requant is None):
         moments = (grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size)
         if requant is None:
             r = (_native or _fast()).adam8_param(*moments, param)
         else:
-            r = (_native or _fast()).adam8_sr(*moments, *requant[:3], *requant[3], *requant[4:])
+            r = (_native or _fast()).adam8_sr(*moments, *requant[:3], *requant[3], *requant[4:], queue)
     if r is not None:
         return r
     _chk(grad, torch.bfloat16, "grad")
@@ -595,15 +596,26 @@ def adam8_ratio(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, 
     return out
 
 
+def adam8_queue():
+    """A queue for the steps of several parameters (adam8_update with requant, adam8_latent_w4_step, adam8_latent_w8_step):
+    adam8_run launches what is in it, up to eight parameters at a time. Until then nothing else may touch the tensors; the
+    queue holds them."""
+    return (_native or _fast()).adam8_queue()
+
+
+def adam8_run(queue) -> None:
+    (_native or _fast()).adam8_run(queue)
+
+
 def adam8_latent_w4_step(grad, codes, residual_int, scales, zeros, shape, state1, state2, scale1, max1, scale2, max2,
-                         dequant_curve, quant_curve, beta1, beta2, eps, step_size):
+                         dequant_curve, quant_curve, beta1, beta2, eps, step_size, queue=None):
     """The Adam step of an lbit = 4 layer in one pass: codes (packed, N*K/2 bytes), residual_int
     (int32[N*K/8]) and the uint8 moments with their block parameters are all updated in place.
     The curves are (k1, b1, k2, b2, k3) tuples: the one the residual was stored with and the
     current one."""
     N, K = shape
     r = (_native or _fast()).adam8_w4(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size, codes, scales,
-                                      zeros, N, K, residual_int, dequant_curve, quant_curve)
+                                      zeros, N, K, residual_int, dequant_curve, quant_curve, queue)
     if r is not None:
         return r
     _chk(grad, torch.bfloat16, "grad")
@@ -638,12 +650,12 @@ def adam8_latent_w4_step(grad, codes, residual_int, scales, zeros, shape, state1
 
 
 def adam8_latent_w8_step(grad, codes, residual_int, qscales, state1, state2, scale1, max1, scale2, max2,
-                         dequant_curve, quant_curve, beta1, beta2, eps, step_size):
+                         dequant_curve, quant_curve, beta1, beta2, eps, step_size, queue=None):
     """The Adam step of an 8-bit-weight layer in lbit = 4 mode in one pass: codes (int8 [N, K]), residual_int
     (int32[N*K/8]) and the uint8 moments with their block parameters are all updated in place; qscales bf16 [N].
     The curves are (k1, b1, k2, b2, k3) tuples: the one the residual was stored with and the current one."""
     r = (_native or _fast()).adam8_w8(grad, state1, state2, scale1, max1, scale2, max2, beta1, beta2, eps, step_size, codes, qscales,
-                                      residual_int, dequant_curve, quant_curve)
+                                      residual_int, dequant_curve, quant_curve, queue)
     if r is not None:
         return r
     _chk(grad, torch.bfloat16, "grad")

@@ -1087,6 +1087,8 @@ class MyAdam(torch.optim.Adam):
 
     ``sr_seed`` seeds the Philox stream of that requantizer; every call consumes N*K/8 counters."""
 
+    _in_step, _queue = False, None  # the fused steps of the step() under way, launched together at its end
+
     def __init__(self, params, lr=1e-3, betas=(0.9, 0.999), obit=8, mu_updata_f=20, cpu=False, sr_seed=0):
         super().__init__(params, lr=lr, betas=betas)
         self.initialized = False
@@ -1124,15 +1126,30 @@ class MyAdam(torch.optim.Adam):
             with torch.enable_grad():
                 loss = closure()
         self._chosen = self._choose_curves()
-        for gindex, group in enumerate(self.param_groups):
-            for pindex, p in enumerate(group["params"]):
-                if p.grad is None:
-                    continue
-                if len(self.state[p]) == 0:
-                    self.init_state(group, p, gindex, pindex)
-                self.update_step(group, p, gindex, pindex)
+        self._in_step, done = True, 0
+        try:
+            for gindex, group in enumerate(self.param_groups):
+                for pindex, p in enumerate(group["params"]):
+                    if p.grad is None:
+                        continue
+                    if len(self.state[p]) == 0:
+                        self.init_state(group, p, gindex, pindex)
+                    self.update_step(group, p, gindex, pindex)
+                    done += 1
+                    if done % 8 == 0 and self._queue is not None:  # a launch's worth: the device need not wait for the rest
+                        ops.adam8_run(self._queue)
+        finally:
+            queue, self._queue, self._in_step = self._queue, None, False
+            if queue is not None:
+                ops.adam8_run(queue)
         self._chosen = frozenset()
         return loss
+
+    def _step_queue(self):
+        """The queue of the step() under way; None where update_step is called by itself."""
+        if self._in_step and self._queue is None:
+            self._queue = ops.adam8_queue()
+        return self._queue
 
     def to_gpu(self):
         for group in self.param_groups:
@@ -1276,7 +1293,7 @@ class MyAdam(torch.optim.Adam):
                 requant = (p.data, scales, zeros, shape, self.sr_seed, self.sr_offset)
             new = ops.adam8_update(grad, state["state1"], state["state2"], state["qmap1"], state["absmax1"], state["qmap2"],
                                    state["absmax2"], beta1, beta2, group["eps"], step_size,
-                                   param=None if sr_mode else pdata, requant=requant)
+                                   param=None if sr_mode else pdata, requant=requant, queue=self._step_queue() if sr_mode else None)
             if sr_mode:
                 p.data = new
                 self.sr_offset += (p.numel() + 7) // 8
@@ -1352,7 +1369,7 @@ class MyAdam(torch.optim.Adam):
             q1, z1, q2, z2 = three_fold_curve_4bit(r.mu)
             ops.adam8_latent_w8_step(grad, p.data, r.residual_int.view(-1), qs.view(-1), *moments,
                                      (p1, y1, p2 - p1, y2, 8 - p2), (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2,
-                                     group["eps"], step_size)
+                                     group["eps"], step_size, self._step_queue())
             r.weight_scale = qs
             r.lock_mu = r.mu
             self._release_grad(p)
@@ -1369,7 +1386,7 @@ class MyAdam(torch.optim.Adam):
         q1, z1, q2, z2 = three_fold_curve_4bit(r.mu)
         ops.adam8_latent_w4_step(grad, p.data, r.residual_int.view(-1), scales, zeros, tuple(shape), *moments,
                                  (p1, y1, p2 - p1, y2, 8 - p2), (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2,
-                                 group["eps"], step_size)
+                                 group["eps"], step_size, self._step_queue())
         r.weight_scale = scales.contiguous().reshape(-1, 1)
         r.lock_mu = r.mu
         self._release_grad(p)
