@@ -91,6 +91,24 @@ __device__ __forceinline__ void lq_dequant_word_f32(unsigned word, float s512, f
     f[6] = fmaf(e1[1], s512, nzs); f[7] = fmaf(o1[1], s512, nzs);
 }
 
+// The same codes as an MFMA operand that needs no rounding: q - zi for an integer zi of at most 240, exact in bf16. A zero
+// point z is zi plus a remainder that is bf16 itself (0 for integer zeros; z, with zi = 0, for larger ones, infinities and NaN):
+//   sum_k x (q - z) = sum_k x (q - zi) + sum_k x (-rest)
+__device__ __forceinline__ void lq_split_zero(float z, float &zi, float &rest) {
+    zi = fabsf(z) <= 240.0f ? rintf(z) : 0.0f;
+    rest = z - zi;
+}
+__device__ __forceinline__ u32x4_t lq_codes_minus(unsigned word, float zi) {
+    float f[8];
+    lq_dequant_word_f32(word, 512.0f, -zi, f);
+    return u32x4_t{lq_pack_bf16(f[0], f[1]), lq_pack_bf16(f[2], f[3]), lq_pack_bf16(f[4], f[5]), lq_pack_bf16(f[6], f[7])};
+}
+// -rest in every place of an operand
+__device__ __forceinline__ u32x4_t lq_minus_rest(float rest) {
+    const unsigned w = lq_pack_bf16(-rest, -rest);
+    return u32x4_t{w, w, w, w};
+}
+
 // ---- Philox4x32-10 ---------------------------------------------------------
 #define LQ_PHILOX_M0 0xD2511F53u
 #define LQ_PHILOX_M1 0xCD9E8D57u

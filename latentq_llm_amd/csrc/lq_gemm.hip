@@ -704,7 +704,7 @@ int lq_gemv_i8_launch(const void *x8, const void *w8, const float *sx, const voi
 // both operands staged, for few workgroups (lq_gemm_staged.hip)
 double lq_gemm_staged_plan(long long M, long long N, int groups, size_t ws_bytes, long long cus, int *rows, int *splits, int *per_split);
 int lq_gemm_staged_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y,
-                          float *partial, int M, int N, int K, int rows, int splits, int per_split, hipStream_t st,
+                          float *partial, int M, int N, int K, int rows, bool exact, int splits, int per_split, hipStream_t st,
                           unsigned long long *clk, const char *who);
 
 int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *scales_g, const void *zeros_g, const void *codes_u,
@@ -781,12 +781,15 @@ struct W4Plan {
     int kernel = LQ_PLAN_STAGED_128;
     int splits = 1, steps_per_split = 0;
     int rows = 128;  // forward LQ_PLAN_STAGED_128: rows of the tile (32, 64 or 128), 128 columns
+    bool exact = false;  // and weights not rounded to bf16
 };
 
 // Forward pass, M > 16. Up to 64 tokens, with 16 columns for each of more than half of the units and at most all of them:
 // the kernel of lq_gemm_few.hip where its time, which grows with the tokens' bytes each unit takes in (2 us + 0.5 us per 1000 k
 // + 0.42 per 16 tokens and 1000 k, less with fewer units asking; 12 % rms over 64 timings), is under the staged kernel's
-// estimate. Otherwise by the number of 128 x 128 output tiles T:
+// estimate. Otherwise, up to 64 tokens the staged kernel on any number of tiles, with weights that are not rounded to bf16
+// (several workgroups to a unit: 32 tokens, 16400 x 4096 23.8 against 35.7 us of the weights-direct kernel, 32000 x 4096 27.1
+// against 40.2, 40960 x 768 10.8 against 16.3), and beyond by the number of 128 x 128 output tiles T:
 //   T <= half of the units             the staged kernel, which plans its row tile and its slices of K itself
 //                                      (1.2 to 1.6 times the speed of the weights-direct kernels there: 11.5 against
 //                                      15.0 us on 1024 x 1536 x 1536, 23.6 against 34 on 384 x 4096 x 4096; level at
@@ -825,10 +828,14 @@ static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, l
     }
     const int groups = (int)(K / LQ_GROUP);
     const long long tiles = (M + 127) / 128 * ((N + 127) / 128);
-    if (tiles * 2 <= cus) {
+    if (M <= 64 || tiles * 2 <= cus) {
         int per = 0;
         lq_gemm_staged_plan(M, N, groups, ws_bytes, cus, &out.rows, &out.splits, &per);
         if (out.splits > 1) out.steps_per_split = 2 * per;
+        // weights as they are for every call that GEMV launches served before, by the estimates of that time (up to 64 tokens
+        // with a workspace, 128 without)
+        out.exact = M <= 64 || (M <= 128 && ws_bytes == 0);
+        if (out.exact && out.rows == 128) out.rows = 64;
         return out;
     }
     if (tiles <= cus && (groups % 2 != 0 || K >= 8192)) return out;  // whole, 128 rows
@@ -909,7 +916,7 @@ static int a16w4_fwd_impl(const char *who, const void *x, const void *codes, con
         return lq_gemm_fwd_direct_launch(x, codes, scales, zeros, bias_or_null, y, (int)M, (int)N, (int)K, (hipStream_t)stream, clk,
                                          plan.kernel == LQ_PLAN_DIRECT_128);
     if (plan.kernel == LQ_PLAN_STAGED_128) {
-        rc = lq_gemm_staged_launch(x, codes, scales, zeros, bias_or_null, y, (float *)workspace, (int)M, (int)N, (int)K, plan.rows,
+        rc = lq_gemm_staged_launch(x, codes, scales, zeros, bias_or_null, y, (float *)workspace, (int)M, (int)N, (int)K, plan.rows, plan.exact,
                                    plan.splits, plan.steps_per_split / 2, (hipStream_t)stream, clk, who);
         if (rc || plan.splits < 2) return rc;
         return launch_split_reduce((const float *)workspace, bias_or_null, y, M, N, plan.splits, (hipStream_t)stream, who);

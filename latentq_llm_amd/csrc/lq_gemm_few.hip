@@ -20,8 +20,12 @@
 // X arrives at 30 bytes a clock and unit, half of what L2 gives a unit reading alone; letting the units start at different
 // groups changes nothing.
 //
-// MFMA 16x16x32, weights first: lane l holds columns 4 (l / 16) .. + 3 of token l % 16. With r = l % 16, h = l / 16 slice w = 0..3 of
-// a group has the lane's operands at k = 32 h + 8 w .. + 7: word w of the 16 bytes of codes of row r, and a 16-byte piece of X.
+// Weights are not rounded to bf16, as they are not in the GEMV (lq_gemv.hip), which ran most of these sizes before: the operand
+// is q - rint(z), exact in bf16, and the scale is applied in fp32 to the sum of a group.
+//
+// MFMA 16x16x32, activations first: lane l holds column l % 16 of tokens 4 (l / 16) .. + 3, so that the scale is one
+// number. With r = l % 16, h = l / 16 slice w = 0..3 of a group has the lane's operands at k = 32 h + 8 w .. + 7: word w of
+// the 16 bytes of codes of row r, and a 16-byte piece of X.
 #include "lq_common.h"
 
 #include <type_traits>
@@ -102,7 +106,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(FewParams p) {
         const u32x4_t c = *reinterpret_cast<const u32x4_t *>(st + A_BYTES + r * 64 + ((h ^ ((r >> 2) & 3)) << 4));
         const unsigned *q = reinterpret_cast<const unsigned *>(st + A_BYTES + 1024);
         const float sc = __uint_as_float(q[r] << 16);
-        const float nzs = -(__uint_as_float(q[16 + r] << 16) * sc), s512 = sc * 512.0f;
+        float zi, rest;
+        lq_split_zero(__uint_as_float(q[16 + r] << 16), zi, rest);
         u32x4_t x[4][MT];
 #pragma unroll
         for (int w = 0; w < 4; ++w)
@@ -113,15 +118,25 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(FewParams p) {
         __builtin_amdgcn_sched_barrier(0);
         issue(wave + kWaves * (i + D < ng ? i + D : ng - 1), st);
         __builtin_amdgcn_sched_barrier(0);
+        f32x4_t P[MT];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            float f[8];
-            lq_dequant_word_f32(c[w], s512, nzs, f);
-            const u32x4_t b = {lq_pack_bf16(f[0], f[1]), lq_pack_bf16(f[2], f[3]), lq_pack_bf16(f[4], f[5]), lq_pack_bf16(f[6], f[7])};
+        for (int j = 0; j < MT; ++j) P[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        auto add = [&](int w, const u32x4_t &b) {
 #pragma unroll
             for (int j = 0; j < MT; ++j)
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, x[w][j]), acc[j], 0, 0, 0);
+                P[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[w][j]), __builtin_bit_cast(bf16x8_t, b), P[j], 0, 0, 0);
+        };
+#pragma unroll
+        for (int w = 0; w < 4; ++w) add(w, lq_codes_minus(c[w], zi));
+        if (__builtin_amdgcn_ballot_w64(rest != 0.0f)) {
+            const u32x4_t b = lq_minus_rest(rest);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) add(w, b);
         }
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[j][e] = fmaf(sc, P[j][e], acc[j][e]);
         __builtin_amdgcn_sched_barrier(0);
     };
     if (ng > 0) {
@@ -145,7 +160,9 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(FewParams p) {
     // ---- partial sums [wave][token][16 columns]
     float *part = reinterpret_cast<float *>(lds);
 #pragma unroll
-    for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4_t *>(part + ((wave * MT + j) * 16 + r) * 16 + 4 * h) = acc[j];
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[((wave * MT + j) * 16 + 4 * h + e) * 16 + r] = acc[j][e];
     __syncthreads();
     for (int q = threadIdx.x; q < MT * 64; q += 64 * kWaves) {
         const int m = q >> 2, c = c0 + 4 * (q & 3);

@@ -6,8 +6,14 @@
 // does about it:
 //   * a stage is a whole group of 128 k (activations, codes, scales and zeros, all by LDS-direct loads), three stages
 //     deep: two groups of loads are in flight while one is multiplied, with one barrier per 128 k;
-//   * codes stay packed in LDS (64 bytes per column and group) and each of the four waves dequantises the 32 columns
+//   * codes stay packed in LDS (64 bytes per column and group) and each of the four waves converts the 32 columns
 //     it multiplies, in registers: no second trip through LDS and no waves that only convert;
+//   * a plain product of up to 64 tokens (128 without a workspace) does not round its weights to bf16, since the GEMV, which
+//     ran many of these sizes before, does not either: the operand is the integer q - rint(z), exact in bf16, and the scale is
+//     applied in fp32 to the sum of a group. Zeros that are no integers of at most 240 add a second product with the
+//     remainder (`rest` below). Against the weights as they are a result is 1.66e-3 off, its own rounding, instead of 2.22e-3;
+//     it takes 2 to 6 % longer (32 / 64 tokens, 11008 x 4096: 17.1 / 19.7 -> 17.7 / 20.7 us, 4096 x 11008: 17.0 / 19.4 -> 17.4 /
+//     20.1; with 128 rows it would be 20 %);
 //   * the row tile is 32, 64 or 128 tokens, so that few tokens are not mostly padding; the planner below picks it
 //     together with the number of slices of K.
 // Bound: LDS reads for 128 rows (one 16-byte fragment read per MFMA), the latency of the chain for 32 and 64.
@@ -55,8 +61,10 @@ constexpr int D = 3;
 //   codes        128 rows of 64 bytes,   chunk c of row i at c ^ ((i >> 2) & 3)
 //   scales, zeros  one dword per column each, the bf16 value in its lower half
 // FM: 32-row fragments of the row tile (32 FM rows)
-template <int FM>
-__global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
+// EXACT: weights as they are (see the top of the file), else rounded to bf16 like those of the kernels for more tokens
+// (launch bounds: with two waves per SIMD asked for, the products of FM < 4 go to vector registers, which the scaling can read)
+template <int FM, bool EXACT>
+__global__ __launch_bounds__(256, FM < 4 ? 2 : 1) void gemm_staged_kernel(StagedParams p) {
     constexpr int BM = 32 * FM;
     constexpr int A_BYTES = BM * 256;
     constexpr int STAGE = A_BYTES + kCodeBytes + kScaleBytes;
@@ -142,23 +150,36 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
             af[j] = *reinterpret_cast<const u32x4_t *>(st + (32 * j + r) * 256 + ((chunk ^ (r & 15)) << 4));
     };
     const int crow = 32 * wave + r;
-    auto read_codes = [&](const unsigned char *st, u32x4_t *c, float &s512, float &nzs) {
+    auto read_codes = [&](const unsigned char *st, u32x4_t *c, float &sc, float &zi, float &rest) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
             c[s] = *reinterpret_cast<const u32x4_t *>(st + A_BYTES + crow * 64 + (((2 * s + h) ^ ((crow >> 2) & 3)) << 4));
         const unsigned *q = reinterpret_cast<const unsigned *>(st + A_BYTES + kCodeBytes);
-        const float sc = __uint_as_float(q[crow] << 16);
-        nzs = -(__uint_as_float(q[kCols + crow] << 16) * sc);
-        s512 = sc * 512.0f;
+        const float z = __uint_as_float(q[kCols + crow] << 16);
+        sc = __uint_as_float(q[crow] << 16);
+        if constexpr (EXACT) {
+            lq_split_zero(z, zi, rest);
+        } else {  // operands of lq_dequant_word_f32
+            zi = -(z * sc);
+            sc *= 512.0f;
+        }
     };
-    auto deq = [&](unsigned word, float s512, float nzs) {
+    auto operand = [](unsigned word, float sc, float zi) {
+        if constexpr (EXACT) return lq_codes_minus(word, zi);
         float f[8];
-        lq_dequant_word_f32(word, s512, nzs, f);
+        lq_dequant_word_f32(word, sc, zi, f);
         return u32x4_t{lq_pack_bf16(f[0], f[1]), lq_pack_bf16(f[2], f[3]), lq_pack_bf16(f[4], f[5]), lq_pack_bf16(f[6], f[7])};
     };
 
     u32x4_t af[2][FM], bf[2], cw[2];
-    float s512, nzs;
+    f32x16_t P[FM];  // EXACT: the group's sums, unscaled
+    float sc, zi, rest;
+    auto mfma = [](const u32x4_t &a, const u32x4_t &b, const f32x16_t &c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+    };
+    f32x16_t zero;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) zero[q] = 0.f;
     auto group = [&](int g, auto si) {
         constexpr int S = decltype(si)::value;
         unsigned char *cur = lds + S * STAGE, *nxt = lds + ((S + 1) % D) * STAGE, *fill = lds + ((S + D - 1) % D) * STAGE;
@@ -166,9 +187,10 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const unsigned word_next = t < 7 ? cw[(t + 1) >> 2][(t + 1) & 3] : 0u;
+            const float sc_cur = sc;
             if (t == 7) {
                 asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 2) * LOADS) : "memory");
-                read_codes(nxt, cw, s512, nzs);
+                read_codes(nxt, cw, sc, zi, rest);
                 read_a(nxt, 0, af[0]);
             } else {
                 read_a(cur, t + 1, af[(t + 1) & 1]);
@@ -179,11 +201,29 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < FM; ++j)
-                acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, bf[t & 1]),
-                                                                 __builtin_bit_cast(bf16x8_t, af[t & 1][j]), acc[j], 0, 0, 0);
-            if (t < 7) bf[(t + 1) & 1] = deq(word_next, s512, nzs);
-            else bf[0] = deq(cw[0][0], s512, nzs);
+            for (int j = 0; j < FM; ++j) {
+                if constexpr (EXACT) P[j] = mfma(af[t & 1][j], bf[t & 1], t ? P[j] : zero);
+                else acc[j] = mfma(af[t & 1][j], bf[t & 1], acc[j]);
+            }
+            bf[(t + 1) & 1] = operand(t < 7 ? word_next : cw[0][0], sc, zi);
+            if constexpr (EXACT) {
+                if (t == 6 && __builtin_amdgcn_ballot_w64(rest != 0.0f)) {
+                    const u32x4_t b = lq_minus_rest(rest);
+#pragma unroll 1
+                    for (int v = 0; v < 8; ++v) {
+                        u32x4_t a[FM];
+                        read_a(cur, v, a);
+#pragma unroll
+                        for (int j = 0; j < FM; ++j) P[j] = mfma(a[j], b, P[j]);
+                    }
+                }
+                if (t == 7) {
+#pragma unroll
+                    for (int j = 0; j < FM; ++j)
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) acc[j][q] = fmaf(sc_cur, P[j][q], acc[j][q]);
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -194,9 +234,9 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) issue(g0 + (d < ng ? d : ng - 1), lds + d * STAGE, i);
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 2) * LOADS) : "memory");
-    read_codes(lds, cw, s512, nzs);
+    read_codes(lds, cw, sc, zi, rest);
     read_a(lds, 0, af[0]);
-    bf[0] = deq(cw[0][0], s512, nzs);
+    bf[0] = operand(cw[0][0], sc, zi);
     __builtin_amdgcn_sched_barrier(0);
     static_assert(D == 3, "the loop below names the three stages");
     int g = 0;
@@ -209,20 +249,18 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
     if (g + 1 < ng) group(g + 1, ic<1>());
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped prefetches of the last groups
 
-    // ---- epilogue: acc[j][q]: row m0 + 32 j + r, column c0 + 32 wave + 8 (q / 4) + 4 h + q % 4
+    // ---- epilogue: acc[j][q]: row m0 + 32 j + 8 (q / 4) + 4 h + q % 4, column c0 + 32 wave + r
+    const int c_mine = c0 + 32 * wave + r;
     if (p.partial) {
         float *part = p.partial + (long long)(blockIdx.z * gridDim.y + blockIdx.y) * p.M * p.N;
+        if (c_mine < p.N) {
 #pragma unroll
-        for (int j = 0; j < FM; ++j) {
-            const int m = m0 + 32 * j + r;
-            if (m >= p.M) continue;
+            for (int j = 0; j < FM; ++j)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int c = c0 + 32 * wave + 8 * q + 4 * h;
-                if (c >= p.N) continue;
-                *reinterpret_cast<f32x4_t *>(part + (long long)m * p.N + c) =
-                    f32x4_t{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
-            }
+                for (int q = 0; q < 16; ++q) {
+                    const int m = m0 + 32 * j + 8 * (q >> 2) + 4 * h + (q & 3);
+                    if (m < p.M) part[(long long)m * p.N + c_mine] = acc[j][q];
+                }
         }
         return;
     }
@@ -231,23 +269,13 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
     unsigned char *ep = lds + wave * (32 * EP);
     const int ep_row = lane >> 2, ep_chunk = lane & 3;
     const int c_lane = c0 + 32 * wave + ep_chunk * 8;
-    float b[4][4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int c = c0 + 32 * wave + 8 * q + 4 * h + e;
-            b[q][e] = (p.bias && c < p.N) ? lq_bf16_bits_to_f32(p.bias[c]) : 0.0f;
-        }
+    const float bias = p.bias && c_mine < p.N ? lq_bf16_bits_to_f32(p.bias[c_mine]) : 0.0f;
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = p.bias ? acc[j][4 * q + e] + b[q][e] : acc[j][4 * q + e];
-            *reinterpret_cast<u32x2_t *>(ep + r * EP + (8 * q + 4 * h) * 2) = u32x2_t{lq_pack_bf16(v[0], v[1]), lq_pack_bf16(v[2], v[3])};
-        }
+        for (int q = 0; q < 16; ++q)
+            *reinterpret_cast<unsigned short *>(ep + (8 * (q >> 2) + 4 * h + (q & 3)) * EP + r * 2) =
+                lq_f32_to_bf16_bits(p.bias ? acc[j][q] + bias : acc[j][q]);
 #pragma unroll
         for (int it = 0; it < 2; ++it) {
             const int row = it * 16 + ep_row, m = m0 + 32 * j + row;
@@ -261,12 +289,19 @@ __global__ __launch_bounds__(256) void gemm_staged_kernel(StagedParams p) {
     }
 }
 
-template <int FM>
-int launch_staged(StagedParams p, int splits, hipStream_t st, const char *who) {
+template <int FM, bool EXACT>
+int launch_staged_tile(StagedParams p, int splits, hipStream_t st, const char *who) {
     p.tiles_m = (p.M + 32 * FM - 1) / (32 * FM);
     p.tiles_n = (p.N + kCols - 1) / kCols;
-    hipLaunchKernelGGL(gemm_staged_kernel<FM>, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits, p.w2 ? 2u : 1u), dim3(256), 0, st, p);
+    const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits, p.w2 ? 2u : 1u);
+    hipLaunchKernelGGL((gemm_staged_kernel<FM, EXACT>), grid, dim3(256), 0, st, p);
     return lq_check_launch(who);
+}
+
+int launch_staged(const StagedParams &p, int rows, bool exact, int splits, hipStream_t st, const char *who) {
+    if (rows == 32) return exact ? launch_staged_tile<1, true>(p, splits, st, who) : launch_staged_tile<1, false>(p, splits, st, who);
+    if (rows == 64) return exact ? launch_staged_tile<2, true>(p, splits, st, who) : launch_staged_tile<2, false>(p, splits, st, who);
+    return launch_staged_tile<4, false>(p, splits, st, who);
 }
 
 }  // namespace
@@ -321,15 +356,14 @@ int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *s
     p.w2 = (const unsigned char *)codes_u; p.scales2 = (const unsigned short *)scales_u; p.zeros2 = (const unsigned short *)zeros_u;
     p.M = M; p.N = N; p.K = K;
     p.partial = partial; p.groups_per_split = per_split;
-    if (rows == 32) return launch_staged<1>(p, splits, st, who);
-    if (rows == 64) return launch_staged<2>(p, splits, st, who);
-    return launch_staged<4>(p, splits, st, who);
+    return launch_staged(p, rows, false, splits, st, who);
 }
 
 // splits > 1: fp32 partial products [splits][M][N] to `partial`, to be added by the caller; else bf16 (x W^T + bias) to y.
-// N % 16 == 0, K % 128 == 0, splits == ceil(K / 128 / per_split) are guaranteed by the caller.
+// exact: weights not rounded to bf16 (32 or 64 rows). N % 16 == 0, K % 128 == 0, splits == ceil(K / 128 / per_split) are
+// guaranteed by the caller.
 int lq_gemm_staged_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y,
-                          float *partial, int M, int N, int K, int rows, int splits, int per_split, hipStream_t st,
+                          float *partial, int M, int N, int K, int rows, bool exact, int splits, int per_split, hipStream_t st,
                           unsigned long long *clk, const char *who) {
     StagedParams p = {};
     p.x = (const unsigned char *)x; p.w = (const unsigned char *)codes;
@@ -337,7 +371,5 @@ int lq_gemm_staged_launch(const void *x, const void *codes, const void *scales, 
     p.bias = (const unsigned short *)bias; p.y = (unsigned short *)y;
     p.M = M; p.N = N; p.K = K; p.clk = clk;
     if (splits > 1) { p.partial = partial; p.groups_per_split = per_split; }
-    if (rows == 32) return launch_staged<1>(p, splits, st, who);
-    if (rows == 64) return launch_staged<2>(p, splits, st, who);
-    return launch_staged<4>(p, splits, st, who);
+    return launch_staged(p, rows, exact, splits, st, who);
 }
