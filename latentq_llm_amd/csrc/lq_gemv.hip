@@ -47,15 +47,17 @@ typedef const __attribute__((address_space(1))) void gbl_void;
 
 constexpr int kUnroll = 4;       // groups per batch (scale/zero batches are 4 x bf16 = 8 bytes)
 constexpr int kXRow = 1024 + 16;  // LDS bytes per staged token row: 4 groups x 256 B, padded against bank conflicts
-
 // MP = number of token rows staged per wave and batch (>= M). NT = 16-row weight tiles per
 // workgroup: every workgroup stages the activations of its K range again, so with many tokens two
 // tiles per workgroup halve that traffic (and share the activation-sum MFMAs).
 // GU (with NT = 2, no QS): gate / up mode. Tile 1 is the same 16 rows of a second matrix (codes2, scales2,
 // zeros2) and the output is silu(tile 0) * tile 1 on the fp32 sums: the gate / up pair of a gated MLP in one
-// pass over both matrices.
-template <int WAVES, int MP, int NT, bool QS, bool GU = false>
-__global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *__restrict__ x,
+// pass over both matrices. There batch b goes into partial sum b % slots, a number that the launcher derives from M and K
+// alone, and a wave works through up to SPW partial sums one after the other: the order of the fp32 sums, and so the bits of
+// the result, do not depend on how many waves the launcher finds best for the grid.
+// (SPW = 2 in at most 128 registers, four waves to a SIMD; more in 168)
+template <int WAVES, int MP, int NT, bool QS, bool GU = false, int SPW = 1>
+__global__ __launch_bounds__(64 * WAVES, SPW == 2 ? 4 : SPW > 2 ? 3 : 1) void gemv_kernel(const unsigned short *__restrict__ x,
                                                           const unsigned char *__restrict__ codes,
                                                           const unsigned short *__restrict__ scales,
                                                           const unsigned short *__restrict__ zeros,
@@ -63,13 +65,18 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
                                                           unsigned short *__restrict__ y, int M, int N, int K,
                                                           const unsigned char *__restrict__ codes2 = nullptr,
                                                           const unsigned short *__restrict__ scales2 = nullptr,
-                                                          const unsigned short *__restrict__ zeros2 = nullptr) {
+                                                          const unsigned short *__restrict__ zeros2 = nullptr, int slots = WAVES) {
     static_assert(!GU || (NT == 2 && !QS), "gate / up mode: two tiles, scales and zeros straight from memory");
     constexpr int RT = GU ? 1 : NT;  // 16-row tiles of output rows per workgroup
-    static_assert(MP * kXRow >= NT * 4 * 64 * 4, "a wave's partial sums fit where its activations were");
-    __shared__ __attribute__((aligned(16))) unsigned char xs[WAVES][MP][kXRow];
-    // a wave's partial sums [tile][4][lane] take the place of the token rows it staged (its reads of them have returned)
-    auto red = [&](int w, int j, int r) -> float & { return reinterpret_cast<float *>(&xs[w][0][0])[(j * 4 + r) * 64 + (threadIdx.x & 63)]; };
+    static_assert(GU || SPW == 1, "several partial sums per wave: gate / up mode only");
+    constexpr int kWaveLds = MP * kXRow > SPW * NT * 1024 ? MP * kXRow : SPW * NT * 1024;
+    __shared__ __attribute__((aligned(16))) unsigned char xs_all[WAVES][kWaveLds];
+    const auto xs = [&](int w, int m) { return &xs_all[w][m * kXRow]; };
+    // partial sums [slot of the wave][tile][4][lane] take the place of the token rows the wave staged (its reads of them
+    // have returned); slot s is slot s / WAVES of wave s % WAVES
+    auto red = [&](int s, int j, int r) -> float & {
+        return reinterpret_cast<float *>(&xs_all[s % WAVES][0])[((s / WAVES * NT + j) * 4 + r) * 64 + (threadIdx.x & 63)];
+    };
     extern __shared__ __attribute__((aligned(16))) unsigned char sq[];  // QS: scales then zeros of the workgroup's rows
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // scalar: uniform control flow
@@ -88,7 +95,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
     const unsigned short *zrow = zeros + (long long)row * G;
     // As an A-fragment lane, `n` is the token index; lanes of tokens >= M re-read the last staged
     // row: they only feed accumulator rows m >= M, which are never stored.
-    const unsigned char *xfrag = &xs[wave][n < M ? n : M - 1][kq * 64];
+    const unsigned char *xfrag = xs(wave, n < M ? n : M - 1) + kq * 64;
 
     const u32x4_t ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
     f32x4_t acc[NT];
@@ -132,7 +139,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
         }
         __syncthreads();
     };
-    for (int g0 = wave * kUnroll; g0 < G; g0 += WAVES * kUnroll) {
+    const int n_slots = GU ? slots : WAVES;
+    f32x4_t done[SPW][NT];  // SPW > 1: the wave's complete partial sums
+#pragma unroll
+    for (int k = 0; k < SPW; ++k)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) done[k][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < SPW; ++i) {
+    const int s = wave + i * WAVES;
+    if (SPW > 1 && s >= n_slots) break;
+    for (int g0 = s * kUnroll; g0 < G; g0 += n_slots * kUnroll) {
         const bool full = g0 + kUnroll <= G;  // a short tail batch re-reads the last group with zero scale
         // ---- activations: one LDS-direct load per token row (1 KB = this batch's 512 k), coalesced.
         //      In a tail batch the lanes past the end of the row re-read its first bytes (dead groups).
@@ -144,7 +160,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
             for (int m = 0; m < MP; ++m)
                 if (m < M)
                     __builtin_amdgcn_global_load_lds((gbl_void *)((const unsigned char *)x + (long long)m * lim + off),
-                                                     (lds_void *)&xs[wave][m][0], 16, 0, 0);
+                                                     (lds_void *)xs(wave, m), 16, 0, 0);
         }
         // ---- codes, scales, zeros
         u32x4_t wv[NT][kUnroll];
@@ -246,14 +262,27 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
         // the next batch overwrites the staged rows: all fragment reads above must have returned
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
+    if constexpr (SPW > 1) {
+#pragma unroll
+        for (int k = 0; k < SPW; ++k)
+            if (i == k) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) done[k][j] = acc[j];
+            }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    }
 
     if constexpr (QS) {
         if (first) publish_q();
     }
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int k = 0; k < SPW; ++k)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red(wave, j, r) = acc[j][r];
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red(wave + k * WAVES, j, r) = SPW > 1 ? done[k][j][r] : acc[j][r];
     __syncthreads();
     if constexpr (GU) {
         if (wave == 0) {
@@ -261,9 +290,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const unsigned short *
             for (int r = 0; r < 4; ++r) {
                 float g = 0.f, u = 0.f;
 #pragma unroll
-                for (int w = 0; w < WAVES; ++w) {
-                    g += red(w, 0, r);
-                    u += red(w, NT - 1, r);
+                for (int s = 0; s < SPW * WAVES; ++s) {  // (those without a batch are zero)
+                    g += red(s, 0, r);
+                    u += red(s, NT - 1, r);
                 }
                 const int m = 4 * kq + r;
                 if (m < M) y[(long long)m * N + row] = lq_f32_to_bf16_bits(g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u);
@@ -299,15 +328,30 @@ struct GemvGuArgs {
     const void *x, *codes, *scales, *zeros, *codes2, *scales2, *zeros2;
     void *y;
     int M, N, K;
+    int slots;
     hipStream_t st;
 };
 
-template <int W, int MP>
-void launch_gu(const GemvGuArgs &a) {
-    hipLaunchKernelGGL((gemv_kernel<W, MP, 2, false, true>), dim3(a.N / 16), dim3(64 * W), 0, a.st, (const unsigned short *)a.x,
+template <int W, int MP, int SPW>
+void launch_gu_spw(const GemvGuArgs &a) {
+    hipLaunchKernelGGL((gemv_kernel<W, MP, 2, false, true, SPW>), dim3(a.N / 16), dim3(64 * W), 0, a.st, (const unsigned short *)a.x,
                        (const unsigned char *)a.codes, (const unsigned short *)a.scales, (const unsigned short *)a.zeros,
                        (const unsigned short *)nullptr, (unsigned short *)a.y, a.M, a.N, a.K, (const unsigned char *)a.codes2,
-                       (const unsigned short *)a.scales2, (const unsigned short *)a.zeros2);
+                       (const unsigned short *)a.scales2, (const unsigned short *)a.zeros2, a.slots);
+}
+
+// Partial sums of a gate / up pass, at most: the waves of the workgroups that stage 4 or 16 rows with one batch each
+constexpr int gu_max_slots(int MP) { return MP == 4 ? 16 : 8; }
+
+template <int W, int MP>
+void launch_gu(const GemvGuArgs &a) {
+    constexpr int kMost = (gu_max_slots(MP) + W - 1) / W;
+    const int batches = (a.K / LQ_GROUP + kUnroll - 1) / kUnroll, used = batches < a.slots ? batches : a.slots;
+    const int spw = (used + W - 1) / W;
+    if (spw <= 1) return launch_gu_spw<W, MP, 1>(a);
+    if constexpr (kMost >= 2)
+        if (spw == 2) return launch_gu_spw<W, MP, 2>(a);
+    if constexpr (MP >= 12 && kMost > 2) launch_gu_spw<W, MP, kMost>(a);
 }
 
 // Waves per workgroup of the gate / up pass, MP staged rows. A grid of c workgroups per CU should be resident at once: the
@@ -318,16 +362,30 @@ void launch_gu(const GemvGuArgs &a) {
 //   8192 x 2560 (c = 2)   8: 13.0 -> 9.3 (5), 12: 13.2 -> 11.0 (3), 16: 13.5 -> 11.3 (3)
 //   6144 x 3072 (c = 2)   8: 12.4 -> 9.5 (6), 12: 12.6 -> 10.4 (3), 16: 12.8 -> 10.8 (3)
 // (12 rows and more on 5 or 6 waves are slower although two such workgroups fit: 6144 x 3072 at 12 tokens 11.7 on 6.)
-int gu_waves(int MP, int N, int batches, int cus) {
+int gu_waves(int MP, int N, int batches, int slots, int cus) {
     const int c = (N / 16 + cus - 1) / cus;
     int most = (160 << 10) / c / (MP * kXRow);
     if (c > 1 && most > 16 / c) most = 16 / c;
     if (c > 1 && MP >= 12 && most > 4) most = 4;
     if (most > (MP == 4 ? 16 : 8)) most = MP == 4 ? 16 : 8;
     if (most < 2) most = 2;
-    const int rounds = (batches + most - 1) / most;
-    const int w = (batches + rounds - 1) / rounds;
-    return w < 2 ? 2 : w <= 6 ? w : w <= 8 ? (most >= 8 ? 8 : 6) : 16;
+    int w = 2;
+    if (batches > slots) {  // a partial sum has several batches, all of one wave: the fewest rounds of wave 0, which has the most
+        int best_rounds = 1 << 30;
+        for (int c : {2, 3, 4, 5, 6, 8, 16}) {
+            int rounds = 0;
+            for (int s = 0; s < slots; s += c) rounds += (batches - s + slots - 1) / slots;
+            if (c <= most && rounds < best_rounds) { w = c; best_rounds = rounds; }
+        }
+    } else {
+        const int rounds = (batches + most - 1) / most;
+        w = (batches + rounds - 1) / rounds;
+    }
+    // More than two partial sums a wave cost few tokens more than workgroups that wait for a place: 20480 x 8192 at 1 token 61
+    // us on 3 waves, 48 on 8; 20480 x 4096 32.3 on 3, 25.4 on 4.
+    const int used = batches < slots ? batches : slots;
+    if (MP <= 8 && w < (used + 1) / 2) w = (used + 1) / 2;
+    return w < 2 ? 2 : w <= 6 ? w : w <= 8 ? (most >= 8 || MP <= 8 ? 8 : 6) : 16;
 }
 
 template <int MP>
@@ -416,10 +474,11 @@ int lq_gemv_a16w4_launch(const void *x, const void *codes, const void *scales, c
 int lq_gemv_a16w4_gate_up_launch(const void *x, const void *codes_g, const void *scales_g, const void *zeros_g,
                                  const void *codes_u, const void *scales_u, const void *zeros_u, void *h, int M, int N, int K,
                                  hipStream_t st) {
-    const GemvGuArgs a = {x, codes_g, scales_g, zeros_g, codes_u, scales_u, zeros_u, h, M, N, K, st};
     const int batches = (K / LQ_GROUP + 3) / 4, cus = lq_device_cu_count();
     const int mp = (M + 3) / 4 * 4;
-    const int w = gu_waves(mp, N, batches, cus);
+    const int slots = pick_waves(batches, gu_max_slots(mp));
+    const GemvGuArgs a = {x, codes_g, scales_g, zeros_g, codes_u, scales_u, zeros_u, h, M, N, K, slots, st};
+    const int w = gu_waves(mp, N, batches, slots, cus);
     if (mp == 4) launch_gu_waves<4>(w, a);
     else if (mp == 8) launch_gu_waves<8>(w, a);
     else if (mp == 12) launch_gu_waves<12>(w, a);

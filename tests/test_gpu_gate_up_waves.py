@@ -28,3 +28,19 @@ def test_gate_up_few_tokens(N, K):
         # a product of every row against the plain pass, which adds the same terms in another order
         y = ops.a16w4_forward(x, *mats[0], (N, K))
         assert rel_l2(y, g) < 5e-3
+
+
+@pytest.mark.parametrize("N,K", [(4112, 2560), (8208, 3584), (12304, 4096), (16400, 640), (20480, 2048), (8224, 4224), (16400, 8704)])
+def test_rows_do_not_depend_on_how_many_there_are(N, K):
+    """The launcher picks the waves of a workgroup by the number of rows; the order of the sums stays that of K alone, so 16
+    rows have the bits they have among N."""
+    from latentq_llm_amd import ops
+    mats = []
+    for seed in (1, 2):
+        _, p, s, z = make_w4(N, K, seed)
+        mats.append((p.cuda(), s.cuda(), z.cuda()))
+    rows = slice(N - 16, N)
+    few = [(p.view(N, -1)[rows].reshape(-1), s.view(N, -1)[rows].reshape(-1, 1), z.view(N, -1)[rows].reshape(-1, 1)) for p, s, z in mats]
+    for M in (1, 3, 4, 5, 8, 9, 12, 13, 16):
+        x = randn_bf16((M, K), M).cuda()
+        assert torch.equal(ops.a16w4_gate_up_silu(x, *mats, (N, K))[:, rows], ops.a16w4_gate_up_silu(x, *few, (16, K))), M
