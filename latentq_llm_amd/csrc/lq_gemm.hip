@@ -713,7 +713,7 @@ int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *s
 
 // 17 to 64 tokens, one launch with 16 columns per compute unit (lq_gemm_few.hip)
 int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
-                       int K, hipStream_t st, const char *who);
+                       int K, hipStream_t st, unsigned long long *clk, const char *who);
 
 // GEMV path (lq_gemv.hip)
 int lq_gemv_a16w4_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias,
@@ -911,7 +911,7 @@ static int a16w4_fwd_impl(const char *who, const void *x, const void *codes, con
         return LQ_OK;
     }
     if (plan.kernel == LQ_PLAN_FEW)
-        return lq_gemm_few_launch(x, codes, scales, zeros, bias_or_null, y, (int)M, (int)N, (int)K, (hipStream_t)stream, who);
+        return lq_gemm_few_launch(x, codes, scales, zeros, bias_or_null, y, (int)M, (int)N, (int)K, (hipStream_t)stream, clk, who);
     if (plan.kernel == LQ_PLAN_DIRECT || plan.kernel == LQ_PLAN_DIRECT_128)
         return lq_gemm_fwd_direct_launch(x, codes, scales, zeros, bias_or_null, y, (int)M, (int)N, (int)K, (hipStream_t)stream, clk,
                                          plan.kernel == LQ_PLAN_DIRECT_128);
@@ -1115,6 +1115,7 @@ extern "C" int lq_calib_gemm_clocks(int backward, const void *a, const void *cod
     const long long wg = plan.kernel == LQ_PLAN_DIRECT ? lq_gemm_fwd_direct_workgroups((int)M, (int)N)
                          : plan.kernel == LQ_PLAN_DIRECT_128 ? lq_gemm_fwd_direct128_workgroups((int)M, (int)N)
                          : plan.kernel == LQ_PLAN_STAGED_256 ? ((M + 255) / 256) * ((cols + 127) / 128)
+                         : plan.kernel == LQ_PLAN_FEW        ? N / 16
                                                              : ((M + plan.rows - 1) / plan.rows) * ((cols + 127) / 128);
     LQ_REQUIRE(4 * wg <= clocks_capacity, "lq_calib_gemm_clocks: clocks must hold %lld values, holds %lld", 4 * wg,
                (long long)clocks_capacity);

@@ -38,6 +38,7 @@ struct FewParams {
     const unsigned short *scales, *zeros, *bias;
     unsigned short *y;       // bf16 [M, N]
     int M, N, K;
+    unsigned long long *clk; // measurement aid, see lq_calib_gemm_clocks; null in normal use
 };
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -59,6 +60,11 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(FewParams p) {
     static_assert((D - 1) * LOADS < 64, "the wait counts loads in six bits");
     __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves * D * STAGE];
 
+    unsigned long long clk_t0 = 0, clk_r0 = 0;
+    if (p.clk) {
+        clk_t0 = __builtin_amdgcn_s_memtime();
+        clk_r0 = __builtin_amdgcn_s_memrealtime();
+    }
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63, r = lane & 15, h = lane >> 4;
     const int c0 = blockIdx.x * 16;
@@ -180,18 +186,22 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(FewParams p) {
         }
         *reinterpret_cast<u32x2_t *>(p.y + (long long)m * p.N + c) = u32x2_t{lq_pack_bf16(v[0], v[1]), lq_pack_bf16(v[2], v[3])};
     }
+    if (p.clk && threadIdx.x == 0) {
+        unsigned long long *c = p.clk + 4ll * blockIdx.x;
+        c[0] = clk_t0; c[1] = __builtin_amdgcn_s_memtime(); c[2] = clk_r0; c[3] = __builtin_amdgcn_s_memrealtime();
+    }
 }
 
 }  // namespace
 
 // 16 < M <= 64, N % 16 == 0, K % 128 == 0 are guaranteed by the caller.
 int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
-                       int K, hipStream_t st, const char *who) {
+                       int K, hipStream_t st, unsigned long long *clk, const char *who) {
     FewParams p = {};
     p.x = (const unsigned char *)x; p.w = (const unsigned char *)codes;
     p.scales = (const unsigned short *)scales; p.zeros = (const unsigned short *)zeros;
     p.bias = (const unsigned short *)bias; p.y = (unsigned short *)y;
-    p.M = M; p.N = N; p.K = K;
+    p.M = M; p.N = N; p.K = K; p.clk = clk;
     // the 32-bit lane offsets of the loads span the tokens' rows and 16 rows of codes
     if (128ll * K >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: K too large", who);
     const dim3 grid((unsigned)(N / 16)), block(64 * kWaves);
