@@ -274,6 +274,12 @@ __global__ __launch_bounds__(256) void adam8_kernel(Adam8Batch b) {
             for (int k = 0; k < 8; ++k) {
                 d[c][k] = lq_bf16r(lq_bf16r_trans(__builtin_sqrtf(v[k])) + a.eps);
                 ratio[k] = m[c][k] / d[c][k];
+            }
+            // the extrema again: the short root of a subnormal is none of the elements
+            clo2 = c ? lo2 : d[c][0];
+            chi2 = c ? hi2 : d[c][0];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
                 clo2 = fminf(clo2, d[c][k]);
                 chi2 = fmaxf(chi2, d[c][k]);
             }

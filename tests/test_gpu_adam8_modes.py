@@ -138,3 +138,24 @@ def test_step_that_chooses_the_residual_curve_fused_equals_the_chain(hip_lib, mo
         assert torch.equal(x.cpu(), y.cpu())
     if lr < 1e-4:
         assert int(fused[0]) == 2  # the curve did change
+
+
+@pytest.mark.parametrize("block", [2048, 128])
+def test_subnormal_second_moments_without_eps(hip_lib, block):
+    """The block's minimum is that of its elements where the hardware's square root takes a subnormal for zero. Between these
+    two gradients the new scale's last place tells the smaller root (2^-64.5) from zero."""
+    from latentq_llm_amd import ops
+    from latentq_llm_amd import quant as Q
+    from tests.test_gpu_adam8 import chain_step, fresh_state
+    n = 4096
+    state = fresh_state(n, n // block, torch.device("cuda"))
+    fused = {k: t.clone() for k, t in state.items()}
+    grad = torch.full((n,), 2.0 ** -64.5, dtype=torch.bfloat16, device="cuda")
+    grad[::64] = 8.8470897e-16
+    want, step_size = chain_step(Q, grad, state, 1, 1e-3, (0.9, 0.0), 0.0)
+    got = torch.empty_like(grad)
+    ops.adam8_update(grad, fused["state1"], fused["state2"], fused["qmap1"], fused["absmax1"], fused["qmap2"], fused["absmax2"],
+                     0.9, 0.0, 0.0, step_size, direction=got)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for k, t in state.items():
+        assert torch.equal(fused[k].view(-1), t.view(-1)), k
