@@ -1079,6 +1079,37 @@ class GradientQTensor(object):
 
 
 # ------------------------------------------------------------------------------ optimizer --
+class _StepQueue(object):
+    """The fused steps of several parameters of one MyAdam.step() on their way to a launch (ops.adam8_queue). What follows a
+    parameter's step - its new codes bound, its gradient released - happens when the launch is out, so that a launch that
+    fails leaves the parameter with what it had."""
+    LAUNCH = 8              # parameters to a launch
+    HELD_BYTES = 64 << 20   # and what the waiting ones may keep allocated: their copied gradients and new codes
+
+    def __init__(self):
+        self._handle = ops.adam8_queue()
+        self._after, self._params, self._held = [], set(), 0
+
+    def add(self, p, call, held, after):
+        self._after.append((after, call(self._handle)))
+        self._params.add(id(p))
+        self._held += held
+
+    def holds(self, p):
+        return id(p) in self._params
+
+    def full(self):
+        return len(self._after) >= self.LAUNCH or self._held >= self.HELD_BYTES
+
+    def run(self):
+        after, self._after = self._after, []
+        self._params.clear()
+        self._held = 0
+        ops.adam8_run(self._handle)
+        for f, result in after:
+            f(result)
+
+
 class MyAdam(torch.optim.Adam):
     """Adam over a mix of nn.Parameters and QuantTensor/FPTensor latents with optional block-wise
     8-bit moments (utils/quant.py:927-1148). For a QuantTensor the latent weight is rebuilt
@@ -1087,7 +1118,7 @@ class MyAdam(torch.optim.Adam):
 
     ``sr_seed`` seeds the Philox stream of that requantizer; every call consumes N*K/8 counters."""
 
-    _in_step, _queue = False, None  # the fused steps of the step() under way, launched together at its end
+    _in_step, _queue = False, None  # a step() that queues its parameters is under way; their queue
 
     def __init__(self, params, lr=1e-3, betas=(0.9, 0.999), obit=8, mu_updata_f=20, cpu=False, sr_seed=0):
         super().__init__(params, lr=lr, betas=betas)
@@ -1125,31 +1156,38 @@ class MyAdam(torch.optim.Adam):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        self._chosen = self._choose_curves()
-        self._in_step, done = True, 0
+        # an update_step that is not this class's own sees every parameter's step finished when it calls the original
+        queued = getattr(self.update_step, "__func__", None) is _UPDATE_STEP
+        self._chosen = self._choose_curves() if queued else frozenset()
+        self._in_step = queued
         try:
             for gindex, group in enumerate(self.param_groups):
                 for pindex, p in enumerate(group["params"]):
+                    if self._queue is not None and self._queue.holds(p):  # listed twice: its gradient is used up first
+                        self._queue.run()
                     if p.grad is None:
                         continue
                     if len(self.state[p]) == 0:
                         self.init_state(group, p, gindex, pindex)
                     self.update_step(group, p, gindex, pindex)
-                    done += 1
-                    if done % 8 == 0 and self._queue is not None:  # a launch's worth: the device need not wait for the rest
-                        ops.adam8_run(self._queue)
+                    if self._queue is not None and self._queue.full():
+                        self._queue.run()
         finally:
             queue, self._queue, self._in_step = self._queue, None, False
             if queue is not None:
-                ops.adam8_run(queue)
+                queue.run()
         self._chosen = frozenset()
         return loss
 
-    def _step_queue(self):
-        """The queue of the step() under way; None where update_step is called by itself."""
-        if self._in_step and self._queue is None:
-            self._queue = ops.adam8_queue()
-        return self._queue
+    def _launch(self, p, call, held, after):
+        """The fused step of one parameter, ``call(queue)``, and what follows it, ``after(result)``: at once, or with other
+        parameters' steps where step() queues them (``held``: bytes that waiting keeps allocated)."""
+        if not self._in_step:
+            after(call(None))
+            return
+        if self._queue is None:
+            self._queue = _StepQueue()
+        self._queue.add(p, call, held, after)
 
     def to_gpu(self):
         for group in self.param_groups:
@@ -1291,15 +1329,18 @@ class MyAdam(torch.optim.Adam):
             if sr_mode:  # the direction goes straight into the requantizer
                 scales, zeros, shape = _flat_qparam(p.qparam)
                 requant = (p.data, scales, zeros, shape, self.sr_seed, self.sr_offset)
-            new = ops.adam8_update(grad, state["state1"], state["state2"], state["qmap1"], state["absmax1"], state["qmap2"],
-                                   state["absmax2"], beta1, beta2, group["eps"], step_size,
-                                   param=None if sr_mode else pdata, requant=requant, queue=self._step_queue() if sr_mode else None)
-            if sr_mode:
-                p.data = new
-                self.sr_offset += (p.numel() + 7) // 8
-                self._release_grad(p)
-            else:
+            moments = (state["state1"], state["state2"], state["qmap1"], state["absmax1"], state["qmap2"], state["absmax2"])
+            if not sr_mode:
+                ops.adam8_update(grad, *moments, beta1, beta2, group["eps"], step_size, param=pdata)
                 self._requantise(p, pdata, None, step_size, is_q, sr_mode)
+                return
+
+            def bind(new):
+                p.data = new
+                self._release_grad(p)
+            self._launch(p, lambda queue: ops.adam8_update(grad, *moments, beta1, beta2, group["eps"], step_size, requant=requant, queue=queue),
+                         self._copied_bytes(p, grad) + p.numel() // 2, bind)
+            self.sr_offset += (p.numel() + 7) // 8
             return
         if q8:
             exp_avg = DeQfunc_8bit_opt(state["state1"].to(grad.device), [state["qmap1"], state["absmax1"]]).to(grad.dtype)
@@ -1367,12 +1408,15 @@ class MyAdam(torch.optim.Adam):
             step_size = config["lr"] * math.sqrt(1 - beta2 ** state["step"]) / (1 - beta1 ** state["step"])
             p1, y1, p2, y2 = three_fold_curve_4bit(r.lock_mu)
             q1, z1, q2, z2 = three_fold_curve_4bit(r.mu)
-            ops.adam8_latent_w8_step(grad, p.data, r.residual_int.view(-1), qs.view(-1), *moments,
-                                     (p1, y1, p2 - p1, y2, 8 - p2), (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2,
-                                     group["eps"], step_size, self._step_queue())
-            r.weight_scale = qs
-            r.lock_mu = r.mu
-            self._release_grad(p)
+            mu = r.mu
+
+            def stored(_):
+                r.weight_scale = qs
+                r.lock_mu = mu
+                self._release_grad(p)
+            self._launch(p, lambda queue: ops.adam8_latent_w8_step(
+                grad, p.data, r.residual_int.view(-1), qs.view(-1), *moments, (p1, y1, p2 - p1, y2, 8 - p2),
+                (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2, group["eps"], step_size, queue), self._copied_bytes(p, grad), stored)
             return True
         scales, zeros, shape = _flat_qparam(p.qparam)
         if not (scales.dtype == torch.bfloat16 and zeros.dtype == torch.bfloat16 and scales.is_contiguous()
@@ -1384,12 +1428,15 @@ class MyAdam(torch.optim.Adam):
         step_size = config["lr"] * math.sqrt(1 - beta2 ** state["step"]) / (1 - beta1 ** state["step"])
         p1, y1, p2, y2 = three_fold_curve_4bit(r.lock_mu)
         q1, z1, q2, z2 = three_fold_curve_4bit(r.mu)
-        ops.adam8_latent_w4_step(grad, p.data, r.residual_int.view(-1), scales, zeros, tuple(shape), *moments,
-                                 (p1, y1, p2 - p1, y2, 8 - p2), (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2,
-                                 group["eps"], step_size, self._step_queue())
-        r.weight_scale = scales.contiguous().reshape(-1, 1)
-        r.lock_mu = r.mu
-        self._release_grad(p)
+        mu = r.mu
+
+        def stored(_):
+            r.weight_scale = scales.contiguous().reshape(-1, 1)
+            r.lock_mu = mu
+            self._release_grad(p)
+        self._launch(p, lambda queue: ops.adam8_latent_w4_step(
+            grad, p.data, r.residual_int.view(-1), scales, zeros, tuple(shape), *moments, (p1, y1, p2 - p1, y2, 8 - p2),
+            (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2, group["eps"], step_size, queue), self._copied_bytes(p, grad), stored)
         return True
 
     def _requantise(self, p, pdata, direction, step_size, is_q, sr_mode):
@@ -1408,8 +1455,16 @@ class MyAdam(torch.optim.Adam):
         self._release_grad(p)
 
     @staticmethod
+    def _copied_bytes(p, grad):
+        """Bytes of a gradient that was made for this step (from an int8 accumulator); 0 for the parameter's own."""
+        return grad.numel() * grad.element_size() if isinstance(p.grad, GradientQTensor) and p.grad.bit <= 8 else 0
+
+    @staticmethod
     def _release_grad(p):
         if isinstance(p.grad, GradientQTensor):
             p.grad.zero()
         else:
             p.grad = None
+
+
+_UPDATE_STEP = MyAdam.update_step
