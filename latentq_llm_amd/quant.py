@@ -572,6 +572,13 @@ class _HookHandle(object):
         self.active = False
 
 
+def _own(module, table, name):
+    """An attribute of a module: from its table of parameters or buffers, which costs the host less than the attribute's own
+    way there, or by that way where the table does not have it (a parametrisation, or a plain attribute that a sharding or
+    replicating wrapper left)."""
+    return table[name] if name in table else getattr(module, name)
+
+
 class _QLinearBase(nn.Module):
     _repr_name = "QLinear"
 
@@ -644,7 +651,7 @@ class QLinearA16W4(_QLinearBase):
 
     def _infer(self, x):
         w = self.weight
-        return ops.linear4(x, w.data, *w.qparam, self._parameters["bias"])
+        return ops.linear4(x, w.data, *w.qparam, _own(self, self._parameters, "bias"))
 
     def to(self, device: Optional[Union[int, torch.device]]):
         """Moves the QuantTensor and re-binds its qparam to the moved buffers; returns None like
@@ -678,7 +685,8 @@ class QLinearA8W8(_QLinearBase):
         return (self.clampv, self.qscales.data)
 
     def _infer(self, x):
-        return ops.infer8(x, self.weight.data, self._buffers["qscales"], self._parameters["bias"], self.act_quant == "per_token")
+        return ops.infer8(x, self.weight.data, _own(self, self._buffers, "qscales"), _own(self, self._parameters, "bias"),
+                          self.act_quant == "per_token")
 
     def to(self, device: Optional[Union[int, torch.device]]):
         self.weight = self.weight.to(device=device)
