@@ -808,9 +808,8 @@ struct W4Plan {
 //                                      the clock: 0.55 up to three quarters of them, 0.61 with all), ~0.74 as soon as a
 //                                      few units hold two, ~1.23 for two everywhere, ~1.38 for three.
 // Up to 32 tokens two GEMV launches of 16 are a little faster where a launch does not wait for the matrix' bytes
-// (4096 x 4096: 10.0 / 10.8 us at 17 / 32 tokens against 10.5 / 11.1; 2048 x 2048: 7.1 / 7.8 against 7.4 / 8.0); at
-// 11008 x 4096 they take 23.3 us against 15.7. One token beyond a GEMV launch keeps the GEMV (the second launch then
-// is the one-token kernel) below K = 8192, although 11008 x 4096 takes 20.0 us so against 15.7.
+// and K is not long (2048 x 2048: 7.4 / 8.1 us at 17 / 32 tokens against 8.6 / 9.0; 1024 x 4096 9.1 / 10.3 against 9.7 / 10.2); at
+// 11008 x 4096 they take 21.0 / 23.4 us against 18.1 / 17.7, at 1536 x 8192 14.4 / 17.0 against 13.1 / 13.7.
 static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     W4Plan out;
     if (M <= 64 && N <= 16 * cus && 2 * N > 16 * cus) {
@@ -822,7 +821,7 @@ static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, l
             return out;
         }
     }
-    if ((M == 17 && K < 8192) || (M <= 32 && N * K <= 4096ll * 4096)) {
+    if (M <= 32 && K < 8192 && N * K <= 4096ll * 4096) {
         out.kernel = LQ_PLAN_GEMV_CHUNKS;
         return out;
     }

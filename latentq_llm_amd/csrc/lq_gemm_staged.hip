@@ -312,8 +312,7 @@ int launch_staged(const StagedParams &p, int rows, bool exact, int splits, hipSt
 // plus 0.19 as soon as there is one. 4.1 us around the loop; a split costs 1.7 us for the second launch and 0.53 us per
 // MB of partial products. Constants fitted to 2000 timings (12 matrices from 1024^2 to 11008 x 4096, 17 to 1536
 // tokens, every row tile, 1 to 8 slices): 5.5 % rms; the choice costs 1.5 % over the best candidate on average.
-// A slice has at least four groups. Few tiles (an eighth of the units) with ten groups or more are always cut: the
-// estimate is a tie there (2048 x 2048 at 192 tokens: 11.1 cut in two, 12.0 whole).
+// A slice has at least four groups.
 double lq_gemm_staged_plan(long long M, long long N, int groups, size_t ws_bytes, long long cus, int *rows, int *splits, int *per_split) {
     static const double lone[3] = {0.45, 0.54, 0.74}, more[3] = {0.30, 0.46, 0.0};
     static const int fit_cu[3] = {3, 2, 1};
@@ -322,12 +321,11 @@ double lq_gemm_staged_plan(long long M, long long N, int groups, size_t ws_bytes
     if (most > cus / tiles128) most = cus / tiles128;
     if (most > 8) most = 8;
     if (most > groups / 4) most = groups / 4;
-    const bool cut = tiles128 * 8 <= cus && groups >= 10 && most >= 2;
     double best = 1e30;
     for (int i = 0; i < 3; ++i) {
         const int h = 32 << i;
         if (i && M <= h / 2) continue;  // half of the rows would be padding
-        for (int s = cut ? 2 : 1; s == 1 || s <= most; ++s) {
+        for (int s = 1; s == 1 || s <= most; ++s) {
             const int per = (groups + s - 1) / s;
             if (s > 1 && (per < 4 || (groups + per - 1) / per != s)) continue;
             const double load = (double)((M + h - 1) / h * cols * s) / (double)cus;
