@@ -6,6 +6,8 @@ does the same checks, allocation and call in a tenth of the host time and return
 plain form; the Python below then runs its own checks and raises what is wrong."""
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from . import _C
@@ -86,12 +88,13 @@ def philox_uniform(n: int, seed: int, offset: int = 0, device="cuda"):
 
 
 # Scratch for the split-reduction GEMM of skinny problems (fp32 partial tiles); the library itself
-# never allocates. Outside graph capture: one buffer of WORKSPACE_MAX_BYTES per (device, stream),
-# allocated on first need and never resized, so its address is stable; at most WORKSPACE_MAX_STREAMS
-# streams per device keep one (least recently used first out; a dropped buffer goes back to the
-# caching allocator's pool of the stream it was allocated on, which orders its reuse after the
-# kernels that still read it). Under graph capture: a buffer of the size the call needs from the
-# capturing graph's own memory pool, which lives as long as the graph and is reused by later
+# never allocates. Outside graph capture: one buffer of WORKSPACE_MAX_BYTES per (device, stream, host
+# thread), allocated on first need and never resized, so its address is stable. (A product is several
+# launches that hand the buffer on: two threads on one stream may launch theirs in between each other.)
+# At most WORKSPACE_MAX_STREAMS of them per device are kept (least recently used first out; a dropped
+# buffer goes back to the caching allocator's pool of the stream it was allocated on, which orders its
+# reuse after the kernels that still read it). Under graph capture: a buffer of the size the call needs
+# from the capturing graph's own memory pool, which lives as long as the graph and is reused by later
 # calls of the same capture.
 _WORKSPACE = {}
 WORKSPACE_MAX_BYTES = 64 << 20
@@ -107,13 +110,13 @@ def _workspace(t, rows, cols):
     if torch.cuda.is_current_stream_capturing():
         buf = torch.empty(min(8 * rows * cols * 4, WORKSPACE_MAX_BYTES), dtype=torch.uint8, device=t.device)
         return buf, buf.data_ptr(), buf.numel()
-    key = (t.device.index, _stream(t))
+    key = (t.device.index, _stream(t), threading.get_ident())
     buf = _WORKSPACE.pop(key, None)
     if buf is None:
         buf = torch.empty(WORKSPACE_MAX_BYTES, dtype=torch.uint8, device=t.device)
-        same_device = [k for k in _WORKSPACE if k[0] == key[0]]
+        same_device = [k for k in list(_WORKSPACE) if k[0] == key[0]]
         for k in same_device[: max(0, len(same_device) - (WORKSPACE_MAX_STREAMS - 1))]:
-            del _WORKSPACE[k]
+            _WORKSPACE.pop(k, None)  # (another thread may have it out to put it last)
     _WORKSPACE[key] = buf  # (re)inserted last: dict order is the recency order
     return buf, buf.data_ptr(), buf.numel()
 
