@@ -52,7 +52,7 @@ class _FusedMLPTrain(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dx = ops.a16w4_dx_pair(dg, _w4(gate), du, _w4(up), (inter, K), split=True)
         for layer, dyl, xin in ((down, dy, h), (up, du, x2), (gate, dg, x2)):
-            if layer.hook_handle is not None:
+            if layer.hook_handle is not None and not quant._removed(layer.hook_handle):
                 dict_temp.append(_pending_dw(dyl, xin))
                 backward_hook_fn(layer, None, None)
         return dx, None

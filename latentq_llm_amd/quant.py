@@ -24,6 +24,7 @@ Deliberate deviations from the reference, all on purpose:
 from __future__ import annotations
 
 import math
+from collections import OrderedDict
 from functools import reduce
 from typing import Optional, Union
 
@@ -561,15 +562,19 @@ _CTX_FORMS = {
 }
 
 
-class _HookHandle(object):
-    """What add_hook leaves in hook_handle: remove() ends the delivery of weight gradients (they then stay in dict_temp,
-    as with the reference's hook removed)."""
+class _HookHandle(torch.utils.hooks.RemovableHandle):
+    """What add_hook leaves in hook_handle, a handle like those of torch's own hooks: remove(), or the end of a with block on
+    it, ends the delivery of weight gradients (a layer's then stay in dict_temp, as with the reference's hook removed; a
+    fused block forms none for it)."""
 
-    def __init__(self):
-        self.active = True
+    @property
+    def active(self):
+        return self.id in (self.hooks_dict_ref() or ())
 
-    def remove(self):
-        self.active = False
+
+def _removed(handle):
+    """Whether a layer's hook_handle is add_hook's and no longer active (a handle of the caller's own is neither)."""
+    return isinstance(handle, _HookHandle) and not handle.active
 
 
 def _own(module, table, name):
@@ -598,7 +603,9 @@ class _QLinearBase(nn.Module):
         """The layer's weight gradients are delivered to weight.grad from now on (until hook_handle.remove()). The
         reference registers backward_hook_fn as a full-backward hook; here the Functions call it themselves, since such a
         hook wraps a layer's inputs and outputs in autograd nodes of their own (47 us of host time per step and layer)."""
-        self.hook_handle = _HookHandle()
+        self._delivery = OrderedDict()
+        self.hook_handle = _HookHandle(self._delivery)
+        self._delivery[self.hook_handle.id] = backward_hook_fn
 
     def _apply_fn(self, fn, x, *layer):
         if not torch._C._are_functorch_transforms_active():
@@ -615,7 +622,7 @@ class _QLinearBase(nn.Module):
     def forward(self, x):
         if self.hook_handle is None:
             return self.forward_eval(x)
-        return self._apply_fn(self._fn_train, x, self if getattr(self.hook_handle, "active", False) else None)
+        return self._apply_fn(self._fn_train, x, self if isinstance(self.hook_handle, _HookHandle) and self.hook_handle.active else None)
 
     def forward_eval(self, x):
         if not torch.is_grad_enabled() and _unwatched():
