@@ -577,13 +577,6 @@ def _removed(handle):
     return isinstance(handle, _HookHandle) and not handle.active
 
 
-def _own(module, table, name):
-    """An attribute of a module: from its table of parameters or buffers, which costs the host less than the attribute's own
-    way there, or by that way where the table does not have it (a parametrisation, or a plain attribute that a sharding or
-    replicating wrapper left)."""
-    return table[name] if name in table else getattr(module, name)
-
-
 class _QLinearBase(nn.Module):
     _repr_name = "QLinear"
 
@@ -612,6 +605,14 @@ class _QLinearBase(nn.Module):
             fn = _CTX_FORMS.get(fn, fn)
         out = fn.apply(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), self.weight.data, self._qparam(), self.bias, *layer)
         return out if x.dim() == 2 else out.reshape(x.shape[:-1] + (self.output_features,))
+
+    def _bias(self):
+        """self.bias from the module's table, which costs the host less than the attribute's own way there; by that way where
+        the table does not have it (a parametrisation, a plain attribute that a sharding or replicating wrapper left)."""
+        try:
+            return self._parameters["bias"]
+        except KeyError:
+            return self.bias
 
     def _infer(self, x):
         """The layer's result where nothing is differentiated and every operand is in the form the kernels take; None
@@ -657,8 +658,11 @@ class QLinearA16W4(_QLinearBase):
         return self.weight.qparam
 
     def _infer(self, x):
-        w = self.weight
-        return ops.linear4(x, w.data, *w.qparam, _own(self, self._parameters, "bias"))
+        w, bias = self.weight, self._bias()
+        y = ops.linear4(x, w.data, *w.qparam, bias)
+        if y is None and bias is not None and bias.dtype != torch.bfloat16:  # as constructed
+            y = ops.linear4(x, w.data, *w.qparam, bias.detach().to(torch.bfloat16))
+        return y
 
     def to(self, device: Optional[Union[int, torch.device]]):
         """Moves the QuantTensor and re-binds its qparam to the moved buffers; returns None like
@@ -692,8 +696,15 @@ class QLinearA8W8(_QLinearBase):
         return (self.clampv, self.qscales.data)
 
     def _infer(self, x):
-        return ops.infer8(x, self.weight.data, _own(self, self._buffers, "qscales"), _own(self, self._parameters, "bias"),
-                          self.act_quant == "per_token")
+        bias, per_token = self._bias(), self.act_quant == "per_token"
+        try:
+            qscales = self._buffers["qscales"]
+        except KeyError:
+            qscales = self.qscales
+        y = ops.infer8(x, self.weight.data, qscales, bias, per_token)
+        if y is None and bias is not None and bias.dtype != torch.bfloat16:  # as constructed
+            y = ops.infer8(x, self.weight.data, qscales, bias.detach().to(torch.bfloat16), per_token)
+        return y
 
     def to(self, device: Optional[Union[int, torch.device]]):
         self.weight = self.weight.to(device=device)

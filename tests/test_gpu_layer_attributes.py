@@ -52,3 +52,16 @@ def test_bias_and_scales_elsewhere(kind, M):
             del m.qscales
             m.qscales = scales
         assert torch.equal(m(x), want)
+
+
+@pytest.mark.parametrize("kind", ["w4", "w8"])
+@pytest.mark.parametrize("M", [1, 40])
+def test_bias_as_constructed(kind, M, monkeypatch):
+    """A bias in fp32, as the constructor leaves it, is rounded to bf16 and takes the direct path too."""
+    x = randn_bf16((M, 512), 6).cuda()
+    m = _layer(kind)
+    m.bias.data = m.bias.data.float() * 1.001
+    want = m(x).detach()  # through the Function
+    monkeypatch.setattr(type(m), "_apply_fn", None)
+    with torch.no_grad():
+        assert m.bias.dtype == torch.float32 and torch.equal(m(x), want)
