@@ -43,6 +43,7 @@ SIGNATURES = {
     "lq_a16w4_gate_up_silu": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "lq_a16w4_gate_up_silu_save": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "lq_a16w4_gate_up_silu_ws": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp],
+    "lq_a16w4_gate_up_plan": [_i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp],
     "lq_a16w4_dx_silu_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "lq_a16w4_dx_acc": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "lq_a16w4_dx_pair": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],

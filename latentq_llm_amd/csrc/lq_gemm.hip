@@ -928,6 +928,35 @@ static int a16w4_fwd_impl(const char *who, const void *x, const void *codes, con
     return launch_gemm<MODE_W4_FWD, 256, 128, 2, 2>(p, (hipStream_t)stream, who);
 }
 
+struct GateUpPlan {
+    int kernel = LQ_PLAN_DIRECT;
+    int rows = 128, splits = 1, per_split = 0;  // LQ_PLAN_STAGED_128: rows of the tile, slices of K and their groups of 128 k
+};
+
+// Gate / up product, M > 16.
+// Few tokens leave most of a 128-row tile empty and most units idle: the staged kernel then runs both products as one
+// launch of 32, 64 or 128 rows, planned as one product of 2 N columns, and a second launch adds its slices and forms h.
+// Both sides estimated: the weights-direct kernel by its pace per 64-deep step (0.58 to 0.68 us for a workgroup with a
+// unit to itself, 1.3 for two) plus 7 us, the staged one by its own plan plus, where that is not in it, the partial
+// products' way through the cache. us against the weights-direct kernel and the two plain products with tensor glue:
+//   11008 x 4096  17 / 45 / 128 tokens  25.7 / 27.7 / 37.3 against 51.1 / 50.4 / 50.5 and 45.5 / 43.9 / 55.7; behind from
+//                 160 on (64.5 against 52.1)
+//   6144 x 3072   17 / 64 / 256         13.4 / 20.2 / 30.9 against 35.8 / 35.9 / 36.4; level at 300
+//   3072 x 1024   17 / 128 / 300        10.3 / 11.7 / 15.3 against 15.0 / 15.1 / 15.5; 19.2 against 15.6 at 400
+static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
+    GateUpPlan out;
+    if (ws_bytes < (size_t)8 * M * N) return out;
+    const int groups = (int)(K / LQ_GROUP);
+    const long long wg = ((M + 127) / 128) * ((N + 127) / 128), rem = wg % (2 * cus);
+    const double est_direct = (1.3 * (double)(wg / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.66 : 1.3)) * (double)(K / 64) + 7.0;
+    out.per_split = groups;
+    double est = lq_gemm_staged_plan(M, 2 * N, groups, ws_bytes, cus, &out.rows, &out.splits, &out.per_split);
+    if (out.splits == 1) est += 1.7 + 0.53e-6 * 8.0 * (double)M * (double)N;
+    if (est >= est_direct) return GateUpPlan();
+    out.kernel = LQ_PLAN_STAGED_128;
+    return out;
+}
+
 static int gate_up_impl(const char *who, const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
                         const void *codes_up, const void *scales_up, const void *zeros_up, void *h, void *g_out, void *u_out,
                         int64_t M, int64_t N, int64_t K, int group, void *workspace, size_t ws_bytes, void *stream) {
@@ -951,31 +980,15 @@ static int gate_up_impl(const char *who, const void *x, const void *codes_gate, 
     }
     LQ_REQUIRE(K % 256 == 0, "%s: K=%lld must be a multiple of 256 for more than 16 tokens", who, (long long)K);
     LQ_REQUIRE(!workspace || lq_aligned(workspace, 16), "%s: the workspace must be 16-byte aligned", who);
-    // Few tokens leave most of a 128-row tile empty and most units idle: the staged kernel then runs both products as one
-    // launch of 32, 64 or 128 rows, planned as one product of 2 N columns, and a second launch adds its slices and forms h.
-    // Both sides estimated: the weights-direct kernel by its pace per 64-deep step (0.58 to 0.68 us for a workgroup with a
-    // unit to itself, 1.3 for two) plus 7 us, the staged one by its own plan plus, where that is not in it, the partial
-    // products' way through the cache. us against the weights-direct kernel and the two plain products with tensor glue:
-    //   11008 x 4096  17 / 45 / 128 tokens  25.7 / 27.7 / 37.3 against 51.1 / 50.4 / 50.5 and 45.5 / 43.9 / 55.7; behind from
-    //                 160 on (64.5 against 52.1)
-    //   6144 x 3072   17 / 64 / 256         13.4 / 20.2 / 30.9 against 35.8 / 35.9 / 36.4; level at 300
-    //   3072 x 1024   17 / 128 / 300        10.3 / 11.7 / 15.3 against 15.0 / 15.1 / 15.5; 19.2 against 15.6 at 400
-    if (ws_bytes >= (size_t)8 * M * N) {
-        const long long cus = lq_device_cu_count();
-        const long long wg = ((M + 127) / 128) * ((N + 127) / 128), rem = wg % (2 * cus);
-        const double est_direct = (1.3 * (double)(wg / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.66 : 1.3)) * (double)(K / 64) + 7.0;
-        int rows = 128, splits = 1, per = (int)(K / LQ_GROUP);
-        double est = lq_gemm_staged_plan(M, 2 * N, (int)(K / LQ_GROUP), ws_bytes, cus, &rows, &splits, &per);
-        if (splits == 1) est += 1.7 + 0.53e-6 * 8.0 * (double)M * (double)N;
-        if (est < est_direct) {
-            rc = lq_gemm_staged_pair_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, (float *)workspace, (int)M,
-                                            (int)N, (int)K, rows, splits, per, (hipStream_t)stream, who);
-            if (rc) return rc;
-            const long long MN = (long long)M * N;
-            hipLaunchKernelGGL(gate_up_reduce_kernel, dim3((unsigned)((MN / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                               (const float *)workspace, (unsigned short *)h, (unsigned short *)g_out, (unsigned short *)u_out, MN, splits);
-            return lq_check_launch(who);
-        }
+    const GateUpPlan plan = plan_gate_up(M, N, K, ws_bytes, lq_device_cu_count());
+    if (plan.kernel == LQ_PLAN_STAGED_128) {
+        rc = lq_gemm_staged_pair_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, (float *)workspace, (int)M,
+                                        (int)N, (int)K, plan.rows, plan.splits, plan.per_split, (hipStream_t)stream, who);
+        if (rc) return rc;
+        const long long MN = (long long)M * N;
+        hipLaunchKernelGGL(gate_up_reduce_kernel, dim3((unsigned)((MN / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                           (const float *)workspace, (unsigned short *)h, (unsigned short *)g_out, (unsigned short *)u_out, MN, plan.splits);
+        return lq_check_launch(who);
     }
     return lq_gemm_fwd_gate_up_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h, g_out, u_out, (int)M,
                                       (int)N, (int)K, (hipStream_t)stream);
@@ -1126,7 +1139,7 @@ extern "C" int lq_calib_gemm_clocks(int backward, const void *a, const void *cod
                           (unsigned long long *)clocks);
 }
 
-// The plan the two entry points above would follow, without launching anything.
+// The plan lq_a16w4_fwd_ws or lq_a16w4_dx_ws would follow, without launching anything.
 extern "C" int lq_a16w4_plan(int backward, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int compute_units,
                              int *kernel, int *splits, int *steps_per_split) {
     LQ_REQUIRE(kernel && splits && steps_per_split, "lq_a16w4_plan: null pointer argument");
@@ -1140,6 +1153,20 @@ extern "C" int lq_a16w4_plan(int backward, int64_t M, int64_t N, int64_t K, int6
     if (!backward && M <= 16) plan.kernel = LQ_PLAN_GEMV;
     else plan = backward ? plan_dx(M, N, K, ws, cus) : plan_fwd(M, N, K, ws, cus);
     *kernel = plan.kernel; *splits = plan.splits; *steps_per_split = plan.steps_per_split;
+    return LQ_OK;
+}
+
+extern "C" int lq_a16w4_gate_up_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int compute_units, int *kernel, int *rows,
+                                     int *splits) {
+    LQ_REQUIRE(kernel && rows && splits, "lq_a16w4_gate_up_plan: null pointer argument");
+    LQ_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31),
+               "lq_a16w4_gate_up_plan: need positive M, N, K");
+    LQ_REQUIRE(N % 16 == 0, "lq_a16w4_gate_up_plan: N=%lld must be a multiple of 16", (long long)N);
+    LQ_REQUIRE(K % (M > 16 ? 256 : LQ_GROUP) == 0, "lq_a16w4_gate_up_plan: K=%lld must be a multiple of %d", (long long)K, M > 16 ? 256 : LQ_GROUP);
+    GateUpPlan plan;
+    if (M <= 16) plan.kernel = LQ_PLAN_GEMV;
+    else plan = plan_gate_up(M, N, K, workspace_bytes > 0 ? (size_t)workspace_bytes : 0, compute_units > 0 ? compute_units : lq_device_cu_count());
+    *kernel = plan.kernel; *rows = plan.rows; *splits = plan.splits;
     return LQ_OK;
 }
 

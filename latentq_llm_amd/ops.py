@@ -339,6 +339,17 @@ def a16w4_plan(M: int, shape, backward: bool = False, workspace_bytes: int = WOR
     return PLAN_KERNELS[k.value], sp.value, per.value
 
 
+def a16w4_gate_up_plan(M: int, shape, workspace_bytes: int = WORKSPACE_MAX_BYTES, compute_units: int = 0):
+    """(kernel name, rows of a tile, slices of K) a16w4_gate_up_silu would use for M tokens on two [N, K] matrices; rows and
+    slices say something for "staged_128x128" only. Launches nothing, as a16w4_plan."""
+    import ctypes
+    N, K = shape
+    k, rows, sp = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    _C.call("lq_a16w4_gate_up_plan", M, N, K, workspace_bytes, compute_units, ctypes.addressof(k), ctypes.addressof(rows),
+            ctypes.addressof(sp))
+    return PLAN_KERNELS[k.value], rows.value, sp.value
+
+
 def a16w4_dequant(codes, scales, zeros, shape):
     N, K = shape
     _codes_ok(codes, N, K)

@@ -202,8 +202,15 @@ def test_dispatch_plan_host_logic(hip_lib):
     # a workspace that holds two slices caps the split at two
     M, N, K = 128, 11008, 4096
     assert plan(M, N, K, True, workspace=2 * M * K * 4)[1] == 2
+    # gate / up: one GEMV pass, small tiles of both matrices (with room for two whole products), the weights-direct kernel
+    def gate_up(M, N, K, workspace=ws):
+        return ops.a16w4_gate_up_plan(M, (N, K), workspace_bytes=workspace, compute_units=256)
+    assert gate_up(16, 11008, 4096)[0] == "gemv" and gate_up(45, 11008, 4096) == ("staged_128x128", 64, 1)
+    assert gate_up(160, 11008, 4096)[0] == gate_up(45, 11008, 4096, 8 * 45 * 11008 - 1)[0] == "direct_128x256"
     # bad arguments
     from latentq_llm_amd._C import LatentQError
+    with pytest.raises(LatentQError, match="multiple of 256"):
+        gate_up(45, 11008, 4096 + 128)
     with pytest.raises(LatentQError, match="multiple of 64"):
         plan(128, 11008 + 16, 4096, backward=True)
     with pytest.raises(LatentQError, match="multiple of 128"):
