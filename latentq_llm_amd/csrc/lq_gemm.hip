@@ -177,26 +177,25 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
     const int bw = rest < GN ? rest : GN;
     const int tile_m = within / bw, tile_n = band * GN + within % bw;
     const int m0 = tile_m * BM, c0 = tile_n * BN;
-    // reduction steps of this workgroup: all of them, or one slice of a split reduction
-    const int k0 = p.partial ? (int)blockIdx.y * p.steps_per_split : 0;
+    // reduction steps of this workgroup: all of them, or (dX) one slice of a split reduction
+    const bool split = kDx && p.partial;
+    const int k0 = split ? (int)blockIdx.y * p.steps_per_split : 0;
     const bool pair = MODE == MODE_W4_DX && p.a2 != nullptr;
     const int n1 = p.R / RT;                                  // steps of the first (or only) product
     const int n_all = pair ? 2 * n1 : n1;
-    const int nk = p.partial && n_all - k0 < p.steps_per_split ? n_all - k0 : p.partial ? p.steps_per_split : n_all;
+    const int nk = split && n_all - k0 < p.steps_per_split ? n_all - k0 : split ? p.steps_per_split : n_all;
     const int n_first = n1 - k0;  // pair: from this step of the workgroup on it is the second product
     const int groups_per_row = p.Kw / LQ_GROUP;
 
     if (is_weight_wave) {
         // ======================= weight waves: B tiles =======================
-        //   W4_FWD  : NW code words (8 k each) of one weight row -> NW 16-byte chunks of that row.
+        //   W4_FWD  : 4 code words (8 k each) of one weight row -> four 16-byte chunks of that row.
         //   W4_DX   : 4 code words (32 k) of one weight row n -> four 16-byte pieces of LDS row n. The
         //             tile stays in the weights' own [n][k] order; the math waves transpose it on
         //             the way out of LDS (ds_read_b64_tr_b16).
-        constexpr int NW = (MODE == MODE_W4_FWD) ? BN * 8 / NT : 1;  // tile has BN rows x 8 words
-        static_assert(MODE != MODE_W4_FWD || NW == 2 || NW == 4 || NW == 8, "bad fwd staging split");
-        static_assert(!kDx || (BN == 128 && NT == 256), "dX staging: 64 rows x 4 threads");
+        static_assert(BN == 128 && NT == 256, "staging: fwd 128 rows x 2 threads, dX 64 rows x 4 threads");
         constexpr int NSZ = 1;
-        constexpr int NWORDS = (MODE == MODE_W4_DX) ? 4 : (MODE == MODE_W8_DX) ? 8 : NW;
+        constexpr int NWORDS = MODE == MODE_W8_DX ? 8 : 4;
 
         const unsigned char *b_src[1];
         const unsigned short *s_src[NSZ];
@@ -206,14 +205,13 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
         int b_row = 0, b_w0 = 0;  // W4_FWD: LDS row and first word; W4_DX: LDS row (n) and quarter of the row
 
         if constexpr (MODE == MODE_W4_FWD) {
-            constexpr int TPR = 8 / NW;  // threads per weight row
-            b_row = tid / TPR;
-            b_w0 = (tid % TPR) * NW;
+            b_row = tid >> 1;
+            b_w0 = (tid & 1) * 4;
             int gr = c0 + b_row;
             gr = gr < p.C ? gr : p.C - 1;
-            b_src[0] = (const unsigned char *)p.b + (long long)gr * (p.Kw / 2) + b_w0 * 4 + (long long)k0 * 32;
-            s_src[0] = p.scales + (long long)gr * groups_per_row + k0 / 2;  // k0 is even: a group is two steps
-            z_src[0] = p.zeros + (long long)gr * groups_per_row + k0 / 2;
+            b_src[0] = (const unsigned char *)p.b + (long long)gr * (p.Kw / 2) + b_w0 * 4;
+            s_src[0] = p.scales + (long long)gr * groups_per_row;
+            z_src[0] = p.zeros + (long long)gr * groups_per_row;
         } else if constexpr (MODE == MODE_W8_DX) {
             b_row = tid >> 2;  // n within the tile
             b_w0 = tid & 3;    // 32 of the tile's 128 output columns k = 32 code bytes
@@ -243,18 +241,9 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
         auto load_b = [&](int kt, Stage &S) {
             if constexpr (MODE == MODE_W4_FWD) {
                 const unsigned char *src = b_src[0] + (long long)kt * 32;
-                if constexpr (NW == 8) {
-                    u32x4_t v0 = *reinterpret_cast<const u32x4_t *>(src), v1 = *reinterpret_cast<const u32x4_t *>(src + 16);
+                const u32x4_t v = *reinterpret_cast<const u32x4_t *>(src);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) { S.w[i] = v0[i]; S.w[4 + i] = v1[i]; }
-                } else if constexpr (NW == 4) {
-                    u32x4_t v = *reinterpret_cast<const u32x4_t *>(src);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) S.w[i] = v[i];
-                } else {
-                    u32x2_t v = *reinterpret_cast<const u32x2_t *>(src);
-                    S.w[0] = v[0]; S.w[1] = v[1];
-                }
+                for (int i = 0; i < 4; ++i) S.w[i] = v[i];
                 S.s[0] = s_src[0][kt >> 1];
                 S.z[0] = z_src[0][kt >> 1];
             } else if constexpr (MODE == MODE_W8_DX) {
@@ -281,7 +270,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
                 const float nzs = -(lq_bf16_bits_to_f32(S.z[0]) * s);
                 const float s512 = s * 512.0f;  // the codes come out of the conversion as q/512
 #pragma unroll
-                for (int w = 0; w < NW; ++w) {
+                for (int w = 0; w < 4; ++w) {
                     float f[8];
                     lq_dequant_word_f32(S.w[w], s512, nzs, f);
                     const int ch = b_w0 + w;
@@ -508,7 +497,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
     // contiguous bytes of a row. The B buffers are free here (the weight waves wrote their last
     // tile before the final barrier, and no load is in flight into them); a wave's staging area
     // is private, row pitch TN*2 + 16 bytes.
-    if (p.partial) {
+    if (split) {
         // split reduction: the fp32 accumulators as they are, 16 bytes per lane; a second kernel adds
         // the slices in a fixed order, adds the bias and rounds
         float *part = p.partial + (long long)blockIdx.y * p.M * p.C;
