@@ -1107,33 +1107,32 @@ class GradientQTensor(object):
 # ------------------------------------------------------------------------------ optimizer --
 class _StepQueue(object):
     """The fused steps of several parameters of one MyAdam.step() on their way to a launch (ops.adam8_queue). What follows a
-    parameter's step - its new codes bound, its gradient released - happens when the launch is out, so that a launch that
-    fails leaves the parameter with what it had."""
-    LAUNCH = 8              # parameters to a launch
-    HELD_BYTES = 64 << 20   # and what the waiting ones may keep allocated: their copied gradients and new codes
+    parameter's step - its new codes or its residual's curve bound, its gradient released - happens when the launch is out,
+    so that a launch that fails leaves the parameter with what it had."""
+    HELD_BYTES = 64 << 20  # what waiting steps may keep allocated: gradients copied for the step, and new codes
+    __slots__ = ("handle", "waiting", "held")
 
     def __init__(self):
-        self._handle = ops.adam8_queue()
-        self._after, self._params, self._held = [], set(), 0
-
-    def add(self, p, call, held, after):
-        self._after.append((after, call(self._handle)))
-        self._params.add(id(p))
-        self._held += held
-
-    def holds(self, p):
-        return id(p) in self._params
-
-    def full(self):
-        return len(self._after) >= self.LAUNCH or self._held >= self.HELD_BYTES
+        self.handle = ops.adam8_queue()
+        self.waiting = {}  # parameter: its new codes, or (weight_scale, lock_mu) of its residual
+        self.held = 0
 
     def run(self):
-        after, self._after = self._after, []
-        self._params.clear()
-        self._held = 0
-        ops.adam8_run(self._handle)
-        for f, result in after:
-            f(result)
+        waiting, self.waiting, self.held = self.waiting, {}, 0
+        ops.adam8_run(self.handle)
+        for p, after in waiting.items():
+            _stepped(p, after)
+
+
+def _stepped(p, after):
+    if after.__class__ is tuple:
+        p.residual.weight_scale, p.residual.lock_mu = after
+    else:
+        p.data = after
+    if p.grad.__class__ is GradientQTensor:
+        p.grad.zero()
+    else:
+        p.grad = None
 
 
 class MyAdam(torch.optim.Adam):
@@ -1186,18 +1185,18 @@ class MyAdam(torch.optim.Adam):
         queued = getattr(self.update_step, "__func__", None) is _UPDATE_STEP
         self._chosen = self._choose_curves() if queued else frozenset()
         self._in_step = queued
+        update = self._update if queued else self.update_step
         try:
             for gindex, group in enumerate(self.param_groups):
                 for pindex, p in enumerate(group["params"]):
-                    if self._queue is not None and self._queue.holds(p):  # listed twice: its gradient is used up first
-                        self._queue.run()
+                    queue = self._queue
+                    if queue is not None and (len(queue.waiting) >= 8 or queue.held >= _StepQueue.HELD_BYTES or p in queue.waiting):
+                        queue.run()  # a launch's worth, or a parameter listed twice: its gradient is used up first
                     if p.grad is None:
                         continue
                     if len(self.state[p]) == 0:
                         self.init_state(group, p, gindex, pindex)
-                    self.update_step(group, p, gindex, pindex)
-                    if self._queue is not None and self._queue.full():
-                        self._queue.run()
+                    update(group, p, gindex, pindex)
         finally:
             queue, self._queue, self._in_step = self._queue, None, False
             if queue is not None:
@@ -1205,15 +1204,16 @@ class MyAdam(torch.optim.Adam):
         self._chosen = frozenset()
         return loss
 
-    def _launch(self, p, call, held, after):
-        """The fused step of one parameter, ``call(queue)``, and what follows it, ``after(result)``: at once, or with other
-        parameters' steps where step() queues them (``held``: bytes that waiting keeps allocated)."""
+    def _step_queue(self, p, grad):
+        """The queue of the step() under way, for p's step; None where that is to be finished at once."""
         if not self._in_step:
-            after(call(None))
-            return
-        if self._queue is None:
-            self._queue = _StepQueue()
-        self._queue.add(p, call, held, after)
+            return None
+        queue = self._queue
+        if queue is None:
+            queue = self._queue = _StepQueue()
+        if grad is not p.grad and p.grad.bit <= 8:  # made from an int8 accumulator
+            queue.held += 2 * grad.numel()
+        return queue
 
     def to_gpu(self):
         for group in self.param_groups:
@@ -1327,6 +1327,10 @@ class MyAdam(torch.optim.Adam):
 
     @torch.no_grad()
     def update_step(self, group, p, gindex, pindex):
+        """One parameter's step, finished when it returns (utils/quant.py:1081-1148)."""
+        self._update(group, p, gindex, pindex)
+
+    def _update(self, group, p, gindex, pindex):
         state = self.state[p]
         config = self.get_config(gindex, pindex, group)
         grad = p.grad
@@ -1361,11 +1365,14 @@ class MyAdam(torch.optim.Adam):
                 self._requantise(p, pdata, None, step_size, is_q, sr_mode)
                 return
 
-            def bind(new):
-                p.data = new
-                self._release_grad(p)
-            self._launch(p, lambda queue: ops.adam8_update(grad, *moments, beta1, beta2, group["eps"], step_size, requant=requant, queue=queue),
-                         self._copied_bytes(p, grad) + p.numel() // 2, bind)
+            queue = self._step_queue(p, grad)
+            new = ops.adam8_update(grad, *moments, beta1, beta2, group["eps"], step_size, requant=requant,
+                                   queue=None if queue is None else queue.handle)
+            if queue is None:
+                _stepped(p, new)
+            else:
+                queue.waiting[p] = new
+                queue.held += new.numel()
             self.sr_offset += (p.numel() + 7) // 8
             return
         if q8:
@@ -1434,15 +1441,14 @@ class MyAdam(torch.optim.Adam):
             step_size = config["lr"] * math.sqrt(1 - beta2 ** state["step"]) / (1 - beta1 ** state["step"])
             p1, y1, p2, y2 = three_fold_curve_4bit(r.lock_mu)
             q1, z1, q2, z2 = three_fold_curve_4bit(r.mu)
-            mu = r.mu
-
-            def stored(_):
-                r.weight_scale = qs
-                r.lock_mu = mu
-                self._release_grad(p)
-            self._launch(p, lambda queue: ops.adam8_latent_w8_step(
-                grad, p.data, r.residual_int.view(-1), qs.view(-1), *moments, (p1, y1, p2 - p1, y2, 8 - p2),
-                (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2, group["eps"], step_size, queue), self._copied_bytes(p, grad), stored)
+            queue = self._step_queue(p, grad)
+            ops.adam8_latent_w8_step(grad, p.data, r.residual_int.view(-1), qs.view(-1), *moments,
+                                     (p1, y1, p2 - p1, y2, 8 - p2), (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2,
+                                     group["eps"], step_size, None if queue is None else queue.handle)
+            if queue is None:
+                _stepped(p, (qs, r.mu))
+            else:
+                queue.waiting[p] = (qs, r.mu)
             return True
         scales, zeros, shape = _flat_qparam(p.qparam)
         if not (scales.dtype == torch.bfloat16 and zeros.dtype == torch.bfloat16 and scales.is_contiguous()
@@ -1454,15 +1460,15 @@ class MyAdam(torch.optim.Adam):
         step_size = config["lr"] * math.sqrt(1 - beta2 ** state["step"]) / (1 - beta1 ** state["step"])
         p1, y1, p2, y2 = three_fold_curve_4bit(r.lock_mu)
         q1, z1, q2, z2 = three_fold_curve_4bit(r.mu)
-        mu = r.mu
-
-        def stored(_):
-            r.weight_scale = scales.contiguous().reshape(-1, 1)
-            r.lock_mu = mu
-            self._release_grad(p)
-        self._launch(p, lambda queue: ops.adam8_latent_w4_step(
-            grad, p.data, r.residual_int.view(-1), scales, zeros, tuple(shape), *moments, (p1, y1, p2 - p1, y2, 8 - p2),
-            (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2, group["eps"], step_size, queue), self._copied_bytes(p, grad), stored)
+        queue = self._step_queue(p, grad)
+        ops.adam8_latent_w4_step(grad, p.data, r.residual_int.view(-1), scales, zeros, tuple(shape), *moments,
+                                 (p1, y1, p2 - p1, y2, 8 - p2), (q1, z1, q2 - q1, z2, 8 - q2), beta1, beta2,
+                                 group["eps"], step_size, None if queue is None else queue.handle)
+        after = (scales.contiguous().reshape(-1, 1), r.mu)
+        if queue is None:
+            _stepped(p, after)
+        else:
+            queue.waiting[p] = after
         return True
 
     def _requantise(self, p, pdata, direction, step_size, is_q, sr_mode):
@@ -1479,11 +1485,6 @@ class MyAdam(torch.optim.Adam):
             elif p.wbit == 4:
                 p.data = Qfunc_4bit_g_res(pdata, p.residual, qparam=p.qparam)
         self._release_grad(p)
-
-    @staticmethod
-    def _copied_bytes(p, grad):
-        """Bytes of a gradient that was made for this step (from an int8 accumulator); 0 for the parameter's own."""
-        return grad.numel() * grad.element_size() if isinstance(p.grad, GradientQTensor) and p.grad.bit <= 8 else 0
 
     @staticmethod
     def _release_grad(p):
