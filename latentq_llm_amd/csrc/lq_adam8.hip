@@ -527,7 +527,9 @@ extern "C" int lq_adam8_latent_w4_step(const void *grad, void *codes, int32_t *r
                                        int dk1, float db1, int dk2, float db2, int dk3, int qk1, float qb1, int qk2,
                                        float qb2, int qk3, double beta1, double beta2, double eps, double step_size,
                                        void *stream) {
-    return lq_adam8_latent_w4_step_queued(grad, codes, residual, scales, zeros, state1, state2, scale1, max1, scale2, max2, N, K, group, block_elems, dk1, db1, dk2, db2, dk3, qk1, qb1, qk2, qb2, qk3, beta1, beta2, eps, step_size, stream, nullptr);
+    return lq_adam8_latent_w4_step_queued(grad, codes, residual, scales, zeros, state1, state2, scale1, max1, scale2,
+                                          max2, N, K, group, block_elems, dk1, db1, dk2, db2, dk3, qk1, qb1, qk2, qb2,
+                                          qk3, beta1, beta2, eps, step_size, stream, nullptr);
 }
 
 extern "C" int lq_adam8_latent_w8_step_queued(const void *grad, int8_t *codes, int32_t *residual, const void *qscales, uint8_t *state1,
@@ -563,7 +565,9 @@ extern "C" int lq_adam8_latent_w8_step(const void *grad, int8_t *codes, int32_t 
                                        int64_t K, int block_elems, int dk1, float db1, int dk2, float db2, int dk3, int qk1,
                                        float qb1, int qk2, float qb2, int qk3, double beta1, double beta2, double eps,
                                        double step_size, void *stream) {
-    return lq_adam8_latent_w8_step_queued(grad, codes, residual, qscales, state1, state2, scale1, max1, scale2, max2, N, K, block_elems, dk1, db1, dk2, db2, dk3, qk1, qb1, qk2, qb2, qk3, beta1, beta2, eps, step_size, stream, nullptr);
+    return lq_adam8_latent_w8_step_queued(grad, codes, residual, qscales, state1, state2, scale1, max1, scale2, max2,
+                                          N, K, block_elems, dk1, db1, dk2, db2, dk3, qk1, qb1, qk2, qb2, qk3, beta1,
+                                          beta2, eps, step_size, stream, nullptr);
 }
 
 extern "C" int lq_adam8_sr_step_queued(const void *grad, const void *codes_in, void *codes_out, const void *scales, const void *zeros,
@@ -593,7 +597,9 @@ extern "C" int lq_adam8_sr_step(const void *grad, const void *codes_in, void *co
                                 uint8_t *state1, uint8_t *state2, float *scale1, float *max1, float *scale2, float *max2,
                                 int64_t N, int64_t K, int group, int block_elems, double beta1, double beta2, double eps,
                                 double step_size, uint64_t philox_seed, uint64_t philox_offset, void *stream) {
-    return lq_adam8_sr_step_queued(grad, codes_in, codes_out, scales, zeros, state1, state2, scale1, max1, scale2, max2, N, K, group, block_elems, beta1, beta2, eps, step_size, philox_seed, philox_offset, stream, nullptr);
+    return lq_adam8_sr_step_queued(grad, codes_in, codes_out, scales, zeros, state1, state2, scale1, max1, scale2,
+                                   max2, N, K, group, block_elems, beta1, beta2, eps, step_size, philox_seed,
+                                   philox_offset, stream, nullptr);
 }
 
 extern "C" int lq_adam8_queue_new(void **queue_out) {

@@ -603,8 +603,8 @@ PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     LQ_METHOD(linear4), LQ_METHOD(dx4), LQ_METHOD(gate_up), LQ_METHOD(dx_silu), LQ_METHOD(dx_pair), LQ_METHOD(linear8), LQ_METHOD(infer8),
     LQ_METHOD(dx8), LQ_METHOD(quant8), LQ_METHOD(quant8_token), LQ_METHOD(dequant8), LQ_METHOD(weight_grad),
-    LQ_METHOD(weight_grad_acc), LQ_METHOD(weight_grad_acc8), LQ_METHOD(gradq8), LQ_METHOD(adam8_param), LQ_METHOD(adam8_sr), LQ_METHOD(adam8_queue), LQ_METHOD(adam8_run),
-    LQ_METHOD(adam8_w4), LQ_METHOD(adam8_w8), LQ_METHOD(current_stream), LQ_METHOD(set_error), {nullptr, nullptr, 0, nullptr}};
+    LQ_METHOD(weight_grad_acc), LQ_METHOD(weight_grad_acc8), LQ_METHOD(gradq8), LQ_METHOD(adam8_param), LQ_METHOD(adam8_sr),
+    LQ_METHOD(adam8_queue), LQ_METHOD(adam8_run), LQ_METHOD(adam8_w4), LQ_METHOD(adam8_w8), LQ_METHOD(current_stream), LQ_METHOD(set_error), {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_lqbind", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -146,132 +146,132 @@ __global__ __launch_bounds__(64 * WAVES, SPW == 2 ? 4 : SPW > 2 ? 3 : 1) void ge
 #pragma unroll
         for (int j = 0; j < NT; ++j) done[k][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int i = 0; i < SPW; ++i) {
-    const int s = wave + i * WAVES;
-    if (SPW > 1 && s >= n_slots) break;
-    for (int g0 = s * kUnroll; g0 < G; g0 += n_slots * kUnroll) {
-        const bool full = g0 + kUnroll <= G;  // a short tail batch re-reads the last group with zero scale
-        // ---- activations: one LDS-direct load per token row (1 KB = this batch's 512 k), coalesced.
-        //      In a tail batch the lanes past the end of the row re-read its first bytes (dead groups).
-        {
-            const long long xoff = (long long)g0 * (LQ_GROUP * 2) + lane * 16;
-            const long long lim = (long long)K * 2;
-            const long long off = xoff < lim ? xoff : 0;
+        const int s = wave + i * WAVES;
+        if (SPW > 1 && s >= n_slots) break;
+        for (int g0 = s * kUnroll; g0 < G; g0 += n_slots * kUnroll) {
+            const bool full = g0 + kUnroll <= G;  // a short tail batch re-reads the last group with zero scale
+            // ---- activations: one LDS-direct load per token row (1 KB = this batch's 512 k), coalesced.
+            //      In a tail batch the lanes past the end of the row re-read its first bytes (dead groups).
+            {
+                const long long xoff = (long long)g0 * (LQ_GROUP * 2) + lane * 16;
+                const long long lim = (long long)K * 2;
+                const long long off = xoff < lim ? xoff : 0;
 #pragma unroll
-            for (int m = 0; m < MP; ++m)
-                if (m < M)
-                    __builtin_amdgcn_global_load_lds((gbl_void *)((const unsigned char *)x + (long long)m * lim + off),
-                                                     (lds_void *)xs(wave, m), 16, 0, 0);
-        }
-        // ---- codes, scales, zeros
-        u32x4_t wv[NT][kUnroll];
-        float sc[NT][kUnroll], zz[NT][kUnroll];
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const int g = g0 + u < G ? g0 + u : G - 1;
-                const unsigned char *wt = (GU && j == 1) ? wrow2 : wrow + j * tile_stride;
-                wv[j][u] = *reinterpret_cast<const u32x4_t *>(wt + g * 64);
+                for (int m = 0; m < MP; ++m)
+                    if (m < M)
+                        __builtin_amdgcn_global_load_lds((gbl_void *)((const unsigned char *)x + (long long)m * lim + off),
+                                                         (lds_void *)xs(wave, m), 16, 0, 0);
             }
-        if constexpr (QS) {
-            if (first) {
-                publish_q();
-                first = false;
-            }
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const unsigned short *ls = reinterpret_cast<const unsigned short *>(sq + (j * 16 + n) * q_pitch);
-                const unsigned short *lz = reinterpret_cast<const unsigned short *>(sq + q_lds + (j * 16 + n) * q_pitch);
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
-                    const bool live = g0 + u < G;
-                    const int g = live ? g0 + u : G - 1;
-                    sc[j][u] = live ? lq_bf16_bits_to_f32(ls[g]) : 0.0f;
-                    zz[j][u] = 128.0f + lq_bf16_bits_to_f32(lz[g]);
-                }
-            }
-        } else
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const unsigned short *sr = GU ? (j == 0 ? srow : scales2 + (long long)row * G) : srow + (long long)j * 16 * G;
-            const unsigned short *zr = GU ? (j == 0 ? zrow : zeros2 + (long long)row * G) : zrow + (long long)j * 16 * G;
-            if (full) {
-                u32x2_t sraw = {0u, 0u}, zraw = {0u, 0u};
-                if (kq == 0) {
-                    sraw = *reinterpret_cast<const u32x2_t *>(sr + g0);
-                    zraw = *reinterpret_cast<const u32x2_t *>(zr + g0);
-                }
-                unsigned s01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sraw[0]);
-                unsigned s23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sraw[1]);
-                unsigned z01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zraw[0]);
-                unsigned z23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zraw[1]);
-                sc[j][0] = lq_bf16_lo(s01); sc[j][1] = lq_bf16_hi(s01); sc[j][2] = lq_bf16_lo(s23); sc[j][3] = lq_bf16_hi(s23);
-                zz[j][0] = 128.0f + lq_bf16_lo(z01); zz[j][1] = 128.0f + lq_bf16_hi(z01);
-                zz[j][2] = 128.0f + lq_bf16_lo(z23); zz[j][3] = 128.0f + lq_bf16_hi(z23);
-            } else {
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
-                    const bool live = g0 + u < G;
-                    const int g = live ? g0 + u : G - 1;
-                    sc[j][u] = live ? lq_bf16_bits_to_f32(sr[g]) : 0.0f;
-                    zz[j][u] = 128.0f + lq_bf16_bits_to_f32(zr[g]);
-                }
-            }
-        }
-        // ---- codes to the MFMA lane layout
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    wv[j][u][t] = (unsigned)__builtin_amdgcn_ds_bpermute(bperm_src, (int)wv[j][u][t]);
-        // ---- MFMAs
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the staged rows have landed in LDS
-        // One group at a time: a single pair of MFMA accumulators (plus one per extra tile) is live,
-        // which keeps the kernel at <= 80 registers (6 waves per SIMD, three 8-wave workgroups per
-        // CU); the unpacking between two MFMAs on the same accumulator covers their latency.
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            f32x4_t P[NT], S = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < NT; ++j) P[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                unsigned a[4];
-                const u32x4_t xv = *reinterpret_cast<const u32x4_t *>(xfrag + u * 256 + t * 16);
-                permute_x(xv, a);
-                const u32x4_t av = {a[0], a[1], a[2], a[3]};
-                S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
-                                                            __builtin_bit_cast(bf16x8_t, ones), S, 0, 0, 0);
-#pragma unroll
-                for (int j = 0; j < NT; ++j) {
-                    unsigned b[4];
-                    unpack_word_128q(wv[j][u][t], b);
-                    const u32x4_t bv = {b[0], b[1], b[2], b[3]};
-                    P[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
-                                                                   __builtin_bit_cast(bf16x8_t, bv), P[j], 0, 0, 0);
-                }
-            }
+            // ---- codes, scales, zeros
+            u32x4_t wv[NT][kUnroll];
+            float sc[NT][kUnroll], zz[NT][kUnroll];
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(sc[j][u], fmaf(-zz[j][u], S[r], P[j][r]), acc[j][r]);
-            __builtin_amdgcn_sched_barrier(0);  // keeps the next group's unpacking from being hoisted (registers)
-        }
-        // the next batch overwrites the staged rows: all fragment reads above must have returned
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-    if constexpr (SPW > 1) {
+                for (int u = 0; u < kUnroll; ++u) {
+                    const int g = g0 + u < G ? g0 + u : G - 1;
+                    const unsigned char *wt = (GU && j == 1) ? wrow2 : wrow + j * tile_stride;
+                    wv[j][u] = *reinterpret_cast<const u32x4_t *>(wt + g * 64);
+                }
+            if constexpr (QS) {
+                if (first) {
+                    publish_q();
+                    first = false;
+                }
 #pragma unroll
-        for (int k = 0; k < SPW; ++k)
-            if (i == k) {
+                for (int j = 0; j < NT; ++j) {
+                    const unsigned short *ls = reinterpret_cast<const unsigned short *>(sq + (j * 16 + n) * q_pitch);
+                    const unsigned short *lz = reinterpret_cast<const unsigned short *>(sq + q_lds + (j * 16 + n) * q_pitch);
 #pragma unroll
-                for (int j = 0; j < NT; ++j) done[k][j] = acc[j];
+                    for (int u = 0; u < kUnroll; ++u) {
+                        const bool live = g0 + u < G;
+                        const int g = live ? g0 + u : G - 1;
+                        sc[j][u] = live ? lq_bf16_bits_to_f32(ls[g]) : 0.0f;
+                        zz[j][u] = 128.0f + lq_bf16_bits_to_f32(lz[g]);
+                    }
+                }
+            } else
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const unsigned short *sr = GU ? (j == 0 ? srow : scales2 + (long long)row * G) : srow + (long long)j * 16 * G;
+                const unsigned short *zr = GU ? (j == 0 ? zrow : zeros2 + (long long)row * G) : zrow + (long long)j * 16 * G;
+                if (full) {
+                    u32x2_t sraw = {0u, 0u}, zraw = {0u, 0u};
+                    if (kq == 0) {
+                        sraw = *reinterpret_cast<const u32x2_t *>(sr + g0);
+                        zraw = *reinterpret_cast<const u32x2_t *>(zr + g0);
+                    }
+                    unsigned s01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sraw[0]);
+                    unsigned s23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sraw[1]);
+                    unsigned z01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zraw[0]);
+                    unsigned z23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zraw[1]);
+                    sc[j][0] = lq_bf16_lo(s01); sc[j][1] = lq_bf16_hi(s01); sc[j][2] = lq_bf16_lo(s23); sc[j][3] = lq_bf16_hi(s23);
+                    zz[j][0] = 128.0f + lq_bf16_lo(z01); zz[j][1] = 128.0f + lq_bf16_hi(z01);
+                    zz[j][2] = 128.0f + lq_bf16_lo(z23); zz[j][3] = 128.0f + lq_bf16_hi(z23);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < kUnroll; ++u) {
+                        const bool live = g0 + u < G;
+                        const int g = live ? g0 + u : G - 1;
+                        sc[j][u] = live ? lq_bf16_bits_to_f32(sr[g]) : 0.0f;
+                        zz[j][u] = 128.0f + lq_bf16_bits_to_f32(zr[g]);
+                    }
+                }
             }
+            // ---- codes to the MFMA lane layout
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        wv[j][u][t] = (unsigned)__builtin_amdgcn_ds_bpermute(bperm_src, (int)wv[j][u][t]);
+            // ---- MFMAs
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the staged rows have landed in LDS
+            // One group at a time: a single pair of MFMA accumulators (plus one per extra tile) is live,
+            // which keeps the kernel at <= 80 registers (6 waves per SIMD, three 8-wave workgroups per
+            // CU); the unpacking between two MFMAs on the same accumulator covers their latency.
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                f32x4_t P[NT], S = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < NT; ++j) P[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    unsigned a[4];
+                    const u32x4_t xv = *reinterpret_cast<const u32x4_t *>(xfrag + u * 256 + t * 16);
+                    permute_x(xv, a);
+                    const u32x4_t av = {a[0], a[1], a[2], a[3]};
+                    S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
+                                                                __builtin_bit_cast(bf16x8_t, ones), S, 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) {
+                        unsigned b[4];
+                        unpack_word_128q(wv[j][u][t], b);
+                        const u32x4_t bv = {b[0], b[1], b[2], b[3]};
+                        P[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
+                                                                       __builtin_bit_cast(bf16x8_t, bv), P[j], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(sc[j][u], fmaf(-zz[j][u], S[r], P[j][r]), acc[j][r]);
+                __builtin_amdgcn_sched_barrier(0);  // keeps the next group's unpacking from being hoisted (registers)
+            }
+            // the next batch overwrites the staged rows: all fragment reads above must have returned
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        if constexpr (SPW > 1) {
+#pragma unroll
+            for (int k = 0; k < SPW; ++k)
+                if (i == k) {
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) done[k][j] = acc[j];
+                }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
     }
 
     if constexpr (QS) {
@@ -358,9 +358,9 @@ void launch_gu(const GemvGuArgs &a) {
 // staged rows (1040 MP bytes a wave) of c of them have to fit the CU's 160 KB and their waves its registers (16 of this
 // kernel). Within that the fewest rounds of batches, and the fewest waves for that number of rounds. us, 8 waves (what
 // every size took before) -> this rule, both matrices:
-//   11008 x 4096 (c = 3)  1 token 15.9 -> 14.1 (4 waves), 8: 22.7 -> 15.2 (4), 12: 23.4 -> 16.0 (4), 16: 24.0 -> 18.5 (3)
-//   8192 x 2560 (c = 2)   8: 13.0 -> 9.3 (5), 12: 13.2 -> 11.0 (3), 16: 13.5 -> 11.3 (3)
-//   6144 x 3072 (c = 2)   8: 12.4 -> 9.5 (6), 12: 12.6 -> 10.4 (3), 16: 12.8 -> 10.8 (3)
+//   11008 x 4096 (c = 3)  1 token 16.7 -> 15.3 (4 waves), 8: 24.2 -> 16.4 (4), 12: 25.0 -> 17.5 (4), 16: 25.3 -> 20.3 (3)
+//   8192 x 2560 (c = 2)   8: 14.9 -> 10.7 (5), 12: 15.0 -> 12.7 (3), 16: 15.3 -> 13.1 (3)
+//   6144 x 3072 (c = 2)   8: 14.4 -> 11.2 (6), 12: 14.7 -> 12.7 (3), 16: 15.1 -> 13.2 (3)
 // (12 rows and more on 5 or 6 waves are slower although two such workgroups fit: 6144 x 3072 at 12 tokens 11.7 on 6.)
 int gu_waves(int MP, int N, int batches, int slots, int cus) {
     const int c = (N / 16 + cus - 1) / cus;
