@@ -722,6 +722,7 @@ def profile_target(device, which, launches=10):
             s2 = torch.randint(0, 256, (n,), device=device, dtype=torch.uint8)
             q = [torch.full((nblk, 1), v, device=device) for v in (1e-5, 1.3e-3, 1e-5, 2.6e-3)]
             o.adam8_update(grad, s1, s2, q[0], q[1], q[2], q[3], 0.9, 0.95, 1e-8, 1e-3, param=param)
+            o.adam8_update(grad, s1, s2, q[0], q[1], q[2], q[3], 0.9, 0.95, 1e-8, 1e-3, requant=(p, s, z, (N, K), 7, i))
             o.adam8_latent_w4_step(grad, p, res, s.view(-1), z.view(-1), (N, K), s1, s2, q[0], q[1], q[2], q[3], curve, curve,
                                    0.9, 0.95, 1e-8, 1e-3)
             w8 = torch.randint(-128, 128, (N, K), device=device, dtype=torch.int8)
