@@ -201,10 +201,10 @@ def test_a16w4_fwd_gemv_many_tokens_staged_scales(ops, co, M, N, K):
 
 
 def test_gemv_and_gemm_agree_on_the_same_tokens_within_the_documented_bound(ops, co):
-    """Up to 16 tokens take the GEMV, which multiplies s * sum((q - z) x) in fp32; more tokens take kernels that
-    round the dequantised weight to bf16 first, as the reference does. The same token therefore gets slightly
+    """Up to 16 tokens take the GEMV, which multiplies s * sum((q - z) x) in fp32, and so do the kernels of up to 64; more
+    tokens take kernels that round the dequantised weight to bf16 first, as the reference does. The same token therefore gets slightly
     different outputs depending on how many tokens ride along: at most 2^-9 relative per weight, i.e. well
-    inside the parity bar. Measured here between M = 16 (GEMV), M = 17 (GEMV chunks or GEMM) and M = 256 (GEMM)."""
+    inside the parity bar. Measured here between M = 16 (GEMV), M = 17 and M = 256 (GEMM)."""
     N, K = 4096, 4096
     codes, packed, scales, zeros = make_w4(N, K, 77)
     x = randn_bf16((256, K), 78)
