@@ -566,10 +566,15 @@ class _HookHandle(torch.utils.hooks.RemovableHandle):
     """What add_hook leaves in hook_handle, a handle like those of torch's own hooks: remove(), or the end of a with block on
     it, ends the delivery of weight gradients (a layer's then stay in dict_temp, as with the reference's hook removed; a
     fused block forms none for it)."""
+    active = True
 
-    @property
-    def active(self):
-        return self.id in (self.hooks_dict_ref() or ())
+    def remove(self):
+        super().remove()
+        self.active = False
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        self.active = self.id in (self.hooks_dict_ref() or ())
 
 
 def _removed(handle):
