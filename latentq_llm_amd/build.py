@@ -26,6 +26,9 @@ COMMON = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # every fp32 rounding is written out (fmaf where a fused operation is meant)
     "-ffp-contract=off",
+    # up to 16 (14 in practice) dwords of leading scalar arguments arrive in registers with the wave instead of by a load that
+    # every address waits for: 0.1 to 0.4 us of a 3 to 12 us kernel. Arguments passed as a structure are not preloaded.
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option",
 ]
 EXTRA: dict[str, list[str]] = {}

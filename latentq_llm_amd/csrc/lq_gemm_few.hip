@@ -52,9 +52,12 @@ constexpr int kWaves = 4;
 //   activations  16 MT rows of 256 bytes, piece c of row i at c ^ (i & 15)
 //   codes        16 rows of 64 bytes, piece c of row i at c ^ ((i >> 2) & 3)
 //   scales, zeros  a dword per row each, the bf16 value in its lower half (and 32 dwords of copies)
-// MT: groups of 16 tokens, D: stages
+// MT: groups of 16 tokens, D: stages. Arguments: those of the first loads first (the leading 14 dwords are preloaded, build.py)
 template <int MT, int D>
-__global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(FewParams p) {
+__global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(
+    const unsigned char *x_, const unsigned char *w_, int M, int N, int K, const unsigned short *scales, const unsigned short *zeros,
+    const unsigned short *bias, unsigned short *y, unsigned long long *clk) {
+    const FewParams p = {x_, w_, scales, zeros, bias, y, M, N, K, clk};
     constexpr int A_BYTES = MT * 4096, STAGE = A_BYTES + 1024 + 256;
     constexpr int LOADS = 4 * MT + 2;
     static_assert((D - 1) * LOADS < 64, "the wait counts loads in six bits");
@@ -205,8 +208,9 @@ int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, con
     // the 32-bit lane offsets of the loads span the tokens' rows and 16 rows of codes
     if (128ll * K >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: K too large", who);
     const dim3 grid((unsigned)(N / 16)), block(64 * kWaves);
-    if (M <= 32) hipLaunchKernelGGL((gemm_few_kernel<2, 4>), grid, block, 0, st, p);
-    else if (M <= 48) hipLaunchKernelGGL((gemm_few_kernel<3, 3>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((gemm_few_kernel<4, 2>), grid, block, 0, st, p);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, p.x, p.w, M, N, K, p.scales, p.zeros, p.bias, p.y, clk); };
+    if (M <= 32) launch(gemm_few_kernel<2, 4>);
+    else if (M <= 48) launch(gemm_few_kernel<3, 3>);
+    else launch(gemm_few_kernel<4, 2>);
     return lq_check_launch(who);
 }

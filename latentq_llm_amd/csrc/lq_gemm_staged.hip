@@ -62,9 +62,14 @@ constexpr int D = 3;
 //   scales, zeros  one dword per column each, the bf16 value in its lower half
 // FM: 32-row fragments of the row tile (32 FM rows)
 // EXACT: weights as they are (see the top of the file), else rounded to bf16 like those of the kernels for more tokens
+// Arguments: those of the first loads first (the leading 14 dwords are preloaded into registers, build.py)
 // (launch bounds: with two waves per SIMD asked for, the products of FM < 4 go to vector registers, which the scaling can read)
 template <int FM, bool EXACT>
-__global__ __launch_bounds__(256, FM < 4 ? 2 : 1) void gemm_staged_kernel(StagedParams p) {
+__global__ __launch_bounds__(256, FM < 4 ? 2 : 1) void gemm_staged_kernel(
+    const unsigned char *x_, const unsigned char *w_, int M, int N, int K, int tiles_m, int tiles_n, int groups_per_split,
+    const unsigned short *scales, const unsigned short *zeros, float *partial, const unsigned short *bias_, unsigned short *y,
+    const unsigned char *w2, const unsigned short *scales2, const unsigned short *zeros2, unsigned long long *clk) {
+    const StagedParams p = {x_, w_, scales, zeros, bias_, w2, scales2, zeros2, y, partial, M, N, K, tiles_m, tiles_n, groups_per_split, clk};
     constexpr int BM = 32 * FM;
     constexpr int A_BYTES = BM * 256;
     constexpr int STAGE = A_BYTES + kCodeBytes + kScaleBytes;
@@ -294,7 +299,8 @@ int launch_staged_tile(StagedParams p, int splits, hipStream_t st, const char *w
     p.tiles_m = (p.M + 32 * FM - 1) / (32 * FM);
     p.tiles_n = (p.N + kCols - 1) / kCols;
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits, p.w2 ? 2u : 1u);
-    hipLaunchKernelGGL((gemm_staged_kernel<FM, EXACT>), grid, dim3(256), 0, st, p);
+    hipLaunchKernelGGL((gemm_staged_kernel<FM, EXACT>), grid, dim3(256), 0, st, p.x, p.w, p.M, p.N, p.K, p.tiles_m, p.tiles_n, p.groups_per_split,
+                       p.scales, p.zeros, p.partial, p.bias, p.y, p.w2, p.scales2, p.zeros2, p.clk);
     return lq_check_launch(who);
 }
 

@@ -56,16 +56,14 @@ constexpr int kXRow = 1024 + 16;  // LDS bytes per staged token row: 4 groups x 
 // alone, and a wave works through up to SPW partial sums one after the other: the order of the fp32 sums, and so the bits of
 // the result, do not depend on how many waves the launcher finds best for the grid.
 // (SPW = 2 in at most 128 registers, four waves to a SIMD; more in 168)
+// The arguments that the first loads need come first: the leading 14 dwords are preloaded into registers (build.py). Weights from
+// HBM, 1 token: 4096 x 4096 5.15 -> 4.77 us, 4096 x 11008 8.01 -> 7.76, 2048 x 2048 3.48 -> 3.31.
 template <int WAVES, int MP, int NT, bool QS, bool GU = false, int SPW = 1>
-__global__ __launch_bounds__(64 * WAVES, SPW == 2 ? 4 : SPW > 2 ? 3 : 1) void gemv_kernel(const unsigned short *__restrict__ x,
-                                                          const unsigned char *__restrict__ codes,
-                                                          const unsigned short *__restrict__ scales,
-                                                          const unsigned short *__restrict__ zeros,
-                                                          const unsigned short *__restrict__ bias,
-                                                          unsigned short *__restrict__ y, int M, int N, int K,
-                                                          const unsigned char *__restrict__ codes2 = nullptr,
-                                                          const unsigned short *__restrict__ scales2 = nullptr,
-                                                          const unsigned short *__restrict__ zeros2 = nullptr, int slots = WAVES) {
+__global__ __launch_bounds__(64 * WAVES, SPW == 2 ? 4 : SPW > 2 ? 3 : 1) void gemv_kernel(
+    const unsigned short *__restrict__ x, const unsigned char *__restrict__ codes, int M, int N, int K, int slots,
+    const unsigned short *__restrict__ scales, const unsigned short *__restrict__ zeros, const unsigned short *__restrict__ bias,
+    unsigned short *__restrict__ y, const unsigned char *__restrict__ codes2, const unsigned short *__restrict__ scales2,
+    const unsigned short *__restrict__ zeros2) {
     static_assert(!GU || (NT == 2 && !QS), "gate / up mode: two tiles, scales and zeros straight from memory");
     constexpr int RT = GU ? 1 : NT;  // 16-row tiles of output rows per workgroup
     static_assert(GU || SPW == 1, "several partial sums per wave: gate / up mode only");
@@ -335,9 +333,9 @@ struct GemvGuArgs {
 template <int W, int MP, int SPW>
 void launch_gu_spw(const GemvGuArgs &a) {
     hipLaunchKernelGGL((gemv_kernel<W, MP, 2, false, true, SPW>), dim3(a.N / 16), dim3(64 * W), 0, a.st, (const unsigned short *)a.x,
-                       (const unsigned char *)a.codes, (const unsigned short *)a.scales, (const unsigned short *)a.zeros,
-                       (const unsigned short *)nullptr, (unsigned short *)a.y, a.M, a.N, a.K, (const unsigned char *)a.codes2,
-                       (const unsigned short *)a.scales2, (const unsigned short *)a.zeros2, a.slots);
+                       (const unsigned char *)a.codes, a.M, a.N, a.K, a.slots, (const unsigned short *)a.scales, (const unsigned short *)a.zeros,
+                       (const unsigned short *)nullptr, (unsigned short *)a.y, (const unsigned char *)a.codes2,
+                       (const unsigned short *)a.scales2, (const unsigned short *)a.zeros2);
 }
 
 // Partial sums of a gate / up pass, at most: the waves of the workgroups that stage 4 or 16 rows with one batch each
@@ -411,14 +409,13 @@ void launch_one(const GemvArgs &a) {
     const int batches = (a.K / LQ_GROUP + kUnroll - 1) / kUnroll;
     const bool qs = MP == 16 && (NT == 2 || batches > W) && lq_aligned(a.scales, 16) && lq_aligned(a.zeros, 16) &&
                     2 * q_bytes <= (size_t)64 * W * 2 * 16;
-    if (qs)
-        hipLaunchKernelGGL((gemv_kernel<W, MP, NT, true>), dim3(a.N / (16 * NT)), dim3(64 * W), 2 * q_bytes + 2 * 16 * NT * 16, a.st,
-                           (const unsigned short *)a.x, (const unsigned char *)a.codes, (const unsigned short *)a.scales,
-                           (const unsigned short *)a.zeros, (const unsigned short *)a.bias, (unsigned short *)a.y, a.M, a.N, a.K);
-    else
-        hipLaunchKernelGGL((gemv_kernel<W, MP, NT, false>), dim3(a.N / (16 * NT)), dim3(64 * W), 0, a.st,
-                           (const unsigned short *)a.x, (const unsigned char *)a.codes, (const unsigned short *)a.scales,
-                           (const unsigned short *)a.zeros, (const unsigned short *)a.bias, (unsigned short *)a.y, a.M, a.N, a.K);
+    auto launch = [&](auto kernel, size_t lds) {
+        hipLaunchKernelGGL(kernel, dim3(a.N / (16 * NT)), dim3(64 * W), lds, a.st, (const unsigned short *)a.x, (const unsigned char *)a.codes,
+                           a.M, a.N, a.K, W, (const unsigned short *)a.scales, (const unsigned short *)a.zeros, (const unsigned short *)a.bias,
+                           (unsigned short *)a.y, (const unsigned char *)nullptr, (const unsigned short *)nullptr, (const unsigned short *)nullptr);
+    };
+    if (qs) launch(gemv_kernel<W, MP, NT, true>, 2 * q_bytes + 2 * 16 * NT * 16);
+    else launch(gemv_kernel<W, MP, NT, false>, 0);
 }
 
 // Waves per workgroup: as many as there are batches, up to the cap, in powers of two. More waves
