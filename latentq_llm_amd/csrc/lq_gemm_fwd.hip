@@ -90,8 +90,18 @@ constexpr int STAGE = BM * ROWB;     // 16 KB per A stage
 // of one fragment read per MFMA instead of half of one).
 // GU (with NT = 2): gate / up mode. The workgroup then covers 128 output columns (both matrices' rows
 // c0 .. c0 + 127) instead of 256.
-template <int NT, bool GU>
-__global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
+// KS: groups of four waves that share the tile and each take a part of K (1 or 2). A workgroup alone on its compute unit has
+// one wave per SIMD, and such a wave issues its MFMAs, conversions and LDS reads one behind the other (0.61 us per step where
+// the MFMAs take 0.25). Two groups on stages of their own fill each other's gaps; their sums meet in LDS at the end.
+// us with one group -> two, weights from HBM:
+//   128 x 128 tiles  1019 tokens, 4096 x 4096 46.7 -> 37.1, 800: 46.6 -> 35.2; 256 tokens, 11008 x 4096 46.3 -> 35.7;
+//                    1024 tokens, 3072 x 768 10.2 -> 10.1
+//   128 x 256 tiles  1536 tokens, 4096 x 4096 56.0 -> 53.3, 2048 tokens, 4096 x 11008 160.4 -> 156.8 (256 workgroups: the
+//                    power limit); gate / up 256 tokens, 11008 x 4096 57.8 -> 54.2
+// Where units get several workgroups, these fill the gaps already, and a workgroup twice as large is slower (2048 tokens,
+// 11008 x 4096 156.3 against 163.8). Three groups: 37.9 on the first size, 92.2 against 95.2 on 1019 tokens, 4096 x 11008.
+template <int NT, bool GU, int KS>
+__global__ __launch_bounds__(256 * KS, 2) void gemm_fwd_direct_kernel(FwdParams p) {
     static_assert(NT == 2 || (NT == 1 && !GU), "gate / up mode uses both column tiles");
     constexpr int BNO = (GU || NT == 1) ? BN / 2 : BN;  // output columns per workgroup
     constexpr int WN = BNO / 4;                         // output columns per wave
@@ -101,15 +111,15 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
     // steps (steps 2j and 2j+1 are 64 contiguous bytes of a row across the two lane halves: fetched
     // together they pull their cache line through L1 twice instead of four times)
     constexpr int NB = 2;
-    __shared__ __attribute__((aligned(16))) unsigned char lds_a0[STAGE];
-    __shared__ __attribute__((aligned(16))) unsigned char lds_a1[STAGE];
-    __shared__ __attribute__((aligned(16))) unsigned char lds_a2[STAGE];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[3 * KS * STAGE];
+    const int wave_all = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int kg = KS == 1 ? 0 : wave_all >> 2, wave = KS == 1 ? wave_all : wave_all & 3;
+    const int tid = KS == 1 ? (int)threadIdx.x : (int)(threadIdx.x & 255);
     auto abuf = [&](auto i) -> unsigned char * {
         constexpr int I = decltype(i)::value;
-        return I == 0 ? lds_a0 : I == 1 ? lds_a1 : lds_a2;
+        return lds + (I * KS + kg) * STAGE;
     };
 
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     const int r = lane & 31, h = lane >> 5;
     unsigned long long clk_t0 = 0, clk_r0 = 0;
@@ -134,21 +144,26 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
     const int bw = rest < GN ? rest : GN;
     const int tile_m = within / bw, tile_n = band * GN + within % bw;
     const int m0 = tile_m * BM, c0 = tile_n * BNO;
-    const int nk = p.K * ESZ / ROWB;
+    const int nk_all = p.K * ESZ / ROWB;
     const long long lda = (long long)p.K * ESZ;
+    // the groups' parts of K: multiples of 256 k (scales and zeros come four groups of 128 k at a time, 4-byte aligned)
+    const int quads = nk_all / 4, q_each = quads / KS, q_more = quads % KS;
+    const int k_first = KS == 1 ? 0 : 4 * (kg * q_each + (kg < q_more ? kg : q_more));
+    const int nk = KS == 1 ? nk_all : 4 * (q_each + (kg < q_more ? 1 : 0));
+    const int nk_most = 4 * (q_each + (q_more ? 1 : 0));
 
     // ---- A staging: 1024 16-byte slots per stage; slot s = i*256 + thread -> row s/8, position s%8
     unsigned a_off[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int row = i * 32 + (int)(threadIdx.x >> 3);
-        const int pos = threadIdx.x & 7;
+        const int row = i * 32 + (tid >> 3);
+        const int pos = tid & 7;
         const int chunk = pos ^ ((row >> 1) & 7);
         int gr = m0 + row;
         gr = gr < p.M ? gr : p.M - 1;
         a_off[i] = (unsigned)((long long)(gr - m0) * lda + chunk * 16);
     }
-    const unsigned char *a_base = p.x + (long long)m0 * lda;
+    const unsigned char *a_base = p.x + (long long)m0 * lda + (long long)k_first * ROWB;
     auto issue_a_one = [&](int kt, unsigned char *la, int i) {
         const unsigned char *src = a_base + (long long)kt * ROWB;
         const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(la + (i * 256 + wave * 64) * 16));
@@ -167,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
 
     // ---- B: buffer descriptors over this workgroup's weight rows (rows past N read as zero), the
     // lane's two rows as 32-bit offsets, the reduction step as the scalar offset
-    const int groups_per_row = p.K / LQ_GROUP;
+    const int groups_per_row = p.K / LQ_GROUP, groups = KS == 1 ? groups_per_row : nk / 2;
     const int rows_here = p.N - c0 < BNO ? p.N - c0 : BNO;
     auto make_rsrc = [](const void *base, unsigned bytes) {
         const unsigned long long a = (unsigned long long)base;
@@ -186,8 +201,8 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const unsigned n = GU ? wave * 32 + r : wave * WN + i * 32 + r;
-        w_off[i] = n * wpitch + h * (WROW / 2);
-        q_off[i] = n * (unsigned)groups_per_row * 2u;
+        w_off[i] = n * wpitch + h * (WROW / 2) + (unsigned)(k_first * WROW);
+        q_off[i] = n * (unsigned)groups_per_row * 2u + (unsigned)k_first;
     }
 
     f32x16_t acc[NT][4];
@@ -333,7 +348,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
                 else if (ODD) deq_one(cn, 0, 0, bf[0], i);
                 else deq_one(cw, 1, 0, bf[0], i);
                 if (t == 0 && !ODD) load_codes_one(kt_codes, cn, i);
-                if (t == 1 && !ODD) load_qparams_one((kt + 2) >> 1 < groups_per_row ? (kt + 2) >> 1 : groups_per_row - 1, i);
+                if (t == 1 && !ODD) load_qparams_one((kt + 2) >> 1 < groups ? (kt + 2) >> 1 : groups - 1, i);
                 if (t >= 2) {
                     if constexpr (NT == 2) {
                         issue_a_one(kt_a, la_load, 2 * (t - 2) + i);
@@ -356,15 +371,15 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
 
     load_qparams(0);
     load_codes(0, cn);
-    issue_a(0, lds_a0);
-    issue_a(nk > 1 ? 1 : 0, lds_a1);
+    issue_a(0, abuf(ic<0>()));
+    issue_a(nk > 1 ? 1 : 0, abuf(ic<1>()));
     wait_and_meet(ic<4>(), ic<1>());
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
         for (int b = 0; b < NB; ++b) cw[i][b] = cn[i][b];
     use_qparams(0);
-    read_a(lds_a0, 0, af[0]);
+    read_a(abuf(ic<0>()), 0, af[0]);
 #pragma unroll
     for (int i = 0; i < NT; ++i) deq_one(cw, 0, 0, bf[0], i);
     __builtin_amdgcn_sched_barrier(0);
@@ -385,10 +400,37 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
     if (rem > 2) step(kt + 2, ic<2>(), ic<0>());
     if (rem > 3) step(kt + 3, ic<0>(), ic<1>());
     if (rem > 4) step(kt + 4, ic<1>(), ic<0>());
+    if constexpr (KS > 1)  // the other group's last steps: every wave meets as many barriers
+        for (int i = nk; i < nk_most; ++i) asm volatile("s_barrier" ::: "memory");
     // the clamped prefetches of the last two steps are still writing LDS: drain them
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     __syncthreads();
+    // KS > 1: half of the wave's rows to the other group, column tile by column tile (64 KB of LDS at a time)
+    auto mine = [&](int j) { return KS == 1 || (j >> 1) == kg; };
+    if constexpr (KS > 1) {
+        f32x4_t *part = reinterpret_cast<f32x4_t *>(lds) + tid;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (!mine(j))
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        part[(j * 4 + q) * 256] = f32x4_t{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (mine(j))
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const f32x4_t v = part[(j * 4 + q) * 256];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += v[e];
+                    }
+            __syncthreads();
+        }
+    }
     if constexpr (GU || NT == 1) {
         // ---- 32 output columns per wave: column c0 + 32*wave + 8*(q/4) + 4h + q%4, row m0 + 32j + r.
         // Gate / up mode: acc[0] and acc[1] hold the same output element of the two products and
@@ -396,7 +438,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
         // columns pass through LDS (row pitch 80 bytes) and leave as 16 bytes per lane, 4 lanes on the 64
         // contiguous bytes of a row.
         constexpr int EP = 80;
-        unsigned char *ep = ((wave & 2) ? lds_a1 : lds_a0) + (wave & 1) * (32 * EP);
+        unsigned char *ep = lds + wave_all * (32 * EP);
         const int ep_row = lane >> 2, ep_chunk = lane & 3;
         const int c_lane = c0 + wave * WN + ep_chunk * 8;
         float bias_n[4][4];
@@ -413,6 +455,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
             unsigned short *dst = which == 0 ? p.y : which == 1 ? p.g_out : p.u_out;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
+                if (!mine(j)) continue;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     float v[4];
@@ -448,7 +491,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
     // loop and its loads have landed; a wave's staging area is private (waves 0,1 in stage 0, waves
     // 2,3 in stage 1), row pitch 144 bytes.
     constexpr int EP = 144;
-    unsigned char *ep = ((wave & 2) ? lds_a1 : lds_a0) + (wave & 1) * (32 * EP);
+    unsigned char *ep = lds + wave_all * (32 * EP);
     const int ep_row = lane >> 3, ep_chunk = lane & 7;
     const int c_lane = c0 + wave * 64 + ep_chunk * 8;  // first of the 8 columns this lane stores
     float bias_v[2][4][4];
@@ -465,6 +508,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fwd_direct_kernel(FwdParams p) {
         }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+        if (!mine(j)) continue;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
 #pragma unroll
@@ -510,7 +554,11 @@ static int launch_direct(FwdParams p, hipStream_t st, const char *who) {
     if (nwg > 0x7FFFFFFFll) return lq_fail(LQ_ERR_BAD_ARG, "%s: problem too large", who);
     // the 32-bit lane offsets of the activation and weight loads span 128 / 256 rows
     if ((long long)BN * p.K * 2 >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: K too large", who);
-    hipLaunchKernelGGL((gemm_fwd_direct_kernel<NT, GU>), dim3((unsigned)nwg), dim3(256), 0, st, p);
+    // Two groups of waves per workgroup where no compute unit gets a second workgroup, and each group has at least 4 steps.
+    if (nwg <= lq_device_cu_count() && p.K >= 512)
+        hipLaunchKernelGGL((gemm_fwd_direct_kernel<NT, GU, 2>), dim3((unsigned)nwg), dim3(512), 0, st, p);
+    else
+        hipLaunchKernelGGL((gemm_fwd_direct_kernel<NT, GU, 1>), dim3((unsigned)nwg), dim3(256), 0, st, p);
     return lq_check_launch(who);
 }
 
