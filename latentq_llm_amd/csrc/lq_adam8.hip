@@ -31,6 +31,13 @@
 // two rounding instructions, two barriers and the exact square root computed beside the short one:
 //   parameter 42.5 -> 37.6 us (33.3), direction 39.3 -> 30.7 (26.6), direction + requantizer 48.2 -> 33.7 in one pass
 //   (23.3), int4 + residual 63.0 -> 46.8 (26.7), int8 + residual 60.4 -> 46.6 (29.9).
+// A block of 2048 has 256 codes at most for each moment, and what the step makes of a stored moment before the gradient
+// comes in (dequantise, round, square, decay, round: 13 instructions for the two) depends on nothing but the code: the block's
+// 128 threads form the 512 values once and an element looks its two up in LDS (random reads; with their
+// bank conflicts LDS is busy for a third of the launch). One block to a workgroup, so that a look-up is a byte shifted and a
+// read. A decoder layer's six weights (50 M elements): stochastic rounding 91.9 -> 85.3 us, int4 + residual 141.9 -> 134.7;
+// 64 M elements: int8 + residual 164.5 -> 155.7, bf16 151.8 -> 147.8. 57 vector instructions an element are left of 65 in
+// the first, and the vector ALUs are busy all the time.
 #include "lq_latent_math.h"
 #include "lq_requant_math.h"
 
@@ -106,12 +113,6 @@ __device__ __forceinline__ float min3_abs(float a, float b, float c) {  // of |a
     return r;
 }
 
-// byte I (0..7) of a pair of words as a float
-template <int I>
-__device__ __forceinline__ float byte_f32(const u32x2_t &w) {
-    return (float)((w[I >> 2] >> (8 * (I & 3))) & 0xFFu);
-}
-
 // x[8] -> uint8 codes with the block's (scale, max); returns them packed, 8 bytes.
 // The quotient (hi - x) / scale must be the correctly rounded one (a quotient one ulp off can fall on the other side of
 // a rounding tie). The divisor is shared by the whole block: with its correctly rounded reciprocal r = RN(1 / scale) and
@@ -175,18 +176,20 @@ __device__ __forceinline__ void requant8_w8(const float (&out)[8], float ws, flo
 }
 
 // BS elements share one (scale, max) pair per moment: TPB threads of CH chunks of 8 elements, chunk c of thread t being
-// elements 8 (c TPB + t) .. + 7 of the block, so that every access of a wave is contiguous.
+// elements 8 (c TPB + t) .. + 7 of the block, so that every access of a wave is contiguous. BPW blocks per workgroup.
 template <int BS, int MODE>
-__global__ __launch_bounds__(256) void adam8_kernel(Adam8Batch b) {
+__global__ __launch_bounds__(BS == 2048 ? 128 : 256) void adam8_kernel(Adam8Batch b) {
     int which = 0;
     for (int i = 1; i < b.n; ++i) which = blockIdx.x >= b.first[i] ? i : which;
     const Adam8Params &a = b.a[which];
-    constexpr int CH = BS == 2048 ? 2 : 1, TPB = BS / 8 / CH, BPW = 256 / TPB;
+    constexpr int CH = BS == 2048 ? 2 : 1, TPB = BS / 8 / CH, BPW = BS == 2048 ? 1 : 256 / TPB;
     __shared__ float red[4][4];
     __shared__ float vtab[16];  // latent modes: dequantised values of the 16 residual nibbles
+    constexpr bool kTables = BS == 2048;
+    __shared__ float tabs[2][256];
     if constexpr (MODE == ADAM_W4 || MODE == ADAM_W8) {
         lq_latent_fill_value_table(vtab, a.dequant_curve);
-        __syncthreads();
+        if constexpr (!kTables) __syncthreads();
     }
     const int t = threadIdx.x % TPB;
     long long blk = (long long)(blockIdx.x - b.first[which]) * BPW + threadIdx.x / TPB;
@@ -217,6 +220,22 @@ __global__ __launch_bounds__(256) void adam8_kernel(Adam8Batch b) {
     }
     const float sc1 = a.scale1[blk], mx1 = a.max1[blk], sc2 = a.scale2[blk], mx2 = a.max2[blk];
 
+    // what a code contributes to the new moments
+    auto first_moment = [&](float q) { return lq_bf16r(lq_bf16r(mx1 - q * sc1) * a.beta1); };
+    auto second_moment = [&](float q) {
+        const float s2 = mx2 - q * sc2;
+        return lq_bf16r(lq_bf16r(s2 * s2) * a.beta2);
+    };
+    if constexpr (kTables) {
+#pragma unroll
+        for (int i = 0; i < 256 / TPB; ++i) {
+            const int q = t + i * TPB;
+            tabs[0][q] = first_moment((float)q);
+            tabs[1][q] = second_moment((float)q);
+        }
+        __syncthreads();
+    }
+
     float m[CH][8], d[CH][8];
     float lo1, hi1, lo2, hi2;
 #pragma unroll
@@ -226,18 +245,12 @@ __global__ __launch_bounds__(256) void adam8_kernel(Adam8Batch b) {
         float g[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) g[k] = (k & 1) ? lq_bf16_hi(g4[c][k >> 1]) : lq_bf16_lo(g4[c][k >> 1]);
-        const float c1[8] = {byte_f32<0>(q1[c]), byte_f32<1>(q1[c]), byte_f32<2>(q1[c]), byte_f32<3>(q1[c]),
-                             byte_f32<4>(q1[c]), byte_f32<5>(q1[c]), byte_f32<6>(q1[c]), byte_f32<7>(q1[c])};
-        const float c2[8] = {byte_f32<0>(q2[c]), byte_f32<1>(q2[c]), byte_f32<2>(q2[c]), byte_f32<3>(q2[c]),
-                             byte_f32<4>(q2[c]), byte_f32<5>(q2[c]), byte_f32<6>(q2[c]), byte_f32<7>(q2[c])};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            float mk = lq_bf16r(mx1 - c1[k] * sc1);
-            const float s2 = mx2 - c2[k] * sc2;
-            float vk = lq_bf16r(s2 * s2);
-            mk = lq_bf16r(mk * a.beta1);
+            const unsigned b1 = (q1[c][k >> 2] >> (8 * (k & 3))) & 0xFFu, b2 = (q2[c][k >> 2] >> (8 * (k & 3))) & 0xFFu;
+            const float mk = kTables ? tabs[0][b1] : first_moment((float)b1);
+            const float vk = kTables ? tabs[1][b2] : second_moment((float)b2);
             m[c][k] = lq_bf16r(fmaf(a.one_minus_beta1, g[k], mk));
-            vk = lq_bf16r(vk * a.beta2);
             v[k] = lq_bf16r(fmaf(a.one_minus_beta2 * g[k], g[k], vk));
             // bf16(sqrt(v)) of a bf16 v: the square root of a number with 8 significant bits never comes closer than
             // 2^-19 (relative) to the midpoint of two bf16 values, so the hardware's one-ulp square root rounds to the
@@ -404,7 +417,7 @@ struct Adam8Item {
 // The items of one mode and block size, kAdam8Batch to a launch
 template <int BS, int MODE>
 int adam8_launch_items(const char *who, const Adam8Item *const *items, int n, hipStream_t st) {
-    constexpr int kPerWg = BS == 2048 ? 2 : 16;  // blocks per workgroup
+    constexpr int kPerWg = BS == 2048 ? 1 : 16;  // blocks per workgroup
     for (int i0 = 0; i0 < n; i0 += kAdam8Batch) {
         Adam8Batch b = {};
         b.n = n - i0 < kAdam8Batch ? n - i0 : kAdam8Batch;
@@ -420,7 +433,7 @@ int adam8_launch_items(const char *who, const Adam8Item *const *items, int n, hi
             wgs += mine;
         }
         b.first[b.n] = (unsigned)wgs;
-        hipLaunchKernelGGL((adam8_kernel<BS, MODE>), dim3((unsigned)wgs), dim3(256), 0, st, b);
+        hipLaunchKernelGGL((adam8_kernel<BS, MODE>), dim3((unsigned)wgs), dim3(BS == 2048 ? 128 : 256), 0, st, b);
         const int rc = lq_check_launch(who);
         if (rc) return rc;
         i0 += b.n - kAdam8Batch;  // (a cut batch: go on behind it)
