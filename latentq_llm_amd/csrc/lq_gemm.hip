@@ -697,8 +697,8 @@ int lq_gemm_staged_launch(const void *x, const void *codes, const void *scales, 
                           unsigned long long *clk, const char *who);
 
 int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *scales_g, const void *zeros_g, const void *codes_u,
-                               const void *scales_u, const void *zeros_u, float *partial, int M, int N, int K, int rows, int splits,
-                               int per_split, hipStream_t st, const char *who);
+                               const void *scales_u, const void *zeros_u, void *h, void *g_out, void *u_out, float *partial, int M, int N,
+                               int K, int rows, int splits, int per_split, hipStream_t st, const char *who);
 
 // 17 to 64 tokens, one launch with 16 columns per compute unit (lq_gemm_few.hip)
 int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
@@ -924,14 +924,13 @@ struct GateUpPlan {
 
 // Gate / up product, M > 16.
 // Few tokens leave most of a 128-row tile empty and most units idle: the staged kernel then runs both products as one
-// launch of 32, 64 or 128 rows, planned as one product of 2 N columns, and a second launch adds its slices and forms h.
+// launch of 32, 64 or 128 rows, planned as one product of 2 N columns. It writes h itself, or where K is cut a second
+// launch adds the slices and forms h.
 // Both sides estimated: the weights-direct kernel by its pace per 64-deep step (0.58 to 0.68 us for a workgroup with a
-// unit to itself, 1.3 for two) plus 7 us, the staged one by its own plan plus, where that is not in it, the partial
-// products' way through the cache. us against the weights-direct kernel and the two plain products with tensor glue:
-//   11008 x 4096  17 / 45 / 128 tokens  25.7 / 27.7 / 37.3 against 51.1 / 50.4 / 50.5 and 45.5 / 43.9 / 55.7; behind from
-//                 160 on (64.5 against 52.1)
-//   6144 x 3072   17 / 64 / 256         13.4 / 20.2 / 30.9 against 35.8 / 35.9 / 36.4; level at 300
-//   3072 x 1024   17 / 128 / 300        10.3 / 11.7 / 15.3 against 15.0 / 15.1 / 15.5; 19.2 against 15.6 at 400
+// unit to itself, 1.3 for two) plus 7 us, the staged one by its own plan plus what the partial products' way through the cache
+// cost when K was not cut either, on the safe side since the kernel writes h. us against the weights-direct kernel:
+//   11008 x 4096  17 / 45 / 128 tokens  19.4 / 23.2 / 36 against 51.1 / 50.4 / 50.5
+//   6144 x 3072   100                   18.5 against 35.9
 static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     GateUpPlan out;
     if (ws_bytes < (size_t)8 * M * N) return out;
@@ -971,9 +970,9 @@ static int gate_up_impl(const char *who, const void *x, const void *codes_gate, 
     LQ_REQUIRE(!workspace || lq_aligned(workspace, 16), "%s: the workspace must be 16-byte aligned", who);
     const GateUpPlan plan = plan_gate_up(M, N, K, ws_bytes, lq_device_cu_count());
     if (plan.kernel == LQ_PLAN_STAGED_128) {
-        rc = lq_gemm_staged_pair_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, (float *)workspace, (int)M,
-                                        (int)N, (int)K, plan.rows, plan.splits, plan.per_split, (hipStream_t)stream, who);
-        if (rc) return rc;
+        rc = lq_gemm_staged_pair_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h, g_out, u_out,
+                                        (float *)workspace, (int)M, (int)N, (int)K, plan.rows, plan.splits, plan.per_split, (hipStream_t)stream, who);
+        if (rc || plan.splits < 2) return rc;
         const long long MN = (long long)M * N;
         hipLaunchKernelGGL(gate_up_reduce_kernel, dim3((unsigned)((MN / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                            (const float *)workspace, (unsigned short *)h, (unsigned short *)g_out, (unsigned short *)u_out, MN, plan.splits);
