@@ -8,13 +8,14 @@
 
 namespace {
 
-// The 8 elements from `base` on, for the clamp value c (uniform over the launch).
+// The 8 elements from `base` on, for the clamp value c (uniform over the launch; kOwnMax: x's maximum).
+template <bool kOwnMax>
 __device__ __forceinline__ void act_quant_piece(const unsigned short *__restrict__ x, signed char *__restrict__ x8, long long base,
                                                 long long n, float c) {
     if (base >= n) return;
     if (base + 8 <= n && (((uintptr_t)(x + base)) & 15) == 0 && (((uintptr_t)(x8 + base)) & 7) == 0) {
         const u32x4_t v = *reinterpret_cast<const u32x4_t *>(x + base);
-        *reinterpret_cast<u32x2_t *>(x8 + base) = act_quant8_any(v, c);
+        *reinterpret_cast<u32x2_t *>(x8 + base) = act_quant8_any<kOwnMax>(v, c);
     } else {
         for (long long i = base; i < n && i < base + 8; ++i) {
             float f = lq_bf16_bits_to_f32(x[i]);
@@ -29,7 +30,7 @@ __device__ __forceinline__ void act_quant_piece(const unsigned short *__restrict
 __global__ __launch_bounds__(256) void act_quant_kernel(const unsigned short *__restrict__ x,
                                                         const float *__restrict__ clampv, signed char *__restrict__ x8,
                                                         long long n) {
-    act_quant_piece(x, x8, ((long long)blockIdx.x * 256 + threadIdx.x) * 8, n, clampv[0]);
+    act_quant_piece<false>(x, x8, ((long long)blockIdx.x * 256 + threadIdx.x) * 8, n, clampv[0]);
 }
 
 // ---- the tensor's own maximum as clamp value ---------------------------------------------------
@@ -48,13 +49,14 @@ constexpr int kMaxPartials = LQ_ACT_WORK_FLOATS - 8;
 __global__ __launch_bounds__(256) void tensor_max_kernel(const unsigned short *__restrict__ x, long long n,
                                                          unsigned *__restrict__ partial) {
     __shared__ unsigned red[4];
-    unsigned k = 0u;  // below every key
+    MaxKeys keys;
     const long long n8 = n / 8;
     const u32x4_t *x16 = reinterpret_cast<const u32x4_t *>(x);
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
         const u32x4_t v = x16[i];
-        k = max_key8(v, k);
+        keys.add8(v);
     }
+    unsigned k = keys.key();
     if (blockIdx.x == 0 && (long long)threadIdx.x < n - n8 * 8) {
         const unsigned t = max_key(x[n8 * 8 + threadIdx.x]);
         k = k > t ? k : t;
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(256) void act_quant_dyn_kernel(const unsigned short
         work[1] = alpha;
     }
     for (long long m = gid; m < M; m += (long long)gridDim.x * 256) sx[m] = alpha;
-    act_quant_piece(x, x8, gid * 8, n, c);
+    act_quant_piece<true>(x, x8, gid * 8, n, c);
 }
 
 // ---- one scale per token row --------------------------------------------------------------------
@@ -103,8 +105,8 @@ __global__ __launch_bounds__(256) void act_quant_token_kernel(const unsigned sho
     u32x2_t *out = reinterpret_cast<u32x2_t *>(x8 + (long long)m * K);
     const int n16 = K / 8, T = (n16 + 63) / 64;
     u32x4_t v[PT];
-    unsigned amax = 0u;
-    auto take = [&](const u32x4_t &w) { amax = act_amax8(w, amax); };
+    act_u16x2_t most = {0, 0};
+    auto take = [&](const u32x4_t &w) { most = act_amax8(w, most); };
 #pragma unroll
     for (int t = 0; t < PT; ++t) {
         const int i = lane + 64 * t;
@@ -117,11 +119,12 @@ __global__ __launch_bounds__(256) void act_quant_token_kernel(const unsigned sho
         const int i = lane + 64 * t;
         if (i < n16) take(row[i]);
     }
-    amax = wave_max_u32(amax);
+    const unsigned amax = wave_max_u32(act_amax_of(most));
     const float am = __uint_as_float(amax << 16);
     const float inv = am == 0.0f ? 0.0f : 127.0f / am;
     if (lane == 0) sx[m] = am / 127.0f;
-    auto quant = [&](const u32x4_t &w) { return act_quant8_token(w, inv); };
+    const bool finite = act_finite_row(am, inv);
+    auto quant = [&](const u32x4_t &w) { return act_quant8_token(w, inv, finite); };
 #pragma unroll
     for (int t = 0; t < PT; ++t) {
         const int i = lane + 64 * t;

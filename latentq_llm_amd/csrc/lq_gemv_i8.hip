@@ -40,8 +40,10 @@ constexpr int kDeep = 4096;  // from this K on a wave has four units to request 
 
 // FM: groups of 16 tokens. UB: units a wave has in flight. PT: pieces of 8 activations a thread holds (kFused, one scale
 // for the tensor): they are requested at once and quantised from registers. Half of them in a loop that read them again
-// cost two more round trips to L2 each time: 12.2 us instead of 10.9 on 2048 x 8192 at 4 tokens, of which some 3 are the
-// vector work of quantising 64 elements per thread.
+// cost two more round trips to L2 each time: 12.2 us instead of 10.9 on 2048 x 8192 at 4 tokens. Every unit quantises all
+// activations, so their instructions count: maxima over pairs of elements and across lanes in registers, no look at each
+// element for NaNs (their maximum shows them) took 184 instructions for 8 elements to 95. us: 4 tokens, 2048 x 2048 4.53 ->
+// 3.96, 8192 x 2048 6.85 -> 5.94, 2048 x 8192 11.67 -> 9.70; 15 tokens, 1536 x 1536 6.86 -> 5.38, per token 7.79 -> 6.89.
 // Arguments: those of the first loads first, the leading 14 dwords are preloaded into registers (build.py): 4 tokens, 8192 x 2048
 // 6.91 -> 6.62 us.
 template <int FM, bool kFused, int UB, int PT = 1>
@@ -107,22 +109,23 @@ __global__ __launch_bounds__(kThreads) void gemv_i8_kernel(const void *x, const 
             // a wave per token row
             for (int m = wave; m < p.M; m += kWaves) {
                 const u32x4_t *row = xp + (long long)m * row16;
-                unsigned amax = 0u;
+                act_u16x2_t most = {0, 0};
 #pragma unroll 4
-                for (int i = lane; i < row16; i += 64) amax = act_amax8(row[i], amax);
-                amax = wave_max_u32(amax);
+                for (int i = lane; i < row16; i += 64) most = act_amax8(row[i], most);
+                const unsigned amax = wave_max_u32(act_amax_of(most));
                 const float am = __uint_as_float(amax << 16);
                 const float inv = am == 0.0f ? 0.0f : 127.0f / am;
+                const bool finite = act_finite_row(am, inv);
                 if (lane == 0) sx_lds[m] = am / 127.0f;
 #pragma unroll 4
-                for (int i = lane; i < row16; i += 64) put(m * row16 + i, act_quant8_token(row[i], inv));
+                for (int i = lane; i < row16; i += 64) put(m * row16 + i, act_quant8_token(row[i], inv, finite));
             }
         } else {
-            unsigned k = 0u;  // below every key
+            MaxKeys keys;
 #pragma unroll
             for (int t = 0; t < PT; ++t)
-                if (tid + t * kThreads < pieces) k = max_key8(xv[t], k);
-            k = wave_max_u32(k);
+                if (tid + t * kThreads < pieces) keys.add8(xv[t]);
+            unsigned k = wave_max_u32(keys.key());
             if (lane == 0) red_key[wave] = k;
             __syncthreads();
 #pragma unroll
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(kThreads) void gemv_i8_kernel(const void *x, const 
             if (tid < 16) sx_lds[tid] = c * (1.0f / 127.0f);
 #pragma unroll
             for (int t = 0; t < PT; ++t)
-                if (tid + t * kThreads < pieces) put(tid + t * kThreads, act_quant8_any(xv[t], c));
+                if (tid + t * kThreads < pieces) put(tid + t * kThreads, act_quant8_any<true>(xv[t], c));
         }
         __syncthreads();
     }
