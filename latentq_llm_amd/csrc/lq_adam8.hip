@@ -37,7 +37,9 @@
 // bank conflicts LDS is busy for a third of the launch). One block to a workgroup, so that a look-up is a byte shifted and a
 // read. A decoder layer's six weights (50 M elements): stochastic rounding 91.9 -> 85.3 us, int4 + residual 141.9 -> 134.7;
 // 64 M elements: int8 + residual 164.5 -> 155.7, bf16 151.8 -> 147.8. 57 vector instructions an element are left of 65 in
-// the first, and the vector ALUs are busy all the time.
+// the first, and the vector ALUs are busy all the time. The extrema across lanes in registers instead of shuffles through LDS,
+// and no minimum of the second moments with an eps that hides their subnormals, 50 M elements: stochastic rounding 90 -> 84 us,
+// int4 + residual 133 -> 125.7, int8 + residual 134 -> 127, bf16 128 -> 124.4.
 #include "lq_latent_math.h"
 #include "lq_requant_math.h"
 
@@ -111,6 +113,25 @@ __device__ __forceinline__ float min3_abs(float a, float b, float c) {  // of |a
     float r;
     asm("v_min3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
+}
+
+// Minima and maxima over the wave's 64 lanes (or each row of 16): across lanes within the vector registers, where shuffles
+// through LDS took six round trips and as many address computations again. A row's results are on all of its lanes, the
+// wave's on lane 63.
+// One block of assembly, since the waits that a register needs between its write and a read across lanes are not put inside
+// or before it: three other instructions lie between, and two wait states in front.
+#define LQ_ADAM8_ACROSS(ctrl)                                       \
+    "v_min_f32_dpp %0, %0, %0 " ctrl " row_mask:0xf bank_mask:0xf\n\t"  \
+    "v_max_f32_dpp %1, %1, %1 " ctrl " row_mask:0xf bank_mask:0xf\n\t"  \
+    "v_min_f32_dpp %2, %2, %2 " ctrl " row_mask:0xf bank_mask:0xf\n\t"  \
+    "v_max_f32_dpp %3, %3, %3 " ctrl " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void row_extrema(float &lo1, float &hi1, float &lo2, float &hi2) {
+    asm volatile("s_nop 1\n\t" LQ_ADAM8_ACROSS("row_ror:8") LQ_ADAM8_ACROSS("row_ror:4") LQ_ADAM8_ACROSS("row_ror:2") LQ_ADAM8_ACROSS("row_ror:1")
+                 : "+v"(lo1), "+v"(hi1), "+v"(lo2), "+v"(hi2));
+}
+__device__ __forceinline__ void wave_extrema(float &lo1, float &hi1, float &lo2, float &hi2) {
+    row_extrema(lo1, hi1, lo2, hi2);
+    asm volatile("s_nop 1\n\t" LQ_ADAM8_ACROSS("row_bcast:15") LQ_ADAM8_ACROSS("row_bcast:31") : "+v"(lo1), "+v"(hi1), "+v"(lo2), "+v"(hi2));
 }
 
 // x[8] -> uint8 codes with the block's (scale, max); returns them packed, 8 bytes.
@@ -267,16 +288,22 @@ __global__ __launch_bounds__(BS == 2048 ? 128 : 256) void adam8_kernel(Adam8Batc
             if constexpr (MODE == ADAM_PARAM || MODE == ADAM_W4 || MODE == ADAM_W8)
                 ratio[k] = fmaf(fmaf(-ratio[k], d[c][k], m[c][k]), r, ratio[k]);
         }
-        float clo1 = m[c][0], chi1 = m[c][0], clo2 = d[c][0], chi2 = d[c][0], mmin = fabsf(m[c][0]), vmin = v[0];
+        float clo1 = m[c][0], chi1 = m[c][0], clo2 = d[c][0], chi2 = d[c][0], mmin = fabsf(m[c][0]), vmin = 1.0f;
         if (c) { clo1 = lo1; chi1 = hi1; clo2 = lo2; chi2 = hi2; }
 #pragma unroll
         for (int k = 0; k < 8; k += 2) {
             clo1 = min3(m[c][k], m[c][k + 1], clo1); chi1 = max3(m[c][k], m[c][k + 1], chi1);
             clo2 = min3(d[c][k], d[c][k + 1], clo2); chi2 = max3(d[c][k], d[c][k + 1], chi2);
             mmin = min3_abs(m[c][k], m[c][k + 1], mmin);
-            vmin = min3(v[k], v[k + 1], vmin);
         }
-        // The short sequences hold for v >= 2^-100 and 2^-80 <= |m| <= 2^80, 2^-40 <= d <= 2^40 (no subnormal, no
+        // an eps of 2^-38 and more swallows every root of a v below 2^-126, the exact one and what the hardware makes of it (at
+        // most 2^-63, a quarter of eps's last place), and normal v have the right root
+        if (!(a.eps >= 0x1p-38f)) {
+            vmin = v[0];
+#pragma unroll
+            for (int k = 0; k < 8; k += 2) vmin = min3(v[k], v[k + 1], vmin);
+        }
+        // The short sequences hold for v >= 2^-100 (or eps >= 2^-38) and 2^-80 <= |m| <= 2^80, 2^-40 <= d <= 2^40 (no subnormal, no
         // underflowing residual, no overflow; NaN and infinity pass through them as through the plain ones). Chunks
         // with anything else, zeros among them, take the plain operations.
         const bool plain = !(vmin >= 0x1p-100f && mmin >= 0x1p-80f && fmaxf(fabsf(clo1), fabsf(chi1)) <= 0x1p80f &&
@@ -375,20 +402,16 @@ __global__ __launch_bounds__(BS == 2048 ? 128 : 256) void adam8_kernel(Adam8Batc
 
     // the moments back to uint8 with the block's new (scale, max): minima and maxima over the block's threads (a
     // 16-lane row of the wave, or two waves, through LDS)
-#pragma unroll
-    for (int off = 1; off < (TPB < 64 ? TPB : 64); off <<= 1) {
-        lo1 = min2(lo1, __shfl_xor(lo1, off, 64));
-        hi1 = max2(hi1, __shfl_xor(hi1, off, 64));
-        lo2 = min2(lo2, __shfl_xor(lo2, off, 64));
-        hi2 = max2(hi2, __shfl_xor(hi2, off, 64));
-    }
-    if constexpr (TPB == 128) {
-        const int wave = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) *reinterpret_cast<f32x4_t *>(red[wave]) = f32x4_t{lo1, hi1, lo2, hi2};
+    static_assert(TPB == 16 || TPB == 128, "a block is a row of lanes or two waves");
+    if constexpr (TPB == 16) {
+        row_extrema(lo1, hi1, lo2, hi2);
+    } else {
+        wave_extrema(lo1, hi1, lo2, hi2);
+        if ((threadIdx.x & 63) == 63) *reinterpret_cast<f32x4_t *>(red[threadIdx.x >> 6]) = f32x4_t{lo1, hi1, lo2, hi2};
         __syncthreads();
-        const f32x4_t other = *reinterpret_cast<const f32x4_t *>(red[wave ^ 1]);
-        lo1 = min2(lo1, other[0]); hi1 = max2(hi1, other[1]);
-        lo2 = min2(lo2, other[2]); hi2 = max2(hi2, other[3]);
+        const f32x4_t w0 = *reinterpret_cast<const f32x4_t *>(red[0]), w1 = *reinterpret_cast<const f32x4_t *>(red[1]);
+        lo1 = min2(w0[0], w1[0]); hi1 = max2(w0[1], w1[1]);
+        lo2 = min2(w0[2], w1[2]); hi2 = max2(w0[3], w1[3]);
     }
     const float inv255 = 1.0f / 255.0f;  // the tensor library divides by a scalar as a multiplication by its reciprocal
     const float ns1 = (hi1 - lo1) * inv255 + 1e-10f;
