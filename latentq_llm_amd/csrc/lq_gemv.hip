@@ -56,16 +56,25 @@ constexpr int kXRow = 1024 + 16;  // LDS bytes per staged token row: 4 groups x 
 // alone, and a wave works through up to SPW partial sums one after the other: the order of the fp32 sums, and so the bits of
 // the result, do not depend on how many waves the launcher finds best for the grid.
 // (SPW = 2 in at most 128 registers, four waves to a SIMD; more in 168)
+// LOADS: how a wave's batches are loaded.
+//   0  at the top of the loop over them, the token rows by the compiler's LDS-direct load, after which it waits for
+//      all loads before any read of LDS
+//   1  the same, the token rows by assembly
+//   2  the next batch's codes before this one's MFMAs (24 to 32 registers more)
+//   3  no loop: one batch a wave. Its loads come before all that is not needed for them; a loop has a hundred
+//      instructions in front of it, a twentieth of a small launch
 // The arguments that the first loads need come first: the leading 14 dwords are preloaded into registers (build.py). Weights from
 // HBM, 1 token: 4096 x 4096 5.15 -> 4.77 us, 4096 x 11008 8.01 -> 7.76, 2048 x 2048 3.48 -> 3.31.
-template <int WAVES, int MP, int NT, bool QS, bool GU = false, int SPW = 1>
-__global__ __launch_bounds__(64 * WAVES, SPW == 2 ? 4 : SPW > 2 ? 3 : 1) void gemv_kernel(
+template <int WAVES, int MP, int NT, bool QS, bool GU = false, int SPW = 1, int LOADS = 0>
+__global__ __launch_bounds__(64 * WAVES, LOADS >= 2 ? 1 : SPW == 2 ? 4 : SPW > 2 ? 3 : 1) void gemv_kernel(
     const unsigned short *__restrict__ x, const unsigned char *__restrict__ codes, int M, int N, int K, int slots,
     const unsigned short *__restrict__ scales, const unsigned short *__restrict__ zeros, const unsigned short *__restrict__ bias,
     unsigned short *__restrict__ y, const unsigned char *__restrict__ codes2, const unsigned short *__restrict__ scales2,
     const unsigned short *__restrict__ zeros2) {
+    constexpr bool PRE = LOADS == 2, ONE = LOADS == 3;
     static_assert(!GU || (NT == 2 && !QS), "gate / up mode: two tiles, scales and zeros straight from memory");
     constexpr int RT = GU ? 1 : NT;  // 16-row tiles of output rows per workgroup
+    static_assert(!ONE || SPW == 1, "one batch a wave");
     static_assert(GU || SPW == 1, "several partial sums per wave: gate / up mode only");
     constexpr int kWaveLds = MP * kXRow > SPW * NT * 1024 ? MP * kXRow : SPW * NT * 1024;
     __shared__ __attribute__((aligned(16))) unsigned char xs_all[WAVES][kWaveLds];
@@ -143,132 +152,203 @@ __global__ __launch_bounds__(64 * WAVES, SPW == 2 ? 4 : SPW > 2 ? 3 : 1) void ge
     for (int k = 0; k < SPW; ++k)
 #pragma unroll
         for (int j = 0; j < NT; ++j) done[k][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < SPW; ++i) {
-        const int s = wave + i * WAVES;
-        if (SPW > 1 && s >= n_slots) break;
-        for (int g0 = s * kUnroll; g0 < G; g0 += n_slots * kUnroll) {
-            const bool full = g0 + kUnroll <= G;  // a short tail batch re-reads the last group with zero scale
-            // ---- activations: one LDS-direct load per token row (1 KB = this batch's 512 k), coalesced.
-            //      In a tail batch the lanes past the end of the row re-read its first bytes (dead groups).
-            {
-                const long long xoff = (long long)g0 * (LQ_GROUP * 2) + lane * 16;
-                const long long lim = (long long)K * 2;
-                const long long off = xoff < lim ? xoff : 0;
+    auto keep = [&](int i) {  // partial sum i is complete
 #pragma unroll
-                for (int m = 0; m < MP; ++m)
-                    if (m < M)
-                        __builtin_amdgcn_global_load_lds((gbl_void *)((const unsigned char *)x + (long long)m * lim + off),
-                                                         (lds_void *)xs(wave, m), 16, 0, 0);
-            }
-            // ---- codes, scales, zeros
-            u32x4_t wv[NT][kUnroll];
-            float sc[NT][kUnroll], zz[NT][kUnroll];
+        for (int k = 0; k < SPW; ++k)
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
-                    const int g = g0 + u < G ? g0 + u : G - 1;
-                    const unsigned char *wt = (GU && j == 1) ? wrow2 : wrow + j * tile_stride;
-                    wv[j][u] = *reinterpret_cast<const u32x4_t *>(wt + g * 64);
-                }
-            if constexpr (QS) {
-                if (first) {
-                    publish_q();
-                    first = false;
-                }
+                for (int r = 0; r < 4; ++r) done[k][j][r] = i == k ? acc[j][r] : done[k][j][r];
 #pragma unroll
-                for (int j = 0; j < NT; ++j) {
-                    const unsigned short *ls = reinterpret_cast<const unsigned short *>(sq + (j * 16 + n) * q_pitch);
-                    const unsigned short *lz = reinterpret_cast<const unsigned short *>(sq + q_lds + (j * 16 + n) * q_pitch);
+        for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    };
+    // ---- loads of the batch that begins with group g0
+    // activations: one LDS-direct load per token row (1 KB = this batch's 512 k), coalesced. In a tail batch the lanes past the
+    // end of the row re-read its first bytes (dead groups). LOADS > 0: written as assembly, with which the compiler does not
+    // wait for the rows (or the next batch's codes) before each of its own reads of LDS.
+    auto load_x = [&](int g0) {
+        const long long xoff = (long long)g0 * (LQ_GROUP * 2) + lane * 16;
+        const long long lim = (long long)K * 2;
+        const long long off = xoff < lim ? xoff : 0;
 #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u) {
-                        const bool live = g0 + u < G;
-                        const int g = live ? g0 + u : G - 1;
-                        sc[j][u] = live ? lq_bf16_bits_to_f32(ls[g]) : 0.0f;
-                        zz[j][u] = 128.0f + lq_bf16_bits_to_f32(lz[g]);
-                    }
-                }
-            } else
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const unsigned short *sr = GU ? (j == 0 ? srow : scales2 + (long long)row * G) : srow + (long long)j * 16 * G;
-                const unsigned short *zr = GU ? (j == 0 ? zrow : zeros2 + (long long)row * G) : zrow + (long long)j * 16 * G;
-                if (full) {
-                    u32x2_t sraw = {0u, 0u}, zraw = {0u, 0u};
-                    if (kq == 0) {
-                        sraw = *reinterpret_cast<const u32x2_t *>(sr + g0);
-                        zraw = *reinterpret_cast<const u32x2_t *>(zr + g0);
-                    }
-                    unsigned s01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sraw[0]);
-                    unsigned s23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sraw[1]);
-                    unsigned z01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zraw[0]);
-                    unsigned z23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zraw[1]);
-                    sc[j][0] = lq_bf16_lo(s01); sc[j][1] = lq_bf16_hi(s01); sc[j][2] = lq_bf16_lo(s23); sc[j][3] = lq_bf16_hi(s23);
-                    zz[j][0] = 128.0f + lq_bf16_lo(z01); zz[j][1] = 128.0f + lq_bf16_hi(z01);
-                    zz[j][2] = 128.0f + lq_bf16_lo(z23); zz[j][3] = 128.0f + lq_bf16_hi(z23);
+        for (int m = 0; m < MP; ++m)
+            if (m < M) {
+                const unsigned char *src = (const unsigned char *)x + (long long)m * lim;
+                if constexpr (LOADS > 0) {
+                    const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)xs(wave, m));
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"((unsigned)off), "s"(src) : "memory");
                 } else {
-#pragma unroll
-                    for (int u = 0; u < kUnroll; ++u) {
-                        const bool live = g0 + u < G;
-                        const int g = live ? g0 + u : G - 1;
-                        sc[j][u] = live ? lq_bf16_bits_to_f32(sr[g]) : 0.0f;
-                        zz[j][u] = 128.0f + lq_bf16_bits_to_f32(zr[g]);
-                    }
+                    __builtin_amdgcn_global_load_lds((gbl_void *)(src + off), (lds_void *)xs(wave, m), 16, 0, 0);
                 }
             }
-            // ---- codes to the MFMA lane layout
+    };
+    // codes, and the scales and zeros of a whole batch (loaded by the 16 lanes kq = 0)
+    u32x4_t wn[NT][kUnroll];
+    u32x2_t sn[NT], zn[NT];
+    constexpr int kCodeLoads = NT * kUnroll + (QS ? 0 : 2 * NT);
+    auto scale_row = [&](int j) { return GU ? (j == 0 ? srow : scales2 + (long long)row * G) : srow + (long long)j * 16 * G; };
+    auto zero_row = [&](int j) { return GU ? (j == 0 ? zrow : zeros2 + (long long)row * G) : zrow + (long long)j * 16 * G; };
+    auto load_scales = [&](int g0, int j) {
+        sn[j] = zn[j] = u32x2_t{0u, 0u};
+        if (kq == 0) {
+            sn[j] = *reinterpret_cast<const u32x2_t *>(scale_row(j) + g0);
+            zn[j] = *reinterpret_cast<const u32x2_t *>(zero_row(j) + g0);
+        }
+    };
+    auto load_codes = [&](int g0) {
 #pragma unroll
-            for (int j = 0; j < NT; ++j)
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u)
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                        wv[j][u][t] = (unsigned)__builtin_amdgcn_ds_bpermute(bperm_src, (int)wv[j][u][t]);
-            // ---- MFMAs
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the staged rows have landed in LDS
-            // One group at a time: a single pair of MFMA accumulators (plus one per extra tile) is live,
-            // which keeps the kernel at <= 80 registers (6 waves per SIMD, three 8-wave workgroups per
-            // CU); the unpacking between two MFMAs on the same accumulator covers their latency.
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
-                f32x4_t P[NT], S = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int j = 0; j < NT; ++j) P[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    unsigned a[4];
-                    const u32x4_t xv = *reinterpret_cast<const u32x4_t *>(xfrag + u * 256 + t * 16);
-                    permute_x(xv, a);
-                    const u32x4_t av = {a[0], a[1], a[2], a[3]};
-                    S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
-                                                                __builtin_bit_cast(bf16x8_t, ones), S, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) {
-                        unsigned b[4];
-                        unpack_word_128q(wv[j][u][t], b);
-                        const u32x4_t bv = {b[0], b[1], b[2], b[3]};
-                        P[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
-                                                                       __builtin_bit_cast(bf16x8_t, bv), P[j], 0, 0, 0);
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(sc[j][u], fmaf(-zz[j][u], S[r], P[j][r]), acc[j][r]);
-                __builtin_amdgcn_sched_barrier(0);  // keeps the next group's unpacking from being hoisted (registers)
+                const int g = g0 + u < G ? g0 + u : G - 1;
+                const unsigned char *wt = (GU && j == 1) ? wrow2 : wrow + j * tile_stride;
+                wn[j][u] = *reinterpret_cast<const u32x4_t *>(wt + g * 64);
             }
-            // the next batch overwrites the staged rows: all fragment reads above must have returned
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        }
-        if constexpr (SPW > 1) {
+        if constexpr ((PRE || ONE) && !QS)
+            if (g0 + kUnroll <= G) {
 #pragma unroll
-            for (int k = 0; k < SPW; ++k)
-                if (i == k) {
+                for (int j = 0; j < NT; ++j) load_scales(g0, j);
+            }
+    };
+    // the batch at group g0, whose loads have been issued; `then` issues what is to travel under its MFMAs and waits for the
+    // staged rows
+    auto multiply = [&](int g0, auto then) {
+        const bool full = g0 + kUnroll <= G;  // a short tail batch re-reads the last group with zero scale
+        u32x4_t wv[NT][kUnroll];
+        float sc[NT][kUnroll], zz[NT][kUnroll];
+        if constexpr (QS) {
+            if (first) {
+                publish_q();
+                first = false;
+            }
 #pragma unroll
-                    for (int j = 0; j < NT; ++j) done[k][j] = acc[j];
+            for (int j = 0; j < NT; ++j) {
+                const unsigned short *ls = reinterpret_cast<const unsigned short *>(sq + (j * 16 + n) * q_pitch);
+                const unsigned short *lz = reinterpret_cast<const unsigned short *>(sq + q_lds + (j * 16 + n) * q_pitch);
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u) {
+                    const bool live = g0 + u < G;
+                    const int g = live ? g0 + u : G - 1;
+                    sc[j][u] = live ? lq_bf16_bits_to_f32(ls[g]) : 0.0f;
+                    zz[j][u] = 128.0f + lq_bf16_bits_to_f32(lz[g]);
                 }
+            }
+        } else if (full) {
+            if constexpr (LOADS == 1) {
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < NT; ++j) load_scales(g0, j);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                if constexpr (LOADS == 0) load_scales(g0, j);
+                const unsigned s01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sn[j][0]);
+                const unsigned s23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)sn[j][1]);
+                const unsigned z01 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zn[j][0]);
+                const unsigned z23 = (unsigned)__builtin_amdgcn_ds_bpermute(bcast_src, (int)zn[j][1]);
+                sc[j][0] = lq_bf16_lo(s01); sc[j][1] = lq_bf16_hi(s01); sc[j][2] = lq_bf16_lo(s23); sc[j][3] = lq_bf16_hi(s23);
+                zz[j][0] = 128.0f + lq_bf16_lo(z01); zz[j][1] = 128.0f + lq_bf16_hi(z01);
+                zz[j][2] = 128.0f + lq_bf16_lo(z23); zz[j][3] = 128.0f + lq_bf16_hi(z23);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u) {
+                    const bool live = g0 + u < G;
+                    const int g = live ? g0 + u : G - 1;
+                    sc[j][u] = live ? lq_bf16_bits_to_f32(scale_row(j)[g]) : 0.0f;
+                    zz[j][u] = 128.0f + lq_bf16_bits_to_f32(zero_row(j)[g]);
+                }
+            }
+        }
+        // ---- codes to the MFMA lane layout
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    wv[j][u][t] = (unsigned)__builtin_amdgcn_ds_bpermute(bperm_src, (int)wn[j][u][t]);
+        then();
+        // ---- MFMAs
+        // One group at a time: a single pair of MFMA accumulators (plus one per extra tile) is live; the unpacking between
+        // two MFMAs on the same accumulator covers their latency.
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            f32x4_t P[NT], S = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NT; ++j) P[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                unsigned a[4];
+                const u32x4_t xv = *reinterpret_cast<const u32x4_t *>(xfrag + u * 256 + t * 16);
+                permute_x(xv, a);
+                const u32x4_t av = {a[0], a[1], a[2], a[3]};
+                S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
+                                                            __builtin_bit_cast(bf16x8_t, ones), S, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    unsigned b[4];
+                    unpack_word_128q(wv[j][u][t], b);
+                    const u32x4_t bv = {b[0], b[1], b[2], b[3]};
+                    P[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
+                                                                   __builtin_bit_cast(bf16x8_t, bv), P[j], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(sc[j][u], fmaf(-zz[j][u], S[r], P[j][r]), acc[j][r]);
+            __builtin_amdgcn_sched_barrier(0);  // keeps the next group's unpacking from being hoisted (registers)
+        }
+        // the next batch overwrites the staged rows: all fragment reads above must have returned
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    if constexpr (ONE) {
+        const int g0 = wave * kUnroll;
+        if (g0 < G) {
+            load_x(g0);
+            load_codes(g0);
+            __builtin_amdgcn_sched_barrier(0);  // the loads before all that is not needed for them
+            multiply(g0, []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); });
+        }
+    } else if constexpr (PRE) {
+        int i = 0, g0 = wave * kUnroll;
+        bool more = g0 < G && (SPW == 1 || wave < n_slots);
+        if (more) {
+            load_x(g0);
+            load_codes(g0);
+        }
+        while (more) {
+            const int i_now = i;
+            multiply(g0, [&]() {
+                g0 += n_slots * kUnroll;
+                if (SPW > 1 && g0 >= G) {  // the wave's next partial sum
+                    ++i;
+                    const int s = wave + i * WAVES;
+                    g0 = i < SPW && s < n_slots ? s * kUnroll : G;
+                }
+                more = g0 < G;
+                if (more) {
+                    load_codes(g0);
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kCodeLoads) : "memory");  // the staged rows are older
+                } else {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                }
+            });
+            if (more) load_x(g0);
+            if (SPW > 1 && (!more || i != i_now)) keep(i_now);
+        }
+    } else {
+        for (int i = 0; i < SPW; ++i) {
+            const int s = wave + i * WAVES;
+            if (SPW > 1 && s >= n_slots) break;
+            for (int g0 = s * kUnroll; g0 < G; g0 += n_slots * kUnroll) {
+                load_x(g0);
+                load_codes(g0);
+                multiply(g0, []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); });
+            }
+            if constexpr (SPW > 1) keep(i);
         }
     }
 
@@ -330,12 +410,30 @@ struct GemvGuArgs {
     hipStream_t st;
 };
 
-template <int W, int MP, int SPW>
-void launch_gu_spw(const GemvGuArgs &a) {
-    hipLaunchKernelGGL((gemv_kernel<W, MP, 2, false, true, SPW>), dim3(a.N / 16), dim3(64 * W), 0, a.st, (const unsigned short *)a.x,
+template <int W, int MP, int SPW, int LOADS>
+void launch_gu_loads(const GemvGuArgs &a) {
+    hipLaunchKernelGGL((gemv_kernel<W, MP, 2, false, true, SPW, LOADS>), dim3(a.N / 16), dim3(64 * W), 0, a.st, (const unsigned short *)a.x,
                        (const unsigned char *)a.codes, a.M, a.N, a.K, a.slots, (const unsigned short *)a.scales, (const unsigned short *)a.zeros,
                        (const unsigned short *)nullptr, (unsigned short *)a.y, (const unsigned char *)a.codes2,
                        (const unsigned short *)a.scales2, (const unsigned short *)a.zeros2);
+}
+
+// How the batches are loaded (LOADS): with one workgroup to a unit registers are free for the next batch's codes; with two they
+// are not, and with three and more than 4 rows the rows' wait for all loads does no harm (8 tokens, 11008 x 4096: 15.9 us
+// against 17.1 by assembly). us, all by the compiler's loads (what every size took before) -> this rule:
+//   4096 x 2048 (c = 1)  2 tokens 5.92 -> 5.47, 12: 6.62 -> 5.97;  4096 x 1792, 8: 6.19 -> 5.46;  3072 x 1024, 16: 5.33 -> 5.01
+//   6144 x 3072 (c = 2)  8: 10.6 -> 9.94, 12: 12.8 -> 11.4, 16: 12.6 -> 11.9;  8192 x 4096, 12: 15.4 -> 13.3, 16: 15.6 -> 14.2
+//   8192 x 2560, 1: 9.2 -> 8.1;  11008 x 4096 (c = 3), 1: 14.2 -> 13.1, 4: 15.1 -> 14.5;  20480 x 8192, 1: 50.1 -> 46.3
+template <int W, int MP, int SPW>
+void launch_gu_spw(const GemvGuArgs &a) {
+    if constexpr (MP == 4) {
+        launch_gu_loads<W, MP, SPW, 1>(a);
+    } else {
+        const int c = (a.N / 16 + lq_device_cu_count() - 1) / lq_device_cu_count();
+        if (c == 1) launch_gu_loads<W, MP, SPW, 2>(a);
+        else if (c == 2) launch_gu_loads<W, MP, SPW, 1>(a);
+        else launch_gu_loads<W, MP, SPW, 0>(a);
+    }
 }
 
 // Partial sums of a gate / up pass, at most: the waves of the workgroups that stage 4 or 16 rows with one batch each
@@ -414,8 +512,24 @@ void launch_one(const GemvArgs &a) {
                            a.M, a.N, a.K, W, (const unsigned short *)a.scales, (const unsigned short *)a.zeros, (const unsigned short *)a.bias,
                            (unsigned short *)a.y, (const unsigned char *)nullptr, (const unsigned short *)nullptr, (const unsigned short *)nullptr);
     };
-    if (qs) launch(gemv_kernel<W, MP, NT, true>, 2 * q_bytes + 2 * 16 * NT * 16);
-    else launch(gemv_kernel<W, MP, NT, false>, 0);
+    // How the batches are loaded (LOADS). us, all by the compiler's loads in a loop (what every size took before) -> this rule:
+    //   one batch a wave        12 tokens, 4096 x 4096 5.95 -> 5.72; 3 tokens, 1280 x 3584 3.94 -> 3.83; 1 token, 32000 x 4096 17.7 -> 17.1
+    //   several, one workgroup  12 tokens, 4096 x 11008 12.7 -> 12.0; 16: 3328 x 9088 11.6 -> 10.5, 2560 x 7680 9.5 -> 8.5,
+    //   to a unit               8192 x 4096 10.9 -> 8.8; 10: 2304 x 6144 6.65 -> 6.15; 8: 2048 x 5504 5.9 -> 5.7
+    //   16 waves (4096 x 11008, up to 8 tokens) have no registers for a second batch, 7.7 -> 8.4 with it at 1 token
+    //   two row tiles           12 tokens, 11008 x 4096 12.3 -> 11.5
+    const size_t qs_lds = 2 * q_bytes + 2 * 16 * NT * 16;
+    const bool pre = W <= 8 && batches > W && a.N / (16 * NT) <= lq_device_cu_count();
+    if (batches <= W) {
+        if (qs) launch(gemv_kernel<W, MP, NT, true, false, 1, 3>, qs_lds);
+        else launch(gemv_kernel<W, MP, NT, false, false, 1, 3>, 0);
+    } else if (pre) {
+        if (qs) launch(gemv_kernel<W, MP, NT, true, false, 1, 2>, qs_lds);
+        else launch(gemv_kernel<W, MP, NT, false, false, 1, 2>, 0);
+    } else {
+        if (qs) launch(gemv_kernel<W, MP, NT, true, false, 1, NT == 2 ? 1 : 0>, qs_lds);
+        else launch(gemv_kernel<W, MP, NT, false, false, 1, NT == 2 ? 1 : 0>, 0);
+    }
 }
 
 // Waves per workgroup: as many as there are batches, up to the cap, in powers of two. More waves
