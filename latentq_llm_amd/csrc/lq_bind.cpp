@@ -13,6 +13,8 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/forward_grad.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/latentq.h"
 
@@ -129,6 +131,14 @@ bool bias_of(PyObject *o, int64_t N, const void **p) {
 #define LQ_ARGS(n) \
     if (nargs != (n)) { PyErr_SetString(PyExc_TypeError, "wrong number of arguments"); return nullptr; }
 
+// Whether something looks at calls that autograd itself does not: a trace being recorded, an open forward-mode level, an active
+// function transform
+bool watched() {
+    const c10::DispatchKeySet included = c10::impl::tls_local_dispatch_key_set().included_;
+    return torch::jit::tracer::isTracing() || torch::autograd::ForwardADLevel::try_get_by_idx(0) ||
+           included.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || included.has(c10::DispatchKey::FuncTorchDynamicLayerBackMode);
+}
+
 // x, codes, scales, zeros, N, K, bias, workspace -> y
 PyObject *linear4(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     LQ_ARGS(8)
@@ -146,6 +156,17 @@ PyObject *linear4(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     LQ_CALL(lq_a16w4_fwd_ws, x->data_ptr(), w.codes->data_ptr(), w.scales->data_ptr(), w.zeros->data_ptr(), bias, y.data_ptr(), M, N,
             K, LQ_GROUP, ws, ws_bytes, on.stream);
     return wrap(std::move(y));
+}
+
+// x, codes, scales, zeros, N, K, bias -> y, for a layer in inference: the whole call where nothing watches and the tokens
+// are few enough to need no workspace
+PyObject *linear4_eval(PyObject *self, PyObject *const *a, Py_ssize_t nargs) {
+    LQ_ARGS(7)
+    const int64_t K = integer(a[5]);
+    const at::Tensor *x = bf16(a[0]);
+    if (!x || K <= 0 || x->numel() > 16 * K || watched()) return none();
+    PyObject *all[8] = {a[0], a[1], a[2], a[3], a[4], a[5], a[6], Py_None};
+    return linear4(self, all, 8);
 }
 
 // dy, codes, scales, zeros, N, K, workspace -> dx
@@ -273,6 +294,11 @@ PyObject *infer8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     LQ_CALL(lq_a8w8_fwd_qs, x8.data_ptr(), w->data_ptr(), (const float *)sx.data_ptr(), qs->data_ptr(), bias, y.data_ptr(), nullptr, M,
             N, K, on.stream);
     return wrap(std::move(y));
+}
+
+// The same for a layer in inference: None where something watches
+PyObject *infer8_eval(PyObject *self, PyObject *const *a, Py_ssize_t nargs) {
+    return watched() ? none() : infer8(self, a, nargs);
 }
 
 // dy, w8, qscales, workspace -> dx
@@ -601,8 +627,8 @@ PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n) {
 }
 
 PyMethodDef methods[] = {
-    LQ_METHOD(linear4), LQ_METHOD(dx4), LQ_METHOD(gate_up), LQ_METHOD(dx_silu), LQ_METHOD(dx_pair), LQ_METHOD(linear8), LQ_METHOD(infer8),
-    LQ_METHOD(dx8), LQ_METHOD(quant8), LQ_METHOD(quant8_token), LQ_METHOD(dequant8), LQ_METHOD(weight_grad),
+    LQ_METHOD(linear4), LQ_METHOD(linear4_eval), LQ_METHOD(dx4), LQ_METHOD(gate_up), LQ_METHOD(dx_silu), LQ_METHOD(dx_pair), LQ_METHOD(linear8), LQ_METHOD(infer8),
+    LQ_METHOD(infer8_eval), LQ_METHOD(dx8), LQ_METHOD(quant8), LQ_METHOD(quant8_token), LQ_METHOD(dequant8), LQ_METHOD(weight_grad),
     LQ_METHOD(weight_grad_acc), LQ_METHOD(weight_grad_acc8), LQ_METHOD(gradq8), LQ_METHOD(adam8_param), LQ_METHOD(adam8_sr),
     LQ_METHOD(adam8_queue), LQ_METHOD(adam8_run), LQ_METHOD(adam8_w4), LQ_METHOD(adam8_w8), LQ_METHOD(current_stream), LQ_METHOD(set_error), {nullptr, nullptr, 0, nullptr}};
 

@@ -93,6 +93,10 @@ class QuantLlamaMLP(nn.Module):
         carries no autograd history (forward() takes the training path where one is needed)."""
         if self._training(x):
             raise RuntimeError("fused_gate_up has no backward: call the module (forward) when training")
+        if x.numel() <= 16 * self.infeatures:  # decoding: no workspace, any number of dimensions
+            h = (ops._native or ops._fast()).gate_up(x, *_w4(self.gate_proj), *_w4(self.up_proj), self.intermediate_size, self.infeatures, False, None)
+            if h is not None:
+                return h
         out_shape = x.shape[:-1] + (self.intermediate_size,)
         x2 = x.reshape(-1, x.shape[-1])
         M, K = x2.shape

@@ -620,8 +620,8 @@ class _QLinearBase(nn.Module):
             return self.bias
 
     def _infer(self, x):
-        """The layer's result where nothing is differentiated and every operand is in the form the kernels take; None
-        otherwise. The same kernels as the autograd Functions run, without the Function around them: in decoding that
+        """The layer's result where nothing watches (see _unwatched) and every operand is in the form the kernels take; None
+        otherwise. Called with autograd switched off. The same kernels as the autograd Functions run, without the Function around them: in decoding that
         costs the host as much as the kernel takes."""
         return None
 
@@ -631,7 +631,7 @@ class _QLinearBase(nn.Module):
         return self._apply_fn(self._fn_train, x, self if isinstance(self.hook_handle, _HookHandle) and self.hook_handle.active else None)
 
     def forward_eval(self, x):
-        if not torch.is_grad_enabled() and _unwatched():
+        if not torch.is_grad_enabled():
             y = self._infer(x)
             if y is not None:
                 return y
@@ -664,9 +664,14 @@ class QLinearA16W4(_QLinearBase):
 
     def _infer(self, x):
         w, bias = self.weight, self._bias()
-        y = ops.linear4(x, w.data, *w.qparam, bias)
+        scales, zeros, shape = w.qparam
+        # all of a decoding call in one: its host time shows where the kernels take 4 us each
+        y = (ops._native or ops._fast()).linear4_eval(x, w.data, scales, zeros, shape[0], shape[1], bias)
+        if y is not None or not _unwatched():
+            return y
+        y = ops.linear4(x, w.data, scales, zeros, shape, bias)
         if y is None and bias is not None and bias.dtype != torch.bfloat16:  # as constructed
-            y = ops.linear4(x, w.data, *w.qparam, bias.detach().to(torch.bfloat16))
+            y = ops.linear4(x, w.data, scales, zeros, shape, bias.detach().to(torch.bfloat16))
         return y
 
     def to(self, device: Optional[Union[int, torch.device]]):
@@ -706,8 +711,8 @@ class QLinearA8W8(_QLinearBase):
             qscales = self._buffers["qscales"]
         except KeyError:
             qscales = self.qscales
-        y = ops.infer8(x, self.weight.data, qscales, bias, per_token)
-        if y is None and bias is not None and bias.dtype != torch.bfloat16:  # as constructed
+        y = (ops._native or ops._fast()).infer8_eval(x, self.weight.data, qscales, bias, per_token)
+        if y is None and bias is not None and bias.dtype != torch.bfloat16 and _unwatched():  # as constructed
             y = ops.infer8(x, self.weight.data, qscales, bias.detach().to(torch.bfloat16), per_token)
         return y
 
