@@ -17,6 +17,8 @@
 //     4096 x 1024    9.9 -> 6.0      9.7 -> 6.2      8.0 -> 6.0      8.0 -> 6.1
 //     2560 x 8192    12.1 -> 9.7     12.9 -> 10.8    14.3 -> 13.2    15.0 / 15.6
 //     4096 x 11008   15.8 -> 14.9    15.7 / 17.2     17.5 / 21.7     18.2 / 25.6   (the last three stay with the staged kernel)
+// (measured then; one load of scales for two groups: 4096 x 4096 at 17 / 32 / 45 / 64 tokens 7.70 / 9.06 / 10.44 / 12.09 -> 7.56 / 8.83 /
+// 10.14 / 11.63 on another card)
 // X arrives at 30 bytes a clock and unit, half of what L2 gives a unit reading alone; letting the units start at different
 // groups changes nothing.
 //
@@ -51,17 +53,19 @@ constexpr int kWaves = 4;
 // LDS layout of a wave's stage (16-byte pieces, swizzled so that 16 lanes reading one piece of 16 rows cover all banks):
 //   activations  16 MT rows of 256 bytes, piece c of row i at c ^ (i & 15)
 //   codes        16 rows of 64 bytes, piece c of row i at c ^ ((i >> 2) & 3)
-//   scales, zeros  a dword per row each, the bf16 value in its lower half (and 32 dwords of copies)
+// and beside the stages four slots of scales and zeros, one load for every two of the wave's groups (each 2-byte value pulls a
+// cache line through L1, 32 of the 144 a group took with 48 tokens; the two groups' are 8 bytes apart):
+//   dword 32 e + i: the scale, 32 e + 16 + i: the zero of row i for the first (e = 0) or second group, in the lower half
 // MT: groups of 16 tokens, D: stages. Arguments: those of the first loads first (the leading 14 dwords are preloaded, build.py)
 template <int MT, int D>
 __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(
     const unsigned char *x_, const unsigned char *w_, int M, int N, int K, const unsigned short *scales, const unsigned short *zeros,
     const unsigned short *bias, unsigned short *y, unsigned long long *clk) {
     const FewParams p = {x_, w_, scales, zeros, bias, y, M, N, K, clk};
-    constexpr int A_BYTES = MT * 4096, STAGE = A_BYTES + 1024 + 256;
-    constexpr int LOADS = 4 * MT + 2;
-    static_assert((D - 1) * LOADS < 64, "the wait counts loads in six bits");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves * D * STAGE];
+    constexpr int A_BYTES = MT * 4096, STAGE = A_BYTES + 1024, WAVE = D * STAGE + 4 * 256;
+    constexpr int LOADS = 4 * MT + 1;  // per stage; one more in the first of two
+    static_assert((D - 1) * (LOADS + 1) < 64, "the wait counts loads in six bits");
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves * WAVE];
 
     unsigned long long clk_t0 = 0, clk_r0 = 0;
     if (p.clk) {
@@ -72,7 +76,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(
     const int lane = threadIdx.x & 63, r = lane & 15, h = lane >> 4;
     const int c0 = blockIdx.x * 16;
     const int G = p.K / LQ_GROUP;
-    unsigned char *const mine = lds + wave * (D * STAGE);
+    unsigned char *const mine = lds + wave * WAVE, *const q_ring = mine + D * STAGE;
 
     // ---- loads: instruction i < 4 MT brings rows 4 i .. 4 i + 3 of the wave's group of X
     const unsigned lda = (unsigned)p.K * 2u;
@@ -88,32 +92,40 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(
     const unsigned char *c_base = p.w + (long long)c0 * (p.K / 2);
     const unsigned char *s_base = (const unsigned char *)(p.scales + (long long)c0 * G);
     const unsigned char *z_base = (const unsigned char *)(p.zeros + (long long)c0 * G);
-    // scales on lanes 0..15 (and 32..47), zeros on 16..31 (and 48..63): one instruction, 64-bit addresses
+    // scales on lanes 0..15, zeros on 16..31, the next group's on 32..63: one instruction, 64-bit addresses
     const unsigned char *q_lane = (h & 1 ? z_base : s_base) + q_off;
     auto to_lds = [&](unsigned char *dst, unsigned off, const unsigned char *src) {
         const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)dst);
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(src) : "memory");
     };
-    // group g into stage st, the codes (from HBM) first
-    auto issue = [&](int g, unsigned char *st) {
+    const int ng = wave < G ? (G - wave + kWaves - 1) / kWaves : 0;  // the wave's groups: wave, wave + 4, ...
+    auto group_at = [&](int i) { return wave + kWaves * (i < ng ? i : ng - 1); };
+    // the wave's group i into stage st, the codes (from HBM) first; past the last group: that one again (nothing uses it)
+    auto issue = [&](int i, unsigned char *st) {
+        const int g = group_at(i);
         to_lds(st + A_BYTES, c_off, c_base + (long long)g * 64);
-        const unsigned q_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(st + A_BYTES + 1024));
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off" ::"s"(q_addr), "v"(q_lane + (long long)g * 2) : "memory");
+        if (!(i & 1)) {
+            const unsigned q_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(q_ring + ((i >> 1) & 3) * 256));
+            const int gq = h < 2 ? g : group_at(i + 1);
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off" ::"s"(q_addr), "v"(q_lane + (long long)gq * 2) : "memory");
+        }
 #pragma unroll
-        for (int i = 0; i < 4 * MT; ++i) to_lds(st + i * 1024, a_off[i], p.x + (long long)g * 256);
+        for (int k = 0; k < 4 * MT; ++k) to_lds(st + k * 1024, a_off[k], p.x + (long long)g * 256);
     };
 
     f32x4_t acc[MT];
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    const int ng = wave < G ? (G - wave + kWaves - 1) / kWaves : 0;  // the wave's groups: wave, wave + 4, ...
     auto group = [&](int i, auto si) {
         constexpr int S = decltype(si)::value;
         unsigned char *st = mine + S * STAGE;
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * LOADS) : "memory");
+        // the D - 1 later stages' loads may be under way; how many of those are first ones of two follows from D and, where D is
+        // even, the stage
+        constexpr int FIRSTS = D == 3 ? 1 : D / 2 - 1 + (S & 1);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * LOADS + FIRSTS) : "memory");
         const u32x4_t c = *reinterpret_cast<const u32x4_t *>(st + A_BYTES + r * 64 + ((h ^ ((r >> 2) & 3)) << 4));
-        const unsigned *q = reinterpret_cast<const unsigned *>(st + A_BYTES + 1024);
+        const unsigned *q = reinterpret_cast<const unsigned *>(q_ring + ((i >> 1) & 3) * 256) + 32 * (i & 1);
         const float sc = __uint_as_float(q[r] << 16);
         float zi, rest;
         lq_split_zero(__uint_as_float(q[16 + r] << 16), zi, rest);
@@ -122,10 +134,10 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(
         for (int w = 0; w < 4; ++w)
 #pragma unroll
             for (int j = 0; j < MT; ++j) x[w][j] = *reinterpret_cast<const u32x4_t *>(st + (16 * j + r) * 256 + (((4 * h + w) ^ r) << 4));
-        // the stage is free once these reads have returned; past the wave's last group: re-read it (nothing uses it)
+        // the stage is free once these reads have returned
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        issue(wave + kWaves * (i + D < ng ? i + D : ng - 1), st);
+        issue(i + D, st);
         __builtin_amdgcn_sched_barrier(0);
         f32x4_t P[MT];
 #pragma unroll
@@ -150,7 +162,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_few_kernel(
     };
     if (ng > 0) {
 #pragma unroll
-        for (int d = 0; d < D; ++d) issue(wave + kWaves * (d < ng ? d : ng - 1), mine + d * STAGE);
+        for (int d = 0; d < D; ++d) issue(d, mine + d * STAGE);
         int i = 0;
         for (; i + D <= ng; i += D) {
             group(i, ic<0>());
