@@ -1,6 +1,6 @@
 // Activation quantisers in front of the int8 GEMM (bf16 -> int8 + the per-row scales its epilogue reads):
 //   lq_act_quant_i8           per-tensor, clamp value given (a device scalar)
-//   lq_act_quant_i8_dynamic   per-tensor, clamp value = the tensor's own maximum (two launches, no host sync)
+//   lq_act_quant_i8_dynamic   per-tensor, clamp value = the tensor's own maximum (one or two launches, no host sync)
 //   lq_act_quant_i8_per_token one scale per token row from the row's absolute maximum (one pass over HBM)
 // and, for the backward passes, lq_act_dequant_i8 (int8 -> bf16) and lq_act_fake_quant (bf16 -> bf16 on the int8 grid)
 #include "lq_common.h"
@@ -65,6 +65,50 @@ __global__ __launch_bounds__(256) void tensor_max_kernel(const unsigned short *_
     if (threadIdx.x == 0) partial[blockIdx.x] = k;
 }
 
+// what follows once the largest key is known: the clamp value and alpha to `work`, the per-row scales, and the thread's 8 elements
+__device__ __forceinline__ void act_quant_with_key(unsigned k, const unsigned short *__restrict__ x, signed char *__restrict__ x8,
+                                                   float *__restrict__ sx, float *__restrict__ work, long long n, long long M, int alpha_bf16) {
+    const float c = max_key_value(k);
+    float alpha = c * (1.0f / 127.0f);
+    if (alpha_bf16) alpha = lq_bf16r(alpha);
+    const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid == 0) {
+        work[0] = c;
+        work[1] = alpha;
+    }
+    for (long long m = gid; m < M; m += (long long)gridDim.x * blockDim.x) sx[m] = alpha;
+    act_quant_piece<true>(x, x8, gid * 8, n, c);
+}
+
+// Both phases in one launch, for few elements: every workgroup finds the maximum of all of them. An int8 layer with two launches
+// and with one, us: 17 x 2048 9.0 / 8.8, 32 x 2048 9.5 / 9.5, 59 x 2048 12.1 / 14.2, 95 x 2048 12.3 / 16.0. A launch is 3 us of
+// the host's time besides, which such calls wait for.
+constexpr long long kOneLaunch = 80 << 10;
+__global__ __launch_bounds__(1024) void act_quant_one_kernel(const unsigned short *__restrict__ x, signed char *__restrict__ x8,
+                                                             float *__restrict__ sx, float *__restrict__ work, int n, int M, int alpha_bf16) {
+    __shared__ __attribute__((aligned(16))) unsigned red[16];
+    MaxKeys keys;
+    const int n8 = n / 8;
+    const u32x4_t *x16 = reinterpret_cast<const u32x4_t *>(x);
+#pragma unroll 8
+    for (int i = threadIdx.x; i < n8; i += 1024) keys.add8(x16[i]);
+    unsigned k = keys.key();
+    if ((int)threadIdx.x < n - n8 * 8) {
+        const unsigned t = max_key(x[n8 * 8 + threadIdx.x]);
+        k = k > t ? k : t;
+    }
+    k = wave_max_u32(k);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = k;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; w += 4) {
+        const u32x4_t r = *reinterpret_cast<const u32x4_t *>(red + w);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) k = k > r[j] ? k : r[j];
+    }
+    act_quant_with_key(k, x, x8, sx, work, n, M, alpha_bf16);
+}
+
 // Phase 2: every workgroup reduces the partial keys to the clamp value, then quantises its 2048 elements;
 // the first M threads of the grid also write the per-row scale alpha = clampv * fl(1/127) (the tensor library
 // divides a tensor by a host scalar as a product with the scalar's fp32 reciprocal), rounded to bf16 when the
@@ -77,16 +121,7 @@ __global__ __launch_bounds__(256) void act_quant_dyn_kernel(const unsigned short
     unsigned k = 0u;
     for (int i = threadIdx.x; i < partials; i += 256) k = k > partial[i] ? k : partial[i];
     k = wg_max_u32(k, red);
-    const float c = max_key_value(k);
-    float alpha = c * (1.0f / 127.0f);
-    if (alpha_bf16) alpha = lq_bf16r(alpha);
-    const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (gid == 0) {
-        work[0] = c;
-        work[1] = alpha;
-    }
-    for (long long m = gid; m < M; m += (long long)gridDim.x * 256) sx[m] = alpha;
-    act_quant_piece<true>(x, x8, gid * 8, n, c);
+    act_quant_with_key(k, x, x8, sx, work, n, M, alpha_bf16);
 }
 
 // ---- one scale per token row --------------------------------------------------------------------
@@ -235,6 +270,11 @@ extern "C" int lq_act_quant_i8_dynamic(const void *x, int8_t *x8, float *sx, flo
     const long long n = M * K;
     const long long blocks = ((n + 7) / 8 + 255) / 256;
     LQ_REQUIRE(blocks <= 0x7FFFFFFFll, "lq_act_quant_i8_dynamic: tensor too large");
+    if (n <= kOneLaunch) {
+        hipLaunchKernelGGL(act_quant_one_kernel, dim3((unsigned)((n + 8191) / 8192)), dim3(1024), 0, (hipStream_t)stream,
+                           (const unsigned short *)x, (signed char *)x8, sx, work, (int)n, (int)M, alpha_bf16);
+        return lq_check_launch("lq_act_quant_i8_dynamic");
+    }
     const int partials = (int)(blocks < kMaxPartials ? blocks : kMaxPartials);
     hipLaunchKernelGGL(tensor_max_kernel, dim3((unsigned)partials), dim3(256), 0, (hipStream_t)stream, (const unsigned short *)x, n,
                        reinterpret_cast<unsigned *>(work + 8));

@@ -283,16 +283,17 @@ PyObject *infer8(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
         LQ_CALL(lq_a8w8_infer, x->data_ptr(), w->data_ptr(), qs->data_ptr(), bias, y.data_ptr(), a[4] == Py_True, M, N, K, on.stream);
         return wrap(std::move(y));
     }
-    at::Tensor x8 = make(x->sizes(), at::kChar, *x), sx = make({M}, at::kFloat, *x);
-    if (a[4] == Py_True) {
-        LQ_CALL(lq_act_quant_i8_per_token, x->data_ptr(), (int8_t *)x8.data_ptr(), (float *)sx.data_ptr(), M, K, on.stream);
-    } else {
-        at::Tensor work = make({LQ_ACT_WORK_FLOATS}, at::kFloat, *x);
-        LQ_CALL(lq_act_quant_i8_dynamic, x->data_ptr(), (int8_t *)x8.data_ptr(), (float *)sx.data_ptr(), (float *)work.data_ptr(), M, K,
-                0, on.stream);
-    }
-    LQ_CALL(lq_a8w8_fwd_qs, x8.data_ptr(), w->data_ptr(), (const float *)sx.data_ptr(), qs->data_ptr(), bias, y.data_ptr(), nullptr, M,
-            N, K, on.stream);
+    // what the quantiser leaves for the product, in one allocation: x8 [M, K], sx [M], the quantiser's scratch
+    const int64_t at_sx = (M * K + 15) / 16 * 16, at_work = at_sx + (M * 4 + 15) / 16 * 16;
+    at::Tensor scratch = make({at_work + LQ_ACT_WORK_FLOATS * 4}, at::kByte, *x);
+    uint8_t *p = (uint8_t *)scratch.data_ptr();
+    int8_t *x8 = (int8_t *)p;
+    float *sx = (float *)(p + at_sx), *work = (float *)(p + at_work);
+    if (a[4] == Py_True)
+        LQ_CALL(lq_act_quant_i8_per_token, x->data_ptr(), x8, sx, M, K, on.stream);
+    else
+        LQ_CALL(lq_act_quant_i8_dynamic, x->data_ptr(), x8, sx, work, M, K, 0, on.stream);
+    LQ_CALL(lq_a8w8_fwd_qs, x8, w->data_ptr(), sx, qs->data_ptr(), bias, y.data_ptr(), nullptr, M, N, K, on.stream);
     return wrap(std::move(y));
 }
 

@@ -84,3 +84,20 @@ def test_quantisers(hip_lib, M, K, name):
             acc = (q.double() @ w.double().t()).float()
             ref = ((acc * s[:, None]) * qs.float().view(1, -1)).to(torch.bfloat16)
             assert torch.equal(torch.nan_to_num(y.float(), nan=7.25), torch.nan_to_num(ref.float(), nan=7.25)), (name, at, per_token)
+
+
+@pytest.mark.parametrize("M,K", [(1, 1), (3, 7), (5, 1021), (10, 8192), (10, 8193), (13, 7867), (60, 7001)])
+@pytest.mark.parametrize("name", SPECIALS)
+def test_maximum_in_one_launch_and_two(hip_lib, M, K, name):
+    """Sizes on both sides of the number of elements up to which every workgroup finds the maximum itself, remainders of eight."""
+    from latentq_llm_amd import ops
+    base = _x(M, K, M + K) if K > 8 else torch.randn(M, K, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    for at in sorted({0, M * K - 1, M * K // 2}):
+        x = _special(base, name, at)
+        want8, c = _per_tensor(x)
+        x8, sx, work = ops.act_quant_i8_dynamic(x.cuda())
+        cv = work[0].cpu()
+        assert (torch.isnan(c) and torch.isnan(cv)) or cv == c.float(), (name, at)
+        assert torch.equal(x8.cpu(), want8), (name, at)
+        alpha = c.float() * torch.tensor(1.0 / 127.0)
+        assert torch.equal(torch.nan_to_num(sx.cpu(), nan=-1.0), torch.nan_to_num(alpha.expand(M), nan=-1.0)), (name, at)
