@@ -1262,6 +1262,12 @@ static int a8w8_fwd_impl(const void *x, const void *w, const float *sx, const vo
     // tokens (two workgroups per unit, each reading all tokens), behind them from 48 tokens on (12.1 against 7.8 there).
     if (M <= 16 || (M <= 32 && N <= 32 * cus))
         return lq_gemv_i8_launch(x, w, sx, sw, sw_bf16, bias_or_null, y, acc_or_null, (int)M, (int)N, (int)K, (hipStream_t)stream);
+    // 32 x 32 tiles while every unit gets one at most: what bounds these tiles is the bytes a unit takes in, K (rows + columns),
+    // and of 64 x 64 tiles at most a quarter as many units would work. us against 64 x 64: 2048 x 8192 at 64 / 128 tokens 14.1 /
+    // 13.9, 22.8 / 22.5; 2560^2 at 40 7.6, 9.2; 2048^2 at 59 / 128 6.8 / 7.0, 7.6 / 7.7. On a short K the four groups have too
+    // few steps to pay for their sums: 1024 x 512 at 33 5.7 against 5.5, 768^2 at 40 5.9 against 5.8.
+    if (K >= 2048 && ((M + 31) / 32) * ((N + 31) / 32) <= cus)
+        return lq_gemm_i8_tile_launch(x, w, sx, sw, sw_bf16, bias_or_null, y, acc_or_null, (int)M, (int)N, (int)K, 32, 4, (hipStream_t)stream);
     // 64 x 64 tiles while no unit gets more than two of them: a step of a 128 x 128 tile fetches 32 KB, which takes a unit
     // twice as long as the 16 KB of this tile, and few tiles leave units idle. us against 128 x 128 tiles: 2048^2 at 64 / 512 / 1024
     // tokens 7.6 / 8.3 / 11.5 against 10.7 / 11.5 / 12.4, 2048 x 8192 at 128 / 512 15.5 / 17.1 against 25.3 / 26.6; with three

@@ -11,7 +11,10 @@
 // 128 x 64 outputs (4 x 2 MFMA 32x32x32 tiles, 128 accumulator registers), two waves per SIMD. One
 // workgroup per CU: two LDS stages of 64 KB (256 rows of A and 256 rows of B, 128 bytes = 128 k
 // each). For small outputs: 128 x 128 tile, 8 waves (2 x 4, 64 x 32 each), with two stages of
-// 32 KB (two workgroups per CU) or four (one workgroup per CU, loads three steps ahead).
+// 32 KB (two workgroups per CU) or four (one workgroup per CU, loads three steps ahead); 64 x 64, 4 waves, four stages of
+// 16 KB. For outputs of at most one 32 x 32 tile per CU: that tile, four groups of one wave, each on a quarter of K with four
+// stages of 8 KB of its own. What bounds the small tiles is the bytes a CU takes in (25 to 30 per clock, K x (rows + columns)
+// of its tile in all), so half the edge on four times the CUs halves the time as long as CUs are idle.
 //
 // Reduction step = 128 k in four slices of 32. Lane l: r = l % 32, h = l / 32. In slice t the
 // lane's operand of row r is chunk 4h + t (16 bytes) of the row's 128 bytes, for A and B alike
@@ -58,8 +61,14 @@ constexpr int ROWB = 128;  // bytes (= k) per tile row and step
 // 128 x 128 with 2 x 4 waves of 64 x 32 (64 KB of LDS: two per CU) for outputs too small to fill the
 // device with the large tile; with 2 x 2 waves of 64 x 64 it was 5-12 % slower (one wave per SIMD
 // when a workgroup has a CU to itself).
-template <int BM, int BN, int WM, int WN, int NS>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) {
+// KS: groups of WM x WN waves that share the tile, each with stages of its own and on a part of K; their int32 sums meet in LDS.
+// 32 x 32 tiles have four groups of one wave, which needs no barrier before the sums. us against 64 x 64 tiles: 2048 x 8192 at
+// 64 / 128 tokens 14.1 / 13.9 against 22.8 / 22.5, 2048^2 6.8 / 7.0 against 7.6 / 7.7, 768 x 3072 at 100 7.5 against 9.0. (Two
+// groups for 64 x 64 tiles are 2 to 8 % slower: there two or more tiles or stages already ask for all that a CU takes in; 32 x 64
+// tiles of three groups gain only from K = 8192 on and lose 15 to 27 % at 2048.)
+template <int BM, int BN, int WM, int WN, int NS, int KS = 1>
+__global__ __launch_bounds__(64 * WM * WN * KS) void gemm_i8_tile_kernel(I8Params p) {
+    static_assert(KS == 1 || WM * WN == 1, "several groups: of one wave each");
     static_assert(NS == 2 || NS == 4, "two or four stages");
     constexpr int NT = 64 * WM * WN;
     constexpr int A_STAGE = BM * ROWB;       // A rows, then B rows
@@ -68,11 +77,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) 
     constexpr int FM = TM / 32, FN = TN / 32;
     constexpr int LA = BM * 8 / NT, LB = BN * 8 / NT;  // 16-byte loads per thread and stage: A, then B
     static_assert(BM * 8 % NT == 0 && BN * 8 % NT == 0 && LA >= 1 && LB >= 1, "a stage divides over the threads");
-    __shared__ __attribute__((aligned(16))) unsigned char lds_all[NS * STAGE];
-    unsigned char *const lds0 = lds_all;
-    auto stage = [&](auto i) -> unsigned char * { return lds_all + decltype(i)::value * STAGE; };
+    __shared__ __attribute__((aligned(16))) unsigned char lds_all[KS * NS * STAGE];
+    const int wave_all = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int kg = KS == 1 ? 0 : wave_all, wave = KS == 1 ? wave_all : 0;
+    const int tid = KS == 1 ? (int)threadIdx.x : (int)(threadIdx.x & 63);
+    unsigned char *const lds0 = lds_all + kg * (NS * STAGE);
+    auto stage = [&](auto i) -> unsigned char * { return lds0 + decltype(i)::value * STAGE; };
 
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     const int r = lane & 31, h = lane >> 5;
     const int wm = wave % WM, wn = wave / WM;
@@ -93,15 +104,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) 
     const int bw = rest < GN ? rest : GN;
     const int tile_m = within / bw, tile_n = band * GN + within % bw;
     const int m0 = tile_m * BM, c0 = tile_n * BN;
-    const int nk = p.K / ROWB;
+    const int nk_all = p.K / ROWB, k_first = nk_all * kg / KS, nk = nk_all * (kg + 1) / KS - k_first;  // this group's steps
 
     // ---- staging: 2048 16-byte slots per operand and stage; slot s = i*512 + thread -> row s/8,
     // position s%8. Rows past the end of a matrix re-read its last row (their results are dropped).
     unsigned a_off[LA], b_off[LB];
 #pragma unroll
     for (int i = 0; i < (LA > LB ? LA : LB); ++i) {
-        const int row = i * (NT / 8) + (int)(threadIdx.x >> 3);
-        const int pos = threadIdx.x & 7;
+        const int row = i * (NT / 8) + (tid >> 3);
+        const int pos = tid & 7;
         const int chunk = pos ^ ((row >> 1) & 7);
         int ga = m0 + row, gb = c0 + row;
         ga = ga < p.M ? ga : p.M - 1;
@@ -109,8 +120,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) 
         if (i < LA) a_off[i] = (unsigned)((long long)(ga - m0) * p.K + chunk * 16);
         if (i < LB) b_off[i] = (unsigned)((long long)(gb - c0) * p.K + chunk * 16);
     }
-    const unsigned char *a_base = p.x + (long long)m0 * p.K;
-    const unsigned char *b_base = p.w + (long long)c0 * p.K;
+    const unsigned char *a_base = p.x + (long long)m0 * p.K + (long long)k_first * ROWB;
+    const unsigned char *b_base = p.w + (long long)c0 * p.K + (long long)k_first * ROWB;
     // load i of a step: 0..LA-1 fill the A rows of the stage, LA..LA+LB-1 its B rows
     auto issue_one = [&](int kt, unsigned char *st, int i) {
         const bool is_b = i >= LA;
@@ -153,7 +164,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) 
         const int kt_b = kt + NS - 1 < nk ? kt + NS - 1 : nk - 1, kt_a = kt + NS < nk ? kt + NS : nk - 1;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            if (t == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * (LA + LB)) : "memory");
+            if (t == 3) {
+                if constexpr (KS == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * (LA + LB)) : "memory");
+                else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * (LA + LB)) : "memory");
+            }
             if (t < 3) read_frags(cur, t + 1, af[(t + 1) & 1], bf[(t + 1) & 1]);
             else read_frags(nxt, 0, af[0], bf[0]);
             if (t == 0) {
@@ -223,6 +237,29 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) 
     constexpr int LPR = TN / 8;        // lanes per staged row (16 bytes each)
     constexpr int RPI = 64 / LPR;      // rows per store instruction
     static_assert(NT / 64 * 32 * EP <= NS * STAGE, "epilogue staging fits the stages");
+    if constexpr (KS > 1) {  // the other groups' sums to the first, behind its staging area
+        static_assert(FM == 1 && 32 * EP + (KS - 1) * FN * 4096 <= KS * NS * STAGE, "the sums fit the stages");
+        i32x4_t *sums = reinterpret_cast<i32x4_t *>(lds_all + 32 * EP) + tid;
+        if (kg)
+#pragma unroll
+            for (int i = 0; i < FN; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    sums[(((kg - 1) * FN + i) * 4 + q) * 64] =
+                        i32x4_t{acc[i][0][4 * q], acc[i][0][4 * q + 1], acc[i][0][4 * q + 2], acc[i][0][4 * q + 3]};
+        __syncthreads();
+        if (kg) return;
+#pragma unroll
+        for (int g = 0; g < KS - 1; ++g)
+#pragma unroll
+            for (int i = 0; i < FN; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const i32x4_t v = sums[((g * FN + i) * 4 + q) * 64];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][0][4 * q + e] += v[e];
+                }
+    }
     unsigned char *ep = lds0 + wave * (32 * EP);
     const int ep_row = lane / LPR, ep_chunk = lane % LPR;
     const int cw0 = c0 + wn * TN;
@@ -280,7 +317,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_tile_kernel(I8Params p) 
 long long lq_gemm_i8_256_workgroups(int M, int N) { return (long long)((M + 255) / 256) * ((N + 255) / 256); }
 
 // Called by lq_a8w8_fwd (lq_gemm.hip) after argument validation: K % 128 == 0, N % 16 == 0.
-// tile = 256 or 128 (square tiles, 8 waves each) or 64 (4 waves); stages = 2, or 4 with the 128 tile (64: always 4).
+// tile = 256 or 128 (square tiles, 8 waves each), 64 or 32 (4 waves; 32: K >= 512, a step for every group); stages = 2, or 4 with the 128 tile (64, 32: always 4).
 int lq_gemm_i8_tile_launch(const void *x8, const void *w8, const float *sx, const void *sw, bool sw_bf16, const void *bias, void *y,
                            int *acc_or_null, int M, int N, int K, int tile, int stages, hipStream_t st) {
     I8Params p = {};
@@ -294,6 +331,7 @@ int lq_gemm_i8_tile_launch(const void *x8, const void *w8, const float *sx, cons
     // the 32-bit lane offsets of the loads span up to 256 rows
     if (256ll * K >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "lq_a8w8_fwd: K too large");
     if (tile == 256) hipLaunchKernelGGL((gemm_i8_tile_kernel<256, 256, 2, 4, 2>), dim3((unsigned)nwg), dim3(512), 0, st, p);
+    else if (tile == 32) hipLaunchKernelGGL((gemm_i8_tile_kernel<32, 32, 1, 1, 4, 4>), dim3((unsigned)nwg), dim3(256), 0, st, p);
     else if (tile == 64) hipLaunchKernelGGL((gemm_i8_tile_kernel<64, 64, 2, 2, 4>), dim3((unsigned)nwg), dim3(256), 0, st, p);
     else if (stages == 4) hipLaunchKernelGGL((gemm_i8_tile_kernel<128, 128, 2, 4, 4>), dim3((unsigned)nwg), dim3(512), 0, st, p);
     else hipLaunchKernelGGL((gemm_i8_tile_kernel<128, 128, 2, 4, 2>), dim3((unsigned)nwg), dim3(512), 0, st, p);
