@@ -537,11 +537,28 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const bool in = c + r < p.C;
-                bias_v[i][q][r] = (p.bias && in) ? lq_bf16_bits_to_f32(p.bias[c + r]) : 0.0f;
+                bias_v[i][q][r] = (!kDx && p.bias && in) ? lq_bf16_bits_to_f32(p.bias[c + r]) : 0.0f;
             }
         }
+    // What the SiLU epilogue reads of g and u goes out for 32 rows at once, ahead of the staging of those rows (rows past the end
+    // read the last one; the columns are a multiple of the tile's). A load behind each row's own test made the epilogue 8 or 16
+    // waits for memory in a row: 500 x 2048 -> 5504 33.0 us before, 29.0 with this; 1500 x 1024 -> 2816 34.0, 27.0; 2048 x 4096
+    // -> 11008 225, 210. (The next 32 rows' loads ahead of this block's arithmetic: no further gain, 0 to 2 % slower.)
+    constexpr int EPI = 32 / RPI;  // row groups of a block of 32 rows
+    u32x4_t g_rows[EPI], u_rows[EPI];
+    auto load_gu = [&](int j) {
+#pragma unroll
+        for (int it = 0; it < EPI; ++it) {
+            const int mm = m0 + wm * TM + j * 32 + it * RPI + ep_row;
+            const long long off = (long long)(mm < p.M ? mm : p.M - 1) * p.C + c_lane;
+            g_rows[it] = *reinterpret_cast<const u32x4_t *>(p.ep_g + off);
+            u_rows[it] = *reinterpret_cast<const u32x4_t *>(p.ep_u + off);
+        }
+    };
+    const bool silu = MODE == MODE_W4_DX && p.ep_mode == EP_SILU_BW;
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
+        if (silu) load_gu(j);
 #pragma unroll
         for (int i = 0; i < FN; ++i) {
 #pragma unroll
@@ -550,14 +567,14 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     v[r] = acc[i][j][4 * q + r];
-                    if (p.bias) v[r] += bias_v[i][q][r];
+                    if (!kDx && p.bias) v[r] += bias_v[i][q][r];
                 }
                 u32x2_t o = {lq_pack_bf16(v[0], v[1]), lq_pack_bf16(v[2], v[3])};
                 *reinterpret_cast<u32x2_t *>(ep + frag_row * EP + (i * 32 + 8 * q + 4 * kh) * 2) = o;
             }
         }
 #pragma unroll
-        for (int it = 0; it < 32 / RPI; ++it) {
+        for (int it = 0; it < EPI; ++it) {
             const int row = it * RPI + ep_row;
             const u32x4_t o = *reinterpret_cast<const u32x4_t *>(ep + row * EP + ep_chunk * 16);
             const int mm = m0 + wm * TM + j * 32 + row;
@@ -570,9 +587,8 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
                     for (int e = 0; e < 4; ++e)
                         sum[e] = lq_pack_bf16(lq_bf16_lo(old[e]) + lq_bf16_lo(o[e]), lq_bf16_hi(old[e]) + lq_bf16_hi(o[e]));
                     *reinterpret_cast<u32x4_t *>(out + off) = sum;
-                } else if (kDx && p.ep_mode == EP_SILU_BW) {
-                    const u32x4_t g8 = *reinterpret_cast<const u32x4_t *>(p.ep_g + off);
-                    const u32x4_t u8 = *reinterpret_cast<const u32x4_t *>(p.ep_u + off);
+                } else if (silu) {
+                    const u32x4_t g8 = g_rows[it], u8 = u_rows[it];
                     u32x4_t dg, du;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
