@@ -152,8 +152,8 @@ int lq_a16w4_gate_up_silu(const void *x, const void *codes_gate, const void *sca
                           int64_t N, int64_t K, int group, void *stream);
 
 /* Both forms (g_out and u_out null: lq_a16w4_gate_up_silu; given: lq_a16w4_gate_up_silu_save below) with a scratch buffer as
- * lq_a16w4_fwd_ws: with 8 M N bytes and more of it, some 17 to 200 tokens run as one launch of small row tiles whose fp32
- * partial products a second launch combines. */
+ * lq_a16w4_fwd_ws: with 8 M N bytes and more of it, some 17 to 200 tokens run as one launch of small row tiles; where the
+ * reduction is cut, a second launch combines its fp32 partial products. */
 int lq_a16w4_gate_up_silu_ws(const void *x, const void *codes_gate, const void *scales_gate, const void *zeros_gate,
                              const void *codes_up, const void *scales_up, const void *zeros_up, void *h, void *g_out_or_null,
                              void *u_out_or_null, int64_t M, int64_t N, int64_t K, int group, void *workspace,
@@ -265,7 +265,7 @@ int lq_act_quant_i8(const void *x, const float *clampv_dev, int8_t *x8, int64_t 
 
 /* The same quantiser with the clamp value the dynamic layers of the reference use, the maximum of the
  * activation tensor itself (`clampv = input.max()`, utils/quant.py:259-266, 319-322), found on the device:
- * two launches, no host synchronisation and no other kernel. A NaN anywhere in x makes the clamp value NaN
+ * one launch (up to some 80 000 elements) or two, no host synchronisation and no other kernel. A NaN anywhere in x makes the clamp value NaN
  * (as the tensor library's max does) and every x8 zero.
  *   clampv = max_i x[i];  x8 as lq_act_quant_i8 with that value;
  *   sx[m]  = alpha for every m < M, alpha = clampv * fl32(1/127) (how the tensor library divides a tensor by

@@ -9,7 +9,7 @@
 //
 // Up to 16 tokens in inference the activations come in as bf16 and every workgroup quantises all of them itself into
 // LDS (kFused; M (K + 16) bytes, at most 64 KB: 16 elements per thread for 4 tokens of 2048): that replaces the
-// two quantiser launches in front of the product, each of which costs more than the work. The first weight pieces are
+// quantiser's launch or two in front of the product, each of which costs more than the work. The first weight pieces are
 // requested behind the activations and travel meanwhile.
 //
 // MFMA operands: weights first, activations second, so that lane l holds columns 4 (l / 16) .. + 3 of token l % 16.
