@@ -498,9 +498,38 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
     // tile before the final barrier, and no load is in flight into them); a wave's staging area
     // is private, row pitch TN*2 + 16 bytes.
     if (split) {
-        // split reduction: the fp32 accumulators as they are, 16 bytes per lane; a second kernel adds
-        // the slices in a fixed order, adds the bias and rounds
+        // split reduction: the fp32 accumulators as they are; a second kernel adds the slices in a fixed order and rounds.
+        // Stored from the registers an instruction touches 32 rows with 32 bytes each. With more rows than a few they pass through
+        // the wave's half of a B buffer, 32 rows at a time, chunk c of row r at position c ^ (r & 15), and leave as 256
+        // contiguous bytes of 4 rows. us before and after: pair of 5504 x 2048 at 500 tokens 38.2, 36.4, of 4096 x 1536 at 1000 39.7,
+        // 38.0; one product 3072 x 768 at 1024 20.3, 19.9; 8192 x 2048 at 2048 81.6, 79.1; 1536^2 at 333 14.0, 13.4. With few rows the way
+        // through LDS is only longer: 4096^2 at 64 tokens 15.9, 16.2; 2048 x 5504 at 130 19.2, 19.5; level at 128 rows.
         float *part = p.partial + (long long)blockIdx.y * p.M * p.C;
+        if (p.M > 192) {
+            static_assert(!kDx || (TN == 64 && 32 * TN * 4 * WM * WN <= 2 * B_BYTES), "a block of 32 rows of fp32 per wave");
+            constexpr int PER_BUF = B_BYTES / (32 * TN * 4);
+            unsigned char *block = (wave >= PER_BUF ? lds_b1 : lds_b0) + (wave % PER_BUF) * (32 * TN * 4);
+            const int p_row = lane >> 4, p_chunk = lane & 15;
+            part += c0 + wn * TN + p_chunk * 4;
+#pragma unroll
+            for (int j = 0; j < FM; ++j) {
+                if (m0 + wm * TM + j * 32 >= p.M) break;
+#pragma unroll
+                for (int i = 0; i < FN; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const f32x4_t v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                        *reinterpret_cast<f32x4_t *>(block + frag_row * (TN * 4) + (((i * 8 + 2 * q + kh) ^ (frag_row & 15)) << 4)) = v;
+                    }
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    const int row = it * 4 + p_row, m = m0 + wm * TM + j * 32 + row;
+                    const f32x4_t v = *reinterpret_cast<const f32x4_t *>(block + row * (TN * 4) + ((p_chunk ^ (row & 15)) << 4));
+                    if (m < p.M) *reinterpret_cast<f32x4_t *>(part + (long long)m * p.C) = v;
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < FM; ++j) {
             const int m = m0 + wm * TM + j * 32 + frag_row;
@@ -509,11 +538,8 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
             for (int i = 0; i < FN; ++i)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int c = c0 + wn * TN + i * 32 + 8 * q + 4 * kh;
-                    if (c >= p.C) continue;
-                    f32x4_t v = {(float)acc[i][j][4 * q], (float)acc[i][j][4 * q + 1], (float)acc[i][j][4 * q + 2],
-                                 (float)acc[i][j][4 * q + 3]};
-                    *reinterpret_cast<f32x4_t *>(part + (long long)m * p.C + c) = v;
+                    const f32x4_t v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                    *reinterpret_cast<f32x4_t *>(part + (long long)m * p.C + c0 + wn * TN + i * 32 + 8 * q + 4 * kh) = v;
                 }
         }
         return;
