@@ -459,6 +459,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
             if (t < 3) read_frags(la, lb, t + 1, af[(t + 1) & 1], bf[(t + 1) & 1]);
             else read_frags(la_next, lb_next, 0, af[0], bf[0]);
             issue_a_part(kt_a, la_load, t);
+            if constexpr (BM == 128) __builtin_amdgcn_sched_barrier(0);
             mfma_step(af[t & 1], bf[t & 1]);
             __builtin_amdgcn_sched_barrier(0);
         }
