@@ -31,6 +31,7 @@
 //     h: 6144 x 3072                                                  25.0 -> 18.5
 //     h: 4096 x 2048                                                  21.2 -> 14.3 (200)
 #include "lq_common.h"
+#include "lq_staged_ring.h"
 
 #include <type_traits>
 
@@ -62,7 +63,7 @@ using ic = std::integral_constant<int, I>;
 constexpr int kCols = 128;
 constexpr int kThreads = 512;
 // LDS stages; a fourth changes nothing, with two the 128-row tile takes 15 % longer
-constexpr int D = 3;
+constexpr int D = kStagedStages;
 
 // LDS (every 16-byte piece swizzled so that the fragment reads, one piece of 32 consecutive rows, spread over all banks).
 // FM < 4: a stage is a pair of groups (256 k); of the two waves on a column block one multiplies the first group, one the second.
@@ -71,9 +72,8 @@ constexpr int D = 3;
 // FM = 4, for which that is too much: a stage is one group, of which each wave takes 64 k
 //   activations  128 rows of 256 bytes,   chunk c of row i at c ^ (i & 15)
 //   codes        as above, a pair of groups in one of two slots, requested every other stage
-// Scales and zeros: a ring of pieces, see issue_q.
+// Scales and zeros: a ring of pieces (lq_staged_ring.h), see issue_q.
 constexpr int kCodeBytes = kCols * 128;
-constexpr int kScaleRing = 8192;
 
 // FM: 32-row fragments of the row tile (32 FM rows)
 // EXACT: weights as they are (see the top of the file), else rounded to bf16 like those of the kernels for more tokens
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
     constexpr int LA = A_BYTES / 16 / kThreads;       // loads per thread and stage: activations
     constexpr int LC = kCodeBytes / 16 / kThreads;    // codes (FM = 4: every other stage)
     constexpr int EP = 136;                           // floats per row of the sums in LDS (4 rows apart: 32 banks)
-    constexpr int LDS_BYTES = D * A_BYTES + C_SLOTS * kCodeBytes + kScaleRing;
+    constexpr int LDS_BYTES = D * A_BYTES + C_SLOTS * kCodeBytes + ScaleRing::bytes(PAIRS);
     static_assert(2 * BM * EP * 4 <= LDS_BYTES, "the sums do not fit");
     static_assert(PAIRS || !EXACT, "128 rows: rounded weights only");
     __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
@@ -122,14 +122,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
     const int G = p.K / LQ_GROUP;
     const int g_first = p.partial ? (int)blockIdx.y * p.groups_per_split : 0;
     const int g_end = p.partial && g_first + p.groups_per_split < G ? g_first + p.groups_per_split : G;
-    const int ng = g_end - g_first;
-    // pairs of groups; the last of an odd number begins a group earlier, and only its second group is new
-    auto pair_start = [&](int j) {
-        const int g = g_first + 2 * j < g_end - 2 ? g_first + 2 * j : g_end - 2;
-        return g > 0 ? g : 0;
-    };
-    const int units = PAIRS ? (ng + 1) / 2 : ng;            // stages of the workgroup
-    const int my_units = PAIRS && kg == 0 ? ng / 2 : units; // and of this wave
+    const StagedSlice slice = {g_first, g_end, PAIRS};
+    const ScaleRing ring = {p.q_log, PAIRS};
+    const int units = slice.units(), my_units = slice.units_of(kg);
     const int half_of_one = G == 1 ? 1 : 0;                 // a row of one group: both halves of a pair are that group
 
     // ---- loads
@@ -169,19 +164,19 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(src) : "memory");
     };
     auto issue_a = [&](int u, unsigned char *st, int i) {
-        const int g = PAIRS ? pair_start(u) : g_first + u;
+        const int g = slice.group_of(u, 0);
         to_lds16(st + (i * kThreads + wave_all * 64) * 16, a_off[i], a_base + (long long)g * 256);
     };
     static_assert(LC == 2, "gate / up: the first load of the codes is the first matrix', the second the second's");
     auto issue_c = [&](int j, unsigned char *slot, int i) {
-        to_lds16(slot + (i * kThreads + wave_all * 64) * 16, c_off[i], (i ? c_base2 : c_base) + (long long)pair_start(j) * 64);
+        to_lds16(slot + (i * kThreads + wave_all * 64) * 16, c_off[i], (i ? c_base2 : c_base) + (long long)slice.pair_start(j) * 64);
     };
     // Scales and zeros of 2^q_log groups in a piece, fetched by the first four waves: 16 bytes per column, 8 values from an even
     // index on: 8 groups, or 4 of rows of an odd number of groups, which may begin at the second value. The last piece
     // ends with the matrix. q_log = 0, matrices that are not 4-byte aligned: one value, in a dword. A slot holds
     // [scales, zeros][128 columns].
     const int q_most = (p.N - c0 < kCols ? p.N - c0 : kCols) * G - 8;
-    const unsigned q_shift = p.q_log ? 4u : 2u, q_slots = p.q_log ? 1u : 7u;
+    const unsigned q_shift = p.q_log ? 4u : 2u;
     auto q_first = [&](int row_at, int piece) {  // index of a piece's first value, for the row that begins at index row_at
         const int at = row_at + (piece << p.q_log);
         if (!p.q_log) return at;
@@ -191,19 +186,18 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
                                      : wave < 2 ? (second ? p.scales2 : p.scales) : second ? p.zeros2 : p.zeros;
     const unsigned char *q_base = scalar((const unsigned char *)(q_mat + (long long)c0 * G));
     const int q_row = tile_row(tid & 127) * G;
-    int q_next = g_first >> p.q_log;  // pieces below have been requested
-    auto issue_q = [&](int g) {       // all pieces up to group g's; whether this wave issued any
-        const bool any = kg == 0 && q_next <= g >> p.q_log;
-        for (; q_next <= g >> p.q_log; ++q_next) {
+    int q_next = ring.piece(g_first);  // pieces below have been requested
+    auto issue_q = [&](int g) {        // all pieces up to group g's; whether this wave issued any
+        const bool any = kg == 0 && q_next <= ring.piece(g);
+        for (; q_next <= ring.piece(g); ++q_next) {
             if (kg) continue;
-            const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(q_ring + ((((unsigned)q_next & q_slots) * 256 + wave * 64) << q_shift)));
+            const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(q_ring + ((ring.slot(q_next) * 256 + wave * 64) << q_shift)));
             const unsigned off = (unsigned)q_first(q_row, q_next) * 2u;
             if (p.q_log) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(q_base) : "memory");
             else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" ::"s"(lds_addr), "v"(off), "s"(q_base) : "memory");
         }
         return any;
     };
-    auto last_group = [&](int u) { return PAIRS ? (g_first + 2 * u + 1 < g_end ? g_first + 2 * u + 1 : g_end - 1) : g_first + u; };
 
     f32x16_t acc[FM];
 #pragma unroll
@@ -223,15 +217,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
     // where a stage's codes and its scale (the zero: kCols entries behind) are in LDS
     int c_at[SLICES / 4], q_at;
     auto find_codes = [&](int u, int stage) {
-        const int start = pair_start(PAIRS ? u : u >> 1), g = PAIRS ? start + kg : g_first + u;
+        const int start = slice.pair_start(PAIRS ? u : u >> 1), g = slice.group_of(u, kg);
         const int half = PAIRS ? kg : g - start, slot = (PAIRS ? stage : (u >> 1) & 1) * kCodeBytes;
 #pragma unroll
         for (int s = 0; s < SLICES / 4; ++s) {
             const int chunk = 4 * half + (PAIRS ? 2 * s : 2 * kg) + h;
             c_at[s] = slot + crow * 128 + ((chunk ^ ((crow >> 1) & 7)) << 4);
         }
-        const int gq = g < g_end ? g : g_end - 1, piece = gq >> p.q_log;
-        q_at = (int)((((unsigned)piece & q_slots) * 256 + crow) << q_shift) + (crow_q + gq - q_first(crow_q, piece)) * 2;
+        const int gq = g < g_end ? g : g_end - 1, piece = ring.piece(gq);
+        q_at = (int)((ring.slot(piece) * 256 + crow) << q_shift) + (crow_q + gq - q_first(crow_q, piece)) * 2;
     };
     auto read_codes = [&](u32x4_t *c, float &sc, float &zi, float &rest) {
         sc = lq_bf16_bits_to_f32(*reinterpret_cast<const unsigned short *>(q_ring + q_at));
@@ -274,7 +268,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
         constexpr int S = decltype(si)::value;
         unsigned char *cur = lds + S * A_BYTES, *nxt = lds + ((S + 1) % D) * A_BYTES, *fill = lds + ((S + D - 1) % D) * A_BYTES;
         const int uf = u + D - 1 < units ? u + D - 1 : units - 1;
-        const bool codes_too = PAIRS || !(u & 1), piece = u + D - 1 < units && issue_q(last_group(uf));
+        const bool codes_too = PAIRS || !(u & 1), piece = u + D - 1 < units && issue_q(slice.last_group(uf));
 #pragma unroll
         for (int t = 0; t < SLICES; ++t) {
             const unsigned word_next = t < SLICES - 1 ? cw[(t + 1) >> 2][(t + 1) & 3] : 0u;
@@ -333,13 +327,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
 
     // prologue: stages 0 .. D - 2
     static_assert(D == 3, "the prologue and the loop below name the three stages");
-    issue_q(last_group(0));
+    issue_q(slice.last_group(0));
 #pragma unroll
     for (int i = 0; i < LC; ++i) issue_c(0, code_slot(0, 0), i);
 #pragma unroll
     for (int i = 0; i < LA; ++i) issue_a(0, lds, i);
     const int u1 = units > 1 ? 1 : 0;
-    if (u1) issue_q(last_group(1));
+    if (u1) issue_q(slice.last_group(1));
     if constexpr (PAIRS)
 #pragma unroll
         for (int i = 0; i < LC; ++i) issue_c(u1, code_slot(1, 1), i);
