@@ -23,6 +23,7 @@
 // broadcast, and activation loads are limited to the lanes of live tokens: what a vector load
 // costs here is cache-line look-ups per quad, not bytes.
 #include "lq_common.h"
+#include "lq_gemv_batches.h"
 
 namespace {
 
@@ -45,7 +46,6 @@ __device__ __forceinline__ void permute_x(const u32x4_t &d, unsigned a[4]) {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
 
-constexpr int kUnroll = 4;       // groups per batch (scale/zero batches are 4 x bf16 = 8 bytes)
 constexpr int kXRow = 1024 + 16;  // LDS bytes per staged token row: 4 groups x 256 B, padded against bank conflicts
 // MP = number of token rows staged per wave and batch (>= M). NT = 16-row weight tiles per
 // workgroup: every workgroup stages the activations of its K range again, so with many tokens two
@@ -185,7 +185,6 @@ __global__ __launch_bounds__(64 * WAVES, LOADS >= 2 ? 1 : SPW == 2 ? 4 : SPW > 2
     // codes, and the scales and zeros of a whole batch (loaded by the 16 lanes kq = 0)
     u32x4_t wn[NT][kUnroll];
     u32x2_t sn[NT], zn[NT];
-    constexpr int kCodeLoads = NT * kUnroll + (QS ? 0 : 2 * NT);
     auto scale_row = [&](int j) { return GU ? (j == 0 ? srow : scales2 + (long long)row * G) : srow + (long long)j * 16 * G; };
     auto zero_row = [&](int j) { return GU ? (j == 0 ? zrow : zeros2 + (long long)row * G) : zrow + (long long)j * 16 * G; };
     auto load_scales = [&](int g0, int j) {
@@ -313,32 +312,8 @@ __global__ __launch_bounds__(64 * WAVES, LOADS >= 2 ? 1 : SPW == 2 ? 4 : SPW > 2
             multiply(g0, []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); });
         }
     } else if constexpr (PRE) {
-        int i = 0, g0 = wave * kUnroll;
-        bool more = g0 < G && (SPW == 1 || wave < n_slots);
-        if (more) {
-            load_x(g0);
-            load_codes(g0);
-        }
-        while (more) {
-            const int i_now = i;
-            multiply(g0, [&]() {
-                g0 += n_slots * kUnroll;
-                if (SPW > 1 && g0 >= G) {  // the wave's next partial sum
-                    ++i;
-                    const int s = wave + i * WAVES;
-                    g0 = i < SPW && s < n_slots ? s * kUnroll : G;
-                }
-                more = g0 < G;
-                if (more) {
-                    load_codes(g0);
-                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kCodeLoads) : "memory");  // the staged rows are older
-                } else {
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                }
-            });
-            if (more) load_x(g0);
-            if (SPW > 1 && (!more || i != i_now)) keep(i_now);
-        }
+        gemv_batches_ahead<WAVES, SPW>(wave, n_slots, G, load_x, load_codes, multiply,
+                                       []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }, keep);
     } else {
         for (int i = 0; i < SPW; ++i) {
             const int s = wave + i * WAVES;
