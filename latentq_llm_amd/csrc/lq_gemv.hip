@@ -74,7 +74,7 @@ __global__ __launch_bounds__(64 * WAVES, LOADS >= 2 ? 1 : SPW == 2 ? 4 : SPW > 2
     constexpr bool PRE = LOADS == 2, ONE = LOADS == 3;
     static_assert(!GU || (NT == 2 && !QS), "gate / up mode: two tiles, scales and zeros straight from memory");
     constexpr int RT = GU ? 1 : NT;  // 16-row tiles of output rows per workgroup
-    static_assert(!ONE || SPW == 1, "one batch a wave");
+    static_assert(LOADS < 2 || SPW == 1, "one partial sum a wave");
     static_assert(GU || SPW == 1, "several partial sums per wave: gate / up mode only");
     constexpr int kWaveLds = MP * kXRow > SPW * NT * 1024 ? MP * kXRow : SPW * NT * 1024;
     __shared__ __attribute__((aligned(16))) unsigned char xs_all[WAVES][kWaveLds];
@@ -312,8 +312,7 @@ __global__ __launch_bounds__(64 * WAVES, LOADS >= 2 ? 1 : SPW == 2 ? 4 : SPW > 2
             multiply(g0, []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); });
         }
     } else if constexpr (PRE) {
-        gemv_batches_ahead<WAVES, SPW>(wave, n_slots, G, load_x, load_codes, multiply,
-                                       []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }, keep);
+        gemv_batches_ahead(wave, n_slots, G, load_x, load_codes, multiply, []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); });
     } else {
         for (int i = 0; i < SPW; ++i) {
             const int s = wave + i * WAVES;
@@ -386,11 +385,12 @@ struct GemvGuArgs {
 };
 
 template <int W, int MP, int SPW, int LOADS>
-void launch_gu_loads(const GemvGuArgs &a) {
+bool launch_gu_loads(const GemvGuArgs &a) {
     hipLaunchKernelGGL((gemv_kernel<W, MP, 2, false, true, SPW, LOADS>), dim3(a.N / 16), dim3(64 * W), 0, a.st, (const unsigned short *)a.x,
                        (const unsigned char *)a.codes, a.M, a.N, a.K, a.slots, (const unsigned short *)a.scales, (const unsigned short *)a.zeros,
                        (const unsigned short *)nullptr, (unsigned short *)a.y, (const unsigned char *)a.codes2,
                        (const unsigned short *)a.scales2, (const unsigned short *)a.zeros2);
+    return true;
 }
 
 // How the batches are loaded (LOADS): with one workgroup to a unit registers are free for the next batch's codes; with two they
@@ -399,15 +399,21 @@ void launch_gu_loads(const GemvGuArgs &a) {
 //   4096 x 2048 (c = 1)  2 tokens 5.92 -> 5.47, 12: 6.62 -> 5.97;  4096 x 1792, 8: 6.19 -> 5.46;  3072 x 1024, 16: 5.33 -> 5.01
 //   6144 x 3072 (c = 2)  8: 10.6 -> 9.94, 12: 12.8 -> 11.4, 16: 12.6 -> 11.9;  8192 x 4096, 12: 15.4 -> 13.3, 16: 15.6 -> 14.2
 //   8192 x 2560, 1: 9.2 -> 8.1;  11008 x 4096 (c = 3), 1: 14.2 -> 13.1, 4: 15.1 -> 14.5;  20480 x 8192, 1: 50.1 -> 46.3
+// Only the forms that gu_waves can ask for are there: with c = 1 every partial sum has a wave of its own, as with c = 2 and 8 rows;
+// with more rows or workgroups the waves are as few as the bounds below say. False for any other form.
 template <int W, int MP, int SPW>
-void launch_gu_spw(const GemvGuArgs &a) {
+bool launch_gu_spw(const GemvGuArgs &a) {
     if constexpr (MP == 4) {
-        launch_gu_loads<W, MP, SPW, 1>(a);
+        return launch_gu_loads<W, MP, SPW, 1>(a);
     } else {
         const int c = (a.N / 16 + lq_device_cu_count() - 1) / lq_device_cu_count();
-        if (c == 1) launch_gu_loads<W, MP, SPW, 2>(a);
-        else if (c == 2) launch_gu_loads<W, MP, SPW, 1>(a);
-        else launch_gu_loads<W, MP, SPW, 0>(a);
+        if constexpr (SPW == 1)
+            if (c == 1) return launch_gu_loads<W, MP, SPW, 2>(a);
+        if constexpr (MP == 8 ? SPW == 1 : W <= 4 && SPW <= 2 && W > SPW)
+            if (c == 2) return launch_gu_loads<W, MP, SPW, 1>(a);
+        if constexpr (W <= (MP == 16 ? 3 : MP == 12 ? 4 : 5))
+            if (c > 2) return launch_gu_loads<W, MP, SPW, 0>(a);
+        return false;
     }
 }
 
@@ -415,14 +421,15 @@ void launch_gu_spw(const GemvGuArgs &a) {
 constexpr int gu_max_slots(int MP) { return MP == 4 ? 16 : 8; }
 
 template <int W, int MP>
-void launch_gu(const GemvGuArgs &a) {
+bool launch_gu(const GemvGuArgs &a) {
     constexpr int kMost = (gu_max_slots(MP) + W - 1) / W;
     const int batches = (a.K / LQ_GROUP + kUnroll - 1) / kUnroll, used = batches < a.slots ? batches : a.slots;
     const int spw = (used + W - 1) / W;
     if (spw <= 1) return launch_gu_spw<W, MP, 1>(a);
     if constexpr (kMost >= 2)
         if (spw == 2) return launch_gu_spw<W, MP, 2>(a);
-    if constexpr (MP >= 12 && kMost > 2) launch_gu_spw<W, MP, kMost>(a);
+    if constexpr (MP >= 12 && kMost > 2) return launch_gu_spw<W, MP, kMost>(a);
+    return false;
 }
 
 // Waves per workgroup of the gate / up pass, MP staged rows. A grid of c workgroups per CU should be resident at once: the
@@ -460,19 +467,20 @@ int gu_waves(int MP, int N, int batches, int slots, int cus) {
 }
 
 template <int MP>
-void launch_gu_waves(int w, const GemvGuArgs &a) {
+bool launch_gu_waves(int w, const GemvGuArgs &a) {
     switch (w) {
-        case 2: launch_gu<2, MP>(a); break;
-        case 3: launch_gu<3, MP>(a); break;
-        case 4: launch_gu<4, MP>(a); break;
-        case 5: launch_gu<5, MP>(a); break;
-        case 6: launch_gu<6, MP>(a); break;
-        case 8: launch_gu<8, MP>(a); break;
-        default: if constexpr (MP == 4) launch_gu<16, MP>(a); else launch_gu<8, MP>(a);
+        case 2: return launch_gu<2, MP>(a);
+        case 3: return launch_gu<3, MP>(a);
+        case 4: return launch_gu<4, MP>(a);
+        case 5: return launch_gu<5, MP>(a);
+        case 6: return launch_gu<6, MP>(a);
+        case 8: return launch_gu<8, MP>(a);
+        default: if constexpr (MP == 4) return launch_gu<16, MP>(a); else return launch_gu<8, MP>(a);
     }
 }
 
-template <int W, int MP, int NT>
+// ONE, LOOP: whether pick_waves takes W for so many batches (one each at most) and for more of them; only what can be launched is there.
+template <int W, int MP, int NT, bool ONE, bool LOOP>
 void launch_one(const GemvArgs &a) {
     // Scales and zeros through LDS: pays with many staged tokens when a wave uses them for more than one
     // batch or for two row tiles (measured: 13.5 -> 12.5 us on 11008 x 4096 at 16 tokens; with one batch
@@ -494,16 +502,24 @@ void launch_one(const GemvArgs &a) {
     //   16 waves (4096 x 11008, up to 8 tokens) have no registers for a second batch, 7.7 -> 8.4 with it at 1 token
     //   two row tiles           12 tokens, 11008 x 4096 12.3 -> 11.5
     const size_t qs_lds = 2 * q_bytes + 2 * 16 * NT * 16;
-    const bool pre = W <= 8 && batches > W && a.N / (16 * NT) <= lq_device_cu_count();
-    if (batches <= W) {
-        if (qs) launch(gemv_kernel<W, MP, NT, true, false, 1, 3>, qs_lds);
-        else launch(gemv_kernel<W, MP, NT, false, false, 1, 3>, 0);
-    } else if (pre) {
-        if (qs) launch(gemv_kernel<W, MP, NT, true, false, 1, 2>, qs_lds);
-        else launch(gemv_kernel<W, MP, NT, false, false, 1, 2>, 0);
-    } else {
-        if (qs) launch(gemv_kernel<W, MP, NT, true, false, 1, NT == 2 ? 1 : 0>, qs_lds);
-        else launch(gemv_kernel<W, MP, NT, false, false, 1, NT == 2 ? 1 : 0>, 0);
+    if constexpr (ONE) {
+        if (batches <= W) {
+            if constexpr (NT == 2)
+                if (qs) return launch(gemv_kernel<W, MP, NT, true, false, 1, 3>, qs_lds);
+            return launch(gemv_kernel<W, MP, NT, false, false, 1, 3>, 0);
+        }
+    }
+    if constexpr (LOOP) {
+        if constexpr (W <= 8) {
+            if (a.N / (16 * NT) <= lq_device_cu_count()) {
+                if constexpr (MP == 16)
+                    if (qs) return launch(gemv_kernel<W, MP, NT, true, false, 1, 2>, qs_lds);
+                return launch(gemv_kernel<W, MP, NT, false, false, 1, 2>, 0);
+            }
+        }
+        if constexpr (MP == 16)
+            if (qs) return launch(gemv_kernel<W, MP, NT, true, false, 1, NT == 2 ? 1 : 0>, qs_lds);
+        launch(gemv_kernel<W, MP, NT, false, false, 1, NT == 2 ? 1 : 0>, 0);
     }
 }
 
@@ -516,14 +532,15 @@ int pick_waves(int batches, int max_waves) {
     return w;
 }
 
+// As many waves as pick_waves finds for a cap of MAXW (8 rows: of 8 up to 16 batches, of 16 beyond)
 template <int MP, int NT, int MAXW>
-void launch_waves(int w, const GemvArgs &a) {
-    switch (w) {
-        case 2: launch_one<2, MP, NT>(a); break;
-        case 4: launch_one<4, MP, NT>(a); break;
-        case 8: if constexpr (MAXW >= 8) launch_one<8, MP, NT>(a); break;
-        default: launch_one<MAXW, MP, NT>(a); break;
-    }
+void launch_waves(const GemvArgs &a, int batches) {
+    const int w = pick_waves(batches, MP == 8 && batches <= 16 ? 8 : MAXW);
+    if (w == 2) return launch_one<2, MP, NT, true, false>(a);
+    if (w == 4) return launch_one<4, MP, NT, true, MAXW == 4>(a);
+    if constexpr (MAXW >= 8)
+        if (w == 8) return launch_one<8, MP, NT, true, MAXW == 8 || MP == 8>(a);
+    if constexpr (MAXW == 16) launch_one<16, MP, NT, MP != 8, true>(a);
 }
 
 }  // namespace
@@ -535,22 +552,22 @@ int lq_gemv_a16w4_launch(const void *x, const void *codes, const void *scales, c
     const int batches = (K / LQ_GROUP + 3) / 4;  // one batch of 4 groups per wave when possible: all of a
                                                  // wave's loads are then in flight at once
     if (M <= 4) {
-        launch_waves<4, 1, 16>(pick_waves(batches, 16), a);
+        launch_waves<4, 1, 16>(a, batches);
     } else if (M <= 8) {
         // 8 staged token rows (8.1 KB of LDS per wave): 8 waves with one 16-row tile, 16 when K has more than 16
         // batches (measured on 11008 x 4096 / 4096 x 11008 / 8192^2 at 8 tokens: 11.1 / 10.9 / 14.9 us against
         // 12.1 / 11.8 / 18.5 with 16 staged rows and the two-tile workgroups below)
-        launch_waves<8, 1, 16>(pick_waves(batches, batches > 16 ? 16 : 8), a);
+        launch_waves<8, 1, 16>(a, batches);
     } else if (N % 32 == 0 && N >= 32 * 256) {
         // many tokens and enough rows for one 32-row workgroup per CU: half the activation traffic;
         // 4 waves = 65 KB of staged activations: two workgroups per CU, all of them resident at once
-        launch_waves<16, 2, 4>(pick_waves(batches, 4), a);
+        launch_waves<16, 2, 4>(a, batches);
     } else if (M <= 12 && batches > 8) {
         // (11.4 -> 10.8 us on 4096 x 11008 at 12 tokens, 8.6 -> 7.8 on 2560 x 8192: the loads of four dead rows)
-        launch_waves<12, 1, 8>(8, a);
+        launch_one<8, 12, 1, false, true>(a);
     } else {
         // 16 staged token rows cost a wave 16.25 KB of LDS, which caps the workgroup at 8 waves
-        launch_waves<16, 1, 8>(pick_waves(batches, 8), a);
+        launch_waves<16, 1, 8>(a, batches);
     }
     return lq_check_launch("lq_a16w4_fwd(gemv)");
 }
@@ -565,9 +582,8 @@ int lq_gemv_a16w4_gate_up_launch(const void *x, const void *codes_g, const void 
     const int slots = pick_waves(batches, gu_max_slots(mp));
     const GemvGuArgs a = {x, codes_g, scales_g, zeros_g, codes_u, scales_u, zeros_u, h, M, N, K, slots, st};
     const int w = gu_waves(mp, N, batches, slots, cus);
-    if (mp == 4) launch_gu_waves<4>(w, a);
-    else if (mp == 8) launch_gu_waves<8>(w, a);
-    else if (mp == 12) launch_gu_waves<12>(w, a);
-    else launch_gu_waves<16>(w, a);
+    const bool there = mp == 4 ? launch_gu_waves<4>(w, a) : mp == 8 ? launch_gu_waves<8>(w, a)
+                       : mp == 12 ? launch_gu_waves<12>(w, a) : launch_gu_waves<16>(w, a);
+    if (!there) return lq_fail(LQ_ERR_BAD_ARG, "lq_a16w4_gate_up_silu(gemv): no kernel of %d waves and %d rows", w, mp);
     return lq_check_launch("lq_a16w4_gate_up_silu(gemv)");
 }

@@ -12,14 +12,13 @@ struct Load {
     int g0;
 };
 
-template <int WAVES, int SPW>
-void walk(int wave, int slots, int G, int M, int NT, bool qs) {
+static void walk(int wave, int waves, int G, int M, int NT, bool qs) {
     std::deque<Load> flying;
     int rows = -1, codes = -1;  // the batch whose rows / codes were requested last
     bool reading = false;
-    std::vector<int> seen, kept;
+    std::vector<int> seen, want;
     auto fail = [&](const char *what, int g0) {
-        printf("%s: wave %d of %d, %d slots, %d groups, %d rows, %d tiles, group %d\n", what, wave, WAVES, slots, G, M, NT, g0);
+        printf("%s: wave %d of %d, %d groups, %d rows, %d tiles, group %d\n", what, wave, waves, G, M, NT, g0);
         exit(1);
     };
     auto load_x = [&](int g0) {
@@ -45,34 +44,18 @@ void walk(int wave, int slots, int G, int M, int NT, bool qs) {
         reading = false;
         seen.push_back(g0);
     };
-    gemv_batches_ahead<WAVES, SPW>(wave, slots, G, load_x, load_codes, multiply, [&]() { flying.clear(); }, [&](int i) {
-        if (i != (int)kept.size()) fail("partial sums out of order", i);
-        kept.push_back((int)seen.size());
-    });
-    std::vector<int> want, ends;
-    for (int i = 0; i < SPW && wave + i * WAVES < slots; ++i) {
-        for (int g0 = (wave + i * WAVES) * kUnroll; g0 < G; g0 += slots * kUnroll) want.push_back(g0);
-        if (SPW > 1 && (int)want.size() > (ends.empty() ? 0 : ends.back())) ends.push_back((int)want.size());
-    }
+    gemv_batches_ahead(wave, waves, G, load_x, load_codes, multiply, [&]() { flying.clear(); });
+    for (int g0 = wave * kUnroll; g0 < G; g0 += waves * kUnroll) want.push_back(g0);
     if (seen != want) fail("not the wave's batches", -1);
-    if (kept != ends) fail("partial sums cut elsewhere", -1);
     if (!flying.empty()) fail("loads in flight at the end", -1);
 }
 
-template <int WAVES, int SPW>
-void all(int slots) {
-    for (int G = 1; G < 90; ++G)
-        for (int wave = 0; wave < WAVES; ++wave)
-            for (int M : {1, 5, 8, 9, 12, 16})
-                for (int NT : {1, 2})
-                    for (bool qs : {false, true}) walk<WAVES, SPW>(wave, slots, G, M, NT, qs);
-}
-
 int main() {
-    all<2, 1>(2);
-    all<4, 1>(4);
-    all<8, 1>(8);
-    all<4, 2>(8);
-    all<3, 3>(8);
+    for (int waves = 2; waves <= 8; ++waves)
+        for (int wave = 0; wave < waves; ++wave)
+            for (int G = 1; G < 90; ++G)
+                for (int M : {1, 5, 8, 9, 12, 16})
+                    for (int NT : {1, 2})
+                        for (bool qs : {false, true}) walk(wave, waves, G, M, NT, qs);
     printf("ok\n");
 }

@@ -44,3 +44,21 @@ def test_rows_do_not_depend_on_how_many_there_are(N, K):
     for M in (1, 3, 4, 5, 8, 9, 12, 13, 16):
         x = randn_bf16((M, K), M).cuda()
         assert torch.equal(ops.a16w4_gate_up_silu(x, *mats, (N, K))[:, rows], ops.a16w4_gate_up_silu(x, *few, (16, K))), M
+
+
+@pytest.mark.parametrize("K", [512 * b - 128 * (b % 3) for b in range(1, 13)] + [8704])
+def test_every_form_has_a_kernel(K):
+    """One to five workgroups to a unit on one to twelve batches of 512 k, and seventeen: the forms the launcher has to have. Rows
+    have the bits they have in the smallest matrix, which the other tests compare with a reference."""
+    from latentq_llm_amd import ops
+    N = 16400
+    mats = []
+    for seed in (1, 2):
+        _, p, s, z = make_w4(N, K, seed)
+        mats.append((p.cuda(), s.cuda(), z.cuda()))
+    for M in (4, 8, 12, 16):
+        x = randn_bf16((M, K), M).cuda()
+        h = {n: ops.a16w4_gate_up_silu(x, *[(p[:n * K // 2], s[:n * K // 128], z[:n * K // 128]) for p, s, z in mats], (n, K))
+             for n in (16, 4096, 8192, 12288, 16384, N)}
+        for n, y in h.items():
+            assert torch.equal(y, h[N][:, :n]) and torch.equal(y[:, :16], h[16]), (M, n)
