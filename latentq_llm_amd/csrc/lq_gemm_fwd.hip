@@ -51,6 +51,7 @@
 // what the loop does besides MFMAs costs throughput even where it overlaps them in time: the forms of the loads
 // above are chosen to keep the bytes moved between L2 and the CU near the bytes used.
 #include "lq_common.h"
+#include "lq_fwd_k_groups.h"
 
 #include <type_traits>
 
@@ -93,13 +94,9 @@ constexpr int STAGE = BM * ROWB;     // 16 KB per A stage
 // KS: groups of four waves that share the tile and each take a part of K (1 or 2). A workgroup alone on its compute unit has
 // one wave per SIMD, and such a wave issues its MFMAs, conversions and LDS reads one behind the other (0.61 us per step where
 // the MFMAs take 0.25). Two groups on stages of their own fill each other's gaps; their sums meet in LDS at the end.
-// us with one group -> two, weights from HBM:
-//   128 x 128 tiles  1019 tokens, 4096 x 4096 46.7 -> 37.1, 800: 46.6 -> 35.2; 256 tokens, 11008 x 4096 46.3 -> 35.7;
-//                    1024 tokens, 3072 x 768 10.2 -> 10.1
-//   128 x 256 tiles  1536 tokens, 4096 x 4096 56.0 -> 53.3, 2048 tokens, 4096 x 11008 160.4 -> 156.8 (256 workgroups: the
-//                    power limit); gate / up 256 tokens, 11008 x 4096 57.8 -> 54.2
-// Where units get several workgroups, these fill the gaps already, and a workgroup twice as large is slower (2048 tokens,
-// 11008 x 4096 156.3 against 163.8). Three groups: 37.9 on the first size, 92.2 against 95.2 on 1019 tokens, 4096 x 11008.
+// (1000 tokens, 4096 x 4096 40.8 -> 36.9 us; the sizes where that pays: lq_fwd_k_groups.h). Where units get several workgroups, these
+// fill the gaps already, and a workgroup twice as large is slower (2048 tokens, 11008 x 4096 156.3 against 163.8). Three groups are
+// no faster on that size (37.9 where two took 37.1) and 3 % on 1019 tokens, 4096 x 11008 (92.2 against 95.2).
 template <int NT, bool GU, int KS>
 __global__ __launch_bounds__(256 * KS, 2) void gemm_fwd_direct_kernel(FwdParams p) {
     static_assert(NT == 2 || (NT == 1 && !GU), "gate / up mode uses both column tiles");
@@ -554,8 +551,7 @@ static int launch_direct(FwdParams p, hipStream_t st, const char *who) {
     if (nwg > 0x7FFFFFFFll) return lq_fail(LQ_ERR_BAD_ARG, "%s: problem too large", who);
     // the 32-bit lane offsets of the activation and weight loads span 128 / 256 rows
     if ((long long)BN * p.K * 2 >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: K too large", who);
-    // Two groups of waves per workgroup where no compute unit gets a second workgroup, and each group has at least 4 steps.
-    if (nwg <= lq_device_cu_count() && p.K >= 512)
+    if (fwd_k_groups(GU ? FWD_GATE_UP : NT == 1 ? FWD_128x128 : FWD_128x256, nwg, lq_device_cu_count(), p.K) == 2)
         hipLaunchKernelGGL((gemm_fwd_direct_kernel<NT, GU, 2>), dim3((unsigned)nwg), dim3(512), 0, st, p);
     else
         hipLaunchKernelGGL((gemm_fwd_direct_kernel<NT, GU, 1>), dim3((unsigned)nwg), dim3(256), 0, st, p);

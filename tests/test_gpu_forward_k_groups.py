@@ -1,5 +1,6 @@
-"""The weights-direct forward kernels with two groups of waves per workgroup, each on its part of K (grids of at most one
-workgroup per compute unit): equal and unequal parts, the shortest K and the one below it, ragged rows and columns, all tiles."""
+"""The weights-direct forward kernels on grids of at most one workgroup per compute unit, with two groups of waves per workgroup,
+each on its part of K, where K is long enough: equal and unequal parts, the shortest K and the one below it, ragged rows and
+columns, all tiles."""
 import pytest
 import torch
 
@@ -15,7 +16,9 @@ TOL = 2.0 ** -8
 @pytest.mark.parametrize("M,N,K,kernel", [(200, 11008, 256, "direct_128x128"), (200, 11008, 512, "direct_128x128"),
                                           (255, 11024, 768, "direct_128x128"), (1000, 4096, 1280, "direct_128x128"),
                                           (513, 4112, 3328, "direct_128x128"), (129, 9008, 7936, "direct_128x128"),
-                                          (1900, 4112, 512, "direct_128x256"), (1537, 4096, 1792, "direct_128x256")])
+                                          (1900, 4112, 512, "direct_128x256"), (1537, 4096, 1792, "direct_128x256"),
+                                          (1000, 4096, 1024, "direct_128x128"), (1000, 4096, 768, "direct_128x128"),
+                                          (1900, 4112, 1536, "direct_128x256"), (1900, 4112, 1280, "direct_128x256")])
 def test_forward(hip_lib, M, N, K, kernel):
     from latentq_llm_amd import ops
     assert ops.a16w4_plan(M, (N, K))[0] == kernel
@@ -36,7 +39,7 @@ def test_forward(hip_lib, M, N, K, kernel):
     assert torch.equal(ops.a16w4_forward(eye, *w, (N, K)).double(), W[:, pick].t())
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 5504, 768), (97, 11024, 512)])
+@pytest.mark.parametrize("M,N,K", [(300, 5504, 768), (97, 11024, 512), (257, 5520, 2816), (257, 5520, 3072), (200, 11008, 3328), (513, 6160, 4096), (500, 8192, 3840)])
 def test_gate_up(hip_lib, M, N, K):
     from latentq_llm_amd import ops
     mats = [tuple(t.cuda() for t in make_w4(N, K, s)[1:]) for s in (1, 2)]
