@@ -59,3 +59,15 @@ def test_forward_quantises_as_the_separate_passes(M, N, K, per_token, special):
         want = ops.a8w8_forward(x8, w8, sx, qs, b)
         assert torch.equal(ops.infer8(x, w8, qs, b, per_token).view(torch.int16), want.view(torch.int16))
         assert torch.equal(ops.infer8(x.view(1, M, K), w8, qs, b, per_token).view(M, N).view(torch.int16), want.view(torch.int16))
+
+
+# a row of exactly one and two steps of 256 pieces, one piece of 16 beyond, half a step; each number of pieces a thread holds
+@pytest.mark.parametrize("M,K", [(3, 2048), (5, 2176), (10, 4096), (12, 4224), (3, 1024), (13, 2560), (5, 8192), (16, 2048)])
+def test_rows_in_steps(M, K):
+    from latentq_llm_amd import ops
+    w8, qs, bias = operands(48, K, M + K)
+    x = randn_bf16((M, K), M).cuda()
+    for row, at in ((0, K - 1), (M - 1, 0), (M // 2, K // 2)):  # the largest in the last, the first and a middle piece
+        x[row, at] = 9.0 + row
+    x8, sx = ops.act_quant_i8_per_token(x)
+    assert torch.equal(ops.infer8(x, w8, qs, bias, True), ops.a8w8_forward(x8, w8, sx, qs, bias))
