@@ -833,16 +833,15 @@ struct W4Plan {
 //                                      a time, rows must be 4-byte aligned): the staged kernel up to one tile per unit,
 //                                      beyond that the kernel with weight waves and 256 x 128 tiles (4224 x 4096:
 //                                      40 against 48 us at T = 256, 70 against 66 at 384)
+//   T <= units, K >= 8192              the staged kernel's 128-row tiles, whole (4096 x 11008: 79.0 against 86.9 us at
+//                                      T = 192, 95.6 against 98.5 at 256); for shorter K the difference is small (0 to
+//                                      4 us) and the weights-direct kernel keeps them
 //   else                               one of the two weights-direct kernels, by rough time per 64-deep step
 //                                      (microseconds, measured): 128 x 256 tiles take ~0.86 with one workgroup on a
 //                                      compute unit and ~1.45 for two sharing it. The kernel with 128 x 128 tiles fits
 //                                      three workgroups on a unit: ~0.55-0.61 alone (the more units are busy, the lower
 //                                      the clock: 0.55 up to three quarters of them, 0.61 with all), ~0.74 as soon as a
 //                                      few units hold two, ~1.23 for two everywhere, ~1.38 for three.
-//                                      (K of 8192 and more with T <= units: the staged kernel's whole tiles, which took
-//                                      these while the weights-direct ones had one group of waves, are 2 to 11 % behind:
-//                                      4096 x 11008 84.6 against 79.6 us at T = 160, 101 against 92.3 at 256, 8192 x 8192
-//                                      78.4 against 73.7 at 256; level on 11008 x 8192 at 172)
 // Up to 32 tokens two GEMV launches of 16 are a little faster where a launch does not wait for the matrix' bytes
 // and K is not long (2048 x 2048: 7.4 / 8.1 us at 17 / 32 tokens against 8.6 / 9.0; 1024 x 4096 9.1 / 10.3 against 9.7 / 10.2); at
 // 11008 x 4096 they take 21.0 / 23.4 us against 18.1 / 17.7, at 1536 x 8192 14.4 / 17.0 against 13.1 / 13.7.
@@ -873,7 +872,7 @@ static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, l
         if (out.exact && out.rows == 128) out.rows = 64;
         return out;
     }
-    if (tiles <= cus && groups % 2 != 0) return out;  // whole, 128 rows
+    if (tiles <= cus && (groups % 2 != 0 || K >= 8192)) return out;  // whole, 128 rows
     if (groups % 2 != 0) {
         out.kernel = LQ_PLAN_STAGED_256;
         return out;
