@@ -7,7 +7,8 @@
 //   * codes stay packed in LDS and each wave converts the 32 columns it multiplies, in registers: no second trip through LDS
 //     and no waves that only convert;
 //   * eight waves, two for each 32 columns, that work on different k and add up at the end: a wave alone on its SIMD issues
-//     its MFMAs, conversions and LDS reads one behind the other;
+//     its MFMAs, conversions and LDS reads one behind the other (128 rows and a long slice of K: four, see
+//     gemm_staged_long_kernel);
 //   * whole cache lines: what a unit takes in through L1 (30 bytes a clock with all units asking) counts in lines of 128
 //     bytes. Codes come in pieces of 128 bytes of a row, two groups of 128 k; scales and zeros 16 bytes at a time;
 //   * a plain product of up to 64 tokens (128 without a workspace) does not round its weights to bf16, since the GEMV, which
@@ -22,8 +23,8 @@
 // MFMAs with 128 (one 16-byte fragment read per MFMA).
 // Measured, weights from HBM, us: before (four waves, a group of 128 k per stage, a 2-byte scale load per column and group, a
 // second launch for h) -> now
-//     plain N x K     17 tokens       45              64              100            384            768
-//     4096 x 11008    16.9 -> 16.4    19.4 -> 18.7    20.0 -> 19.2    24.2 -> 24.2                   96.8 -> 91-95
+//     plain N x K     17 tokens       45              64              100            384
+//     4096 x 11008    16.9 -> 16.4    19.4 -> 18.7    20.0 -> 19.2    24.2 -> 24.2
 //     4096 x 4096                                                                    26.0 -> 23.6
 //     11008 x 4096                    21.0 -> 18.6
 //     32000 x 4096    26.2 -> 22.8 (32 tokens)        32.4 -> 27.9 (60)
@@ -422,6 +423,215 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
     }
 }
 
+// Long slices of K in 128-row tiles: four waves of 32 columns, a group of 128 k per stage, codes in pieces of 64 bytes, scales
+// and zeros 2 bytes at a time. Once a loop runs long the kernel above is the slower one: its two waves on a column block wait
+// for each other at every barrier without filling each other's gaps, since LDS reads beside MFMAs fill them already; and where
+// rows are an odd number of groups, or a slice begins at an odd one, its 128-byte pieces of codes lie across two cache lines. us,
+// weights from HBM, eight waves -> four:
+//   in one line  4096 x 11008 at 1019 tokens 100.3 -> 97.8, 2560 x 8192 at 1500 72.4 -> 70.8
+//   across two   3840 x 9088 at 632 69.7 -> 64.5, 2816 x 10880 at 876 81.8 -> 72.8; two slices: 3840 x 11008 at 370 54.6 -> 51.1,
+//                6272 x 7936 at 245 43.8 -> 39.4
+// LDS of a stage, swizzled like the one above:
+//   activations  128 rows of 256 bytes, chunk c of row i at c ^ (i & 15)
+//   codes        128 rows of 64 bytes,  chunk c of row i at c ^ ((i >> 2) & 3)
+//   scales, zeros  one dword per column each, the bf16 value in its lower half
+constexpr int kLongThreads = 256;
+__global__ __launch_bounds__(kLongThreads) void gemm_staged_long_kernel(StagedParams p) {
+    constexpr int FM = 4, BM = 32 * FM, A_BYTES = BM * 256, C_BYTES = kCols * 64, STAGE = A_BYTES + C_BYTES + kCols * 8;
+    constexpr int LA = A_BYTES / 16 / kLongThreads, LC = C_BYTES / 16 / kLongThreads;
+    constexpr int LOADS = LA + LC + 1;  // per thread and stage: activations, codes, one scale or zero
+    __shared__ __attribute__((aligned(16))) unsigned char lds[D * STAGE];
+
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    unsigned long long clk_t0 = 0, clk_r0 = 0;
+    if (p.clk) {
+        clk_t0 = __builtin_amdgcn_s_memtime();
+        clk_r0 = __builtin_amdgcn_s_memrealtime();
+    }
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
+
+    const int nwg = p.tiles_m * p.tiles_n;
+    int id = blockIdx.x;
+    {
+        const int per = nwg / 8;
+        if (id < per * 8) id = (id % 8) * per + id / 8;
+    }
+    const int tile_m = id % p.tiles_m, tile_n = id / p.tiles_m;
+    const int m0 = tile_m * BM, c0 = tile_n * kCols;
+    const int G = p.K / LQ_GROUP;
+    const int g0 = p.partial ? (int)blockIdx.y * p.groups_per_split : 0;
+    const int g1 = p.partial && g0 + p.groups_per_split < G ? g0 + p.groups_per_split : G;
+    const int ng = g1 - g0;
+
+    // ---- loads
+    unsigned a_off[LA], c_off[LC];
+    const unsigned lda = (unsigned)p.K * 2u, ldw = (unsigned)p.K / 2u;
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+        const int s = i * kLongThreads + tid, row = s >> 4, chunk = (s & 15) ^ (row & 15);
+        a_off[i] = (unsigned)((m0 + row < p.M ? m0 + row : p.M - 1) - m0) * lda + chunk * 16;
+    }
+    auto tile_row = [&](int row) { return (unsigned)(c0 + row < p.N ? row : p.N - 1 - c0); };
+#pragma unroll
+    for (int i = 0; i < LC; ++i) {
+        const int s = i * kLongThreads + tid, row = s >> 2, chunk = (s & 3) ^ ((row >> 2) & 3);
+        c_off[i] = tile_row(row) * ldw + chunk * 16;
+    }
+    const unsigned q_off = tile_row(tid & 127) * (unsigned)G * 2u;
+    const unsigned char *a_base = p.x + (long long)m0 * lda, *c_base = p.w + (long long)c0 * ldw;
+    const unsigned char *q_base = (const unsigned char *)((wave < 2 ? p.scales : p.zeros) + (long long)c0 * G);
+    auto to_lds16 = [&](unsigned char *dst, unsigned off, const unsigned char *src) {
+        const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)dst);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(src) : "memory");
+    };
+    auto issue = [&](int g, unsigned char *st, int i) {
+        if (i < LA) {
+            to_lds16(st + (i * kLongThreads + wave * 64) * 16, a_off[i < LA ? i : 0], a_base + (long long)g * 256);
+        } else if (i < LA + LC) {
+            to_lds16(st + A_BYTES + ((i - LA) * kLongThreads + wave * 64) * 16, c_off[i - LA < LC ? i - LA : 0], c_base + (long long)g * 64);
+        } else {
+            const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(st + A_BYTES + C_BYTES + wave * 256));
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" ::"s"(lds_addr), "v"(q_off), "s"(q_base + (long long)g * 2) : "memory");
+        }
+    };
+
+    f32x16_t acc[FM];
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc[j][q] = 0.f;
+
+    // ---- operands: slice t = 0..7 of a group: step t / 4 (64 k), the lane's 8 k at 64 (t / 4) + 32 h + 8 (t % 4)
+    auto read_a = [&](const unsigned char *st, int t, u32x4_t *af) {
+        const int chunk = (t >> 2) * 8 + 4 * h + (t & 3);
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+            af[j] = *reinterpret_cast<const u32x4_t *>(st + (32 * j + r) * 256 + ((chunk ^ (r & 15)) << 4));
+    };
+    const int crow = 32 * wave + r;
+    auto read_codes = [&](const unsigned char *st, u32x4_t *c, float &sc, float &zs) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            c[s] = *reinterpret_cast<const u32x4_t *>(st + A_BYTES + crow * 64 + (((2 * s + h) ^ ((crow >> 2) & 3)) << 4));
+        const unsigned *q = reinterpret_cast<const unsigned *>(st + A_BYTES + C_BYTES);
+        sc = __uint_as_float(q[crow] << 16);
+        zs = -(__uint_as_float(q[kCols + crow] << 16) * sc);  // operands of lq_dequant_word_f32
+        sc *= 512.0f;
+    };
+    auto operand = [](unsigned word, float sc, float zs) {
+        float f[8];
+        lq_dequant_word_f32(word, sc, zs, f);
+        return u32x4_t{lq_pack_bf16(f[0], f[1]), lq_pack_bf16(f[2], f[3]), lq_pack_bf16(f[4], f[5]), lq_pack_bf16(f[6], f[7])};
+    };
+
+    u32x4_t af[2][FM], bf[2], cw[2];
+    float sc, zs;
+    auto group = [&](int g, auto si) {
+        constexpr int S = decltype(si)::value;
+        unsigned char *cur = lds + S * STAGE, *nxt = lds + ((S + 1) % D) * STAGE, *fill = lds + ((S + D - 1) % D) * STAGE;
+        const int gf = g0 + (g + D - 1 < ng ? g + D - 1 : ng - 1);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const unsigned word_next = t < 7 ? cw[(t + 1) >> 2][(t + 1) & 3] : 0u;
+            if (t == 7) {
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 2) * LOADS) : "memory");
+                read_codes(nxt, cw, sc, zs);
+                read_a(nxt, 0, af[0]);
+            } else {
+                read_a(cur, t + 1, af[(t + 1) & 1]);
+                // the loads of the stage the previous group left, spread over the slices
+#pragma unroll
+                for (int i = 0; i < LOADS; ++i)
+                    if (i * 7 / LOADS == t) issue(gf, fill, i);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < FM; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, af[t & 1][j]),
+                                                                 __builtin_bit_cast(bf16x8_t, bf[t & 1]), acc[j], 0, 0, 0);
+            bf[(t + 1) & 1] = operand(t < 7 ? word_next : cw[0][0], sc, zs);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    // prologue: groups 0 .. D - 2
+    static_assert(D == 3, "the loop below names the three stages");
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue(g0 + (d < ng ? d : ng - 1), lds + d * STAGE, i);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 2) * LOADS) : "memory");
+    read_codes(lds, cw, sc, zs);
+    read_a(lds, 0, af[0]);
+    bf[0] = operand(cw[0][0], sc, zs);
+    __builtin_amdgcn_sched_barrier(0);
+    int g = 0;
+    for (; g + D <= ng; g += D) {
+        group(g, ic<0>());
+        group(g + 1, ic<1>());
+        group(g + 2, ic<2>());
+    }
+    if (g < ng) group(g, ic<0>());
+    if (g + 1 < ng) group(g + 1, ic<1>());
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped prefetches of the last groups
+
+    // ---- epilogue: acc[j][q]: row m0 + 32 j + 8 (q / 4) + 4 h + q % 4, column c0 + 32 wave + r
+    const int c_mine = c0 + 32 * wave + r;
+    if (p.partial) {
+        float *part = p.partial + (long long)blockIdx.y * p.M * p.N;
+        if (c_mine < p.N) {
+#pragma unroll
+            for (int j = 0; j < FM; ++j)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const int m = m0 + 32 * j + 8 * (q >> 2) + 4 * h + (q & 3);
+                    if (m < p.M) part[(long long)m * p.N + c_mine] = acc[j][q];
+                }
+        }
+        return;
+    }
+    __syncthreads();
+    constexpr int EP = 80;  // row pitch of the wave's 32 x 32 staging area
+    unsigned char *ep = lds + wave * (32 * EP);
+    const int ep_row = lane >> 2, ep_chunk = lane & 3;
+    const int c_lane = c0 + 32 * wave + ep_chunk * 8;
+    const float bias = p.bias && c_mine < p.N ? lq_bf16_bits_to_f32(p.bias[c_mine]) : 0.0f;
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            *reinterpret_cast<unsigned short *>(ep + (8 * (q >> 2) + 4 * h + (q & 3)) * EP + r * 2) =
+                lq_f32_to_bf16_bits(p.bias ? acc[j][q] + bias : acc[j][q]);
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+            const int row = it * 16 + ep_row, m = m0 + 32 * j + row;
+            const u32x4_t o = *reinterpret_cast<const u32x4_t *>(ep + row * EP + ep_chunk * 16);
+            if (m < p.M && c_lane < p.N) *reinterpret_cast<u32x4_t *>(p.y + (long long)m * p.N + c_lane) = o;
+        }
+    }
+    if (p.clk && threadIdx.x == 0) {
+        unsigned long long *c = p.clk + 4ll * blockIdx.x;
+        c[0] = clk_t0; c[1] = __builtin_amdgcn_s_memtime(); c[2] = clk_r0; c[3] = __builtin_amdgcn_s_memrealtime();
+    }
+}
+
+// Which kernel takes a slice of so many groups in 128-row tiles: four waves where it is long, and sooner where the other kernel's
+// pieces of codes, two groups, lie across cache lines (rows of an odd number of groups; slices that begin at an odd one). Speed of
+// four waves over eight, medians over 2330 sizes (1024 to 8192 columns, 65 to 2048 tokens, every slice the planner cuts):
+//     groups of the slice   6-17   18-29  30-41  42-49  50-59  60-71  72-95  96-
+//     pieces in one line    0.964  0.968  0.978  0.985  0.98   1.014  1.022  1.025
+//     across two            0.985  1.000  1.013  1.019  1.04   1.055  1.076  1.10
+constexpr bool staged_long(int groups_of_row, int groups_of_slice) {
+    return groups_of_slice >= (groups_of_row % 2 || (groups_of_slice < groups_of_row && groups_of_slice % 2) ? 30 : 60);
+}
+
+int launch_staged_long(StagedParams p, int splits, hipStream_t st, const char *who) {
+    p.tiles_m = (p.M + 127) / 128;
+    p.tiles_n = (p.N + kCols - 1) / kCols;
+    hipLaunchKernelGGL(gemm_staged_long_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits), dim3(kLongThreads), 0, st, p);
+    return lq_check_launch(who);
+}
+
 template <int FM, bool EXACT, bool GU>
 int launch_staged_tile(StagedParams p, int splits, hipStream_t st, const char *who) {
     const int cols = GU ? kCols / 2 : kCols;
@@ -442,6 +652,7 @@ int launch_staged(const StagedParams &p, int rows, bool exact, int splits, hipSt
                             : launch_staged_tile<4, false, true>(p, 1, st, who);
     if (rows == 32) return exact ? launch_staged_tile<1, true, false>(p, splits, st, who) : launch_staged_tile<1, false, false>(p, splits, st, who);
     if (rows == 64) return exact ? launch_staged_tile<2, true, false>(p, splits, st, who) : launch_staged_tile<2, false, false>(p, splits, st, who);
+    if (!p.w2 && staged_long(p.K / LQ_GROUP, p.partial ? p.groups_per_split : p.K / LQ_GROUP)) return launch_staged_long(p, splits, st, who);
     return launch_staged_tile<4, false, false>(p, splits, st, who);
 }
 
