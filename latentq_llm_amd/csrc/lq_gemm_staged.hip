@@ -7,8 +7,8 @@
 //   * codes stay packed in LDS and each wave converts the 32 columns it multiplies, in registers: no second trip through LDS
 //     and no waves that only convert;
 //   * eight waves, two for each 32 columns, that work on different k and add up at the end: a wave alone on its SIMD issues
-//     its MFMAs, conversions and LDS reads one behind the other (128 rows and a long slice of K: four, see
-//     gemm_staged_long_kernel);
+//     its MFMAs, conversions and LDS reads one behind the other (128 rows and a long slice of K, or
+//     rows of an odd number of groups: four, see gemm_staged_four_kernel);
 //   * whole cache lines: what a unit takes in through L1 (30 bytes a clock with all units asking) counts in lines of 128
 //     bytes. Codes come in pieces of 128 bytes of a row, two groups of 128 k; scales and zeros 16 bytes at a time;
 //   * a plain product of up to 64 tokens (128 without a workspace) does not round its weights to bf16, since the GEMV, which
@@ -423,22 +423,22 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_staged_kernel(
     }
 }
 
-// Long slices of K in 128-row tiles: four waves of 32 columns, a group of 128 k per stage, codes in pieces of 64 bytes, scales
-// and zeros 2 bytes at a time. Once a loop runs long the kernel above is the slower one: its two waves on a column block wait
+// 128-row tiles on four waves of 32 columns, a group of 128 k per stage, codes in pieces of 64 bytes, scales
+// and zeros 2 bytes at a time. Where the loop is long the kernel above is the slower one: its two waves on a column block wait
 // for each other at every barrier without filling each other's gaps, since LDS reads beside MFMAs fill them already; and where
 // rows are an odd number of groups, or a slice begins at an odd one, its 128-byte pieces of codes lie across two cache lines. us,
 // weights from HBM, eight waves -> four:
 //   in one line  4096 x 11008 at 1019 tokens 100.3 -> 97.8, 2560 x 8192 at 1500 72.4 -> 70.8
-//   across two   3840 x 9088 at 632 69.7 -> 64.5, 2816 x 10880 at 876 81.8 -> 72.8; two slices: 3840 x 11008 at 370 54.6 -> 51.1,
+//   across two   3840 x 9088 at 632 69.7 -> 64.5, 2816 x 10880 at 876 81.8 -> 72.8, 7808 x 1408 at 336 14.7 -> 14.0; two slices: 3840 x 11008 at 370 54.6 -> 51.1,
 //                6272 x 7936 at 245 43.8 -> 39.4
 // LDS of a stage, swizzled like the one above:
 //   activations  128 rows of 256 bytes, chunk c of row i at c ^ (i & 15)
 //   codes        128 rows of 64 bytes,  chunk c of row i at c ^ ((i >> 2) & 3)
 //   scales, zeros  one dword per column each, the bf16 value in its lower half
-constexpr int kLongThreads = 256;
-__global__ __launch_bounds__(kLongThreads) void gemm_staged_long_kernel(StagedParams p) {
+constexpr int kFourThreads = 256;
+__global__ __launch_bounds__(kFourThreads) void gemm_staged_four_kernel(StagedParams p) {
     constexpr int FM = 4, BM = 32 * FM, A_BYTES = BM * 256, C_BYTES = kCols * 64, STAGE = A_BYTES + C_BYTES + kCols * 8;
-    constexpr int LA = A_BYTES / 16 / kLongThreads, LC = C_BYTES / 16 / kLongThreads;
+    constexpr int LA = A_BYTES / 16 / kFourThreads, LC = C_BYTES / 16 / kFourThreads;
     constexpr int LOADS = LA + LC + 1;  // per thread and stage: activations, codes, one scale or zero
     __shared__ __attribute__((aligned(16))) unsigned char lds[D * STAGE];
 
@@ -468,13 +468,13 @@ __global__ __launch_bounds__(kLongThreads) void gemm_staged_long_kernel(StagedPa
     const unsigned lda = (unsigned)p.K * 2u, ldw = (unsigned)p.K / 2u;
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
-        const int s = i * kLongThreads + tid, row = s >> 4, chunk = (s & 15) ^ (row & 15);
+        const int s = i * kFourThreads + tid, row = s >> 4, chunk = (s & 15) ^ (row & 15);
         a_off[i] = (unsigned)((m0 + row < p.M ? m0 + row : p.M - 1) - m0) * lda + chunk * 16;
     }
     auto tile_row = [&](int row) { return (unsigned)(c0 + row < p.N ? row : p.N - 1 - c0); };
 #pragma unroll
     for (int i = 0; i < LC; ++i) {
-        const int s = i * kLongThreads + tid, row = s >> 2, chunk = (s & 3) ^ ((row >> 2) & 3);
+        const int s = i * kFourThreads + tid, row = s >> 2, chunk = (s & 3) ^ ((row >> 2) & 3);
         c_off[i] = tile_row(row) * ldw + chunk * 16;
     }
     const unsigned q_off = tile_row(tid & 127) * (unsigned)G * 2u;
@@ -486,9 +486,9 @@ __global__ __launch_bounds__(kLongThreads) void gemm_staged_long_kernel(StagedPa
     };
     auto issue = [&](int g, unsigned char *st, int i) {
         if (i < LA) {
-            to_lds16(st + (i * kLongThreads + wave * 64) * 16, a_off[i < LA ? i : 0], a_base + (long long)g * 256);
+            to_lds16(st + (i * kFourThreads + wave * 64) * 16, a_off[i < LA ? i : 0], a_base + (long long)g * 256);
         } else if (i < LA + LC) {
-            to_lds16(st + A_BYTES + ((i - LA) * kLongThreads + wave * 64) * 16, c_off[i - LA < LC ? i - LA : 0], c_base + (long long)g * 64);
+            to_lds16(st + A_BYTES + ((i - LA) * kFourThreads + wave * 64) * 16, c_off[i - LA < LC ? i - LA : 0], c_base + (long long)g * 64);
         } else {
             const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(st + A_BYTES + C_BYTES + wave * 256));
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" ::"s"(lds_addr), "v"(q_off), "s"(q_base + (long long)g * 2) : "memory");
@@ -615,20 +615,22 @@ __global__ __launch_bounds__(kLongThreads) void gemm_staged_long_kernel(StagedPa
     }
 }
 
-// Which kernel takes a slice of so many groups in 128-row tiles: four waves where it is long, and sooner where the other kernel's
+// Whether a slice of so many groups goes to four waves in 128-row tiles: where it is long, and sooner where the other kernel's
 // pieces of codes, two groups, lie across cache lines (rows of an odd number of groups; slices that begin at an odd one). Speed of
 // four waves over eight, medians over 2330 sizes (1024 to 8192 columns, 65 to 2048 tokens, every slice the planner cuts):
-//     groups of the slice   6-17   18-29  30-41  42-49  50-59  60-71  72-95  96-
-//     pieces in one line    0.964  0.968  0.978  0.985  0.98   1.014  1.022  1.025
-//     across two            0.985  1.000  1.013  1.019  1.04   1.055  1.076  1.10
-constexpr bool staged_long(int groups_of_row, int groups_of_slice) {
-    return groups_of_slice >= (groups_of_row % 2 || (groups_of_slice < groups_of_row && groups_of_slice % 2) ? 30 : 60);
+//     groups of the slice    6-17   18-29  30-41  42-49  50-59  60-71  72-95  96-
+//     pieces in one line     0.964  0.968  0.978  0.985  0.98   1.014  1.022  1.025
+//     across two, K whole    1.013  1.006  1.010  1.020  1.04   1.055  1.076  1.10
+//     across two, K cut      0.983  0.994  1.015  1.019  1.04
+constexpr bool four_waves(int groups_of_row, int groups_of_slice) {
+    const bool whole = groups_of_slice >= groups_of_row, across = whole ? groups_of_row % 2 : groups_of_row % 2 || groups_of_slice % 2;
+    return groups_of_slice >= (!across ? 60 : whole ? 0 : 30);
 }
 
-int launch_staged_long(StagedParams p, int splits, hipStream_t st, const char *who) {
+int launch_staged_four(StagedParams p, int splits, hipStream_t st, const char *who) {
     p.tiles_m = (p.M + 127) / 128;
     p.tiles_n = (p.N + kCols - 1) / kCols;
-    hipLaunchKernelGGL(gemm_staged_long_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits), dim3(kLongThreads), 0, st, p);
+    hipLaunchKernelGGL(gemm_staged_four_kernel, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)splits), dim3(kFourThreads), 0, st, p);
     return lq_check_launch(who);
 }
 
@@ -652,7 +654,7 @@ int launch_staged(const StagedParams &p, int rows, bool exact, int splits, hipSt
                             : launch_staged_tile<4, false, true>(p, 1, st, who);
     if (rows == 32) return exact ? launch_staged_tile<1, true, false>(p, splits, st, who) : launch_staged_tile<1, false, false>(p, splits, st, who);
     if (rows == 64) return exact ? launch_staged_tile<2, true, false>(p, splits, st, who) : launch_staged_tile<2, false, false>(p, splits, st, who);
-    if (!p.w2 && staged_long(p.K / LQ_GROUP, p.partial ? p.groups_per_split : p.K / LQ_GROUP)) return launch_staged_long(p, splits, st, who);
+    if (!p.w2 && four_waves(p.K / LQ_GROUP, p.partial ? p.groups_per_split : p.K / LQ_GROUP)) return launch_staged_four(p, splits, st, who);
     return launch_staged_tile<4, false, false>(p, splits, st, who);
 }
 
