@@ -616,15 +616,18 @@ __global__ __launch_bounds__(kFourThreads) void gemm_staged_four_kernel(StagedPa
 }
 
 // Whether a slice of so many groups goes to four waves in 128-row tiles: where it is long, and sooner where the other kernel's
-// pieces of codes, two groups, lie across cache lines (rows of an odd number of groups; slices that begin at an odd one). Speed of
-// four waves over eight, medians over 2330 sizes (1024 to 8192 columns, 65 to 2048 tokens, every slice the planner cuts):
-//     groups of the slice    6-17   18-29  30-41  42-49  50-59  60-71  72-95  96-
-//     pieces in one line     0.964  0.968  0.978  0.985  0.98   1.014  1.022  1.025
-//     across two, K whole    1.013  1.006  1.010  1.020  1.04   1.055  1.076  1.10
-//     across two, K cut      0.983  0.994  1.015  1.019  1.04
-constexpr bool four_waves(int groups_of_row, int groups_of_slice) {
-    const bool whole = groups_of_slice >= groups_of_row, across = whole ? groups_of_row % 2 : groups_of_row % 2 || groups_of_slice % 2;
-    return groups_of_slice >= (!across ? 60 : whole ? 0 : 30);
+// pieces of codes, two groups, lie across cache lines (rows of an odd number of groups; slices that begin at an odd one), the more
+// so the fewer row tiles read the codes after the first. Speed of four waves over eight, medians over 3500 sizes (1024 to 8192
+// columns, 65 to 2048 tokens, every slice the planner cuts):
+//     groups of the slice                 6-17   18-23  24-31  32-41  42-49  50-59  60-71  72-95  96-
+//     pieces in one line                  0.964  0.970  0.977  0.980  0.99   0.998  1.014  1.022  1.025
+//     across two, K whole                 1.013  1.006  1.006  1.010  1.020  1.04   1.055  1.076  1.10
+//     across two, K cut, 2 row tiles      0.982  1.013  1.026  1.04
+//                        3                0.972  0.985  1.008  1.024  1.04
+//                        4 and more       0.972  0.980  0.988  1.002  1.011  1.036
+constexpr bool four_waves(int groups_of_row, int groups_of_slice, int row_tiles) {
+    const bool whole = groups_of_slice >= groups_of_row, across = groups_of_row % 2 || (!whole && groups_of_slice % 2);
+    return groups_of_slice >= (!across ? 60 : whole ? 0 : row_tiles <= 2 ? 18 : row_tiles == 3 ? 25 : 32);
 }
 
 int launch_staged_four(StagedParams p, int splits, hipStream_t st, const char *who) {
@@ -654,7 +657,8 @@ int launch_staged(const StagedParams &p, int rows, bool exact, int splits, hipSt
                             : launch_staged_tile<4, false, true>(p, 1, st, who);
     if (rows == 32) return exact ? launch_staged_tile<1, true, false>(p, splits, st, who) : launch_staged_tile<1, false, false>(p, splits, st, who);
     if (rows == 64) return exact ? launch_staged_tile<2, true, false>(p, splits, st, who) : launch_staged_tile<2, false, false>(p, splits, st, who);
-    if (!p.w2 && four_waves(p.K / LQ_GROUP, p.partial ? p.groups_per_split : p.K / LQ_GROUP)) return launch_staged_four(p, splits, st, who);
+    if (!p.w2 && four_waves(p.K / LQ_GROUP, p.partial ? p.groups_per_split : p.K / LQ_GROUP, (p.M + 127) / 128))
+        return launch_staged_four(p, splits, st, who);
     return launch_staged_tile<4, false, false>(p, splits, st, who);
 }
 

@@ -14,11 +14,12 @@ pytestmark = pytest.mark.gpu
 TOL = 2.0 ** -8
 
 
-@pytest.mark.parametrize("M,N,K,slices", [(336, 7808, 11 * 128, 1), (1100, 2064, 3 * 128, 1), (1100, 2064, 128, 1), (1100, 2064, 31 * 128, 1),
-                                          (379, 3840, 73 * 128, 2), (245, 3072, 57 * 128, 5), (800, 2816, 66 * 128, 1), (245, 6272, 58 * 128, 2),
-                                          (245, 6272, 62 * 128, 2), (300, 4096, 116 * 128, 2), (300, 4096, 120 * 128, 2)])
-def test_forward(hip_lib, M, N, K, slices):
+@pytest.mark.parametrize("M,N,groups,slices", [(336, 7808, 11, 1), (1100, 2064, 3, 1), (1100, 2064, 1, 1), (1100, 2064, 31, 1), (379, 3840, 73, 2),
+                                               (245, 3072, 57, 5), (800, 2816, 66, 1), (245, 4096, 68, 4), (245, 4096, 76, 4), (380, 4608, 46, 2),
+                                               (380, 4608, 54, 2), (500, 2944, 62, 2), (500, 2944, 66, 2), (300, 4096, 116, 2), (300, 4096, 120, 2)])
+def test_forward(hip_lib, M, N, groups, slices):
     from latentq_llm_amd import ops
+    K = groups * 128
     assert ops.a16w4_plan(M, (N, K))[:2] == ("staged_128x128", slices)
     _, packed, scales, zeros = make_w4(N, K, M + N + K)
     w = (packed.cuda(), scales.cuda(), zeros.cuda())
