@@ -35,8 +35,8 @@
 // comes in (dequantise, round, square, decay, round: 13 instructions for the two) depends on nothing but the code: the block's
 // 128 threads form the 512 values once and an element looks its two up in LDS (random reads; with their
 // bank conflicts LDS is busy for a third of the launch). One block to a workgroup, so that a look-up is a byte shifted and a
-// read. A decoder layer's six weights (50 M elements): stochastic rounding 91.9 -> 85.3 us, int4 + residual 141.9 -> 134.7;
-// 64 M elements: int8 + residual 164.5 -> 155.7, bf16 151.8 -> 147.8. 57 vector instructions an element are left of 65 in
+// read. (Launches of few blocks: neither, see adam8_launch_items.) A decoder layer's six weights (50 M elements): stochastic
+// rounding 91.9 -> 85.3 us, int4 + residual 141.9 -> 134.7; 64 M elements: int8 + residual 164.5 -> 155.7, bf16 151.8 -> 147.8. 57 vector instructions an element are left of 65 in
 // the first, and the vector ALUs are busy all the time. The extrema across lanes in registers instead of shuffles through LDS,
 // and no minimum of the second moments with an eps that hides their subnormals, 50 M elements: stochastic rounding 90 -> 84 us,
 // int4 + residual 133 -> 125.7, int8 + residual 134 -> 127, bf16 128 -> 124.4.
@@ -198,19 +198,20 @@ __device__ __forceinline__ void requant8_w8(const float (&out)[8], float ws, flo
 
 // BS elements share one (scale, max) pair per moment: TPB threads of CH chunks of 8 elements, chunk c of thread t being
 // elements 8 (c TPB + t) .. + 7 of the block, so that every access of a wave is contiguous. BPW blocks per workgroup.
-template <int BS, int MODE>
-__global__ __launch_bounds__(BS == 2048 ? 128 : 256) void adam8_kernel(Adam8Batch b) {
+// TABLES: the block's 512 values by code in LDS (see the top of the file), else computed for each element
+template <int BS, int MODE, bool TABLES>
+__global__ __launch_bounds__(TABLES ? 128 : 256) void adam8_kernel(Adam8Batch b) {
     int which = 0;
     for (int i = 1; i < b.n; ++i) which = blockIdx.x >= b.first[i] ? i : which;
     const Adam8Params &a = b.a[which];
-    constexpr int CH = BS == 2048 ? 2 : 1, TPB = BS / 8 / CH, BPW = BS == 2048 ? 1 : 256 / TPB;
+    constexpr int CH = BS == 2048 ? 2 : 1, TPB = BS / 8 / CH, BPW = (TABLES ? 128 : 256) / TPB;
     __shared__ float red[4][4];
     __shared__ float vtab[16];  // latent modes: dequantised values of the 16 residual nibbles
-    constexpr bool kTables = BS == 2048;
-    __shared__ float tabs[2][256];
+    static_assert(!TABLES || TPB == 128, "a workgroup is one block");
+    __shared__ float tabs[2][TABLES ? 256 : 1];
     if constexpr (MODE == ADAM_W4 || MODE == ADAM_W8) {
         lq_latent_fill_value_table(vtab, a.dequant_curve);
-        if constexpr (!kTables) __syncthreads();
+        if constexpr (!TABLES) __syncthreads();
     }
     const int t = threadIdx.x % TPB;
     long long blk = (long long)(blockIdx.x - b.first[which]) * BPW + threadIdx.x / TPB;
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(BS == 2048 ? 128 : 256) void adam8_kernel(Adam8Batc
         const float s2 = mx2 - q * sc2;
         return lq_bf16r(lq_bf16r(s2 * s2) * a.beta2);
     };
-    if constexpr (kTables) {
+    if constexpr (TABLES) {
 #pragma unroll
         for (int i = 0; i < 256 / TPB; ++i) {
             const int q = t + i * TPB;
@@ -269,8 +270,8 @@ __global__ __launch_bounds__(BS == 2048 ? 128 : 256) void adam8_kernel(Adam8Batc
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const unsigned b1 = (q1[c][k >> 2] >> (8 * (k & 3))) & 0xFFu, b2 = (q2[c][k >> 2] >> (8 * (k & 3))) & 0xFFu;
-            const float mk = kTables ? tabs[0][b1] : first_moment((float)b1);
-            const float vk = kTables ? tabs[1][b2] : second_moment((float)b2);
+            const float mk = TABLES ? tabs[0][b1] : first_moment((float)b1);
+            const float vk = TABLES ? tabs[1][b2] : second_moment((float)b2);
             m[c][k] = lq_bf16r(fmaf(a.one_minus_beta1, g[k], mk));
             v[k] = lq_bf16r(fmaf(a.one_minus_beta2 * g[k], g[k], vk));
             // bf16(sqrt(v)) of a bf16 v: the square root of a number with 8 significant bits never comes closer than
@@ -409,7 +410,8 @@ __global__ __launch_bounds__(BS == 2048 ? 128 : 256) void adam8_kernel(Adam8Batc
         wave_extrema(lo1, hi1, lo2, hi2);
         if ((threadIdx.x & 63) == 63) *reinterpret_cast<f32x4_t *>(red[threadIdx.x >> 6]) = f32x4_t{lo1, hi1, lo2, hi2};
         __syncthreads();
-        const f32x4_t w0 = *reinterpret_cast<const f32x4_t *>(red[0]), w1 = *reinterpret_cast<const f32x4_t *>(red[1]);
+        const int w = TABLES ? 0 : threadIdx.x >> 7 << 1;  // the block's first wave
+        const f32x4_t w0 = *reinterpret_cast<const f32x4_t *>(red[w]), w1 = *reinterpret_cast<const f32x4_t *>(red[w + 1]);
         lo1 = min2(w0[0], w1[0]); hi1 = max2(w0[1], w1[1]);
         lo2 = min2(w0[2], w1[2]); hi2 = max2(w0[3], w1[3]);
     }
@@ -437,29 +439,38 @@ struct Adam8Item {
     int mode, block;
 };
 
-// The items of one mode and block size, kAdam8Batch to a launch
+// Items of one mode and block size in one launch: as many as leave a grid that can be launched, their number to *taken
+template <int BS, int MODE, bool TABLES>
+int adam8_launch_batch(const char *who, const Adam8Item *const *items, int n, hipStream_t st, int *taken) {
+    constexpr int kPerWg = BS == 128 ? 16 : TABLES ? 1 : 2;  // blocks per workgroup
+    Adam8Batch b = {};
+    unsigned long long wgs = 0;
+    for (b.n = 0; b.n < n; ++b.n) {
+        const unsigned long long mine = (unsigned long long)((items[b.n]->a.n_blocks + kPerWg - 1) / kPerWg);
+        if (wgs + mine > 0x7FFFFFFFull) break;  // (one item alone fits: adam8_check)
+        b.a[b.n] = items[b.n]->a;
+        b.first[b.n] = (unsigned)wgs;
+        wgs += mine;
+    }
+    b.first[b.n] = (unsigned)wgs;
+    *taken = b.n;
+    hipLaunchKernelGGL((adam8_kernel<BS, MODE, TABLES>), dim3((unsigned)wgs), dim3(TABLES ? 128 : 256), 0, st, b);
+    return lq_check_launch(who);
+}
+
+// The items of one mode and block size, kAdam8Batch to a launch. Up to two blocks of 2048 to a compute unit: two to a workgroup and
+// no tables, which are for busy vector ALUs and only lengthen the chain here. us this way / with tables: 0.6 M elements, stochastic
+// rounding 5.6 / 6.4, parameter 5.1 / 5.9; 1.05 M (two blocks) 5.7 / 6.6, 5.3 / 6.2; 1.6 M (three and four) 7.6 / 6.9, 7.2 / 6.5. (One
+// block to a workgroup without tables: 6.8 and 6.95 for the first and third.)
 template <int BS, int MODE>
 int adam8_launch_items(const char *who, const Adam8Item *const *items, int n, hipStream_t st) {
-    constexpr int kPerWg = BS == 2048 ? 1 : 16;  // blocks per workgroup
-    for (int i0 = 0; i0 < n; i0 += kAdam8Batch) {
-        Adam8Batch b = {};
-        b.n = n - i0 < kAdam8Batch ? n - i0 : kAdam8Batch;
-        unsigned long long wgs = 0;
-        for (int i = 0; i < b.n; ++i) {
-            const unsigned long long mine = (unsigned long long)((items[i0 + i]->a.n_blocks + kPerWg - 1) / kPerWg);
-            if (wgs + mine > 0x7FFFFFFFull) {  // (one item alone fits: adam8_check)
-                b.n = i;
-                break;
-            }
-            b.a[i] = items[i0 + i]->a;
-            b.first[i] = (unsigned)wgs;
-            wgs += mine;
-        }
-        b.first[b.n] = (unsigned)wgs;
-        hipLaunchKernelGGL((adam8_kernel<BS, MODE>), dim3((unsigned)wgs), dim3(BS == 2048 ? 128 : 256), 0, st, b);
-        const int rc = lq_check_launch(who);
+    for (int i0 = 0, taken = 0; i0 < n; i0 += taken) {
+        const int most = n - i0 < kAdam8Batch ? n - i0 : kAdam8Batch;
+        long long blocks = 0;
+        for (int i = 0; i < most; ++i) blocks += items[i0 + i]->a.n_blocks;
+        const int rc = BS == 2048 && blocks > 2 * lq_device_cu_count() ? adam8_launch_batch<BS, MODE, BS == 2048>(who, items + i0, most, st, &taken)
+                                                                       : adam8_launch_batch<BS, MODE, false>(who, items + i0, most, st, &taken);
         if (rc) return rc;
-        i0 += b.n - kAdam8Batch;  // (a cut batch: go on behind it)
     }
     return LQ_OK;
 }
