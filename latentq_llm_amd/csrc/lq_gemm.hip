@@ -973,10 +973,15 @@ struct GateUpPlan {
 // launch of 32, 64 or 128 rows, planned as one product of 2 N columns. It writes h itself, or where K is cut a second
 // launch adds the slices and forms h.
 // Both sides estimated: the weights-direct kernel by its pace per 64-deep step (0.58 to 0.68 us for a workgroup with a
-// unit to itself, 1.3 for two) plus 7 us, the staged one by its own plan plus what the partial products' way through the cache
-// cost when K was not cut either, on the safe side since the kernel writes h. us against the weights-direct kernel:
+// unit to itself, 1.3 for two) plus 7 us, the staged one by its own plan, plus, where K is not cut, what the way of partial
+// products through the cache would cost (they have none; on a K of some hundred, where that counts, the weights-direct kernel is
+// level). us against the weights-direct kernel:
 //   11008 x 4096  17 / 45 / 128 tokens  19.4 / 23.2 / 36 against 51.1 / 50.4 / 50.5
 //   6144 x 3072   100                   18.5 against 35.9
+// More tiles than units: their rounds, one workgroup to a unit (its stages fill LDS), 0.66 us a group and round of 64 rows. The
+// plan's own estimate, less by up to a third, had sent products of just over four rounds to five of them: 11008 x 4096 at 337
+// tokens 110 against 92 us, 9472 x 3328 at 417 93 against 78; up to four rounds both are level (11008 x 4096 at 300 88 / 91, 9088 x
+// 3328 at 397 72 / 76).
 static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     GateUpPlan out;
     if (ws_bytes < (size_t)8 * M * N) return out;
@@ -985,7 +990,12 @@ static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_
     const double est_direct = (1.3 * (double)(wg / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.66 : 1.3)) * (double)(K / 64) + 7.0;
     out.per_split = groups;
     double est = lq_gemm_staged_plan(M, 2 * N, groups, ws_bytes, cus, &out.rows, &out.splits, &out.per_split);
-    if (out.splits == 1) est += 1.7 + 0.53e-6 * 8.0 * (double)M * (double)N;
+    if (out.splits == 1) {
+        est += 1.7 + 0.53e-6 * 8.0 * (double)M * (double)N;
+        const long long rounds = ((M + out.rows - 1) / out.rows * ((2 * N + 127) / 128) + cus - 1) / cus;
+        const double whole = 4.1 + (out.rows == 32 ? 0.55 : out.rows == 64 ? 0.66 : 0.90) * (double)groups * (double)rounds;
+        if (rounds > 1 && est < whole) est = whole;
+    }
     if (est >= est_direct) return GateUpPlan();
     out.kernel = LQ_PLAN_STAGED_128;
     return out;

@@ -207,6 +207,9 @@ def test_dispatch_plan_host_logic(hip_lib):
         return ops.a16w4_gate_up_plan(M, (N, K), workspace_bytes=workspace, compute_units=256)
     assert gate_up(16, 11008, 4096)[0] == "gemv" and gate_up(45, 11008, 4096) == ("staged_128x128", 64, 1)
     assert gate_up(160, 11008, 4096)[0] == gate_up(45, 11008, 4096, 8 * 45 * 11008 - 1)[0] == "direct_128x256"
+    # four rounds of small tiles, but not five
+    assert gate_up(320, 11008, 4096)[0] == gate_up(397, 9088, 3328)[0] == "staged_128x128"
+    assert gate_up(321, 11008, 4096)[0] == gate_up(417, 9472, 3328)[0] == gate_up(329, 11008, 3072)[0] == "direct_128x256"
     # bad arguments
     from latentq_llm_amd._C import LatentQError
     with pytest.raises(LatentQError, match="multiple of 256"):
