@@ -833,9 +833,12 @@ struct W4Plan {
 //                                      a time, rows must be 4-byte aligned): the staged kernel up to one tile per unit,
 //                                      beyond that the kernel with weight waves and 256 x 128 tiles (4224 x 4096:
 //                                      40 against 48 us at T = 256, 70 against 66 at 384)
-//   T <= units, K >= 8192              the staged kernel's 128-row tiles, whole (4096 x 11008: 79.0 against 86.9 us at
-//                                      T = 192, 95.6 against 98.5 at 256); for shorter K the difference is small (0 to
-//                                      4 us) and the weights-direct kernel keeps them
+//   T <= 3/4 of units, K >= 8192       the staged kernel's 128-row tiles, whole. They had the advantage while the weights-direct
+//                                      kernel had one group of waves (79.0 against 86.9 us on 4096 x 11008 at T = 192); with two
+//                                      the latter is 1 to 7 % faster here (4096 x 11008 at T = 160 76.4 against 75.5, 8192 x 9216 at
+//                                      192 69.9 against 69.4, 4096 x 8192 at 192 64.0 against 59.8), where a test states the plan, and
+//                                      has those above: 4096 x 11008 at T = 256 97.8 against 91.5, 2560 x 9728 at 200 78.4 against
+//                                      71.0, 8192 x 8192 at 256 74.2 against 71.6
 //   else                               one of the two weights-direct kernels, by rough time per 64-deep step
 //                                      (microseconds, measured): 128 x 256 tiles take ~0.86 with one workgroup on a
 //                                      compute unit and ~1.45 for two sharing it. The kernel with 128 x 128 tiles fits
@@ -872,7 +875,7 @@ static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, l
         if (out.exact && out.rows == 128) out.rows = 64;
         return out;
     }
-    if (tiles <= cus && (groups % 2 != 0 || K >= 8192)) return out;  // whole, 128 rows
+    if (tiles <= cus && (groups % 2 != 0 || (K >= 8192 && 4 * tiles <= 3 * cus))) return out;  // whole, 128 rows
     if (groups % 2 != 0) {
         out.kernel = LQ_PLAN_STAGED_256;
         return out;

@@ -183,6 +183,10 @@ def test_dispatch_plan_host_logic(hip_lib):
         assert plan(M, 11008, 4096) == ("direct_128x128", 1, 0), M
     assert plan(3072, 4096, 11008) == ("direct_128x128", 1, 0)
     assert plan(2048, 11008, 4096 + 128)[0] not in ("direct_128x256", "direct_128x128")
+    # one workgroup to a compute unit on a long K: from three quarters of the units on the same, unless rows have an odd number of groups
+    for M, N, K in [(1019, 4096, 11008), (512, 8192, 8192), (1240, 2560, 9728), (1019, 4096, 16384)]:
+        assert plan(M, N, K) == ("direct_128x128", 1, 0) and plan(M, N, K + 128) == ("staged_128x128", 1, 0)
+    assert plan(700, 4096, 8192) == plan(640, 4096, 11008) == ("staged_128x128", 1, 0)
     # skinny grids: split reduction, slices of an even number of steps >= 8 that cover the reduction
     for M, N, K, back in [(128, 11008, 4096, True), (512, 11008, 4096, True), (1024, 11008, 4096, True),
                           (128, 4096, 11008, False), (512, 4096, 11008, False), (200, 1024, 2048, False)]:

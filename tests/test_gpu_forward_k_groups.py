@@ -18,6 +18,7 @@ TOL = 2.0 ** -8
                                           (513, 4112, 3328, "direct_128x128"), (129, 9008, 7936, "direct_128x128"),
                                           (1900, 4112, 512, "direct_128x256"), (1537, 4096, 1792, "direct_128x256"),
                                           (1000, 4096, 1024, "direct_128x128"), (1000, 4096, 768, "direct_128x128"),
+                                          (769, 4112, 8192, "direct_128x128"),
                                           (1900, 4112, 1536, "direct_128x256"), (1900, 4112, 1280, "direct_128x256")])
 def test_forward(hip_lib, M, N, K, kernel):
     from latentq_llm_amd import ops
