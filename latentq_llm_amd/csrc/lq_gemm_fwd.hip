@@ -485,8 +485,9 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_fwd_direct_kernel(FwdParams 
     // instruction would touch 32 rows with 16 bytes each. Instead every wave passes its block
     // through LDS, 32 rows (one j) at a time, and stores 16 bytes per lane with 8 lanes on the 128
     // contiguous bytes of a row: full cache lines. The stages are free once every wave has left the
-    // loop and its loads have landed; a wave's staging area is private (waves 0,1 in stage 0, waves
-    // 2,3 in stage 1), row pitch 144 bytes.
+    // loop and its loads have landed (KS = 2: and the sums have been read); a wave's staging area is
+    // private, one behind the other from the first stage on, row pitch 144 bytes. With KS = 2 each
+    // group stores the two of the four 32-row blocks whose sums it has.
     constexpr int EP = 144;
     unsigned char *ep = lds + wave_all * (32 * EP);
     const int ep_row = lane >> 3, ep_chunk = lane & 7;
