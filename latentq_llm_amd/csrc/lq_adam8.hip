@@ -35,11 +35,12 @@
 // comes in (dequantise, round, square, decay, round: 13 instructions for the two) depends on nothing but the code: the block's
 // 128 threads form the 512 values once and an element looks its two up in LDS (random reads; with their
 // bank conflicts LDS is busy for a third of the launch). One block to a workgroup, so that a look-up is a byte shifted and a
-// read. (Launches of few blocks: neither, see adam8_launch_items.) A decoder layer's six weights (50 M elements): stochastic
+// read. (Launches of few blocks and of two numbers between: neither, see adam8_tables.) A decoder layer's six weights (50 M elements): stochastic
 // rounding 91.9 -> 85.3 us, int4 + residual 141.9 -> 134.7; 64 M elements: int8 + residual 164.5 -> 155.7, bf16 151.8 -> 147.8. 57 vector instructions an element are left of 65 in
 // the first, and the vector ALUs are busy all the time. The extrema across lanes in registers instead of shuffles through LDS,
 // and no minimum of the second moments with an eps that hides their subnormals, 50 M elements: stochastic rounding 90 -> 84 us,
 // int4 + residual 133 -> 125.7, int8 + residual 134 -> 127, bf16 128 -> 124.4.
+#include "lq_adam8_tables.h"
 #include "lq_latent_math.h"
 #include "lq_requant_math.h"
 
@@ -458,17 +459,15 @@ int adam8_launch_batch(const char *who, const Adam8Item *const *items, int n, hi
     return lq_check_launch(who);
 }
 
-// The items of one mode and block size, kAdam8Batch to a launch. Up to two blocks of 2048 to a compute unit: two to a workgroup and
-// no tables, which are for busy vector ALUs and only lengthen the chain here. us this way / with tables: 0.6 M elements, stochastic
-// rounding 5.6 / 6.4, parameter 5.1 / 5.9; 1.05 M (two blocks) 5.7 / 6.6, 5.3 / 6.2; 1.6 M (three and four) 7.6 / 6.9, 7.2 / 6.5. (One
-// block to a workgroup without tables: 6.8 and 6.95 for the first and third.)
+// The items of one mode and block size, kAdam8Batch to a launch; with tables or without by adam8_tables. (Without them one block to
+// a workgroup: 6.8 and 6.95 us for 0.6 and 1.6 M elements, stochastic rounding, where two take 5.6 and 7.6.)
 template <int BS, int MODE>
 int adam8_launch_items(const char *who, const Adam8Item *const *items, int n, hipStream_t st) {
     for (int i0 = 0, taken = 0; i0 < n; i0 += taken) {
         const int most = n - i0 < kAdam8Batch ? n - i0 : kAdam8Batch;
         long long blocks = 0;
         for (int i = 0; i < most; ++i) blocks += items[i0 + i]->a.n_blocks;
-        const int rc = BS == 2048 && blocks > 2 * lq_device_cu_count() ? adam8_launch_batch<BS, MODE, BS == 2048>(who, items + i0, most, st, &taken)
+        const int rc = BS == 2048 && adam8_tables(blocks, lq_device_cu_count()) ? adam8_launch_batch<BS, MODE, BS == 2048>(who, items + i0, most, st, &taken)
                                                                        : adam8_launch_batch<BS, MODE, false>(who, items + i0, most, st, &taken);
         if (rc) return rc;
     }
