@@ -96,7 +96,7 @@ constexpr int STAGE = BM * ROWB;     // 16 KB per A stage
 // the MFMAs take 0.25). Two groups on stages of their own fill each other's gaps; their sums meet in LDS at the end.
 // (1000 tokens, 4096 x 4096 40.8 -> 36.9 us; the sizes where that pays: lq_fwd_k_groups.h). Where units get several workgroups, these
 // fill the gaps already, and a workgroup twice as large is slower (2048 tokens, 11008 x 4096 156.3 against 163.8). Three groups are
-// no faster on that size (37.9 where two took 37.1) and 3 % on 1019 tokens, 4096 x 11008 (92.2 against 95.2).
+// no faster on 4096 x 4096 (37.9 where two took 37.1) and 3 % faster on 1019 tokens, 4096 x 11008 (92.2 against 95.2).
 template <int NT, bool GU, int KS>
 __global__ __launch_bounds__(256 * KS, 2) void gemm_fwd_direct_kernel(FwdParams p) {
     static_assert(NT == 2 || (NT == 1 && !GU), "gate / up mode uses both column tiles");

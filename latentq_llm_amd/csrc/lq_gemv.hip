@@ -27,7 +27,6 @@
 
 namespace {
 
-
 // k-slot order produced by the AND-OR unpack of one code word: slots (2i, 2i+1) of dword i
 // hold codes (1,5), (0,4), (3,7), (2,6). The activation fragment is permuted to match.
 __device__ __forceinline__ void unpack_word_128q(unsigned w, unsigned o[4]) {
