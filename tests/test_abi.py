@@ -187,6 +187,9 @@ def test_dispatch_plan_host_logic(hip_lib):
     for M, N, K in [(1019, 4096, 11008), (512, 8192, 8192), (1240, 2560, 9728), (1019, 4096, 16384)]:
         assert plan(M, N, K) == ("direct_128x128", 1, 0) and plan(M, N, K + 128) == ("staged_128x128", 1, 0)
     assert plan(700, 4096, 8192) == plan(640, 4096, 11008) == ("staged_128x128", 1, 0)
+    # up to 64 tokens: slices of whole pairs of groups, unless they are short, rows are an odd number of groups or it would be a slice less
+    assert plan(61, 4096, 9216) == ("staged_128x128", 8, 20) and plan(64, 4112, 1792)[2] == plan(56, 1280, 1280)[2] == 10
+    assert plan(61, 4096, 9088) == ("staged_128x128", 8, 18) and plan(65, 4096, 9216)[2] % 4 == 2
     # skinny grids: split reduction, slices of an even number of steps >= 8 that cover the reduction
     for M, N, K, back in [(128, 11008, 4096, True), (512, 11008, 4096, True), (1024, 11008, 4096, True),
                           (128, 4096, 11008, False), (512, 4096, 11008, False), (200, 1024, 2048, False)]:

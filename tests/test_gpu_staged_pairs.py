@@ -29,7 +29,7 @@ def _x(M, K):
 
 
 SMALL = [(33, 16, 128), (64, 272, 128), (40, 5504, 256), (64, 1040, 384), (17, 4112, 640), (20, 8208, 1152), (64, 6160, 896),
-         (50, 2048, 5504), (128, 144, 3200), (100, 2064, 1408), (300, 528, 1152), (129, 256, 128), (30, 160, 11008)]
+         (50, 2048, 5504), (128, 144, 3200), (100, 2064, 1408), (300, 528, 1152), (129, 256, 128), (30, 160, 11008), (61, 4112, 3328), (20, 6160, 4352)]
 LARGE = [(500, 1024, 5504), (257, 2048, 11008), (1000, 2064, 8320)]  # (whose alignment the small ones cover)
 
 
