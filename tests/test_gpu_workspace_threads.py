@@ -15,12 +15,14 @@ def test_threads_on_one_stream(hip_lib):
     mine = ops._workspace(x, 45, 4096)[0]
     assert ops._workspace(x, 45, 4096)[0] is mine
     other, errors = [], []
+    both = threading.Barrier(2, timeout=60)  # a thread that ended may leave its number, and the buffer with it, to the next
     mats = [tuple(t.cuda() for t in make_w4(2048, 4096, seed)[1:]) for seed in (2, 3)]
     want = [(ops.a16w4_forward(x, *m, (2048, 4096)), ops.a16w4_gate_up_silu(x, m, mats[0], (2048, 4096))) for m in mats]
 
     def work(i):
         try:
             other.append(ops._workspace(x, 45, 4096)[0])
+            both.wait()
             for _ in range(50):
                 y, h = ops.a16w4_forward(x, *mats[i], (2048, 4096)), ops.a16w4_gate_up_silu(x, mats[i], mats[0], (2048, 4096))
                 assert torch.equal(y, want[i][0]) and torch.equal(h, want[i][1])
