@@ -819,6 +819,18 @@ struct W4Plan {
     bool exact = false;  // and weights not rounded to bf16
 };
 
+// Groups per slice of a row's `groups`, an even number if there are as many slices of one group more. Small tiles take groups in pairs: a
+// slice of an odd number is no shorter than of one more, and the next one's pieces of codes would lie across cache lines, which had made
+// some slower than with pieces of one group. Up to 64 tokens, slices of seven groups and more:
+//   plain    3400 sizes 1.020, for each length of a slice and grid (4096 x 9216 at 18 / 34 / 61 tokens 15.3 / 18.5 / 20.0 -> 15.0 / 18.0 / 18.9 us)
+//   gate / up  tiles of 32 rows 1.018, of 64 rows in slices of seven 1.015 (5376 x 2560 at 55 18.3 -> 17.5); 64 rows in longer ones are level
+//            or, on grids that leave no unit idle, 2 % slower
+// Slices of five gain nothing (1280 x 1280 0.994), nor do rows of an odd number of groups, which lie across lines anyway (0.990), nor
+// more than 64 tokens, whose row tiles share the codes (1.00).
+static int whole_pairs(int per, int splits, int groups) {
+    return splits > 1 && groups % 2 == 0 && per % 2 && (groups + per) / (per + 1) == splits ? per + 1 : per;
+}
+
 // Forward pass, M > 16. Up to 64 tokens, with 16 columns for each of more than half of the units and at most all of them:
 // the kernel of lq_gemm_few.hip where its time, which grows with the tokens' bytes each unit takes in (2 us + 0.5 us per 1000 k
 // + 0.42 per 16 tokens and 1000 k, less with fewer units asking; 12 % rms over 64 timings), is under the staged kernel's
@@ -868,12 +880,7 @@ static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, l
     if (M <= 64 || tiles * 2 <= cus) {
         int per = 0;
         lq_gemm_staged_plan(M, N, groups, ws_bytes, cus, &out.rows, &out.splits, &per);
-        // Small tiles take groups in pairs: a slice of an odd number is no shorter than of one more, and the next one's pieces of codes
-        // would lie across cache lines, which had made slices of 9 up to 5 % slower than with pieces of one group. 3400 sizes of up to 64
-        // tokens 1.020 by this, for each length of a slice and grid (4096 x 9216 at 18 / 34 / 61 tokens 15.3 / 18.5 / 20.0 -> 15.0 / 18.0 / 18.9 us). Not
-        // slices of five (1280 x 1280 0.994), rows of an odd number of groups, which lie across lines anyway (0.990), nor above 64
-        // tokens, where more rows share the codes (1.00).
-        if (M <= 64 && out.splits > 1 && groups % 2 == 0 && per % 2 && per >= 7 && (groups + per) / (per + 1) == out.splits) ++per;
+        if (M <= 64 && per >= 7) per = whole_pairs(per, out.splits, groups);
         if (out.splits > 1) out.steps_per_split = 2 * per;
         // weights as they are for every call that GEMV launches served before, by the estimates of that time (up to 64 tokens
         // with a workspace, 128 without)
@@ -999,6 +1006,7 @@ static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_
     const double est_direct = (1.3 * (double)(wg / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.66 : 1.3)) * (double)(K / 64) + 7.0;
     out.per_split = groups;
     double est = lq_gemm_staged_plan(M, 2 * N, groups, ws_bytes, cus, &out.rows, &out.splits, &out.per_split);
+    if (M <= 64 && out.per_split >= 7 && (out.rows == 32 || out.per_split == 7)) out.per_split = whole_pairs(out.per_split, out.splits, groups);
     if (out.splits == 1) {
         est += 1.7 + 0.53e-6 * 8.0 * (double)M * (double)N;
         const long long rounds = ((M + out.rows - 1) / out.rows * ((2 * N + 127) / 128) + cus - 1) / cus;

@@ -52,7 +52,7 @@ def test_forward(hip_lib, M, N, K, offset):
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 11008, 256), (32, 5520, 768), (45, 11024, 512), (64, 8208, 1280), (100, 5504, 512), (150, 2064, 256),
-                                   (40, 144, 2048), (45, 1040, 2816)])
+                                   (40, 144, 2048), (45, 1040, 2816), (55, 5392, 2560), (20, 8176, 2816)])
 def test_gate_up(hip_lib, M, N, K):
     from latentq_llm_amd import ops
     mats = [_weights(N, K, s, 0) for s in (1, 2)]
