@@ -14,13 +14,13 @@
 // straddle a 128-element quantisation group, so scale, zero and reciprocal are per-thread constants,
 // the codes move as one 16-byte load and one 16-byte store, and the 4 Philox blocks of the thread
 // (one per word: 8 draws of 16 bits) have consecutive counters. The kernel is bound by vector-ALU
-// issue (about 16 instructions per element, 5 of them Philox4x32-10), so the tail is written to
+// issue (about 15 instructions per element, 5 of them Philox4x32-10), so the tail is written to
 // keep that count down:
 //   - (q - z) * s comes from one fma on the code read as an FP8 number (exact for an integer zero,
 //     see below) and is rounded to bf16 as the high half of a packed conversion whose low half is 0;
 //   - the float -> fixed conversion saturates in hardware (v_cvt_u32_f32), the 16-bit draw is added
-//     straight from its half of the Philox word with a saturating v_mad_u32_u16, and the eight codes
-//     of a word are gathered from byte 2 of the eight sums with v_perm_b32.
+//     straight from its half of the Philox word with a saturating v_mad_u32_u16, and a code, the sum's
+//     top nibble, is appended to its word with one v_alignbit_b32.
 // Threads whose (scale, zero) do not allow the one-fma dequantisation (non-integer zero, extreme
 // scale) redo their 32 elements on a rolled cold path with the operations written out one by one.
 //
