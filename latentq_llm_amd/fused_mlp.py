@@ -41,21 +41,34 @@ class _FusedMLPTrain(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        from .quant import _pending_dw, backward_hook_fn, dict_temp
-        x2, g, u, h = ctx.saved_tensors
-        mlp = ctx.mlp
-        gate, up, down = mlp.gate_proj, mlp.up_proj, mlp.down_proj
-        inter, K = mlp.intermediate_size, mlp.infeatures
-        dy = grad_output.to(torch.bfloat16).contiguous()
-        dg, du = ops.a16w4_dx_silu_bwd(dy, *_w4(down), (mlp.outfeatures, inter), g, u)
-        dx = None
-        if ctx.needs_input_grad[0]:
-            dx = ops.a16w4_dx_pair(dg, _w4(gate), du, _w4(up), (inter, K), split=True)
-        for layer, dyl, xin in ((down, dy, h), (up, du, x2), (gate, dg, x2)):
-            if layer.hook_handle is not None and not quant._removed(layer.hook_handle):
-                dict_temp.append(_pending_dw(dyl, xin))
-                backward_hook_fn(layer, None, None)
-        return dx, None
+        return _mlp_backward(ctx.mlp, ctx.saved_tensors, grad_output, ctx.needs_input_grad[0]), None
+
+
+def _mlp_backward(mlp, saved, grad_output, wanted):
+    from .quant import _pending_dw, _rows, backward_hook_fn, dict_temp
+    x2, g, u, h = saved
+    x2 = _rows(x2)
+    gate, up, down = mlp.gate_proj, mlp.up_proj, mlp.down_proj
+    inter, K = mlp.intermediate_size, mlp.infeatures
+    dy = grad_output.to(torch.bfloat16).contiguous()
+    dg, du = ops.a16w4_dx_silu_bwd(dy, *_w4(down), (mlp.outfeatures, inter), g, u)
+    dx = None
+    if wanted:
+        dx = ops.a16w4_dx_pair(dg, _w4(gate), du, _w4(up), (inter, K), split=True)
+    for layer, dyl, xin in ((down, dy, h), (up, du, x2), (gate, dg, x2)):
+        if layer.hook_handle is not None and not quant._removed(layer.hook_handle):
+            dict_temp.append(_pending_dw(dyl, xin))
+            backward_hook_fn(layer, None, None)
+    return dx
+
+
+def _mlp_node(mlp, x):
+    """_FusedMLPTrain without an autograd Function of Python's (quant._NODES)."""
+    down, inter = mlp.down_proj, mlp.intermediate_size
+    h, g, u = ops.a16w4_gate_up_silu(quant._rows(x.detach()), _w4(mlp.gate_proj), _w4(mlp.up_proj), (inter, mlp.infeatures), save=True)
+    bias = None if down.bias is None else down.bias.detach().to(torch.bfloat16).contiguous()
+    y = ops.linear4(h if x.dim() == 2 else h.view(x.shape[:-1] + (inter,)), *_w4(down), (mlp.outfeatures, inter), bias)
+    return None if y is None else quant._attach(y, x, None, (x, g, u, h), _mlp_backward, mlp, _FusedMLPTrain)
 
 
 class QuantLlamaMLP(nn.Module):
@@ -79,11 +92,13 @@ class QuantLlamaMLP(nn.Module):
     def forward(self, x):
         if not self._training(x):
             return self.down_proj(self.fused_gate_up(x))
-        x2 = x.reshape(-1, x.shape[-1])
-        M, K = x2.shape
-        if (x2.dtype == torch.bfloat16 and M > 0 and K % 256 == 0 and self.intermediate_size % 64 == 0
+        if (x.dtype == torch.bfloat16 and x.numel() > 0 and x.shape[-1] % 256 == 0 and self.intermediate_size % 64 == 0
                 and self.outfeatures % 64 == 0):
-            y = _FusedMLPTrain.apply(x2.contiguous(), self)
+            if quant._plain_activations(x) and quant._records_plainly(x):
+                y = _mlp_node(self, x)
+                if y is not None:
+                    return y
+            y = _FusedMLPTrain.apply(x.reshape(-1, x.shape[-1]).contiguous(), self)
             return y.reshape(x.shape[:-1] + (self.outfeatures,))
         # shapes the fused launches do not take: the layers' own forward, which autograd follows
         return self.down_proj(torch.nn.functional.silu(self.gate_proj(x)) * self.up_proj(x))

@@ -254,11 +254,19 @@ def a16w4_dx_silu_bwd(dy, codes, scales, zeros, shape, g, u):
     return dg, du
 
 
+def dx4(dy, codes, scales, zeros, shape):
+    """a16w4_dx of rows dy; None if an operand is not in the plain form the native binding takes."""
+    if dy.dim() != 2 or not dy.is_cuda or not dy.shape[0]:
+        return None
+    N, K = shape
+    return (_native or _fast()).dx4(dy, codes, scales, zeros, N, K, _workspace(dy, dy.shape[0], K)[0])
+
+
 def a16w4_dx(dy, codes, scales, zeros, shape, out=None, accumulate=False):
     """dX[M,K] = dY[M,N] . deq(W)[N,K]; accumulate=True: out = bf16(out + bf16(dY . deq(W))) (lq_a16w4_dx_acc)."""
     N, K = shape
-    if out is None and not accumulate and dy.dim() == 2 and dy.is_cuda and dy.shape[0]:
-        r = (_native or _fast()).dx4(dy, codes, scales, zeros, N, K, _workspace(dy, dy.shape[0], K)[0])
+    if out is None and not accumulate:
+        r = dx4(dy, codes, scales, zeros, shape)
         if r is not None:
             return r
     _chk(dy, torch.bfloat16, "dy")

@@ -239,6 +239,21 @@ def _w4_linear(input, weight_d, qparamw4, bias):
     return y if input.dtype == torch.bfloat16 else y.to(input.dtype)
 
 
+def _w4_backward(layer, qparam, input, weight_d, grad_output, wanted):
+    """The input's gradient of rows, where wanted; the weight's to its layer."""
+    dy = _as_bf16_2d(grad_output)
+    grad_input = None
+    if wanted:
+        grad_input = ops.dx4(dy, weight_d, *qparam)
+        if grad_input is None:
+            scales, zeros, shape = _flat_qparam(qparam)
+            grad_input = ops.a16w4_dx(dy, weight_d, scales, zeros, shape)
+        if grad_input.dtype != input.dtype:
+            grad_input = grad_input.to(input.dtype)
+    _hand_over(layer, _pending_dw(dy, _as_bf16_2d(input)))  # dW = dY^T X (utils/quant.py:141-142)
+    return grad_input
+
+
 class QLinearFunctionW4(torch.autograd.Function):
     """Training A16W4 linear (utils/quant.py:112-146): Y = X deq(W)^T + b; backward re-reads the
     packed codes (never a materialised W): dX on the HIP dequant-GEMM, dW = dY^T X pushed to
@@ -258,14 +273,8 @@ class QLinearFunctionW4(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         input, weight_d, bias = ctx.saved_tensors
-        scales, zeros, shape = _flat_qparam(ctx.save_qparamw4)
-        grad_input = grad_bias = None
-        dy = _as_bf16_2d(grad_output)
-        if ctx.needs_input_grad[0]:
-            grad_input = ops.a16w4_dx(dy, weight_d, scales, zeros, shape)
-            if grad_input.dtype != input.dtype:
-                grad_input = grad_input.to(input.dtype)
-        _hand_over(ctx.layer, _pending_dw(dy, _as_bf16_2d(input)))  # dW = dY^T X (utils/quant.py:141-142)
+        grad_input = _w4_backward(ctx.layer, ctx.save_qparamw4, input, weight_d, grad_output, ctx.needs_input_grad[0])
+        grad_bias = None
         if bias is not None and ctx.needs_input_grad[_BIAS_FLAG]:
             grad_bias = grad_output.sum(0)
         return grad_input, None, None, grad_bias, None
@@ -354,13 +363,12 @@ def _fake_quant_activation(input, clampv):
     return (input * s).round_().clamp_(-128, 127).div_(s)
 
 
-def _a8w8_backward_common(ctx, grad_output, input_f, weight_f, bias, detach_dw=False):
-    """grad_input = dY . Wf and dW = dY^T . Xf on the dequantised operands (utils/quant.py:203-210). weight_f is the
-    dense weight, or an (int8 codes, qscales) pair: then dX comes from the codes (ops.a8w8_dx: bf16(W8 * qs) is formed
-    inside the GEMM, the values the reference's `weight_d.to(dtype) * qscales` holds) whenever the kernel takes the
-    shapes. detach_dw is kept for the call sites' symmetry with the reference (the product has no history here)."""
-    grad_input = grad_bias = None
-    if ctx.needs_input_grad[0]:
+def _a8w8_grads(layer, grad_output, input_f, weight_f, wanted):
+    """grad_input = dY . Wf, where wanted, and dW = dY^T . Xf on the dequantised operands (utils/quant.py:203-210), to its layer.
+    weight_f is the dense weight, or an (int8 codes, qscales) pair: then dX comes from the codes (ops.a8w8_dx: bf16(W8 * qs) is
+    formed inside the GEMM, the values the reference's `weight_d.to(dtype) * qscales` holds) whenever the kernel takes the shapes."""
+    grad_input = None
+    if wanted:
         if isinstance(weight_f, tuple):
             w8, qscales = weight_f
             dy = grad_output if grad_output.is_contiguous() else grad_output.contiguous()
@@ -371,10 +379,37 @@ def _a8w8_backward_common(ctx, grad_output, input_f, weight_f, bias, detach_dw=F
                 grad_input = grad_output.mm((w8.to(grad_output.dtype) * qscales).to(grad_output.dtype))
         else:
             grad_input = grad_output.mm(weight_f)
-    _hand_over(ctx.layer, _pending_dw(grad_output, input_f))
+    _hand_over(layer, _pending_dw(grad_output, input_f))
+    return grad_input
+
+
+def _a8w8_backward_common(ctx, grad_output, input_f, weight_f, bias, detach_dw=False):
+    """What a Function's backward returns. detach_dw is kept for the call sites' symmetry with the reference (the product has no
+    history here)."""
+    grad_input, grad_bias = _a8w8_grads(ctx.layer, grad_output, input_f, weight_f, ctx.needs_input_grad[0]), None
     if bias is not None and ctx.needs_input_grad[_BIAS_FLAG]:
         grad_bias = grad_output.sum(0)
     return grad_input, None, None, grad_bias, None
+
+
+def _dequantised_input(x8, scale, per_token, dtype):
+    """The int8 activations of a dynamic layer times their scale, as its backward multiplies them."""
+    # x8 * (clampv / 127.): the quantiser left that bf16-valued alpha in scale[1]; per token: the row scales
+    sv = scale.view(-1) if per_token else scale.view(-1)[1:2]
+    if dtype == torch.bfloat16 and ops.act_dequant_ok(x8, sv, per_token):
+        return ops.act_dequant_i8(x8, sv, per_token)  # the two tensor operations below as one pass
+    s = scale.view(-1, 1) if per_token else scale[1]
+    return x8.to(dtype) * s.to(dtype)
+
+
+def _qat_backward_operands(input, weight_f, work, qscales):
+    """The fake-quantised activations and weight of a QAT layer's backward."""
+    input_f = _fake_quant_activation(input, work[0].to(input.dtype))
+    # the fake-quantised weight (utils/quant.py:363-365) is bf16(w8 * qscales) for the int8 codes of the forward:
+    # handed over as codes, so that the input gradient forms it inside its GEMM
+    if weight_f.dtype == torch.bfloat16 and input.dtype == torch.bfloat16:
+        return input_f, (_qat_weight_i8(weight_f, qscales), qscales)
+    return input_f, (weight_f / qscales).round_().clamp_(-128, 127).mul_(qscales).to(input.dtype)
 
 
 class QLinearFunctionA8W8_static(torch.autograd.Function):
@@ -438,13 +473,7 @@ class QLinearFunctionA8W8_dynamic(torch.autograd.Function):
     def backward(ctx, grad_output):
         x8, weight_d, bias = ctx.saved_tensors
         scale, qscales, per_token = ctx.save_qparamaw
-        # x8 * (clampv / 127.): the quantiser left that bf16-valued alpha in scale[1]; per token: the row scales
-        sv = scale.view(-1) if per_token else scale.view(-1)[1:2]
-        if grad_output.dtype == torch.bfloat16 and ops.act_dequant_ok(x8, sv, per_token):
-            input_f = ops.act_dequant_i8(x8, sv, per_token)  # the two tensor operations below as one pass
-        else:
-            s = scale.view(-1, 1) if per_token else scale[1]
-            input_f = x8.to(grad_output.dtype) * s.to(grad_output.dtype)
+        input_f = _dequantised_input(x8, scale, per_token, grad_output.dtype)
         return _a8w8_backward_common(ctx, grad_output, input_f, (weight_d, qscales), bias, detach_dw=True)
 
 
@@ -500,13 +529,7 @@ class QLinearFunctionQAT_dynamic(torch.autograd.Function):
     def backward(ctx, grad_output):
         input, weight_f, bias = ctx.saved_tensors
         work, qscales = ctx.save_qparamaw
-        input_f = _fake_quant_activation(input, work[0].to(input.dtype))
-        # the fake-quantised weight (utils/quant.py:363-365) is bf16(w8 * qscales) for the int8 codes of the forward:
-        # handed over as codes, so that the input gradient forms it inside its GEMM
-        if weight_f.dtype == torch.bfloat16 and input.dtype == torch.bfloat16:
-            weight_q = (_qat_weight_i8(weight_f, qscales), qscales)
-        else:
-            weight_q = (weight_f / qscales).round_().clamp_(-128, 127).mul_(qscales).to(input.dtype)
+        input_f, weight_q = _qat_backward_operands(input, weight_f, work, qscales)
         return _a8w8_backward_common(ctx, grad_output, input_f, weight_q, bias, detach_dw=False)
 
 
@@ -562,6 +585,84 @@ _CTX_FORMS = {
 }
 
 
+# Training without an autograd Function of Python's (see LayerNode in csrc/lq_bind.cpp), for activations in the form the kernels take: a
+# layer's forward, which attaches the backward beside it to its result. None: the Function.
+def _plain_activations(x):
+    return type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.numel() > 0 and x.dim() >= 1
+
+
+def _rows(x):
+    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+
+
+def _attach(y, x, bias, saved, backward, left, fn):
+    return ops._native.attach(y, x, bias, saved if bias is None else saved + (bias,), backward, left, fn.__name__ + "Backward")
+
+
+def _w4_node(m, x, layer):
+    qparam, bias, codes = m._qparam(), m._bias(), m.weight.data
+    y = ops.linear4(x, codes, *qparam, bias)
+    if y is None:
+        return None
+    return _attach(y, x, bias, (x, codes.data), _w4_node_backward, (layer, qparam), QLinearFunctionW4)
+
+
+def _w4_node_backward(left, saved, dy, wanted):
+    return _w4_backward(*left, _rows(saved[0]), saved[1], dy, wanted)
+
+
+def _int8_product(x, w8, qscales, bias, alpha_in_bf16, per_token):
+    """_a8w8_linear_dynamic for activations of any number of dimensions; (None, ..) where the kernels do not take an operand."""
+    x2 = _rows(x.detach())
+    if per_token:
+        x8, sx = ops.act_quant_i8_per_token(x2)
+        scale = sx
+    else:
+        x8, sx, scale = ops.act_quant_i8_dynamic(x2, alpha_in_bf16)
+    sw, b = _qs_bias(qscales, bias)
+    return ops._native.linear8(x8.view(x.shape), w8.contiguous(), sx, sw, b), x8, scale
+
+
+def _a8w8_node(m, x, layer):
+    qparam, bias, w8 = m._qparam(), m._bias(), m.weight.data
+    qscales, per_token = qparam[1], _per_token(qparam)
+    if not _plain_activations(x) or x.shape[-1] != m.input_features:
+        return None
+    y, x8, scale = _int8_product(x, w8, qscales, bias, True, per_token)
+    if y is None:
+        return None
+    return _attach(y, x, bias, (x8, w8.data), _a8w8_node_backward, (layer, scale, qscales, per_token), QLinearFunctionA8W8_dynamic)
+
+
+def _a8w8_node_backward(left, saved, dy, wanted):
+    layer, scale, qscales, per_token = left
+    return _a8w8_grads(layer, dy, _dequantised_input(saved[0], scale, per_token, dy.dtype), (saved[1], qscales), wanted)
+
+
+def _qat_node(m, x, layer):
+    qscales, bias, w = m._qparam()[1], m._bias(), m.weight.data
+    if not _plain_activations(x) or x.shape[-1] != m.input_features or w.dtype != torch.bfloat16:
+        return None
+    y, _, work = _int8_product(x, _qat_weight_i8(w, qscales), qscales, bias, False, False)
+    if y is None:
+        return None
+    return _attach(y, x, bias, (x, w.data), _qat_node_backward, (layer, work, qscales), QLinearFunctionQAT_dynamic)
+
+
+def _qat_node_backward(left, saved, dy, wanted):
+    layer, work, qscales = left
+    input_f, weight_q = _qat_backward_operands(_rows(saved[0]), saved[1], work, qscales)
+    return _a8w8_grads(layer, dy, input_f, weight_q, wanted)
+
+
+_NODES = {QLinearFunctionW4: _w4_node, QLinearFunctionA8W8_dynamic: _a8w8_node, QLinearFunctionQAT_dynamic: _qat_node}
+
+
+def _records_plainly(x):
+    """Whether a layer in training may attach its backward itself (see the binding's records_plainly)."""
+    return x.is_cuda and not torch.compiler.is_compiling() and (ops._native or ops._fast()).records_plainly()
+
+
 class _HookHandle(torch.utils.hooks.RemovableHandle):
     """What add_hook leaves in hook_handle, a handle like those of torch's own hooks: remove(), or the end of a with block on
     it, ends the delivery of weight gradients (a layer's then stay in dict_temp, as with the reference's hook removed; a
@@ -606,6 +707,10 @@ class _QLinearBase(nn.Module):
         self._delivery[self.hook_handle.id] = backward_hook_fn
 
     def _apply_fn(self, fn, x, *layer):
+        if layer and fn in _NODES and _records_plainly(x):
+            y = _NODES[fn](self, x, *layer)
+            if y is not None:
+                return y
         if not torch._C._are_functorch_transforms_active():
             fn = _CTX_FORMS.get(fn, fn)
         out = fn.apply(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), self.weight.data, self._qparam(), self.bias, *layer)
