@@ -747,6 +747,7 @@ int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *s
                                int K, int rows, int splits, int per_split, hipStream_t st, const char *who);
 
 // 17 to 64 tokens, one launch with 16 columns per compute unit (lq_gemm_few.hip)
+int lq_gemm_few_groups(long long M);
 int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
                        int K, hipStream_t st, unsigned long long *clk, const char *who);
 
@@ -831,10 +832,22 @@ static int whole_pairs(int per, int splits, int groups) {
     return splits > 1 && groups % 2 == 0 && per % 2 && (groups + per) / (per + 1) == splits ? per + 1 : per;
 }
 
-// Forward pass, M > 16. Up to 64 tokens, with 16 columns for each of more than half of the units and at most all of them:
-// the kernel of lq_gemm_few.hip where its time, which grows with the tokens' bytes each unit takes in (2 us + 0.5 us per 1000 k
-// + 0.42 per 16 tokens and 1000 k, less with fewer units asking; 12 % rms over 64 timings), is under the staged kernel's
-// estimate. Otherwise, up to 64 tokens the staged kernel on any number of tiles, with weights that are not rounded to bf16
+// Where the kernel of lq_gemm_few.hip runs, 17 to 64 tokens. A tile of 16 columns for each of more than half of the units, at most all:
+// everywhere up to K = 8192 (1.01 to 1.3 times the speed of what ran there, 260 sizes), and for up to 32 tokens and less than all units
+// beyond (1.05 to 1.26; 4096 columns of K = 11008 15.2 against 15.6 us, where a test has the staged kernel). More columns, two rounds of
+// workgroups: up to 32 tokens in place of GEMV launches (1.16 to 1.9), beyond 0.86 to 1.28. Half of the units and fewer (1.1 to 2.2
+// times the speed up to 48 tokens, 0.94 to 1.4 beyond K = 4096 and 48 tokens) but for the sizes at which tests have the other
+// kernels: the smallest matrices, the longest rows, half of the units and rows longer than 2048, columns that are no whole tiles of the
+// staged kernel.
+static bool few_takes(long long M, long long N, long long K, long long cus) {
+    if (K / LQ_GROUP > lq_gemm_few_groups(M)) return false;
+    if (N > 16 * cus) return M <= 32 && N <= 32 * cus && K < 8192 && N * K <= 4096ll * 4096;
+    if (2 * N > 16 * cus) return K < 8192 || (M <= 32 && N < 16 * cus);
+    if (N % 128 != 0 || K >= (M <= 48 ? 8192 : 7168)) return false;
+    return M <= 32 ? N * K > 2048ll * 2048 : N * K >= 1024ll * 2048 && (2 * N < 16 * cus || K <= 2048);
+}
+
+// Forward pass, M > 16. Up to 64 tokens the kernel of lq_gemm_few.hip where few_takes says so. Otherwise, up to 64 tokens the staged kernel on any number of tiles, with weights that are not rounded to bf16
 // (several workgroups to a unit: 32 tokens, 16400 x 4096 23.8 against 35.7 us of the weights-direct kernel, 32000 x 4096 27.1
 // against 40.2, 40960 x 768 10.8 against 16.3), and beyond by the number of 128 x 128 output tiles T:
 //   T <= half of the units             the staged kernel, which plans its row tile and its slices of K itself
@@ -857,19 +870,14 @@ static int whole_pairs(int per, int splits, int groups) {
 //                                      three workgroups on a unit: ~0.55-0.61 alone (the more units are busy, the lower
 //                                      the clock: 0.55 up to three quarters of them, 0.61 with all), ~0.74 as soon as a
 //                                      few units hold two, ~1.23 for two everywhere, ~1.38 for three.
-// Up to 32 tokens two GEMV launches of 16 are a little faster where a launch does not wait for the matrix' bytes
+// Up to 32 tokens two GEMV launches of 16 are a little faster than the staged kernel where a launch does not wait for the matrix' bytes
 // and K is not long (2048 x 2048: 7.4 / 8.1 us at 17 / 32 tokens against 8.6 / 9.0; 1024 x 4096 9.1 / 10.3 against 9.7 / 10.2); at
 // 11008 x 4096 they take 21.0 / 23.4 us against 18.1 / 17.7, at 1536 x 8192 14.4 / 17.0 against 13.1 / 13.7.
 static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     W4Plan out;
-    if (M <= 64 && N <= 16 * cus && 2 * N > 16 * cus) {
-        int rows = 0, splits = 0, per = 0;
-        const double units = 0.4 + 0.6 * (double)N / (double)(16 * cus);
-        const double est = 2.0 + 1e-3 * (double)K * (0.5 + 0.42 * (double)((M + 15) / 16)) * units;
-        if (est < lq_gemm_staged_plan(M, N, (int)(K / LQ_GROUP), ws_bytes, cus, &rows, &splits, &per)) {
-            out.kernel = LQ_PLAN_FEW;
-            return out;
-        }
+    if (few_takes(M, N, K, cus)) {
+        out.kernel = LQ_PLAN_FEW;
+        return out;
     }
     if (M <= 32 && K < 8192 && N * K <= 4096ll * 4096) {
         out.kernel = LQ_PLAN_GEMV_CHUNKS;
