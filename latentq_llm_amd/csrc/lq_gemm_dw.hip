@@ -113,9 +113,10 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     const int bw = rest < GN ? rest : GN;
     const int tile_n = within / bw, tile_k = band * GN + within % bw;
     const int n0 = tile_n * TILE, k0 = tile_k * TILE;
-    // A number of tokens that is no multiple of the step leaves the FIRST step short: it covers tokens 0 .. first - 1 (its
-    // other rows re-read the last of them and are masked out of both operands), and every later step starts on a full
-    // stride. The steps after it are then those of a multiple of 64.
+    // A number of tokens that is no multiple of the step leaves the FIRST step short: its last rows are tokens 0 .. first - 1
+    // (the rows ahead of them re-read the last of these and are masked out of both operands), and every later step starts on
+    // a full stride. Counted from the end the tokens then fall into the same slices of 16 whatever the step, so that the tile
+    // sizes add in one order and the store and accumulate forms agree in every bit where they take different ones.
     const int nk = (p.M + STEP_M - 1) / STEP_M;
     const int first = p.M - (nk - 1) * STEP_M;
 
@@ -147,10 +148,10 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
         const int ii = i >= LOADS ? i - LOADS : i;
         issue_off((long long)kt * STEP_M - (STEP_M - first), st, i, i >= LOADS ? b_off[ii < LOADS ? ii : 0] : a_off[ii < LOADS ? ii : 0]);
     };
-    auto issue_first = [&](unsigned char *st, int i) {  // step 0: rows past `first` re-read the last one
+    auto issue_first = [&](unsigned char *st, int i) {  // step 0: rows ahead of token 0 read the step's last token
         const int ii = i >= LOADS ? i - LOADS : i;
-        const int over = (ii * NT + (int)threadIdx.x) / (TILE / 8) - (first - 1);
-        const unsigned back = over > 0 ? (unsigned)over : 0u;
+        const int row = (ii * NT + (int)threadIdx.x) / (TILE / 8), ahead = STEP_M - first;
+        const unsigned back = (unsigned)(row >= ahead ? ahead : row - (first - 1));  // (modulo 2^32: the offsets stay within the step's tokens)
         issue_off(0, st, i, i >= LOADS ? b_off[ii < LOADS ? ii : 0] - back * (unsigned)(p.K * 2) : a_off[ii < LOADS ? ii : 0] - back * (unsigned)(p.N * 2));
     };
 
@@ -168,12 +169,12 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
 #pragma unroll
     for (int i = 0; i < FN; ++i) b_col[i] = OP_STAGE + col_off(wn * TN + 32 * i);
     const int row_lane = (8 * h + (i16 >> 2)) * ROWB;  // + 16 t rows for slice t, + 4 rows for the second read
-    // a short first step: the lane's tokens 16 t + 8 h + e of slice t with 16 t + 8 h + e >= first become zero
+    // a short first step: the lane's rows 16 t + 8 h + e of slice t ahead of the first token become zero
     auto mask_frag = [&](u32x4_t &f, int t) {
-        const int valid = first - (16 * t + 8 * h);
+        const int ahead = STEP_M - first - (16 * t + 8 * h);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const unsigned keep = valid >= 2 * e + 2 ? 0xFFFFFFFFu : valid == 2 * e + 1 ? 0x0000FFFFu : 0u;
+            const unsigned keep = ahead <= 2 * e ? 0xFFFFFFFFu : ahead == 2 * e + 1 ? 0xFFFF0000u : 0u;
             f[e] &= keep;
         }
     };
@@ -434,26 +435,38 @@ static int launch_dw_tile(DwParams p, hipStream_t st, const char *who) {
 }
 
 // Which tile a product takes: the smaller of two estimates in microseconds, both of the form (time per 64-token step,
-// summed over the rounds of workgroups) x steps + fixed, fitted to 30 shapes from 64 to 4096 tokens and 768^2 to
-// 11008 x 4096 outputs. A round of 256 x 256 tiles steps in 1.13 us while it leaves two fifths of the CUs idle and in 1.55
-// with all of them busy (power); 128 x 128 tiles step in 0.40 to 0.48 us alone on a CU, in 0.62 to 0.85 as the second
-// workgroup of a CU joins. Both sides, small and large: 2048 tokens, 2048^2 20.4 / 39.8 us; 2048 x 4096 36.2 / 43.9;
-// 3072^2 47.6 / 44.1; 11008 x 4096 176 / 157; 1024 tokens, 3072 x 768 12.0 / 23.1; 300 tokens, 2048 x 4096 16.0 / 13.3.
-static bool dw_takes_small_tiles(long long M, long long N, long long K, long long cus) {
-    const double steps = (double)M / 64.0;
+// summed over the rounds of workgroups) x steps + the ways in and out, fitted to 760 products of 64 to 4096 tokens, 768^2 to
+// 11008 x 4096 outputs. The last round is never empty: 256 tiles on 256 CUs are one full "last" round. A round of 256 x 256
+// tiles steps in 1.09 us while it leaves half of the CUs idle and in 1.48 with all of them busy (power); 128 x 128 tiles
+// step in 0.43 to 0.50 us alone on a CU, in 0.66 to 0.89 as the second workgroup of a CU joins. What comes around the steps
+// depends on the form: bf16 stores, a gradient read and added as well, or the int8 accumulator's arithmetic, some 17
+// instructions an element, which want every CU and another workgroup's steps beside them. The choice costs 0.2 % over the
+// faster of both on average and 6 % at most; one estimate, of the store form, for all three cost 3, 4 and 9 %. us, small / large:
+//   tokens, outputs     2048, 2048^2   2000, 8192 x 3072   500, 8192 x 3072   500, 5504 x 2048   64, 4096 x 1536   2000, 11008 x 4096
+//   store               20.4 / 39.8    94.9 / 92.6         32.2 / 34.9        18.3 / 18.0        6.5 / 7.7         171 / 153
+//   int8                23.9 / 51.0    105 / 115           41.9 / 50.7        25.0 / 26.8        11.3 / 17.4       188 / 186
+enum DwForm { DW_STORE, DW_ACC, DW_ACC8 };
+
+static bool dw_takes_small_tiles(DwForm form, long long M, long long N, long long K, long long cus) {
+    struct Ways { double once, round, share, second; };  // us per launch, full round, share of the last one, second workgroup on a CU
+    constexpr Ways kWays256[] = {{5.2, 6.6, 4.2, 0}, {7.5, 12.4, 6.8, 0}, {14.9, 14.9, 3.2, 0}};
+    constexpr Ways kWays128[] = {{3.9, 3.5, 1.0, 1.5}, {5.0, 6.1, 1.9, 2.1}, {7.3, 7.2, 0.8, 2.8}};
     const long long t256 = ((N + 255) / 256) * ((K + 255) / 256), t128 = ((N + 127) / 128) * ((K + 127) / 128);
-    const double r256 = (double)(t256 % cus) / (double)cus;          // the last round's share of the CUs
-    const double r128 = (double)(t128 % (2 * cus)) / (double)cus;    // 0 .. 2 workgroups per CU
-    const double last256 = r256 == 0 ? 0 : r256 <= 0.56 ? 1.13 : 1.13 + 0.42 * (r256 - 0.56) / 0.44;
-    const double last128 = r128 == 0 ? 0 : r128 <= 1 ? 0.40 + 0.08 * r128 : 0.62 + 0.23 * (r128 - 1);
-    const double rounds256 = (double)(t256 / cus), rounds128 = (double)(t128 / (2 * cus));
-    const double est256 = (1.55 * rounds256 + last256) * steps + 8 + 4 * rounds256;
-    const double est128 = (0.85 * rounds128 + last128) * steps + (t128 <= cus ? 5 : 9) + 4 * rounds128;
+    const long long rounds256 = (t256 - 1) / cus, rounds128 = (t128 - 1) / (2 * cus);
+    const double r256 = (double)(t256 - rounds256 * cus) / (double)cus;      // the last round's share of the CUs, 0 .. 1
+    const double r128 = (double)(t128 - rounds128 * 2 * cus) / (double)cus;  // 0 .. 2 workgroups per CU
+    const double step256 = 1.47 * rounds256 + 1.09 + (r256 > 0.5 ? 0.78 * (r256 - 0.5) : 0.0);
+    const double step128 = 0.83 * rounds128 + (r128 <= 1 ? 0.43 + 0.07 * r128 : 0.66 + 0.23 * (r128 - 1));
+    const Ways &w256 = kWays256[form], &w128 = kWays128[form];
+    const double est256 = step256 * (double)((M + 63) / 64) + w256.once + w256.round * rounds256 + w256.share * r256;
+    const double est128 = step128 * 0.5 * (double)((M + 31) / 32) + w128.once + w128.round * rounds128 +
+                          (r128 <= 1 ? w128.share * r128 : w128.second + w128.share * (r128 - 1));
     return est128 < est256;
 }
 
-static int launch_dw(const DwParams &p, bool acc8, hipStream_t st, const char *who) {
-    if (dw_takes_small_tiles(p.M, p.N, p.K, lq_device_cu_count()))
+static int launch_dw(const DwParams &p, DwForm form, hipStream_t st, const char *who) {
+    const bool acc8 = form == DW_ACC8;
+    if (dw_takes_small_tiles(form, p.M, p.N, p.K, lq_device_cu_count()))
         return acc8 ? launch_dw_tile<128, 256, 32, 4, true>(p, st, who) : launch_dw_tile<128, 256, 32, 4, false>(p, st, who);
     if (acc8) return launch_dw_tile<256, 512, 64, 2, true>(p, st, who);
     // 4 waves of 128 x 128 from where their faster steps outweigh the longer way in and out (see the top of the file)
@@ -477,7 +490,7 @@ extern "C" int lq_weight_grad(const void *dy, const void *x, void *dw_out, int64
     DwParams p = {};
     p.dy = (const unsigned char *)dy; p.x = (const unsigned char *)x; p.dw = (unsigned short *)dw_out;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
-    return launch_dw(p, false, (hipStream_t)stream, "lq_weight_grad");
+    return launch_dw(p, DW_STORE, (hipStream_t)stream, "lq_weight_grad");
 }
 
 extern "C" int lq_weight_grad_acc(const void *dy, const void *x, void *dw_inout, int64_t M, int64_t N, int64_t K, void *stream) {
@@ -488,7 +501,7 @@ extern "C" int lq_weight_grad_acc(const void *dy, const void *x, void *dw_inout,
     p.dy = (const unsigned char *)dy; p.x = (const unsigned char *)x; p.dw = (unsigned short *)dw_inout;
     p.accumulate = 1;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
-    return launch_dw(p, false, (hipStream_t)stream, "lq_weight_grad_acc");
+    return launch_dw(p, DW_ACC, (hipStream_t)stream, "lq_weight_grad_acc");
 }
 
 extern "C" int lq_weight_grad_acc8(const void *dy, const void *x, int8_t *q_inout, const void *scale, int64_t M, int64_t N,
@@ -503,5 +516,5 @@ extern "C" int lq_weight_grad_acc8(const void *dy, const void *x, int8_t *q_inou
     p.scale = (const unsigned short *)scale; p.noise = (const unsigned short *)noise_or_null;
     p.seed = philox_seed; p.offset = philox_offset;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
-    return launch_dw(p, true, (hipStream_t)stream, "lq_weight_grad_acc8");
+    return launch_dw(p, DW_ACC8, (hipStream_t)stream, "lq_weight_grad_acc8");
 }
