@@ -7,7 +7,7 @@
 // 16-lane block, lane i receives the four elements of column i of the 4 x 16 block the 16 lanes address. No
 // transposed copy of dY is made anywhere.
 //
-// Two tile sizes (dw_takes_small_tiles below chooses) and two ways through the large one:
+// Three tile sizes (dw_tile below chooses) and two ways through the large one:
 //   256 (n) x 256 (k) outputs, 512 threads = 8 waves in a 2 (n) x 4 (k) grid; a wave owns 128 x 64 outputs (4 x 2 MFMA
 //     32x32x16 tiles, 128 accumulator registers). Steps of 64 tokens, two LDS stages of 64 KB (64 rows of dY and 64 rows
 //     of X, 512 bytes each); one workgroup per CU.
@@ -27,11 +27,17 @@
 //     20.4 us against 26.4 with two stages of 64 tokens). Deeper stages gain the large tile nothing (159 against 157 us
 //     on 11008 x 4096: it is bound by power, 79 % of the matrix pipe's cycles when few CUs run it).
 //
+//   192 (n) x 256 (k) outputs in the 8-wave form, 96 x 64 a wave: for outputs of which 256 x 256 tiles leave a third of the CUs idle
+//     or begin another round, and 128 x 128 ones pay more ways in and out. 500 tokens, 5504 x 2048 outputs are 172 / 232 large /
+//     medium tiles on 256 CUs: 20.0 -> 17.9 us, with the int8 accumulator 26.1 (small tiles) -> 23.9; 1024 tokens, 3072^2 (144 / 192)
+//     25.3 -> 22.1 and 32.5 -> 28.0; 2240 tokens, 4736 x 1792 46.2 -> 39.4.
+//
 // A slice is 16 tokens. Lane l: r = l % 32, h = l / 32; in slice t the lane's operand for column r of a 32-column
 // fragment is tokens 16 t + 8 h .. + 7: two transposing reads (tokens .. + 3 and + 4 .. + 7). In each read block lane i
 // (of 16) addresses row i / 4 of the block's 4 token rows at columns 4 (i % 4) .. + 3 of its 16 columns. A row is a
 // number of 32-byte segments; segment s of token row m sits at position s ^ 2 (m & 3), which spreads the 4 rows x 2
-// column blocks that 32 lanes read over all 64 banks; the swizzle is free, since an LDS-direct load lets a lane choose
+// column blocks that 32 lanes read over all 64 banks (rows of 384 bytes alternate between the halves of the banks by themselves and
+// have 12 segments: s ^ (m & 2)); the swizzle is free, since an LDS-direct load lets a lane choose
 // the global 16 bytes that land in its slot.
 //
 // Any number of tokens: see `first` below. Against the tensor library's product, which took the token counts that are
@@ -72,17 +78,15 @@ typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 template <int I>
 using ic = std::integral_constant<int, I>;
 
-// TILE: outputs per workgroup along n and along k, NT: its threads. STEP_M: tokens per reduction step; NST: LDS stages of
-// one step.
-template <int TILE, int NT, int STEP_M, int NST, bool ACC8>
+// TILE_N, TILE_K: outputs per workgroup, NT: its threads. STEP_M: tokens per reduction step; NST: LDS stages of one step.
+template <int TILE_N, int TILE_K, int NT, int STEP_M, int NST, bool ACC8>
 __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
-    constexpr int ROWB = TILE * 2;           // bytes per staged token row of one operand
-    constexpr int OP_STAGE = STEP_M * ROWB;  // bytes per operand and stage
-    constexpr int STAGE = 2 * OP_STAGE;
-    constexpr int LOADS = OP_STAGE / 16 / NT;  // 16-byte loads per thread, operand and stage
+    constexpr int ROW_A = TILE_N * 2, ROW_B = TILE_K * 2;  // bytes per staged token row of dY, of X
+    constexpr int A_STAGE = STEP_M * ROW_A, STAGE = A_STAGE + STEP_M * ROW_B;
+    constexpr int LA = A_STAGE / 16 / NT, LB = STEP_M * ROW_B / 16 / NT;  // 16-byte loads per thread and stage
     constexpr int SL = STEP_M / 16;            // slices of a step (an even number)
     constexpr int WM = 2, WN = NT / 64 / WM;       // waves along n, along k
-    constexpr int TM = TILE / WM, TN = TILE / WN;  // wave tile: 128 n x 64 k, or 64 x 64
+    constexpr int TM = TILE_N / WM, TN = TILE_K / WN;  // wave tile: 128 n x 64 k, 96 x 64, or 64 x 64
     constexpr int FM = TM / 32, FN = TN / 32;
     constexpr bool kLone = FM * FN == 16;  // 256 accumulators: one wave per SIMD
     static_assert(!kLone || !ACC8, "the int8 epilogue wants two waves per SIMD");
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     const int rest = p.tiles_k - band * GN;
     const int bw = rest < GN ? rest : GN;
     const int tile_n = within / bw, tile_k = band * GN + within % bw;
-    const int n0 = tile_n * TILE, k0 = tile_k * TILE;
+    const int n0 = tile_n * TILE_N, k0 = tile_k * TILE_K;
     // A number of tokens that is no multiple of the step leaves the FIRST step short: its last rows are tokens 0 .. first - 1
     // (the rows ahead of them re-read the last of these and are masked out of both operands), and every later step starts on
     // a full stride. Counted from the end the tokens then fall into the same slices of 16 whatever the step, so that the tile
@@ -121,54 +125,52 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     const int first = p.M - (nk - 1) * STEP_M;
 
     // ---- staging: slot s = i * NT + thread of an operand's stage is token row s / (TILE / 8), 16-byte position
-    // s % (TILE / 8); it receives the 16 bytes of segment (pos / 2) ^ 2 (row & 3), half pos & 1. Columns past the end of a matrix
+    // s % (TILE / 8); it receives the 16 bytes of segment (pos / 2) ^ flip(row), half pos & 1. Columns past the end of a matrix
     // re-read its last 8 columns (their results are dropped).
-    unsigned a_off[LOADS], b_off[LOADS];
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
+    auto flip = [](int row, int row_bytes) { return row_bytes % 256 == 0 ? 2 * (row & 3) : row & 2; };
+    unsigned a_off[LA], b_off[LB];
+    auto offset = [&](int i, int tile, int first_col, int cols) {
         const int s = i * NT + (int)threadIdx.x;
-        const int row = s / (TILE / 8), pos = s % (TILE / 8);
-        const int c16 = ((((pos >> 1) ^ (2 * (row & 3))) << 1) | (pos & 1));
-        int ca = n0 / 8 + c16, cb = k0 / 8 + c16;
-        ca = ca < p.N / 8 ? ca : p.N / 8 - 1;
-        cb = cb < p.K / 8 ? cb : p.K / 8 - 1;
-        a_off[i] = (unsigned)((long long)row * p.N * 2 + (long long)ca * 16);
-        b_off[i] = (unsigned)((long long)row * p.K * 2 + (long long)cb * 16);
-    }
-    // load i of a step: 0 .. LOADS-1 fill the dY rows of the stage, LOADS .. 2 LOADS-1 its X rows
+        const int row = s / (tile / 8), pos = s % (tile / 8);
+        const int c = first_col / 8 + ((((pos >> 1) ^ flip(row, tile * 2)) << 1) | (pos & 1));
+        return (unsigned)((long long)row * cols * 2 + (long long)(c < cols / 8 ? c : cols / 8 - 1) * 16);
+    };
+#pragma unroll
+    for (int i = 0; i < LA; ++i) a_off[i] = offset(i, TILE_N, n0, p.N);
+#pragma unroll
+    for (int i = 0; i < LB; ++i) b_off[i] = offset(i, TILE_K, k0, p.K);
+    // load i of a step: 0 .. LA - 1 fill the dY rows of the stage, the LB others its X rows
     auto issue_off = [&](long long row0, unsigned char *st, int i, unsigned off) {
-        const bool is_b = i >= LOADS;
-        const int ii = is_b ? i - LOADS : i;
+        const bool is_b = i >= LA;
+        const int ii = is_b ? i - LA : i;
         const unsigned char *src = is_b ? p.x + row0 * p.K * 2 : p.dy + row0 * p.N * 2;
         const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>(
-            (lds_void *)(st + (is_b ? OP_STAGE : 0) + (ii * NT + wave * 64) * 16));
+            (lds_void *)(st + (is_b ? A_STAGE : 0) + (ii * NT + wave * 64) * 16));
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds_addr), "v"(off), "s"(src) : "memory");
     };
     auto issue_one = [&](int kt, unsigned char *st, int i) {  // kt >= 1, or a full first step
-        const int ii = i >= LOADS ? i - LOADS : i;
-        issue_off((long long)kt * STEP_M - (STEP_M - first), st, i, i >= LOADS ? b_off[ii < LOADS ? ii : 0] : a_off[ii < LOADS ? ii : 0]);
+        issue_off((long long)kt * STEP_M - (STEP_M - first), st, i, i >= LA ? b_off[i >= LA ? i - LA : 0] : a_off[i < LA ? i : 0]);
     };
     auto issue_first = [&](unsigned char *st, int i) {  // step 0: rows ahead of token 0 read the step's last token
-        const int ii = i >= LOADS ? i - LOADS : i;
-        const int row = (ii * NT + (int)threadIdx.x) / (TILE / 8), ahead = STEP_M - first;
+        const int row = ((i >= LA ? i - LA : i) * NT + (int)threadIdx.x) / ((i >= LA ? TILE_K : TILE_N) / 8), ahead = STEP_M - first;
         const unsigned back = (unsigned)(row >= ahead ? ahead : row - (first - 1));  // (modulo 2^32: the offsets stay within the step's tokens)
-        issue_off(0, st, i, i >= LOADS ? b_off[ii < LOADS ? ii : 0] - back * (unsigned)(p.K * 2) : a_off[ii < LOADS ? ii : 0] - back * (unsigned)(p.N * 2));
+        issue_off(0, st, i, i >= LA ? b_off[i >= LA ? i - LA : 0] - back * (unsigned)(p.K * 2) : a_off[i < LA ? i : 0] - back * (unsigned)(p.N * 2));
     };
 
     // ---- fragments. Read block = lane / 16: column block (lane / 16) & 1 of the fragment's 32 columns, token half
     // h; block lane i16 addresses token row (i16 / 4) of the block's 4 and columns 4 (i16 % 4) .. + 3.
     const int i16 = lane & 15, cblk = (lane >> 4) & 1;
     // byte offset of the lane's 8 bytes within a staged row of fragment f (32 columns from column 32 f of the wave's part)
-    auto col_off = [&](int col0) {
+    auto col_off = [&](int col0, int row_bytes) {
         const int seg = (col0 >> 4) + cblk;  // 32-byte segment of the row
-        return ((seg ^ (2 * (i16 >> 2))) << 5) + ((i16 & 3) << 3);
+        return ((seg ^ flip(i16 >> 2, row_bytes)) << 5) + ((i16 & 3) << 3);
     };
     int a_col[FM], b_col[FN];
 #pragma unroll
-    for (int j = 0; j < FM; ++j) a_col[j] = col_off(wm * TM + 32 * j);
+    for (int j = 0; j < FM; ++j) a_col[j] = col_off(wm * TM + 32 * j, ROW_A);
 #pragma unroll
-    for (int i = 0; i < FN; ++i) b_col[i] = OP_STAGE + col_off(wn * TN + 32 * i);
-    const int row_lane = (8 * h + (i16 >> 2)) * ROWB;  // + 16 t rows for slice t, + 4 rows for the second read
+    for (int i = 0; i < FN; ++i) b_col[i] = A_STAGE + col_off(wn * TN + 32 * i, ROW_B);
+    const int row_a = (8 * h + (i16 >> 2)) * ROW_A, row_b = (8 * h + (i16 >> 2)) * ROW_B;  // + 16 t rows for slice t, + 4 rows for the second read
     // a short first step: the lane's rows 16 t + 8 h + e of slice t ahead of the first token become zero
     auto mask_frag = [&](u32x4_t &f, int t) {
         const int ahead = STEP_M - first - (16 * t + 8 * h);
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     };
     // half e (tokens .. + 3, .. + 7) of fragment f of slice t: dY fragments 0 .. FM - 1, then X fragments
     auto read_half = [&](const unsigned char *st, int t, u32x4_t *af, u32x4_t *bf, int f, int e) {
-        const unsigned char *base = st + row_lane + (t * 16 + 4 * e) * ROWB;
+        const unsigned char *base = st + (f < FM ? row_a + (t * 16 + 4 * e) * ROW_A : row_b + (t * 16 + 4 * e) * ROW_B);
         const u32x2_t v = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(base + (f < FM ? a_col[f < FM ? f : 0] : b_col[f >= FM ? f - FM : 0]))));
         u32x4_t &d = f < FM ? af[f < FM ? f : 0] : bf[f >= FM ? f - FM : 0];
         d[2 * e] = v[0];
@@ -227,13 +229,13 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
         };
 #pragma unroll
         for (int t = 0; t < SL; ++t) {
-            if (t == SL - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * 2 * LOADS) : "memory");
+            if (t == SL - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * (LA + LB)) : "memory");
             const unsigned char *src = t < SL - 1 ? cur : nxt;
             const int tn = t < SL - 1 ? t + 1 : 0;
             if constexpr (kLone && !MASKED) {
                 // one wave per SIMD: everything else is dealt out between the MFMAs, the reads of the next slice (in the
                 // order in which it uses them) over the first half of them, so that they are back when it starts
-                static_assert(FM == FN && LOADS <= FM * FN, "one load per MFMA at most");
+                static_assert(FM == FN && LA == LB && LA <= FM * FN, "one load per MFMA at most");
 #pragma unroll
                 for (int m = 0; m < FM * FN; ++m) {
                     constexpr int kReads = 2 * (FM + FN), kPer = kReads / (FM * FN / 2);
@@ -242,8 +244,8 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
                         const int n = m * kPer + q;  // halves: dY 0, X 0, dY 1, X 1, ...
                         if (n < kReads) read_half(src, tn, af[tn & 1], bf[tn & 1], (n >> 1) % 2 == 0 ? (n >> 2) : FM + (n >> 2), n & 1);
                     }
-                    if (m % 2 == 1 && m / 2 < LOADS) {
-                        if (t == 0) load(kt_x, left, LOADS + m / 2);
+                    if (m % 2 == 1 && m / 2 < LA) {
+                        if (t == 0) load(kt_x, left, LA + m / 2);
                         if (t == SL - 1) load(kt_dy, cur, m / 2);
                     }
                     const int i = m / FM, j = m % FM;
@@ -256,11 +258,11 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
             read_frags(src, tn, af[tn & 1], bf[tn & 1]);
             if (t == 0) {
 #pragma unroll
-                for (int i = LOADS; i < 2 * LOADS; ++i) load(kt_x, left, i);
+                for (int i = LA; i < LA + LB; ++i) load(kt_x, left, i);
             }
             if (t == SL - 1) {
 #pragma unroll
-                for (int i = 0; i < LOADS; ++i) load(kt_dy, cur, i);
+                for (int i = 0; i < LA; ++i) load(kt_dy, cur, i);
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (MASKED) {
@@ -280,12 +282,12 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
 #pragma unroll
     for (int s = 0; s < NST; ++s)
 #pragma unroll
-        for (int i = 0; i < (s == NST - 1 ? LOADS : 2 * LOADS); ++i) {
+        for (int i = 0; i < (s == NST - 1 ? LA : LA + LB); ++i) {
             const int k = s < nk ? s : nk - 1;
             if (k == 0) issue_first(stage(s + shift), i);
             else issue_one(k, stage(s + shift), i);
         }
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * 2 * LOADS + LOADS) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * (LA + LB) + LA) : "memory");
     read_frags(stage(shift), 0, af[0], bf[0]);
     __builtin_amdgcn_sched_barrier(0);
     int kt = 0;
@@ -421,56 +423,71 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
     }
 }
 
-template <int TILE, int NT, int STEP_M, int NST, bool ACC8>
+template <int TILE_N, int TILE_K, int NT, int STEP_M, int NST, bool ACC8>
 static int launch_dw_tile(DwParams p, hipStream_t st, const char *who) {
-    p.tiles_n = (p.N + TILE - 1) / TILE;
-    p.tiles_k = (p.K + TILE - 1) / TILE;
+    p.tiles_n = (p.N + TILE_N - 1) / TILE_N;
+    p.tiles_k = (p.K + TILE_K - 1) / TILE_K;
     const long long nwg = (long long)p.tiles_n * p.tiles_k;
     if (nwg > 0x7FFFFFFFll) return lq_fail(LQ_ERR_BAD_ARG, "%s: problem too large", who);
     // the 32-bit lane offsets of the loads span a step's token rows
     if (64ll * 2 * (p.N > p.K ? p.N : p.K) >= (1ll << 32)) return lq_fail(LQ_ERR_BAD_ARG, "%s: rows too long", who);
     const dim3 grid((unsigned)nwg), block(NT);
-    hipLaunchKernelGGL((gemm_dw_kernel<TILE, NT, STEP_M, NST, ACC8>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((gemm_dw_kernel<TILE_N, TILE_K, NT, STEP_M, NST, ACC8>), grid, block, 0, st, p);
     return lq_check_launch(who);
 }
 
-// Which tile a product takes: the smaller of two estimates in microseconds, both of the form (time per 64-token step,
+// Which tile a product takes: the smallest of three estimates in microseconds, all of the form (time per 64-token step,
 // summed over the rounds of workgroups) x steps + the ways in and out, fitted to 760 products of 64 to 4096 tokens, 768^2 to
-// 11008 x 4096 outputs. The last round is never empty: 256 tiles on 256 CUs are one full "last" round. A round of 256 x 256
-// tiles steps in 1.09 us while it leaves half of the CUs idle and in 1.48 with all of them busy (power); 128 x 128 tiles
-// step in 0.43 to 0.50 us alone on a CU, in 0.66 to 0.89 as the second workgroup of a CU joins. What comes around the steps
-// depends on the form: bf16 stores, a gradient read and added as well, or the int8 accumulator's arithmetic, some 17
-// instructions an element, which want every CU and another workgroup's steps beside them. The choice costs 0.2 % over the
-// faster of both on average and 6 % at most; one estimate, of the store form, for all three cost 3, 4 and 9 %. us, small / large:
-//   tokens, outputs     2048, 2048^2   2000, 8192 x 3072   500, 8192 x 3072   500, 5504 x 2048   64, 4096 x 1536   2000, 11008 x 4096
-//   store               20.4 / 39.8    94.9 / 92.6         32.2 / 34.9        18.3 / 18.0        6.5 / 7.7         171 / 153
-//   int8                23.9 / 51.0    105 / 115           41.9 / 50.7        25.0 / 26.8        11.3 / 17.4       188 / 186
+// 11008 x 4096 outputs (192 x 256 tiles: to 430, so that the sum of what a wrong choice costs is smallest). The last round is never
+// empty: 256 tiles on 256 CUs are one full "last" round. A round of 256 x 256 tiles steps in 1.09 us while it leaves half of the CUs
+// idle and in 1.48 with all of them busy (power), of 192 x 256 in 0.81 and 1.13; 128 x 128 tiles step in 0.43 to 0.50 us alone on a CU,
+// in 0.66 to 0.89 as the second workgroup of a CU joins. What comes around the steps depends on the form: bf16 stores, a gradient read
+// and added as well, or the int8 accumulator's arithmetic, some 17 instructions an element, which want every CU and another
+// workgroup's steps beside them. us, 128 x 128 / 192 x 256 / 256 x 256:
+//   tokens, outputs     2048, 2048^2   2000, 8192 x 3072   500, 8192 x 3072   500, 5504 x 2048     64, 4096 x 1536   2000, 11008 x 4096
+//   store               20.4 / - / 39.8    94.9 / - / 92.6     32.2 / 40.4 / 34.1   19.9 / 17.9 / 20.0   6.5 / - / 7.7     171 / - / 153
+//   int8                23.9 / - / 51.0    105 / - / 115       43.8 / 60.7 / 52.8   26.1 / 23.9 / 32.1   11.3 / - / 17.4   188 / - / 186
+// Over the 430 products the medium tile makes the store 1.8 % faster on average, the bf16 add 1.4 and the int8 add 1.6 (up to
+// 17, 16 and 35 %; three are 1 to 3 % slower); the choice costs 0.1, 0.2 and 1.4 % over the fastest of the three.
 enum DwForm { DW_STORE, DW_ACC, DW_ACC8 };
+enum DwTile { DW_128, DW_192, DW_256 };
 
-static bool dw_takes_small_tiles(DwForm form, long long M, long long N, long long K, long long cus) {
+static DwTile dw_tile(DwForm form, long long M, long long N, long long K, long long cus) {
     struct Ways { double once, round, share, second; };  // us per launch, full round, share of the last one, second workgroup on a CU
     constexpr Ways kWays256[] = {{5.2, 6.6, 4.2, 0}, {7.5, 12.4, 6.8, 0}, {14.9, 14.9, 3.2, 0}};
+    constexpr Ways kWays192[] = {{4.94, 4.96, 2.5, 0}, {6.48, 10.0, 4.77, 0}, {13.14, 12.14, 1.12, 0}};
     constexpr Ways kWays128[] = {{3.9, 3.5, 1.0, 1.5}, {5.0, 6.1, 1.9, 2.1}, {7.3, 7.2, 0.8, 2.8}};
-    const long long t256 = ((N + 255) / 256) * ((K + 255) / 256), t128 = ((N + 127) / 128) * ((K + 127) / 128);
-    const long long rounds256 = (t256 - 1) / cus, rounds128 = (t128 - 1) / (2 * cus);
-    const double r256 = (double)(t256 - rounds256 * cus) / (double)cus;      // the last round's share of the CUs, 0 .. 1
+    const double steps = (double)((M + 63) / 64);
+    // one workgroup to a CU: a step in a full round, in the last one, and more of it from half of the CUs on
+    auto whole = [&](long long tiles, double full, double last, double busy, const Ways &w) {
+        const long long rounds = (tiles - 1) / cus;
+        const double share = (double)(tiles - rounds * cus) / (double)cus;  // the last round's share of the CUs, 0 .. 1
+        const double step = full * (double)rounds + last + (share > 0.5 ? busy * (share - 0.5) : 0.0);
+        return step * steps + w.once + w.round * (double)rounds + w.share * share;
+    };
+    const long long tiles_k = (K + 255) / 256, t128 = ((N + 127) / 128) * ((K + 127) / 128);
+    const double est256 = whole((N + 255) / 256 * tiles_k, 1.47, 1.09, 0.78, kWays256[form]);
+    const double est192 = whole((N + 191) / 192 * tiles_k, 1.35, 0.81, 0.63, kWays192[form]);
+    const long long rounds128 = (t128 - 1) / (2 * cus);
     const double r128 = (double)(t128 - rounds128 * 2 * cus) / (double)cus;  // 0 .. 2 workgroups per CU
-    const double step256 = 1.47 * rounds256 + 1.09 + (r256 > 0.5 ? 0.78 * (r256 - 0.5) : 0.0);
-    const double step128 = 0.83 * rounds128 + (r128 <= 1 ? 0.43 + 0.07 * r128 : 0.66 + 0.23 * (r128 - 1));
-    const Ways &w256 = kWays256[form], &w128 = kWays128[form];
-    const double est256 = step256 * (double)((M + 63) / 64) + w256.once + w256.round * rounds256 + w256.share * r256;
-    const double est128 = step128 * 0.5 * (double)((M + 31) / 32) + w128.once + w128.round * rounds128 +
+    const double step128 = 0.83 * (double)rounds128 + (r128 <= 1 ? 0.43 + 0.07 * r128 : 0.66 + 0.23 * (r128 - 1));
+    const Ways &w128 = kWays128[form];
+    const double est128 = step128 * 0.5 * (double)((M + 31) / 32) + w128.once + w128.round * (double)rounds128 +
                           (r128 <= 1 ? w128.share * r128 : w128.second + w128.share * (r128 - 1));
-    return est128 < est256;
+    const double large = est192 < est256 ? est192 : est256;
+    return est128 < large ? DW_128 : est192 < est256 ? DW_192 : DW_256;
 }
 
 static int launch_dw(const DwParams &p, DwForm form, hipStream_t st, const char *who) {
-    const bool acc8 = form == DW_ACC8;
-    if (dw_takes_small_tiles(form, p.M, p.N, p.K, lq_device_cu_count()))
-        return acc8 ? launch_dw_tile<128, 256, 32, 4, true>(p, st, who) : launch_dw_tile<128, 256, 32, 4, false>(p, st, who);
-    if (acc8) return launch_dw_tile<256, 512, 64, 2, true>(p, st, who);
+    const DwTile tile = dw_tile(form, p.M, p.N, p.K, lq_device_cu_count());
+    if (form == DW_ACC8)
+        return tile == DW_128   ? launch_dw_tile<128, 128, 256, 32, 4, true>(p, st, who)
+               : tile == DW_192 ? launch_dw_tile<192, 256, 512, 64, 2, true>(p, st, who)
+                                : launch_dw_tile<256, 256, 512, 64, 2, true>(p, st, who);
+    if (tile == DW_128) return launch_dw_tile<128, 128, 256, 32, 4, false>(p, st, who);
+    if (tile == DW_192) return launch_dw_tile<192, 256, 512, 64, 2, false>(p, st, who);
     // 4 waves of 128 x 128 from where their faster steps outweigh the longer way in and out (see the top of the file)
-    return p.M >= 1536 ? launch_dw_tile<256, 256, 64, 2, false>(p, st, who) : launch_dw_tile<256, 512, 64, 2, false>(p, st, who);
+    return p.M >= 1536 ? launch_dw_tile<256, 256, 256, 64, 2, false>(p, st, who) : launch_dw_tile<256, 256, 512, 64, 2, false>(p, st, who);
 }
 
 static int check_dw(const char *who, const void *dy, const void *x, int64_t M, int64_t N, int64_t K, int k_mult) {

@@ -15,8 +15,7 @@ def ops(hip_lib):
     return ops
 
 
-# on 256 compute units, tiles of (store, add, int8): large, large, small; small, large, small; all large; a short first step
-# of less and of more than half of a large tile's, the tile of four waves (1537)
+# a short first step of less and of more than half of a large tile's, rows and columns beyond the last whole tile
 @pytest.mark.parametrize("M,N,K", [(33, 3072, 3072), (49, 2056, 4112), (97, 3080, 3088), (129, 3072, 3072), (500, 2048, 5504),
                                    (1500, 3072, 3072), (1537, 2048, 5504)])
 def test_forms_on_different_tiles_agree(ops, M, N, K):
