@@ -351,8 +351,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
     // lane offset) so that the compiler's wait-count insertion does not see an LDS write it cannot
     // tell apart from the fragment reads and park a vmcnt(0) in front of them: the explicit
     // s_waitcnt before each barrier is the only ordering these loads need.
-    static_assert(APT % 4 == 0, "A loads are issued in four parts per tile");
-    // part q (0..3) of a tile's loads: APT/4 of them
+    // part q (0..3) of a tile's loads: a quarter of them (of six: 1, 2, 1, 2)
     auto issue_a_part = [&](int kt, unsigned char *la, int q) {
         const bool second = kt >= n_first && pair;
         const unsigned long long addr = (unsigned long long)((second ? a_base2 : a_base) + (long long)(second ? kt - n1 : kt) * ROWB);
@@ -360,7 +359,7 @@ __global__ __launch_bounds__(128 * WM * WN) void gemm_kernel(GemmParams p) {
         const unsigned char *src = (const unsigned char *)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(addr >> 32)) << 32) |
                                                            (unsigned)__builtin_amdgcn_readfirstlane((int)addr));
 #pragma unroll
-        for (int i = q * (APT / 4); i < (q + 1) * (APT / 4); ++i) {
+        for (int i = q * APT / 4; i < (q + 1) * APT / 4; ++i) {
             const unsigned lds_addr = (unsigned)reinterpret_cast<size_t>((lds_void *)(la + (i * NT + wave * 64) * 16));
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                          :: "s"(lds_addr), "v"(a_off[i]), "s"(src) : "memory");
@@ -772,46 +771,6 @@ static int check_w4_common(const char *who, const void *a, const void *codes, co
     return LQ_OK;
 }
 
-// Split reduction of the dX kernels for grids that fill less than half of the compute units: the reduction is cut
-// into up to 8 slices of an even number of steps (at least 8) so that every unit gets at most one
-// workgroup, fp32 partial tiles go to the caller's workspace, then a reduce kernel adds them. Both
-// staged tile heights are tried (128 x 128 at ~0.56 us per step, 256 x 128 at pace_big); the plan
-// with the smaller estimated time is returned (splits = 1: do not split). The estimate counts the
-// partial tiles written and read back through the last-level cache at ~5 TB/s and ~3 us for the
-// second launch.
-struct SplitPlan {
-    int splits = 1, steps_per_split = 0;
-    bool big = false;
-    double est_us = 1e30;
-};
-
-static SplitPlan plan_split(long long M, long long C, int total_steps, size_t ws_bytes, double pace_big, long long cus) {
-    SplitPlan best;
-    if (!ws_bytes) return best;
-    const long long fit = (long long)(ws_bytes / ((size_t)M * C * 4));
-    for (int big = 0; big < 2; ++big) {
-        const long long tiles = ((M + (big ? 255 : 127)) / (big ? 256 : 128)) * ((C + 127) / 128);
-        if (tiles * 2 > cus) continue;
-        long long S = cus / tiles;
-        if (S > 8) S = 8;
-        if (S > fit) S = fit;
-        if (S < 2) continue;
-        int per = (int)((total_steps + S - 1) / S);
-        per += per & 1;
-        if (per < 8) per = 8;
-        S = (total_steps + per - 1) / per;
-        if (S < 2) continue;
-        // with more than three quarters of the units busy the clock gives ~9 % (as for the unsplit kernels)
-        const double busy = 4 * tiles * S > 3 * cus ? 1.09 : 1.0;
-        const double est = busy * (big ? pace_big : 0.56) * (per + 3) * (double)((tiles * S + cus - 1) / cus) + 4.0 + 3.0 +
-                           2.0 * S * M * C * 4 / 5.0e6;
-        if (est < best.est_us) {
-            best.splits = (int)S; best.steps_per_split = per; best.big = big != 0; best.est_us = est;
-        }
-    }
-    return best;
-}
-
 // Which kernel runs a product, and how its reduction is cut (the values of LQ_PLAN_* in latentq.h).
 struct W4Plan {
     int kernel = LQ_PLAN_STAGED_128;
@@ -916,44 +875,90 @@ static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, l
     return out;
 }
 
-// dX: rounds of one workgroup per compute unit at ~0.54 us per 64-deep step for 128 x 128 tiles (0.62 in a last round that
-// fills more than three quarters of the units: 1024 x 4096 x 4096 takes 44.5 us), ~0.75 for 256 x 128 (a second small-tile
-// workgroup on the same unit adds its full time), or a split reduction. Two products into one output (lq_a16w4_dx_pair_ws)
-// are planned as one over twice the rows of W. Unsplit -> this plan, weights from HBM, us (M x N x K, output M x K):
-//   pair of 5504 x 2048   100 tokens 94 -> 21, 500: 98 -> 38, 1000: 100 -> 56
-//   pair of 11008 x 4096  256 tokens 193 -> 57, 512: 194 -> 94, 1024: 212 -> 172; 2048 stays whole (316 against 338)
-//   int8 8192 x 2048      64 tokens 68 -> 17, 512: 79 -> 32, 1024: 84 -> 45, 2048: 91 -> 74
+// ---- dX. Tiles of 128, 192 or 256 rows by 128 columns, one workgroup to a compute unit, and the reduction whole or in slices: the plan
+// with the smallest estimate in microseconds. A tile has one order of its sums, so the height changes no bit; slices do.
+struct DxTile {
+    long long rows;
+    int kernel;
+};
+constexpr DxTile kDxTiles[] = {{128, LQ_PLAN_STAGED_128}, {192, LQ_PLAN_STAGED_192}, {256, LQ_PLAN_STAGED_256}};
+static long long dx_tiles(const DxTile &t, long long M, long long C) { return (M + t.rows - 1) / t.rows * ((C + 127) / 128); }
+
+// Whole: a 64-deep step in a full round of workgroups, in the last one, what that is slower with all units busy than with half of
+// them (clock), the ways in and out of a launch, of a full round, of all of the last one
+struct DxWhole {
+    double full, last, busy, once, round, share;
+};
+static double dx_whole_us(const DxWhole &p, long long tiles, double steps, long long cus) {
+    const long long rounds = (tiles - 1) / cus;
+    const double share = (double)(tiles - rounds * cus) / (double)cus;  // of the last round, 0 .. 1
+    const double step = p.full * (double)rounds + p.last + (share > 0.5 ? p.busy * (share - 0.5) * 2 : 0.0);
+    return step * (steps + 3) + p.once + p.round * (double)rounds + p.share * share;
+}
+// Cut into up to 8 slices of an even number of steps (at least 8), with a workgroup for every unit at most, where whole tiles fill half of
+// the units or less: a step, its slowdown from three quarters of the units on, both launches, the fp32 partial tiles written
+// and read at 5 TB/s, each slice
+struct DxCut {
+    double step, busy, once, traffic, slice;
+};
+
+// 1100 products timed whole and cut with all three heights (64 to 4096 tokens, 1024^2 to 11008 x 4096, 256 units, weights from HBM): the
+// estimates' choice costs 0.2 % over the fastest, and is 2.3 % faster for one product, 4.6 for a pair, 2.7 for int8 weights than
+// the choice between 128 and 256 rows it replaces (at worst 7 % slower, one of 850). us, 128 / 192 / 256 rows:
+//   whole  3648 tokens, int8 6912 x 2560 178 / 163 / 190    3428, pair of 3712 x 1536 113 / 87 / 96    1664, 9088 x 3840 148 / 195 / 128
+//   cut    299 tokens, pair of 9344 x 4096 89 / 68 / 77     500, 5504 x 2048 23.0 / 25.6 / 26.5        384, pair of 11008 x 3584 81 / 77 / 88
+// Unsplit -> cut: pair of 5504 x 2048 at 500 tokens 97 -> 37, of 11008 x 4096 at 512 194 -> 94; int8 8192 x 2048 at 64 68 -> 17, at 2048 84 -> 79.
+// Two products into one output (lq_a16w4_dx_pair_ws) are planned as one over twice the rows of W.
 static W4Plan plan_dx(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
+    constexpr DxWhole kWhole[] = {{0.52, 0.51, 0.09, 0.79, 1.35, 2.42}, {0.76, 0.60, 0.13, 1.19, 2.02, 4.76}, {0.90, 0.66, 0.24, 1.74, 2.41, 6.65}};
+    constexpr DxCut kCut[] = {{0.51, 0.02, 3.71, 1.08, 0.24}, {0.63, 0.05, 4.63, 0.90, 0.15}, {0.72, 0.09, 6.10, 0.76, 0.02}};
+    const long long steps = N / 64, fit = (long long)(ws_bytes / ((size_t)M * K * 4));
     W4Plan out;
-    const long long cols = (K + 127) / 128, small = (M + 127) / 128 * cols, last = small % cus;
-    const double pace_last = last == 0 || 4 * last > 3 * cus ? 0.62 : 0.54;
-    const double est_small = 0.54 * (double)((small + cus - 1) / cus - 1) + pace_last;
-    const double est_big = 0.75 * (double)((((M + 255) / 256) * cols + cus - 1) / cus);
-    out.kernel = est_small < est_big ? LQ_PLAN_STAGED_128 : LQ_PLAN_STAGED_256;
-    const double est_gemm = (est_small < est_big ? est_small : est_big) * (double)(N / 64 + 3) + 4.0;
-    const SplitPlan sp = plan_split(M, K, (int)(N / 64), ws_bytes, 0.75, cus);
-    if (sp.splits >= 2 && sp.est_us < est_gemm) {
-        out.kernel = sp.big ? LQ_PLAN_STAGED_256 : LQ_PLAN_STAGED_128;
-        out.splits = sp.splits;
-        out.steps_per_split = sp.steps_per_split;
+    double best = 1e30;
+    for (int i = 0; i < 3; ++i) {
+        const long long tiles = dx_tiles(kDxTiles[i], M, K);
+        const double whole = dx_whole_us(kWhole[i], tiles, (double)steps, cus);
+        if (whole < best) {
+            best = whole;
+            out.kernel = kDxTiles[i].kernel; out.splits = 1; out.steps_per_split = 0;
+        }
+        long long S = cus / tiles;
+        if (S > 8) S = 8;
+        if (S > fit) S = fit;
+        if (S < 2) continue;
+        long long per = (steps + S - 1) / S;
+        per += per & 1;
+        if (per < 8) per = 8;
+        S = (steps + per - 1) / per;
+        if (S < 2) continue;
+        const DxCut &c = kCut[i];
+        const double share = (double)(tiles * S) / (double)cus;
+        const double cut = (c.step + (share > 0.75 ? c.busy * (share - 0.75) * 4 : 0.0)) * (double)(per + 3) + c.once + c.slice * (double)S +
+                           c.traffic * 8.0 * (double)S * (double)M * (double)K / 5.0e6;
+        if (cut < best) {
+            best = cut;
+            out.kernel = kDxTiles[i].kernel; out.splits = (int)S; out.steps_per_split = (int)per;
+        }
     }
     return out;
 }
 
 // dX with the backward of silu(g) * u behind it: whole, since the slices' sum has no such form. The way out reads and writes four
-// matrices, which a round of 256 x 128 tiles does all at once and 128 x 128 tiles beside the next one's steps: 10 us a round against
-// 2 to 4 (194 products fitted, the slower tile chosen once, by 3 %; with plan_dx's estimate for plain stores 1.6 % slower on average,
-// 20 % at most). us, 128 / 256 rows: 1920 tokens, 1792 -> 5120 55.0 / 64.4; 1722, 2304 -> 4992 66.5 / 76.2; 1928, 2560 -> 7936 102.8 / 95.5.
+// matrices, which a round of 256-row tiles does all at once and 128-row tiles beside the next one's steps (260 products fitted, the
+// choice costs 0.1 % over the fastest; 1.5 % faster than the choice between 128 and 256 rows, one of them 1 % slower). us, 128 / 192 / 256 rows:
+// 716 tokens, 2048 -> 6400 39.7 / 31.6 / 35.8; 744, 3328 -> 11008 93 / 89 / 102; 500, 2048 -> 5504 25.4 / 30.6 / 34.7; 1928, 2560 -> 7936
+// 102.8 / - / 95.5.
 static W4Plan plan_dx_silu(long long M, long long N, long long K, long long cus) {
-    struct Pace { double round, last, busy, once, out_round, out_share; };  // us a step, and a launch's and a round's ways in and out
-    auto est = [&](long long rows, const Pace &p) {
-        const long long tiles = (M + rows - 1) / rows * ((K + 127) / 128), rounds = (tiles - 1) / cus;
-        const double share = (double)(tiles - rounds * cus) / (double)cus;  // of the last round, 0 .. 1
-        const double step = p.round * (double)rounds + p.last + (share > 0.75 ? p.busy * (share - 0.75) * 4 : 0.0);
-        return step * (double)(N / 64 + 3) + p.once + p.out_round * (double)rounds + p.out_share * share;
-    };
+    constexpr DxWhole kWhole[] = {{0.58, 0.46, 0.07, 4.54, 0.15, 4.01}, {0.79, 0.58, 0.11, 5.52, 6.10, 6.02}, {0.99, 0.66, 0.20, 7.16, 7.20, 7.03}};
     W4Plan out;
-    out.kernel = est(128, {0.49, 0.53, 0.07, 3.2, 2.0, 4.4}) < est(256, {0.83, 0.72, 0.14, 5.3, 10.4, 10.1}) ? LQ_PLAN_STAGED_128 : LQ_PLAN_STAGED_256;
+    double best = 1e30;
+    for (int i = 0; i < 3; ++i) {
+        const double est = dx_whole_us(kWhole[i], dx_tiles(kDxTiles[i], M, K), (double)(N / 64), cus);
+        if (est < best) {
+            best = est;
+            out.kernel = kDxTiles[i].kernel;
+        }
+    }
     return out;
 }
 
@@ -1124,7 +1129,9 @@ static int launch_dx(GemmParams p, const W4Plan &plan, void *workspace, hipStrea
         p.partial = (float *)workspace;
         p.steps_per_split = plan.steps_per_split;
     }
-    const int rc = plan.kernel == LQ_PLAN_STAGED_256 ? launch_gemm<MODE, 256, 128, 2, 2>(p, st, who) : launch_gemm<MODE, 128, 128, 2, 2>(p, st, who);
+    const int rc = plan.kernel == LQ_PLAN_STAGED_256   ? launch_gemm<MODE, 256, 128, 2, 2>(p, st, who)
+                   : plan.kernel == LQ_PLAN_STAGED_192 ? launch_gemm<MODE, 192, 128, 2, 2>(p, st, who)
+                                                       : launch_gemm<MODE, 128, 128, 2, 2>(p, st, who);
     if (rc || plan.splits < 2) return rc;
     return launch_split_reduce(p.partial, nullptr, p.c, p.M, p.C, plan.splits, st, who);
 }
@@ -1214,6 +1221,7 @@ extern "C" int lq_calib_gemm_clocks(int backward, const void *a, const void *cod
     const long long wg = plan.kernel == LQ_PLAN_DIRECT ? lq_gemm_fwd_direct_workgroups((int)M, (int)N)
                          : plan.kernel == LQ_PLAN_DIRECT_128 ? lq_gemm_fwd_direct128_workgroups((int)M, (int)N)
                          : plan.kernel == LQ_PLAN_STAGED_256 ? ((M + 255) / 256) * ((cols + 127) / 128)
+                         : plan.kernel == LQ_PLAN_STAGED_192 ? ((M + 191) / 192) * ((cols + 127) / 128)
                          : plan.kernel == LQ_PLAN_FEW        ? N / 16
                                                              : ((M + plan.rows - 1) / plan.rows) * ((cols + 127) / 128);
     LQ_REQUIRE(4 * wg <= clocks_capacity, "lq_calib_gemm_clocks: clocks must hold %lld values, holds %lld", 4 * wg,

@@ -332,7 +332,7 @@ def a16w4_dx_pair(dy1, w1, dy2, w2, shape, out=None, split: bool = False):
 
 
 PLAN_KERNELS = {0: "gemv", 1: "gemv_chunks", 2: "direct_128x256", 3: "staged_128x128", 4: "staged_256x128",
-                5: "direct_128x128", 6: "few_x16"}
+                5: "direct_128x128", 6: "few_x16", 7: "staged_192x128"}
 
 
 def a16w4_plan(M: int, shape, backward: bool = False, workspace_bytes: int = WORKSPACE_MAX_BYTES, compute_units: int = 0):
