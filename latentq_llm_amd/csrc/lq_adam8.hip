@@ -169,34 +169,6 @@ __device__ __forceinline__ u32x2_t quantize8(const float (&x)[8], float scale, f
     return u32x2_t{w[0], w[1]};
 }
 
-// A chunk's 8 updated latent values back to one code word and one residual word (codec parameters by value)
-template <bool kFast>
-__device__ __forceinline__ void requant8(const float (&out)[8], float ws, float wz, float wr, const CodecParams pq,
-                                         unsigned &cnew, unsigned &rnew) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        unsigned nib, code;
-        lq_latent_requant_elem<kFast>(out[k], ws, wz, wr, pq, nib, code);
-        rnew = (rnew << 4) | nib;
-        cnew |= code << (4 * (k ^ 1));
-    }
-}
-
-// The same for an 8-bit-weight layer: 8 code bytes and one residual word per chunk
-template <bool kFast>
-__device__ __forceinline__ void requant8_w8(const float (&out)[8], float ws, float wr, const CodecParams pq, u32x2_t &cnew,
-                                            unsigned &rnew) {
-    unsigned cw[2] = {0u, 0u};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        unsigned nib, byte;
-        lq_latent_w8_requant_elem<kFast>(out[k], ws, wr, pq, nib, byte);
-        rnew = (rnew << 4) | nib;
-        cw[k >> 2] |= byte << (8 * (k & 3));
-    }
-    cnew = u32x2_t{cw[0], cw[1]};
-}
-
 // BS elements share one (scale, max) pair per moment: TPB threads of CH chunks of 8 elements, chunk c of thread t being
 // elements 8 (c TPB + t) .. + 7 of the block, so that every access of a wave is contiguous. BPW blocks per workgroup.
 // TABLES: the block's 512 values by code in LDS (see the top of the file), else computed for each element
@@ -332,32 +304,34 @@ __global__ __launch_bounds__(TABLES ? 128 : 256) void adam8_kernel(Adam8Batch b)
             const float ws = lq_bf16_bits_to_f32(wsb[c]), wz = lq_bf16_bits_to_f32(wzb[c]);
             float out[8], wq[8];
             lq_latent_weights(cword[c], ws, wz, lq_latent_one_fma(ws, wz), wq);
+            const lq_latent_offsets rq = lq_latent_value_offsets(rword[c]);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                const float p = lq_bf16r(lq_latent_value(wq[k], vtab[(rword[c] >> (28 - 4 * k)) & 0xFu], ws));
+                const float p = lq_bf16r(lq_latent_value(wq[k], lq_latent_value_of(vtab, rq, k), ws));
                 out[k] = lq_bf16r(fmaf(a.neg_step, ratio[k], p));
             }
             const float wr = 1.0f / ws;
-            unsigned cnew = 0, rnew = 0;
-            if ((ws >= 0x1p-40f) && (ws <= 0x1p40f)) requant8<true>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
-            else requant8<false>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
+            unsigned cnew, rnew;
+            if ((ws >= 0x1p-40f) && (ws <= 0x1p40f)) lq_latent_requant8<true>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
+            else lq_latent_requant8<false>(out, ws, wz, wr, a.quant_curve, cnew, rnew);
             if (live) {
                 a.codes[T] = cnew;
                 a.residual[T] = rnew;
             }
         } else if constexpr (MODE == ADAM_W8) {
             const float ws = lq_bf16_bits_to_f32(wsb[c]);
+            const lq_latent_offsets rq = lq_latent_value_offsets(rword[c]);
             float out[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                const float p = lq_bf16r(lq_latent_w8_value(c8[c][k >> 2] >> (8 * (k & 3)), vtab[(rword[c] >> (28 - 4 * k)) & 0xFu], ws));
+                const float p = lq_bf16r(lq_latent_w8_value(c8[c][k >> 2] >> (8 * (k & 3)), lq_latent_value_of(vtab, rq, k), ws));
                 out[k] = lq_bf16r(fmaf(a.neg_step, ratio[k], p));
             }
             const float wr = 1.0f / ws;
             u32x2_t cnew;
-            unsigned rnew = 0;
-            if ((fabsf(ws) >= 0x1p-40f) && (fabsf(ws) <= 0x1p40f)) requant8_w8<true>(out, ws, wr, a.quant_curve, cnew, rnew);
-            else requant8_w8<false>(out, ws, wr, a.quant_curve, cnew, rnew);
+            unsigned rnew;
+            if ((fabsf(ws) >= 0x1p-40f) && (fabsf(ws) <= 0x1p40f)) lq_latent_w8_requant8<true>(out, ws, wr, a.quant_curve, cnew, rnew);
+            else lq_latent_w8_requant8<false>(out, ws, wr, a.quant_curve, cnew, rnew);
             if (live) {
                 a.codes8[T] = cnew;
                 a.residual[T] = rnew;

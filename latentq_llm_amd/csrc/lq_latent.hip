@@ -60,15 +60,11 @@ __device__ __forceinline__ void requant_thread(const u32x4_t (&in)[4], float s, 
                                                u32x4_t &cout, u32x4_t &rout) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        unsigned cword = 0, rword = 0;
+        float t[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float t = (k & 1) ? lq_bf16_hi(in[i][k >> 1]) : lq_bf16_lo(in[i][k >> 1]);
-            unsigned nib, code;
-            lq_latent_requant_elem<kFast>(t, s, z, r, p, nib, code);
-            rword = (rword << 4) | nib;
-            cword |= code << (4 * (k ^ 1));
-        }
+        for (int k = 0; k < 8; ++k) t[k] = (k & 1) ? lq_bf16_hi(in[i][k >> 1]) : lq_bf16_lo(in[i][k >> 1]);
+        unsigned cword, rword;
+        lq_latent_requant8<kFast>(t, s, z, r, p, cword, rword);
         cout[i] = cword;
         rout[i] = rword;
     }
@@ -129,16 +125,14 @@ __device__ __forceinline__ void requant_w8_thread(const u32x4_t (&in)[2], float 
     unsigned cw[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        unsigned rword = 0;
+        float t[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float t = (k & 1) ? lq_bf16_hi(in[i][k >> 1]) : lq_bf16_lo(in[i][k >> 1]);
-            unsigned nib, byte;
-            lq_latent_w8_requant_elem<kFast>(t, s, r, p, nib, byte);
-            rword = (rword << 4) | nib;
-            const int e = 8 * i + k;
-            cw[e >> 2] |= byte << (8 * (e & 3));
-        }
+        for (int k = 0; k < 8; ++k) t[k] = (k & 1) ? lq_bf16_hi(in[i][k >> 1]) : lq_bf16_lo(in[i][k >> 1]);
+        u32x2_t codes;
+        unsigned rword;
+        lq_latent_w8_requant8<kFast>(t, s, r, p, codes, rword);
+        cw[2 * i] = codes[0];
+        cw[2 * i + 1] = codes[1];
         rout[i] = rword;
     }
     cout = u32x4_t{cw[0], cw[1], cw[2], cw[3]};
@@ -154,7 +148,7 @@ __global__ __launch_bounds__(256) void latent_w8_requant_kernel(const u32x4_t *_
     in[0] = latent[L * 2];
     in[1] = latent[L * 2 + 1];
     const float s = lq_bf16_bits_to_f32(qscales[L / chunks_per_row]);
-    // the quotient of two bf16 numbers as a product with the reciprocal: see lq_latent_requant_elem
+    // the quotient of two bf16 numbers as a product with the reciprocal: see lq_latent_requant8
     const bool fast = (fabsf(s) >= 0x1p-40f) && (fabsf(s) <= 0x1p40f);
     const float r = 1.0f / s;
     u32x4_t cout;

@@ -24,10 +24,13 @@ __device__ __forceinline__ float lq_round_half_away(float x) {
 __device__ __forceinline__ float lq_round_half_up_nonneg(float x) { return truncf(x + 0.49999997f); }
 
 // Branch-free: the segment only selects the operands of one fused multiply-add and one rounding.
+// kHalf: an |x| of at most 1/2 with no more than 8 significant bits (or NaN). 499 |x| is then exact and half an integer for |x| = 1/2
+// alone, where 249.5 rounds to 250 either way, so that rounding half to even, one instruction, is rounding half up.
+template <bool kHalf = false>
 __device__ __forceinline__ float level_3fold(float x, const CodecParams &p) {
     const float S = fabsf(x);
     float v = fmaf(S, 499.0f, 0.0f);
-    v -= lq_round_half_up_nonneg(v);
+    v -= kHalf ? rintf(v) : lq_round_half_up_nonneg(v);
     const bool in1 = S < p.b1, in2 = S < p.b2;
     const float arg = in1 ? x : (S - (in2 ? p.b1 : p.b2));
     const float slope = in1 ? p.c1 : (in2 ? p.c2 : p.c3);
@@ -52,15 +55,6 @@ __device__ __forceinline__ unsigned nibble_of(float lv, bool &carry) {
     unsigned t;
     asm("v_cvt_u32_f32 %0, %1" : "=v"(t) : "v"(lv + 8.0f));
     return carry ? 1u : (t & 0xFu);
-}
-
-// The same for a level of level_3fold of an |x| <= 1/2, which is no wild input: without a carry it is at most 7, and the
-// conversion's saturation is all that a level below -8 needs
-__device__ __forceinline__ unsigned nibble_of_half(float lv, bool &carry) {
-    carry = lv > 7.5f;
-    unsigned t;
-    asm("v_cvt_u32_f32 %0, %1" : "=v"(t) : "v"(lv + 8.0f));
-    return carry ? 1u : t;
 }
 
 // nibble - 8 -> value of the three-segment curve (inverse slopes in p), branch-free
