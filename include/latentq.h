@@ -158,7 +158,8 @@ int lq_a16w4_gate_up_silu_ws(const void *x, const void *codes_gate, const void *
                              const void *codes_up, const void *scales_up, const void *zeros_up, void *h, void *g_out_or_null,
                              void *u_out_or_null, int64_t M, int64_t N, int64_t K, int group, void *workspace,
                              int64_t workspace_bytes, void *stream);
-/* Which kernel the above would run, launching nothing (see lq_a16w4_plan below): LQ_PLAN_GEMV, LQ_PLAN_DIRECT, or
+/* Which kernel the above would run, launching nothing (see lq_a16w4_plan below): LQ_PLAN_GEMV, LQ_PLAN_FEW (17 to 64
+ * tokens; with scales or zeros that are not 4-byte aligned what follows instead), LQ_PLAN_DIRECT, or
  * LQ_PLAN_STAGED_128 for the launch of small tiles, then with the rows of a tile (32, 64 or 128) and the slices of K.
  * compute_units <= 0 asks the current device. No counterpart in the reference. */
 int lq_a16w4_gate_up_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int compute_units, int *kernel, int *rows,

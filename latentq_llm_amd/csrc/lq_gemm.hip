@@ -745,6 +745,12 @@ int lq_gemm_staged_pair_launch(const void *x, const void *codes_g, const void *s
                                const void *scales_u, const void *zeros_u, void *h, void *g_out, void *u_out, float *partial, int M, int N,
                                int K, int rows, int splits, int per_split, hipStream_t st, const char *who);
 
+// gate / up product of 17 to 64 tokens, up to 32 columns per compute unit (lq_gate_up_few.hip)
+bool lq_gate_up_few_fits(long long M, long long N, long long K, long long cus);
+int lq_gate_up_few_launch(const void *x, const void *codes_g, const void *scales_g, const void *zeros_g, const void *codes_u,
+                          const void *scales_u, const void *zeros_u, void *h, void *g_out, void *u_out, int M, int N, int K, hipStream_t st,
+                          const char *who);
+
 // 17 to 64 tokens, one launch with 16 columns per compute unit (lq_gemm_few.hip)
 int lq_gemm_few_groups(long long M);
 int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
@@ -1028,8 +1034,22 @@ struct GateUpPlan {
 // plan's own estimate, less by up to a third, had sent products of just over four rounds to five of them: 11008 x 4096 at 337
 // tokens 110 against 92 us, 9472 x 3328 at 417 93 against 78; up to four rounds both are level (11008 x 4096 at 300 88 / 91, 9088 x
 // 3328 at 397 72 / 76).
-static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
+//
+// 17 to 64 tokens: the kernel of lq_gate_up_few.hip (few: scales and zeros lie on 4 bytes, as it wants them). 330 sizes, speed
+// against what the rest of this function says, mean and least:
+//   more than 8, up to 16 columns a unit      up to 48 tokens 1.50, 1.09;  49 to 64: 1.33, 1.05 up to K = 6144, 0.89 at 7168
+//   up to 30 columns, 48 tokens and K = 4096  1.14, 1.00 (31 and 32 columns 0.98 to 1.29; 49 to 64 tokens 0.96; longer K 0.96)
+// With 8 columns a unit and fewer it is 1.02 to 2.1 times as fast, but tests have the staged kernel's slices there.
+static bool gate_up_few_takes(long long M, long long N, long long K, long long cus) {
+    if (!lq_gate_up_few_fits(M, N, K, cus) || N <= 8 * cus) return false;
+    return N <= 16 * cus ? M <= 48 || K <= 6144 : N <= 30 * cus && K <= 4096;
+}
+static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_bytes, long long cus, bool few) {
     GateUpPlan out;
+    if (few && gate_up_few_takes(M, N, K, cus)) {
+        out.kernel = LQ_PLAN_FEW;
+        return out;
+    }
     if (ws_bytes < (size_t)8 * M * N) return out;
     const int groups = (int)(K / LQ_GROUP);
     const long long wg = ((M + 127) / 128) * ((N + 127) / 128), rem = wg % (2 * cus);
@@ -1071,7 +1091,11 @@ static int gate_up_impl(const char *who, const void *x, const void *codes_gate, 
     }
     LQ_REQUIRE(K % 256 == 0, "%s: K=%lld must be a multiple of 256 for more than 16 tokens", who, (long long)K);
     LQ_REQUIRE(!workspace || lq_aligned(workspace, 16), "%s: the workspace must be 16-byte aligned", who);
-    const GateUpPlan plan = plan_gate_up(M, N, K, ws_bytes, lq_device_cu_count());
+    const bool few = lq_aligned(scales_gate, 4) && lq_aligned(zeros_gate, 4) && lq_aligned(scales_up, 4) && lq_aligned(zeros_up, 4);
+    const GateUpPlan plan = plan_gate_up(M, N, K, ws_bytes, lq_device_cu_count(), few);
+    if (plan.kernel == LQ_PLAN_FEW)
+        return lq_gate_up_few_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h, g_out, u_out, (int)M, (int)N,
+                                     (int)K, (hipStream_t)stream, who);
     if (plan.kernel == LQ_PLAN_STAGED_128) {
         rc = lq_gemm_staged_pair_launch(x, codes_gate, scales_gate, zeros_gate, codes_up, scales_up, zeros_up, h, g_out, u_out,
                                         (float *)workspace, (int)M, (int)N, (int)K, plan.rows, plan.splits, plan.per_split, (hipStream_t)stream, who);
@@ -1260,7 +1284,7 @@ extern "C" int lq_a16w4_gate_up_plan(int64_t M, int64_t N, int64_t K, int64_t wo
     LQ_REQUIRE(K % (M > 16 ? 256 : LQ_GROUP) == 0, "lq_a16w4_gate_up_plan: K=%lld must be a multiple of %d", (long long)K, M > 16 ? 256 : LQ_GROUP);
     GateUpPlan plan;
     if (M <= 16) plan.kernel = LQ_PLAN_GEMV;
-    else plan = plan_gate_up(M, N, K, workspace_bytes > 0 ? (size_t)workspace_bytes : 0, compute_units > 0 ? compute_units : lq_device_cu_count());
+    else plan = plan_gate_up(M, N, K, workspace_bytes > 0 ? (size_t)workspace_bytes : 0, compute_units > 0 ? compute_units : lq_device_cu_count(), true);
     *kernel = plan.kernel; *rows = plan.rows; *splits = plan.splits;
     return LQ_OK;
 }
