@@ -213,7 +213,7 @@ int lq_a16w4_dx_pair_ws(const void *dy1, const void *codes1, const void *scales1
 #define LQ_PLAN_STAGED_128 3   /* staged kernel, 128 x 128 tiles (forward: 32, 64 or 128 rows) */
 #define LQ_PLAN_STAGED_256 4   /* staged kernel, 256 x 128 tiles */
 #define LQ_PLAN_DIRECT_128 5   /* weights-direct forward kernel, 128 x 128 tiles */
-#define LQ_PLAN_FEW 6          /* 17..64 tokens forward: 16 columns per workgroup, K shared by its waves */
+#define LQ_PLAN_FEW 6          /* 17..128 tokens forward: 16 columns per workgroup, K shared by its waves */
 #define LQ_PLAN_STAGED_192 7   /* dX: staged kernel, 192 x 128 tiles */
 int lq_a16w4_plan(int backward, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int compute_units,
                   int *kernel, int *splits, int *steps_per_split);

@@ -751,7 +751,7 @@ int lq_gate_up_few_launch(const void *x, const void *codes_g, const void *scales
                           const void *scales_u, const void *zeros_u, void *h, void *g_out, void *u_out, int M, int N, int K, hipStream_t st,
                           const char *who);
 
-// 17 to 64 tokens, one launch with 16 columns per compute unit (lq_gemm_few.hip)
+// 17 to 128 tokens, one launch with 16 columns per compute unit (lq_gemm_few.hip)
 int lq_gemm_few_groups(long long M);
 int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
                        int K, hipStream_t st, unsigned long long *clk, const char *who);
@@ -797,22 +797,36 @@ static int whole_pairs(int per, int splits, int groups) {
     return splits > 1 && groups % 2 == 0 && per % 2 && (groups + per) / (per + 1) == splits ? per + 1 : per;
 }
 
-// Where the kernel of lq_gemm_few.hip runs, 17 to 64 tokens. A tile of 16 columns for each of more than half of the units, at most all:
+// Where the kernel of lq_gemm_few.hip runs, 17 to 128 tokens. A tile of 16 columns for each of more than half of the units, at most all:
 // everywhere up to K = 8192 (1.01 to 1.3 times the speed of what ran there, 260 sizes), and for up to 32 tokens and less than all units
 // beyond (1.05 to 1.26; 4096 columns of K = 11008 15.2 against 15.6 us, where a test has the staged kernel). More columns, two rounds of
 // workgroups: up to 32 tokens in place of GEMV launches (1.16 to 1.9), beyond 0.86 to 1.28. Half of the units and fewer (1.1 to 2.2
 // times the speed up to 48 tokens, 0.94 to 1.4 beyond K = 4096 and 48 tokens) but for the sizes at which tests have the other
 // kernels: the smallest matrices, the longest rows, half of the units and rows longer than 2048, columns that are no whole tiles of the
 // staged kernel.
+//
+// 65 tokens and more, against the staged kernel's slices and their sum (310 sizes from K = 1024 on, speed: mean and least; every
+// workgroup reads all of X, so a longer K and fewer columns are what ends it; an even number of groups, and whole tiles of the staged
+// kernel on half of the units and fewer, since tests have that kernel beside them):
+//                                65 to 96 tokens                          97 to 128
+//   up to 4 columns a unit       1.28, 1.08 to K = 3072; 0.97 at 4096     1.16, 1.13 to K = 2048; 0.94, 0.91 to 3072
+//   up to 8                      1.25, 1.01 to K = 5376; 0.92 beyond      1.18, 1.15 to K = 2048; 1.02, 0.93 to 3072
+//   up to 12                     1.27, 1.09 to K = 5376; 1.02, 0.95       1.19, 1.05 to K = 3072; 1.06, 0.98 to 4096
+//   up to 16                     1.25, 0.99 to K = 7168                   1.15, 1.01 to K = 4096; 1.00, 0.98 to 5376
 static bool few_takes(long long M, long long N, long long K, long long cus) {
     if (K / LQ_GROUP > lq_gemm_few_groups(M)) return false;
+    if (M > 64) {
+        if (K < 1024 || K % 256 != 0 || N > 16 * cus || (N <= 8 * cus && N % 128 != 0)) return false;
+        if (M <= 96) return K <= (N <= 4 * cus ? 3072 : N <= 12 * cus ? 5376 : 7168);
+        return K <= (N <= 8 * cus ? 2048 : N <= 12 * cus ? 3072 : 4096);
+    }
     if (N > 16 * cus) return M <= 32 && N <= 32 * cus && K < 8192 && N * K <= 4096ll * 4096;
     if (2 * N > 16 * cus) return K < 8192 || (M <= 32 && N < 16 * cus);
     if (N % 128 != 0 || K >= (M <= 48 ? 8192 : 7168)) return false;
     return M <= 32 ? N * K > 2048ll * 2048 : N * K >= 1024ll * 2048 && (2 * N < 16 * cus || K <= 2048);
 }
 
-// Forward pass, M > 16. Up to 64 tokens the kernel of lq_gemm_few.hip where few_takes says so. Otherwise, up to 64 tokens the staged kernel on any number of tiles, with weights that are not rounded to bf16
+// Forward pass, M > 16. Up to 128 tokens the kernel of lq_gemm_few.hip where few_takes says so. Otherwise, up to 64 tokens the staged kernel on any number of tiles, with weights that are not rounded to bf16
 // (several workgroups to a unit: 32 tokens, 16400 x 4096 23.8 against 35.7 us of the weights-direct kernel, 32000 x 4096 27.1
 // against 40.2, 40960 x 768 10.8 against 16.3), and beyond by the number of 128 x 128 output tiles T:
 //   T <= half of the units             the staged kernel, which plans its row tile and its slices of K itself
