@@ -799,7 +799,8 @@ static int whole_pairs(int per, int splits, int groups) {
 
 // Where the kernel of lq_gemm_few.hip runs, 17 to 128 tokens. A tile of 16 columns for each of more than half of the units, at most all:
 // everywhere up to K = 8192 (1.01 to 1.3 times the speed of what ran there, 260 sizes), and for up to 32 tokens and less than all units
-// beyond (1.05 to 1.26; 4096 columns of K = 11008 15.2 against 15.6 us, where a test has the staged kernel). More columns, two rounds of
+// beyond (1.05 to 1.26); beyond, whole tiles of the staged kernel and an even number of groups, up to 48 tokens and
+// K = 10752 1.01 to 1.29 (11008 0.95 to 1.08; 64 tokens 0.84 to 1.11; 1.14 to 1.33 at K = 8192 as well, where a test has the staged kernel). More columns, two rounds of
 // workgroups: up to 32 tokens in place of GEMV launches (1.16 to 1.9), beyond 0.86 to 1.28. Half of the units and fewer (1.1 to 2.2
 // times the speed up to 48 tokens, 0.94 to 1.4 beyond K = 4096 and 48 tokens) but for the sizes at which tests have the other
 // kernels: the smallest matrices, the longest rows, half of the units and rows longer than 2048, columns that are no whole tiles of the
@@ -821,7 +822,8 @@ static bool few_takes(long long M, long long N, long long K, long long cus) {
         return K <= (N <= 8 * cus ? 2048 : N <= 12 * cus ? 3072 : 4096);
     }
     if (N > 16 * cus) return M <= 32 && N <= 32 * cus && K < 8192 && N * K <= 4096ll * 4096;
-    if (2 * N > 16 * cus) return K < 8192 || (M <= 32 && N < 16 * cus);
+    if (2 * N > 16 * cus) return K < 8192 || (M <= 32 && N < 16 * cus) ||
+                                    (M <= 48 && N % 128 == 0 && K % 256 == 0 && K > 8192 && K <= 10752);
     if (N % 128 != 0 || K >= (M <= 48 ? 8192 : 7168)) return false;
     return M <= 32 ? N * K > 2048ll * 2048 : N * K >= 1024ll * 2048 && (2 * N < 16 * cus || K <= 2048);
 }

@@ -23,11 +23,12 @@
 // against the kernels of other sizes (GEMV launches up to 32 tokens, staged):
 //     2048 x 4096    8.3 -> 5.8       9.4 -> 5.9       10.3 -> 6.9      10.8 -> 7.9
 //     1536 x 1536                                      8.0 -> 4.5       8.2 -> 5.3
-// From 65 tokens on (rows of X in halves of a group, gemm_few_half_kernel), against the staged kernel's slices and the launch that adds them:
+// From 65 tokens on and on long rows (rows of X in halves of a group, gemm_few_half_kernel), against the staged kernel's slices and the launch that adds them:
 //                    65 tokens        80              96              128
 //     4096 x 4096    12.6 -> 10.0                     13.5 -> 11.5    15.1 -> 13.9
 //     1536 x 1536                     8.0 -> 5.6
 //     2560 x 2560                                     11.3 -> 9.4 (97)
+//     4096 x 9728 at 20 / 32 / 48 tokens 14.6 -> 12.9, 15.1 -> 13.0, 17.8 -> 15.4;  3072 x 9216 at 45 16.4 -> 13.3
 // Also measured, 4096 x 4096 at 45 tokens: 32 columns a workgroup on half of the units 12.4; no rows of X after the first group 7.2, of
 // the weights 8.0; no conversions 8.5, no LDS reads 8.6; units starting at different groups 8.8; codes of neighbouring groups in one
 // piece of 128 bytes 8.7; X requested ahead of all but the first group's codes 8.6 (2560 x 2560 5.8).
@@ -215,8 +216,8 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(
     }
 }
 
-// The same for 65 to 128 tokens, whose rows of a whole group would leave LDS room for few waves: rows of X come 64 k at a time, and the
-// sums of a group are scaled after both halves. LDS of a wave: codes, scales and zeros as above;
+// The same for 65 to 128 tokens and for long rows, where rows of X of a whole group would leave LDS room for few waves: they come 64 k at
+// a time, and the sums of a group are scaled after both halves. LDS of a wave: codes, scales and zeros as above;
 //   activations  16 MT rows of 128 bytes, piece c of row i at c ^ ((i >> 1) & 7)
 // With r, h as above slice w = 0, 1 of half s has the lane's operands at k = 64 s + 16 h + 8 w .. + 7.
 constexpr int few_half_lds(int MT, int NG, int W) { return W * (NG * 1024 + (NG + 1) / 2 * 256 + MT * 2048); }
@@ -315,15 +316,18 @@ __global__ __launch_bounds__(64 * W) void gemm_few_half_kernel(
 }
 
 // The forms, by groups of 16 tokens: eight waves where LDS holds their codes, and the most waves for longer rows. A row of G groups
-// takes the first whose waves have room for it. (More than 32 tokens of rows from K = 8192 on are the staged kernel's.)
+// takes the first whose waves have room for it. Rows of X in halves of a group where whole ones would leave room for fewer waves: 4096 x 5120
+// at 45 / 60 tokens 9.2 / 10.7 us on six and five waves with whole groups, 9.0 / 9.9 on eight with halves.
 struct FewForm {
     int waves, groups;  // groups a wave has room for
+    bool half;          // rows of X in halves of a group
 };
 template <int MT>
-constexpr int kFewForms = MT == 2 ? 3 : 2;
+constexpr int kFewForms = MT <= 3 ? 3 : 2;
 template <int MT>
 constexpr FewForm few_form(int i) {
-    constexpr FewForm forms[5][3] = {{{8, 4}, {8, 8}, {6, 15}}, {{8, 4}, {6, 11}, {}}, {{7, 5}, {5, 13}, {}}, {{8, 4}, {8, 7}, {}}, {{8, 3}, {7, 6}, {}}};
+    constexpr FewForm forms[5][3] = {{{8, 4, false}, {8, 8, false}, {6, 15, false}}, {{8, 4, false}, {8, 8, true}, {8, 11, true}},
+                                     {{7, 5, false}, {8, 8, true}, {}}, {{8, 4, true}, {8, 7, true}, {}}, {{8, 3, true}, {7, 6, true}, {}}};
     return forms[MT <= 4 ? MT - 2 : MT / 2][i];  // 2, 3, 4, 6, 8
 }
 template <int MT>
@@ -334,7 +338,7 @@ void few_launch(int G, Launch &&launch) {
     constexpr FewForm f = few_form<MT>(I);
     if constexpr (I + 1 < kFewForms<MT>)
         if (G > f.waves * f.groups) return few_launch<MT, I + 1>(G, launch);
-    if constexpr (MT <= 4) launch(gemm_few_kernel<MT, f.groups, f.waves>, f.waves);
+    if constexpr (!f.half) launch(gemm_few_kernel<MT, f.groups, f.waves>, f.waves);
     else launch(gemm_few_half_kernel<MT, f.groups, f.waves>, f.waves);
 }
 
