@@ -13,13 +13,11 @@
 #include <ATen/SavedTensorHooks.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
-#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/forward_grad.h>
-#include <torch/csrc/autograd/function.h>
-#include <torch/csrc/autograd/functions/utils.h>
-#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/latentq.h"
@@ -618,96 +616,13 @@ PyObject *set_error(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     return none();
 }
 
-// -> whether a layer in training can have its result's history from attach: autograd records, and nothing looks at the call that an
-// autograd Function's own machinery would answer (a trace, a transform, hooks on saved tensors, a dispatch mode)
-PyObject *records_plainly(PyObject *, PyObject *const *, Py_ssize_t nargs) {
-    LQ_ARGS(0)
-    return PyBool_FromLong(c10::GradMode::is_enabled() && !c10::InferenceMode::is_enabled() && !watched() &&
-                           !c10::impl::dispatch_mode_enabled() && at::SavedTensorDefaultHooks::get_tls_state().stack.empty());
-}
-
-// The node of a layer in training: its backward is a Python function, called with what the layer left for it, the tensors saved
-// (as autograd saves them: checked for changes in place, gone after the backward unless the graph is kept), dy as rows, and whether dx
-// is wanted. A Python autograd Function's own way there and back costs the host 15 us a call, and the views around one that takes
-// rows another 12; the kernels of a small layer's step run for 40. Two micro-batches of 1024 tokens through 3072 x 768 with int4
-// weights: 209.7 -> 164.5 us, of which the engine's thread, woken for the backward and waited for, takes 35 each.
-struct LayerNode : torch::autograd::Node {
-    std::vector<torch::autograd::SavedVariable> saved;
-    at::DimVector shape;  // of dx
-    c10::SafePyObject backward, left;
-    std::string called;
-
-    LayerNode(PyObject *f, PyObject *l, const char *name)
-        : backward((Py_INCREF(f), f), getPyInterpreter()), left((Py_INCREF(l), l), getPyInterpreter()), called(name) {}
-    std::string name() const override { return called; }
-    void release_variables() override {
-        std::lock_guard<std::mutex> lock(mutex_);
-        for (auto &v : saved) v.reset_data();
-    }
-
-    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
-        at::Tensor dy = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
-        dy = dy.dim() == 2 ? dy : dy.reshape({-1, dy.size(-1)});
-        torch::autograd::variable_list tensors;
-        {
-            std::lock_guard<std::mutex> lock(mutex_);
-            for (const auto &v : saved) tensors.push_back(v.unpack());
-        }
-        const bool wanted = task_should_compute_output(0);
-        at::Tensor dx;
-        {
-            pybind11::gil_scoped_acquire gil;
-            auto one = [](PyObject *o) {
-                if (!o) {  // to the thread that called backward
-                    python_error e;
-                    e.persist();
-                    throw e;
-                }
-                return pybind11::reinterpret_steal<pybind11::object>(o);
-            };
-            const pybind11::object list = one(PyTuple_New((Py_ssize_t)tensors.size())), d = one(THPVariable_Wrap(dy));
-            for (size_t i = 0; i < tensors.size(); ++i) PyTuple_SET_ITEM(list.ptr(), i, one(THPVariable_Wrap(tensors[i])).release().ptr());
-            PyObject *args[4] = {left.ptr(getPyInterpreter()), list.ptr(), d.ptr(), wanted ? Py_True : Py_False};
-            const pybind11::object r = one(PyObject_Vectorcall(backward.ptr(getPyInterpreter()), args, 4, nullptr));
-            if (THPVariable_Check(r.ptr())) dx = THPVariable_Unpack(r.ptr());
-        }
-        torch::autograd::variable_list out(num_outputs());
-        if (wanted && dx.defined()) out[0] = dx.sizes() == at::IntArrayRef(shape) ? dx : dx.reshape(shape);
-        return out;
-    }
-};
-
-// y, x, bias or None, saved tensors (a tuple), backward, what it is called with, name -> y, which from here on has the history of a
-// function of x and bias
-PyObject *attach(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    LQ_ARGS(7)
-    if (!THPVariable_Check(a[0]) || !THPVariable_Check(a[1]) || (a[2] != Py_None && !THPVariable_Check(a[2])) || !PyTuple_CheckExact(a[3])) {
-        PyErr_SetString(PyExc_TypeError, "attach: tensors expected");
-        return nullptr;
-    }
-    const char *name = PyUnicode_AsUTF8(a[6]);
-    if (!name) return nullptr;
-    const at::Tensor &y = THPVariable_Unpack(a[0]), &x = THPVariable_Unpack(a[1]);
-    at::Tensor bias;
-    if (a[2] != Py_None) bias = THPVariable_Unpack(a[2]);
-    Py_INCREF(a[0]);
-    const pybind11::object result = pybind11::reinterpret_steal<pybind11::object>(a[0]);
-    if (torch::autograd::compute_requires_grad(x, bias)) {
-        std::shared_ptr<LayerNode> node(new LayerNode(a[4], a[5], name), torch::autograd::deleteNode);
-        node->set_next_edges(torch::autograd::collect_next_edges(x, bias));
-        node->shape = at::DimVector(x.sizes().begin(), x.sizes().end());
-        const Py_ssize_t n = PyTuple_GET_SIZE(a[3]);
-        for (Py_ssize_t i = 0; i < n; ++i) {
-            PyObject *t = PyTuple_GET_ITEM(a[3], i);
-            if (!THPVariable_Check(t)) {
-                PyErr_SetString(PyExc_TypeError, "attach: tensors expected");
-                return nullptr;
-            }
-            node->saved.emplace_back(THPVariable_Unpack(t), false);
-        }
-        torch::autograd::set_history(y, node);
-    }
-    return pybind11::object(result).release().ptr();
+// x -> whether a layer in training can take its short way: activations in plain form, autograd records, and nothing looks at the call
+// that is given the tensors of the Function over rows otherwise (a trace, a transform, hooks on saved tensors, a dispatch mode)
+PyObject *records_plainly(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
+    LQ_ARGS(1)
+    const at::Tensor *x = bf16(a[0]);
+    return PyBool_FromLong(x && x->dim() >= 1 && x->numel() > 0 && c10::GradMode::is_enabled() && !c10::InferenceMode::is_enabled() &&
+                           !watched() && !c10::impl::dispatch_mode_enabled() && at::SavedTensorDefaultHooks::get_tls_state().stack.empty());
 }
 
 #define LQ_METHOD(f) {#f, (PyCFunction)(void (*)(void))guarded<f>, METH_FASTCALL, nullptr}
@@ -730,7 +645,7 @@ PyMethodDef methods[] = {
     LQ_METHOD(infer8_eval), LQ_METHOD(dx8), LQ_METHOD(quant8), LQ_METHOD(quant8_token), LQ_METHOD(dequant8), LQ_METHOD(weight_grad),
     LQ_METHOD(weight_grad_acc), LQ_METHOD(weight_grad_acc8), LQ_METHOD(gradq8), LQ_METHOD(adam8_param), LQ_METHOD(adam8_sr),
     LQ_METHOD(adam8_queue), LQ_METHOD(adam8_run), LQ_METHOD(adam8_w4), LQ_METHOD(adam8_w8), LQ_METHOD(current_stream),
-    LQ_METHOD(records_plainly), LQ_METHOD(attach), LQ_METHOD(set_error), {nullptr, nullptr, 0, nullptr}};
+    LQ_METHOD(records_plainly), LQ_METHOD(set_error), {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_lqbind", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

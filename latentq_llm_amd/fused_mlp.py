@@ -47,7 +47,7 @@ class _FusedMLPTrain(torch.autograd.Function):
 def _mlp_backward(mlp, saved, grad_output, wanted):
     from .quant import _pending_dw, _rows, backward_hook_fn, dict_temp
     x2, g, u, h = saved
-    x2 = _rows(x2)
+    x2, grad_output = _rows(x2), _rows(grad_output)
     gate, up, down = mlp.gate_proj, mlp.up_proj, mlp.down_proj
     inter, K = mlp.intermediate_size, mlp.infeatures
     dy = grad_output.to(torch.bfloat16).contiguous()
@@ -63,7 +63,7 @@ def _mlp_backward(mlp, saved, grad_output, wanted):
 
 
 def _mlp_node(mlp, x):
-    """_FusedMLPTrain without an autograd Function of Python's (quant._NODES)."""
+    """_FusedMLPTrain on activations of any number of dimensions (quant._attach)."""
     down, inter = mlp.down_proj, mlp.intermediate_size
     h, g, u = ops.a16w4_gate_up_silu(quant._rows(x.detach()), _w4(mlp.gate_proj), _w4(mlp.up_proj), (inter, mlp.infeatures), save=True)
     bias = None if down.bias is None else down.bias.detach().to(torch.bfloat16).contiguous()
@@ -94,7 +94,7 @@ class QuantLlamaMLP(nn.Module):
             return self.down_proj(self.fused_gate_up(x))
         if (x.dtype == torch.bfloat16 and x.numel() > 0 and x.shape[-1] % 256 == 0 and self.intermediate_size % 64 == 0
                 and self.outfeatures % 64 == 0):
-            if quant._plain_activations(x) and quant._records_plainly(x):
+            if quant._records_plainly(x):
                 y = _mlp_node(self, x)
                 if y is not None:
                     return y

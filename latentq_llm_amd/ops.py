@@ -255,17 +255,17 @@ def a16w4_dx_silu_bwd(dy, codes, scales, zeros, shape, g, u):
 
 
 def dx4(dy, codes, scales, zeros, shape):
-    """a16w4_dx of rows dy; None if an operand is not in the plain form the native binding takes."""
-    if dy.dim() != 2 or not dy.is_cuda or not dy.shape[0]:
+    """a16w4_dx for dy of any number of dimensions; None if an operand is not in the plain form the native binding takes."""
+    if not dy.is_cuda or not dy.numel():
         return None
     N, K = shape
-    return (_native or _fast()).dx4(dy, codes, scales, zeros, N, K, _workspace(dy, dy.shape[0], K)[0])
+    return (_native or _fast()).dx4(dy, codes, scales, zeros, N, K, _workspace(dy, dy.numel() // N, K)[0])
 
 
 def a16w4_dx(dy, codes, scales, zeros, shape, out=None, accumulate=False):
     """dX[M,K] = dY[M,N] . deq(W)[N,K]; accumulate=True: out = bf16(out + bf16(dY . deq(W))) (lq_a16w4_dx_acc)."""
     N, K = shape
-    if out is None and not accumulate:
+    if out is None and not accumulate and dy.dim() == 2:
         r = dx4(dy, codes, scales, zeros, shape)
         if r is not None:
             return r

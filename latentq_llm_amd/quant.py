@@ -25,7 +25,7 @@ from __future__ import annotations
 
 import math
 from collections import OrderedDict
-from functools import reduce
+from functools import lru_cache, reduce
 from typing import Optional, Union
 
 import torch
@@ -225,6 +225,10 @@ def _ctx_form(fn, forward):
 # biases never receive a gradient there. Kept as is so that training runs match the reference.
 _BIAS_FLAG = 2
 
+def _rows(x):
+    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+
+
 def _as_bf16_2d(x):
     return x.contiguous() if x.dtype == torch.bfloat16 else x.to(torch.bfloat16).contiguous()
 
@@ -240,17 +244,17 @@ def _w4_linear(input, weight_d, qparamw4, bias):
 
 
 def _w4_backward(layer, qparam, input, weight_d, grad_output, wanted):
-    """The input's gradient of rows, where wanted; the weight's to its layer."""
+    """The input's gradient, where wanted (as rows, or shaped as the result's); the weight's to its layer."""
     dy = _as_bf16_2d(grad_output)
     grad_input = None
     if wanted:
         grad_input = ops.dx4(dy, weight_d, *qparam)
         if grad_input is None:
             scales, zeros, shape = _flat_qparam(qparam)
-            grad_input = ops.a16w4_dx(dy, weight_d, scales, zeros, shape)
+            grad_input = ops.a16w4_dx(_rows(dy), weight_d, scales, zeros, shape)
         if grad_input.dtype != input.dtype:
             grad_input = grad_input.to(input.dtype)
-    _hand_over(layer, _pending_dw(dy, _as_bf16_2d(input)))  # dW = dY^T X (utils/quant.py:141-142)
+    _hand_over(layer, _pending_dw(_rows(dy), _rows(_as_bf16_2d(input))))  # dW = dY^T X (utils/quant.py:141-142)
     return grad_input
 
 
@@ -585,18 +589,33 @@ _CTX_FORMS = {
 }
 
 
-# Training without an autograd Function of Python's (see LayerNode in csrc/lq_bind.cpp), for activations in the form the kernels take: a
-# layer's forward, which attaches the backward beside it to its result. None: the Function.
-def _plain_activations(x):
-    return type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.numel() > 0 and x.dim() >= 1
+# Training on activations in the form the kernels take: a layer's forward, whose result gets its history from a Function that takes
+# any number of dimensions. The Functions above take rows, and the views around them, forward and backward, cost the host 12 us a
+# call; the kernels of a small layer's step run for 40. None: the Function above.
+@lru_cache(maxsize=None)
+def _history(fn, grads):
+    """apply of an autograd Function named as fn, for a result that is there already: grads is called with what the layer left for it,
+    the tensors saved, dy and whether the input's gradient is wanted, and returns that gradient (as rows, or shaped as dy), or None."""
+    def forward(ctx, x, bias, y, saved, left):
+        ctx.save_for_backward(*saved)
+        ctx.left = left
+        return y[0]
+
+    def backward(ctx, dy):
+        dx = grads(ctx.left, ctx.saved_tensors, dy, ctx.needs_input_grad[0])
+        if dx is not None and dx.dim() != dy.dim():
+            dx = dx.view(dy.shape[:-1] + dx.shape[-1:])
+        return dx, None, None, None, None
+    cls = type(torch.autograd.Function)(fn.__name__, (torch.autograd.Function,),
+                                        {"forward": staticmethod(forward), "backward": staticmethod(backward)})
+    # what Function.apply calls once it has seen that no transform is active and no operand is a wrapper of one that has ended (3 us),
+    # which is known here (see _records_plainly)
+    return super(torch.autograd.Function, cls).apply
 
 
-def _rows(x):
-    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-
-
-def _attach(y, x, bias, saved, backward, left, fn):
-    return ops._native.attach(y, x, bias, saved if bias is None else saved + (bias,), backward, left, fn.__name__ + "Backward")
+def _attach(y, x, bias, saved, grads, left, fn):
+    """y as a function of x and bias. (In a list y is no input of the Function, and so its output rather than a view of it.)"""
+    return _history(fn, grads)(x, bias, [y], saved if bias is None else saved + (bias,), left)
 
 
 def _w4_node(m, x, layer):
@@ -608,7 +627,7 @@ def _w4_node(m, x, layer):
 
 
 def _w4_node_backward(left, saved, dy, wanted):
-    return _w4_backward(*left, _rows(saved[0]), saved[1], dy, wanted)
+    return _w4_backward(*left, saved[0], saved[1], dy, wanted)
 
 
 def _int8_product(x, w8, qscales, bias, alpha_in_bf16, per_token):
@@ -626,7 +645,7 @@ def _int8_product(x, w8, qscales, bias, alpha_in_bf16, per_token):
 def _a8w8_node(m, x, layer):
     qparam, bias, w8 = m._qparam(), m._bias(), m.weight.data
     qscales, per_token = qparam[1], _per_token(qparam)
-    if not _plain_activations(x) or x.shape[-1] != m.input_features:
+    if x.shape[-1] != m.input_features:
         return None
     y, x8, scale = _int8_product(x, w8, qscales, bias, True, per_token)
     if y is None:
@@ -636,12 +655,13 @@ def _a8w8_node(m, x, layer):
 
 def _a8w8_node_backward(left, saved, dy, wanted):
     layer, scale, qscales, per_token = left
+    dy = _rows(dy)
     return _a8w8_grads(layer, dy, _dequantised_input(saved[0], scale, per_token, dy.dtype), (saved[1], qscales), wanted)
 
 
 def _qat_node(m, x, layer):
     qscales, bias, w = m._qparam()[1], m._bias(), m.weight.data
-    if not _plain_activations(x) or x.shape[-1] != m.input_features or w.dtype != torch.bfloat16:
+    if x.shape[-1] != m.input_features or w.dtype != torch.bfloat16:
         return None
     y, _, work = _int8_product(x, _qat_weight_i8(w, qscales), qscales, bias, False, False)
     if y is None:
@@ -652,15 +672,17 @@ def _qat_node(m, x, layer):
 def _qat_node_backward(left, saved, dy, wanted):
     layer, work, qscales = left
     input_f, weight_q = _qat_backward_operands(_rows(saved[0]), saved[1], work, qscales)
-    return _a8w8_grads(layer, dy, input_f, weight_q, wanted)
+    return _a8w8_grads(layer, _rows(dy), input_f, weight_q, wanted)
 
 
 _NODES = {QLinearFunctionW4: _w4_node, QLinearFunctionA8W8_dynamic: _a8w8_node, QLinearFunctionQAT_dynamic: _qat_node}
 
 
 def _records_plainly(x):
-    """Whether a layer in training may attach its backward itself (see the binding's records_plainly)."""
-    return x.is_cuda and not torch.compiler.is_compiling() and (ops._native or ops._fast()).records_plainly()
+    """Whether a layer's result in training may get its history from _attach: the activations have the form the kernels take, autograd
+    records, and nothing looks at the call that would see other tensors than the Function's over rows (see the binding's
+    records_plainly)."""
+    return x.is_cuda and not torch.compiler.is_compiling() and (ops._native or ops._fast()).records_plainly(x)
 
 
 class _HookHandle(torch.utils.hooks.RemovableHandle):

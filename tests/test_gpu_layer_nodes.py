@@ -183,3 +183,38 @@ def test_the_node_is_taken(hip_lib):
     assert kind_of(y) == "QLinearFunctionW4Backward" and len(y.grad_fn.next_functions) == 2
     with through_function():
         assert "View" in kind_of(m(x))  # the Function's rows, shaped again
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("lead", [(4,), (2, 33)])
+def test_compiled_autograd(hip_lib, kind, lead):
+    """The forward as ever, the backward captured and run as a graph."""
+    from torch._dynamo import compiled_autograd
+    m, layers = make(kind)
+    dy = x_of(lead + (K if kind == "mlp" else N,), 7)
+    grads = []
+    for captured in (False, True):
+        for layer in layers:
+            layer.weight.grad = None
+        x = x_of(lead + (K,)).requires_grad_(True)
+        y = m(x)
+        if captured:
+            with compiled_autograd._enable(lambda graph: graph):
+                y.backward(dy)
+        else:
+            y.backward(dy)
+        grads.append([x.grad] + [layer.weight.grad for layer in layers])
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_layer_that_keeps_its_result_is_collected(hip_lib, kind):
+    import gc
+    import weakref
+    m, layers = make(kind)
+    m.out = m(x_of((4, K)).requires_grad_(True))
+    gone = weakref.ref(m)
+    del m, layers
+    gc.collect()
+    assert gone() is None
