@@ -503,6 +503,9 @@ int lq_weight_grad_acc(const void *dy, const void *x, void *dw_inout, int64_t M,
 int lq_weight_grad_acc8(const void *dy, const void *x, int8_t *q_inout, const void *scale, int64_t M, int64_t N,
                         int64_t K, const void *noise_or_null, uint64_t philox_seed, uint64_t philox_offset,
                         void *stream);
+/* Which tile the above would take, launching nothing: the rows and columns of dW in a workgroup's tile and its waves, for form = 0
+ * (lq_weight_grad), 1 (_acc) or 2 (_acc8). compute_units <= 0 asks the current device. No counterpart in the reference. */
+int lq_weight_grad_plan(int form, int64_t M, int64_t N, int64_t K, int compute_units, int *rows, int *columns, int *waves);
 
 /* ---------------------------------------------------------------------------
  * Layout converters (device side).

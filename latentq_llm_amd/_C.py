@@ -54,6 +54,7 @@ SIGNATURES = {
     "lq_weight_grad": [_vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "lq_weight_grad_acc": [_vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "lq_weight_grad_acc8": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _u64, _u64, _vp],
+    "lq_weight_grad_plan": [_i32, _i64, _i64, _i64, _i32, _vp, _vp, _vp],
     "lq_repack_gptq_to_native": [_vp, _vp, _i64, _i64, _vp],
     "lq_repack_native_to_gptq": [_vp, _vp, _i64, _i64, _vp],
     "lq_calib_copy": [_vp, _vp, _i64, _vp],

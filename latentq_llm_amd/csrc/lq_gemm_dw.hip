@@ -366,7 +366,7 @@ __global__ __launch_bounds__(NT) void gemm_dw_kernel(DwParams p) {
         else emit(ic<0>());
     } else {
         // The whole block of the wave goes to LDS as bf16 first (straight-line code), then a rolled loop of
-        // 8 passes of 16 rows does the accumulator arithmetic: unrolled over the accumulator registers that
+        // TM / RPP passes of 16 rows does the accumulator arithmetic: unrolled over the accumulator registers that
         // arithmetic would be some 50 KB of code, more than the instruction cache holds. 16 consecutive k per lane
         // (one Philox block), 4 lanes per row.
         unsigned char *ep = lds_all + wave * (TM * EP);
@@ -436,46 +436,56 @@ static int launch_dw_tile(DwParams p, hipStream_t st, const char *who) {
     return lq_check_launch(who);
 }
 
-// Which tile a product takes: the smallest of three estimates in microseconds, all of the form (time per 64-token step,
-// summed over the rounds of workgroups) x steps + the ways in and out, fitted to 760 products of 64 to 4096 tokens, 768^2 to
-// 11008 x 4096 outputs (192 x 256 tiles: to 430, so that the sum of what a wrong choice costs is smallest). The last round is never
-// empty: 256 tiles on 256 CUs are one full "last" round. A round of 256 x 256 tiles steps in 1.09 us while it leaves half of the CUs
-// idle and in 1.48 with all of them busy (power), of 192 x 256 in 0.81 and 1.13; 128 x 128 tiles step in 0.43 to 0.50 us alone on a CU,
-// in 0.66 to 0.89 as the second workgroup of a CU joins. What comes around the steps depends on the form: bf16 stores, a gradient read
-// and added as well, or the int8 accumulator's arithmetic, some 17 instructions an element, which want every CU and another
-// workgroup's steps beside them. us, 128 x 128 / 192 x 256 / 256 x 256:
+// Which tile a product takes: the smallest of three estimates in microseconds, all of the form (time per 64-token step, summed
+// over the rounds of workgroups) x steps + the ways in and out. The last round is never empty: 256 tiles on 256 CUs are one full "last"
+// round. A round of large tiles steps more slowly with more than half of the CUs busy (power), one of 128 x 128 tiles as the
+// second workgroup of a CU joins. What comes around the steps depends on the form: bf16 stores, a gradient read and added as well, or the
+// int8 accumulator's arithmetic, some 17 instructions an element, which want every CU and another workgroup's steps beside
+// them; the four-wave form has steps and ways of its own. us, 128 x 128 / 192 x 256 / 256 x 256:
 //   tokens, outputs     2048, 2048^2   2000, 8192 x 3072   500, 8192 x 3072   500, 5504 x 2048     64, 4096 x 1536   2000, 11008 x 4096
 //   store               20.4 / - / 39.8    94.9 / - / 92.6     32.2 / 40.4 / 34.1   19.9 / 17.9 / 20.0   6.5 / - / 7.7     171 / - / 153
 //   int8                23.9 / - / 51.0    105 / - / 115       43.8 / 60.7 / 52.8   26.1 / 23.9 / 32.1   11.3 / - / 17.4   188 / - / 186
-// Over the 430 products the medium tile makes the store 1.8 % faster on average, the bf16 add 1.4 and the int8 add 1.6 (up to
-// 17, 16 and 35 %; three are 1 to 3 % slower); the choice costs 0.1, 0.2 and 1.4 % over the fastest of the three.
+// The constants are fitted to 2500 products (8 to 4096 tokens, 768^2 to 11008 x 4096) timed in each form with each tile: to the times
+// (off by 5 % on average), but above all to the choice, which costs 0.19 / 0.13 / 0.02 % (store, add, int8) over the fastest tile. Against the
+// choice between 128 x 128 and 256 x 256 by one estimate for all forms it takes 0.968 / 0.962 / 0.936 of the time, 18 products of the
+// 7500 are more than 2 % slower (at most 9), and 7 of 1500 that it was not fitted to (at most 7). Constants with one set for both
+// 256 x 256 forms and nothing for a masked step had 108 of the 7500: 13 tokens, 4096^2 store 11.9 against 10.9; 3316, 3584 x 11008 add 262 against 242; 64, 3584 x 8832 int8 41.5 against 39.1. Level
+// tiles are not told apart: 65 to 95 tokens, 11008 x 4096 store 28.8 against 27.7, 4096 x 11008 28.5 against 29.1.
 enum DwForm { DW_STORE, DW_ACC, DW_ACC8 };
-enum DwTile { DW_128, DW_192, DW_256 };
+enum DwTile { DW_128, DW_192, DW_256, DW_256_LONE };
 
 static DwTile dw_tile(DwForm form, long long M, long long N, long long K, long long cus) {
-    struct Ways { double once, round, share, second; };  // us per launch, full round, share of the last one, second workgroup on a CU
-    constexpr Ways kWays256[] = {{5.2, 6.6, 4.2, 0}, {7.5, 12.4, 6.8, 0}, {14.9, 14.9, 3.2, 0}};
-    constexpr Ways kWays192[] = {{4.94, 4.96, 2.5, 0}, {6.48, 10.0, 4.77, 0}, {13.14, 12.14, 1.12, 0}};
-    constexpr Ways kWays128[] = {{3.9, 3.5, 1.0, 1.5}, {5.0, 6.1, 1.9, 2.1}, {7.3, 7.2, 0.8, 2.8}};
+    struct Step { double full, last, busy, ragged; };  // us per step of a full round, of the last one, and more by the share of the CUs beyond
+                                                       // half; a masked first step, per round
+    struct Ways { double once, round, share; };        // us per launch, per full round, by the last one's share of the CUs
+    constexpr Step kStep256 = {1.727, 1.002, 0.733, 0.173}, kStepLone = {1.313, 1.009, 1.076, 0.344}, kStep192 = {1.297, 0.806, 0.672, 0.227};
+    constexpr Ways kWays256[] = {{5.592, 7.523, 3.459}, {8.216, 16.138, 6.378}, {15.406, 19.057, 4.035}};
+    constexpr Ways kWaysLone[] = {{5.195, 12.784, 3.316}, {4.709, 22.364, 10.903}};
+    constexpr Ways kWays192[] = {{3.873, 6.196, 3.281}, {8.216, 12.575, 4.083}, {11.188, 14.900, 5.485}};
+    constexpr Ways kWays128[] = {{3.967, 3.740, 1.090}, {4.001, 7.607, 4.524}, {7.150, 8.756, 1.542}};
+    constexpr double kSecond[] = {1.024, 2.759, 4.916};  // 128 x 128: once more, where CUs have two workgroups
     const double steps = (double)((M + 63) / 64);
-    // one workgroup to a CU: a step in a full round, in the last one, and more of it from half of the CUs on
-    auto whole = [&](long long tiles, double full, double last, double busy, const Ways &w) {
+    // one workgroup to a compute unit
+    auto whole = [&](long long tiles, const Step &s, const Ways &w) {
         const long long rounds = (tiles - 1) / cus;
         const double share = (double)(tiles - rounds * cus) / (double)cus;  // the last round's share of the CUs, 0 .. 1
-        const double step = full * (double)rounds + last + (share > 0.5 ? busy * (share - 0.5) : 0.0);
-        return step * steps + w.once + w.round * (double)rounds + w.share * share;
+        const double step = s.full * (double)rounds + s.last + (share > 0.5 ? s.busy * (share - 0.5) : 0.0);
+        return step * steps + w.once + w.round * (double)rounds + w.share * share + (M % 64 ? s.ragged * (double)(rounds + 1) : 0.0);
     };
+    // 4 waves of 128 x 128 from where their faster steps outweigh the longer way in and out (see the top of the file)
+    const bool lone = form != DW_ACC8 && M >= 1536;
     const long long tiles_k = (K + 255) / 256, t128 = ((N + 127) / 128) * ((K + 127) / 128);
-    const double est256 = whole((N + 255) / 256 * tiles_k, 1.47, 1.09, 0.78, kWays256[form]);
-    const double est192 = whole((N + 191) / 192 * tiles_k, 1.35, 0.81, 0.63, kWays192[form]);
+    const double est256 = whole((N + 255) / 256 * tiles_k, lone ? kStepLone : kStep256, lone ? kWaysLone[form] : kWays256[form]);
+    const double est192 = whole((N + 191) / 192 * tiles_k, kStep192, kWays192[form]);
     const long long rounds128 = (t128 - 1) / (2 * cus);
     const double r128 = (double)(t128 - rounds128 * 2 * cus) / (double)cus;  // 0 .. 2 workgroups per CU
-    const double step128 = 0.83 * (double)rounds128 + (r128 <= 1 ? 0.43 + 0.07 * r128 : 0.66 + 0.23 * (r128 - 1));
+    const double step128 = 0.858 * (double)rounds128 + (r128 <= 1 ? 0.355 + 0.204 * r128 : 0.745 + 0.049 * (r128 - 1));
     const Ways &w128 = kWays128[form];
     const double est128 = step128 * 0.5 * (double)((M + 31) / 32) + w128.once + w128.round * (double)rounds128 +
-                          (r128 <= 1 ? w128.share * r128 : w128.second + w128.share * (r128 - 1));
+                          (r128 <= 1 ? w128.share * r128 : kSecond[form] + w128.share * (r128 - 1)) +
+                          (M % 32 ? 0.185 * (double)(rounds128 + 1) : 0.0);
     const double large = est192 < est256 ? est192 : est256;
-    return est128 < large ? DW_128 : est192 < est256 ? DW_192 : DW_256;
+    return est128 < large ? DW_128 : est192 < est256 ? DW_192 : lone ? DW_256_LONE : DW_256;
 }
 
 static int launch_dw(const DwParams &p, DwForm form, hipStream_t st, const char *who) {
@@ -484,21 +494,39 @@ static int launch_dw(const DwParams &p, DwForm form, hipStream_t st, const char 
         return tile == DW_128   ? launch_dw_tile<128, 128, 256, 32, 4, true>(p, st, who)
                : tile == DW_192 ? launch_dw_tile<192, 256, 512, 64, 2, true>(p, st, who)
                                 : launch_dw_tile<256, 256, 512, 64, 2, true>(p, st, who);
-    if (tile == DW_128) return launch_dw_tile<128, 128, 256, 32, 4, false>(p, st, who);
-    if (tile == DW_192) return launch_dw_tile<192, 256, 512, 64, 2, false>(p, st, who);
-    // 4 waves of 128 x 128 from where their faster steps outweigh the longer way in and out (see the top of the file)
-    return p.M >= 1536 ? launch_dw_tile<256, 256, 256, 64, 2, false>(p, st, who) : launch_dw_tile<256, 256, 512, 64, 2, false>(p, st, who);
+    return tile == DW_128   ? launch_dw_tile<128, 128, 256, 32, 4, false>(p, st, who)
+           : tile == DW_192 ? launch_dw_tile<192, 256, 512, 64, 2, false>(p, st, who)
+           : tile == DW_256 ? launch_dw_tile<256, 256, 512, 64, 2, false>(p, st, who)
+                            : launch_dw_tile<256, 256, 256, 64, 2, false>(p, st, who);
+}
+
+static int check_dw_sizes(const char *who, int64_t M, int64_t N, int64_t K, int k_mult) {
+    LQ_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "%s: M, N, K must be positive", who);
+    LQ_REQUIRE(N % 8 == 0 && K % k_mult == 0, "%s: N=%lld must be a multiple of 8 and K=%lld of %d", who, (long long)N, (long long)K, k_mult);
+    return LQ_OK;
 }
 
 static int check_dw(const char *who, const void *dy, const void *x, int64_t M, int64_t N, int64_t K, int k_mult) {
     LQ_REQUIRE(dy && x, "%s: null pointer argument", who);
-    LQ_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "%s: M, N, K must be positive", who);
-    LQ_REQUIRE(N % 8 == 0 && K % k_mult == 0, "%s: N=%lld must be a multiple of 8 and K=%lld of %d", who, (long long)N, (long long)K, k_mult);
+    const int rc = check_dw_sizes(who, M, N, K, k_mult);
+    if (rc) return rc;
     LQ_REQUIRE(lq_aligned(dy, 16) && lq_aligned(x, 16), "%s: dy and x must be 16-byte aligned", who);
     return LQ_OK;
 }
 
 }  // namespace
+
+extern "C" int lq_weight_grad_plan(int form, int64_t M, int64_t N, int64_t K, int compute_units, int *rows, int *columns, int *waves) {
+    LQ_REQUIRE(rows && columns && waves, "lq_weight_grad_plan: null pointer argument");
+    LQ_REQUIRE(form >= DW_STORE && form <= DW_ACC8, "lq_weight_grad_plan: form=%d must be 0, 1 or 2", form);
+    int rc = check_dw_sizes("lq_weight_grad_plan", M, N, K, form == DW_ACC8 ? 16 : 8);
+    if (rc) return rc;
+    const DwTile tile = dw_tile((DwForm)form, M, N, K, compute_units > 0 ? compute_units : lq_device_cu_count());
+    *rows = tile == DW_128 ? 128 : tile == DW_192 ? 192 : 256;
+    *columns = tile == DW_128 ? 128 : 256;
+    *waves = tile == DW_128 || tile == DW_256_LONE ? 4 : 8;
+    return LQ_OK;
+}
 
 extern "C" int lq_weight_grad(const void *dy, const void *x, void *dw_out, int64_t M, int64_t N, int64_t K, void *stream) {
     int rc = check_dw("lq_weight_grad", dy, x, M, N, K, 8);

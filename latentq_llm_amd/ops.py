@@ -358,6 +358,17 @@ def a16w4_gate_up_plan(M: int, shape, workspace_bytes: int = WORKSPACE_MAX_BYTES
     return PLAN_KERNELS[k.value], rows.value, sp.value
 
 
+def weight_grad_plan(form: str, M: int, shape, compute_units: int = 0):
+    """(rows, columns, waves) of the tile that weight_grad ("store"), weight_grad_acc ("add") or weight_grad_acc8 ("int8") would take
+    for M tokens and an [N, K] gradient. Launches nothing, as a16w4_plan."""
+    import ctypes
+    N, K = shape
+    rows, columns, waves = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    _C.call("lq_weight_grad_plan", ("store", "add", "int8").index(form), M, N, K, compute_units, ctypes.addressof(rows),
+            ctypes.addressof(columns), ctypes.addressof(waves))
+    return rows.value, columns.value, waves.value
+
+
 def a16w4_dequant(codes, scales, zeros, shape):
     N, K = shape
     _codes_ok(codes, N, K)

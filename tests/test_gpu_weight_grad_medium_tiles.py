@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 5504, 2048), (33, 3080, 3088), (64, 3072, 3072), (65, 4616, 2064), (127, 3080, 3088), (129, 5504, 2048), (333, 4616, 2064),
          (1600, 4616, 2320)]
-# and beside them, tiles of (store, add, int8): 128, 256, 128; 256, 256, 128; 192, 128, 128; 256, 128, 128
+# and beside them, 256 x 256 tiles, and 192 x 256 for the store with 128 x 128 for the two others (117 tokens)
 MIXED = [(18, 4488, 2800), (48, 3432, 3632), (117, 2968, 5616), (88, 4328, 2864)]
 
 

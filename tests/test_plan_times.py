@@ -1,0 +1,26 @@
+"""The tiles that the backward products take, at sizes where a choice by the step times alone, or by one set of constants for two kernels,
+took one that is 3 % slower and more. Host arithmetic for 256 compute units, no launch."""
+import pytest
+
+
+# (store, add or int8), tokens, [N, K]; us on 128 x 128 / 192 x 256 / 256 x 256
+@pytest.mark.parametrize("form,M,shape,tile", [
+    ("store", 13, (4096, 4096), (256, 256, 8)),     # 11.9 / 13.9 / 10.9
+    ("store", 20, (6400, 2304), (256, 256, 8)),     # 11.1 / 13.7 / 10.3
+    ("store", 2956, (11008, 3584), (256, 256, 4)),  # 229 / 231 / 213
+    ("store", 256, (8576, 2304), (192, 256, 8)),    # 24.3 / 20.4 / 22.8
+    ("add", 3316, (3584, 11008), (256, 256, 4)),    # 262 / 266 / 242
+    ("int8", 64, (3584, 8832), (256, 256, 8)),      # 41.5 / 44.3 / 39.1
+    ("int8", 25, (5888, 2816), (256, 256, 8)),      # 22.8 / 31.0 / 21.7
+])
+def test_weight_gradient(hip_lib, form, M, shape, tile):
+    from latentq_llm_amd import ops
+    assert ops.weight_grad_plan(form, M, shape, 256) == tile
+
+
+def test_weight_gradient_plan_refuses_what_the_product_does(hip_lib):
+    from latentq_llm_amd import ops
+    from latentq_llm_amd._C import LatentQError
+    for form, shape, text in (("store", (100, 128), "multiple of 8"), ("int8", (128, 136), "K=136 of 16"), ("add", (0, 128), "positive")):
+        with pytest.raises(LatentQError, match=text):
+            ops.weight_grad_plan(form, 64, shape, 256)
