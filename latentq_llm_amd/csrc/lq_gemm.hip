@@ -924,16 +924,19 @@ struct DxCut {
     double step, busy, once, traffic, slice;
 };
 
-// 1100 products timed whole and cut with all three heights (64 to 4096 tokens, 1024^2 to 11008 x 4096, 256 units, weights from HBM): the
-// estimates' choice costs 0.2 % over the fastest, and is 2.3 % faster for one product, 4.6 for a pair, 2.7 for int8 weights than
-// the choice between 128 and 256 rows it replaces (at worst 7 % slower, one of 850). us, 128 / 192 / 256 rows:
+// The constants are fitted to 5900 products (8 to 4096 tokens, 768^2 to 11008 x 4096, weights from HBM; one product, a pair, int8
+// weights) timed whole and cut with all three heights: to the times (off by 6 % on average), but above all to the choice, which costs 0.1 %
+// over the fastest. It takes 0.982 (one), 0.978 (pair) and 0.983 (int8) of the time of the choice between 128 and 256 rows it replaces;
+// 7 products are more than 2 % slower, 7 % at most, and 3 of 1200 that it was not fitted to. A fit to the times of fewer had 49 of the
+// 5900: 256 tokens, int8 10752 x 4096 39.6 against 36.0; 640, pair of 11008 x 3072 123 against 112; 3461, int8 4096 x 1024 41.0 against
+// 37.6. us, 128 / 192 / 256 rows:
 //   whole  3648 tokens, int8 6912 x 2560 178 / 163 / 190    3428, pair of 3712 x 1536 113 / 87 / 96    1664, 9088 x 3840 148 / 195 / 128
 //   cut    299 tokens, pair of 9344 x 4096 89 / 68 / 77     500, 5504 x 2048 23.0 / 25.6 / 26.5        384, pair of 11008 x 3584 81 / 77 / 88
 // Unsplit -> cut: pair of 5504 x 2048 at 500 tokens 97 -> 37, of 11008 x 4096 at 512 194 -> 94; int8 8192 x 2048 at 64 68 -> 17, at 2048 84 -> 79.
 // Two products into one output (lq_a16w4_dx_pair_ws) are planned as one over twice the rows of W.
 static W4Plan plan_dx(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
-    constexpr DxWhole kWhole[] = {{0.52, 0.51, 0.09, 0.79, 1.35, 2.42}, {0.76, 0.60, 0.13, 1.19, 2.02, 4.76}, {0.90, 0.66, 0.24, 1.74, 2.41, 6.65}};
-    constexpr DxCut kCut[] = {{0.51, 0.02, 3.71, 1.08, 0.24}, {0.63, 0.05, 4.63, 0.90, 0.15}, {0.72, 0.09, 6.10, 0.76, 0.02}};
+    constexpr DxWhole kWhole[] = {{0.647, 0.518, 0.054, 0.686, 0.796, 1.973}, {0.946, 0.587, 0.088, 1.885, 0.816, 3.272}, {1.073, 0.770, 0.075, 0.272, 1.926, 6.166}};
+    constexpr DxCut kCut[] = {{0.527, 0.028, 3.631, 1.075, 0.149}, {0.631, 0.058, 4.356, 0.894, 0.142}, {0.709, 0.111, 6.626, 0.688, 0.005}};
     const long long steps = N / 64, fit = (long long)(ws_bytes / ((size_t)M * K * 4));
     W4Plan out;
     double best = 1e30;
@@ -966,12 +969,12 @@ static W4Plan plan_dx(long long M, long long N, long long K, size_t ws_bytes, lo
 }
 
 // dX with the backward of silu(g) * u behind it: whole, since the slices' sum has no such form. The way out reads and writes four
-// matrices, which a round of 256-row tiles does all at once and 128-row tiles beside the next one's steps (260 products fitted, the
-// choice costs 0.1 % over the fastest; 1.5 % faster than the choice between 128 and 256 rows, one of them 1 % slower). us, 128 / 192 / 256 rows:
+// matrices, which a round of 256-row tiles does all at once and 128-row tiles beside the next one's steps (the
+// choice costs 0.01 % over the fastest of 1900 products, and takes 0.985 of the time of the choice between 128 and 256 rows). us, 128 / 192 / 256 rows:
 // 716 tokens, 2048 -> 6400 39.7 / 31.6 / 35.8; 744, 3328 -> 11008 93 / 89 / 102; 500, 2048 -> 5504 25.4 / 30.6 / 34.7; 1928, 2560 -> 7936
 // 102.8 / - / 95.5.
 static W4Plan plan_dx_silu(long long M, long long N, long long K, long long cus) {
-    constexpr DxWhole kWhole[] = {{0.58, 0.46, 0.07, 4.54, 0.15, 4.01}, {0.79, 0.58, 0.11, 5.52, 6.10, 6.02}, {0.99, 0.66, 0.20, 7.16, 7.20, 7.03}};
+    constexpr DxWhole kWhole[] = {{0.596, 0.468, 0.07, 4.54, 0.147, 4.043}, {0.79, 0.58, 0.11, 5.52, 6.10, 6.02}, {0.97, 0.66, 0.195, 5.946, 7.20, 7.03}};
     W4Plan out;
     double best = 1e30;
     for (int i = 0; i < 3; ++i) {

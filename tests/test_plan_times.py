@@ -18,6 +18,21 @@ def test_weight_gradient(hip_lib, form, M, shape, tile):
     assert ops.weight_grad_plan(form, M, shape, 256) == tile
 
 
+# two products into one input gradient are planned as one of twice the rows of W; us on 128 / 192 / 256 rows
+@pytest.mark.parametrize("M,shape,kernel,cut", [
+    (256, (10752, 4096), "staged_256x128", True),   # int8 39.6 / 44.7 / 36.0
+    (640, (22016, 3072), "staged_256x128", True),   # pair 123 / 128 / 112
+    (832, (17408, 2304), "staged_256x128", True),   # pair 99.3 / 100 / 90.9
+    (601, (8064, 2304), "staged_256x128", True),    # 42.6 / 40.4 / 39.6
+    (3461, (4096, 1024), "staged_128x128", False),  # int8 37.6 / 43.0 / 50.5 whole, 41.0 in slices of 256 rows
+    (1664, (4352, 2048), "staged_128x128", False),  # 39.3 / 45.6 / 51.7 whole, 42.0 in slices of 256 rows
+])
+def test_input_gradient(hip_lib, M, shape, kernel, cut):
+    from latentq_llm_amd import ops
+    got, slices, _ = ops.a16w4_plan(M, shape, backward=True, compute_units=256)
+    assert (got, slices > 1) == (kernel, cut)
+
+
 def test_weight_gradient_plan_refuses_what_the_product_does(hip_lib):
     from latentq_llm_amd import ops
     from latentq_llm_amd._C import LatentQError
