@@ -23,6 +23,7 @@ def ops(hip_lib):
 @pytest.mark.parametrize("M,N,K", SIZES)
 def test_every_token_counts_once(ops, M, N, K):
     """Integers whose sums fp32 holds, and bf16 up to 256; beyond that the one rounding of the exact sum."""
+    assert all(ops.weight_grad_plan(form, M, (N, K), 256) == (192, 256, 8) for form in ("store", "add", "int8"))
     gen = torch.Generator().manual_seed(M)
     dy = torch.randint(-1, 2, (M, N), generator=gen).to(torch.bfloat16).cuda()
     x = torch.randint(-1, 2, (M, K), generator=gen).to(torch.bfloat16).cuda()
