@@ -201,8 +201,8 @@ int lq_a16w4_dx_pair_ws(const void *dy1, const void *codes1, const void *scales1
                         const void *codes2, const void *scales2, const void *zeros2, void *dx, int64_t M, int64_t N,
                         int64_t K, int group, void *workspace, int64_t workspace_bytes, void *stream);
 
-/* Which kernel lq_a16w4_fwd(_ws) (backward = 0) or lq_a16w4_dx(_ws) (backward = 1) would run for a
- * shape and a workspace size, and how it would cut the reduction; launches nothing. *kernel is
+/* Which kernel lq_a16w4_fwd(_ws) (backward = 0), lq_a16w4_dx(_ws) (backward = 1) or lq_a16w4_dx_silu_bwd
+ * (backward = 2) would run for a shape and a workspace size, and how it would cut the reduction; launches nothing. *kernel is
  * one of LQ_PLAN_*; *splits > 1 means a split reduction of *steps_per_split 64-deep steps per slice
  * followed by the reduce kernel. compute_units <= 0 asks the current device. The choice follows a
  * rough cost model of measured per-step times (see lq_gemm.hip); it is exposed so that callers and

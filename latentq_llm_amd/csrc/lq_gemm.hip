@@ -1289,7 +1289,7 @@ extern "C" int lq_a16w4_plan(int backward, int64_t M, int64_t N, int64_t K, int6
     const size_t ws = workspace_bytes > 0 ? (size_t)workspace_bytes : 0;
     W4Plan plan;
     if (!backward && M <= 16) plan.kernel = LQ_PLAN_GEMV;
-    else plan = backward ? plan_dx(M, N, K, ws, cus) : plan_fwd(M, N, K, ws, cus);
+    else plan = backward == 2 ? plan_dx_silu(M, N, K, cus) : backward ? plan_dx(M, N, K, ws, cus) : plan_fwd(M, N, K, ws, cus);
     *kernel = plan.kernel; *splits = plan.splits; *steps_per_split = plan.steps_per_split;
     return LQ_OK;
 }

@@ -335,14 +335,15 @@ PLAN_KERNELS = {0: "gemv", 1: "gemv_chunks", 2: "direct_128x256", 3: "staged_128
                 5: "direct_128x128", 6: "few_x16", 7: "staged_192x128"}
 
 
-def a16w4_plan(M: int, shape, backward: bool = False, workspace_bytes: int = WORKSPACE_MAX_BYTES, compute_units: int = 0):
+def a16w4_plan(M: int, shape, backward: bool = False, workspace_bytes: int = WORKSPACE_MAX_BYTES, compute_units: int = 0,
+               silu: bool = False):
     """(kernel name, splits, steps per slice) the forward / dX entry points would use for M tokens on an
-    [N, K] matrix; compute_units = 0 asks the current device. Launches nothing (works without a GPU when
-    compute_units is given)."""
+    [N, K] matrix; compute_units = 0 asks the current device. silu: dX with the SiLU backward behind it
+    (a16w4_dx_silu_bwd). Launches nothing (works without a GPU when compute_units is given)."""
     import ctypes
     N, K = shape
     k, sp, per = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
-    _C.call("lq_a16w4_plan", int(bool(backward)), M, N, K, workspace_bytes, compute_units, ctypes.addressof(k),
+    _C.call("lq_a16w4_plan", 2 if silu else int(bool(backward)), M, N, K, workspace_bytes, compute_units, ctypes.addressof(k),
             ctypes.addressof(sp), ctypes.addressof(per))
     return PLAN_KERNELS[k.value], sp.value, per.value
 

@@ -57,9 +57,10 @@ def test_slices(hip_lib, M, N, K):
     check(ops.a8w8_dx(dy, w8, qs), [(dy, (w8.to(torch.bfloat16) * qs[:, None]).to(torch.bfloat16).double())])
 
 
-@pytest.mark.parametrize("M,N,K", [(716, 2048, 6400), (577, 128, 6656)])
-def test_silu_backward(hip_lib, M, N, K):
+@pytest.mark.parametrize("M,N,K,rows", [(716, 2048, 6400, 192), (769, 2048, 6400, 192), (577, 128, 6656, 128)])
+def test_silu_backward(hip_lib, M, N, K, rows):
     from latentq_llm_amd import ops
+    assert ops.a16w4_plan(M, (N, K), silu=True, compute_units=256) == ("staged_%dx128" % rows, 1, 0)
     w, _ = weights(N, K, 3)
     dy, g, u = randn_bf16((M, N), 4).cuda(), randn_bf16((M, K), 6, 2.0).cuda(), randn_bf16((M, K), 7).cuda()
     want = ops.a16w4_dx_silu_bwd(dy, *w, (N, K), g, u)

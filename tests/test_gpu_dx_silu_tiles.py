@@ -8,10 +8,13 @@ from tests.util import make_w4, randn_bf16
 pytestmark = pytest.mark.gpu
 
 
-# on 256 compute units: 256 rows a tile for all the tokens, 128 for the first of them; outputs that end inside a tile
-@pytest.mark.parametrize("full,few,N,K", [(1928, 257, 2560, 7936), (1916, 130, 3584, 8064)])
-def test_tile_heights_agree(full, few, N, K):
+# rows of a tile for all the tokens and for the first of them, on 256 compute units; outputs that end inside a tile
+@pytest.mark.parametrize("full,few,N,K,heights", [(1928, 257, 2560, 7936, (256, 128)), (1916, 130, 3584, 8064, (256, 128)),
+                                                  (716, 257, 2048, 6400, (192, 128)), (1928, 716, 2048, 6400, (256, 192))])
+def test_tile_heights_agree(full, few, N, K, heights):
     from latentq_llm_amd import ops
+    for M, rows in zip((full, few), heights):
+        assert ops.a16w4_plan(M, (N, K), silu=True, compute_units=256) == ("staged_%dx128" % rows, 1, 0)
     _, packed, scales, zeros = make_w4(N, K, 3)
     w = (packed.cuda(), scales.cuda(), zeros.cuda())
     dy, g, u = randn_bf16((full, N), 4).cuda(), randn_bf16((full, K), 6, 2.0).cuda(), randn_bf16((full, K), 7).cuda()

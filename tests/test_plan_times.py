@@ -33,6 +33,15 @@ def test_input_gradient(hip_lib, M, shape, kernel, cut):
     assert (got, slices > 1) == (kernel, cut)
 
 
+# with the SiLU backward behind it; us on 128 / 192 / 256 rows
+@pytest.mark.parametrize("M,shape", [(3462, (3840, 7936)),   # 266 / 265 / 255
+                                     (1728, (4096, 11008)),  # 195 / 203 / 187
+                                     (2432, (3840, 11008))])  # 253 / 257 / 245
+def test_input_gradient_with_silu(hip_lib, M, shape):
+    from latentq_llm_amd import ops
+    assert ops.a16w4_plan(M, shape, silu=True, compute_units=256) == ("staged_256x128", 1, 0)
+
+
 def test_weight_gradient_plan_refuses_what_the_product_does(hip_lib):
     from latentq_llm_amd import ops
     from latentq_llm_amd._C import LatentQError
