@@ -1056,16 +1056,18 @@ struct GateUpPlan {
 //
 // 17 to 64 tokens: the kernel of lq_gate_up_few.hip (few: scales and zeros lie on 4 bytes, as it wants them). 330 sizes, speed
 // against what the rest of this function says, mean and least:
-//   more than 8, up to 16 columns a unit      up to 48 tokens 1.50, 1.09;  49 to 64: 1.33, 1.05 up to K = 6144, 0.89 at 7168
+//   more than 8, up to 16 columns a unit      up to 48 tokens 1.50, 1.09, from K = 6912 on 1.00, 0.93
+//                                             49 to 64: 1.20, 1.15 up to K = 4352; 1.14 and 1.03 at the next two; 1.00 (0.93 to 1.08) at
+//                                             5120; 1.06, 1.01 and 1.04, 0.97 at 5376 and 5632; 0.94, 0.89 beyond, where K can be cut (2200 sizes)
 //   up to 30 columns, 48 tokens and K = 4096  1.14, 1.00 (31 and 32 columns 0.98 to 1.29; 49 to 64 tokens 0.96; longer K 0.96)
 // With 8 columns a unit and fewer it is 1.02 to 2.1 times as fast, but tests have the staged kernel's slices there.
-static bool gate_up_few_takes(long long M, long long N, long long K, long long cus) {
+static bool gate_up_few_takes(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     if (!lq_gate_up_few_fits(M, N, K, cus) || N <= 8 * cus) return false;
-    return N <= 16 * cus ? M <= 48 || K <= 6144 : N <= 30 * cus && K <= 4096;
+    return N <= 16 * cus ? M <= 48 || K <= 5632 || ws_bytes < (size_t)16 * M * N : N <= 30 * cus && K <= 4096;
 }
 static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_bytes, long long cus, bool few) {
     GateUpPlan out;
-    if (few && gate_up_few_takes(M, N, K, cus)) {
+    if (few && gate_up_few_takes(M, N, K, ws_bytes, cus)) {
         out.kernel = LQ_PLAN_FEW;
         return out;
     }

@@ -1,5 +1,5 @@
-"""The tiles that the backward products take, at sizes where a choice by the step times alone, or by one set of constants for two kernels,
-took one that is 3 % slower and more. Host arithmetic for 256 compute units, no launch."""
+"""The kernels and tiles that products take, at sizes where a choice by the step times alone, or by one set of constants for two kernels,
+or a line drawn from too few sizes, took one that is 2 % slower and more. Host arithmetic for 256 compute units, no launch."""
 import pytest
 
 
@@ -40,6 +40,17 @@ def test_input_gradient(hip_lib, M, shape, kernel, cut):
 def test_input_gradient_with_silu(hip_lib, M, shape):
     from latentq_llm_amd import ops
     assert ops.a16w4_plan(M, shape, silu=True, compute_units=256) == ("staged_256x128", 1, 0)
+
+
+# gate / up of 49 to 64 tokens; us in slices of K / in one launch
+@pytest.mark.parametrize("M,shape", [(54, (3584, 6144)),   # 17.2 / 18.8
+                                     (62, (2336, 5888)),   # 17.3 / 18.0
+                                     (50, (4096, 5888))])  # 17.2 / 18.9
+def test_gate_up_on_a_long_k(hip_lib, M, shape):
+    from latentq_llm_amd import ops
+    kernel, _, slices = ops.a16w4_gate_up_plan(M, shape, compute_units=256)
+    assert kernel == "staged_128x128" and slices > 1
+    assert ops.a16w4_gate_up_plan(M, shape, workspace_bytes=0, compute_units=256)[0] == "few_x16"  # K cannot be cut
 
 
 def test_weight_gradient_plan_refuses_what_the_product_does(hip_lib):
