@@ -810,7 +810,7 @@ static int whole_pairs(int per, int splits, int groups) {
 // workgroup reads all of X, so a longer K and fewer columns are what ends it; an even number of groups, and whole tiles of the staged
 // kernel on half of the units and fewer, since tests have that kernel beside them):
 //                                65 to 96 tokens                          97 to 128
-//   up to 4 columns a unit       1.28, 1.08 to K = 3072; 0.97 at 4096     1.16, 1.13 to K = 2048; 0.94, 0.91 to 3072
+//   up to 4 columns a unit       1.28, 1.08 to K = 3072; 0.97 at 4096     1.15, 1.07 to K = 1792; 0.99, 0.96 at 2048; 0.94, 0.91 to 3072
 //   up to 8                      1.25, 1.01 to K = 5376; 0.92 beyond      1.18, 1.15 to K = 2048; 1.02, 0.93 to 3072
 //   up to 12                     1.27, 1.09 to K = 5376; 1.02, 0.95       1.19, 1.05 to K = 3072; 1.06, 0.98 to 4096
 //   up to 16                     1.25, 0.99 to K = 7168                   1.15, 1.01 to K = 4096; 1.00, 0.98 to 5376

@@ -352,7 +352,7 @@ int lq_gemm_few_groups(long long M) {
 // 16 < M <= 128, N % 16 == 0, K % 128 == 0 and K / 128 <= lq_gemm_few_groups(M) are guaranteed by the caller.
 int lq_gemm_few_launch(const void *x, const void *codes, const void *scales, const void *zeros, const void *bias, void *y, int M, int N,
                        int K, hipStream_t st, unsigned long long *clk, const char *who) {
-    // the 32-bit lane offsets of the loads span the tokens' rows and 16 rows of codes
+    // what the waves' LDS holds (and with it the 32-bit lane offsets of the loads, which span the tokens' rows and 16 rows of codes)
     if (K / LQ_GROUP > lq_gemm_few_groups(M)) return lq_fail(LQ_ERR_BAD_ARG, "%s: K too large", who);
     auto launch = [&](auto kernel, int waves) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)(N / 16)), dim3(64 * waves), 0, st, (const unsigned char *)x, (const unsigned char *)codes, M, N, K,
