@@ -797,35 +797,35 @@ static int whole_pairs(int per, int splits, int groups) {
     return splits > 1 && groups % 2 == 0 && per % 2 && (groups + per) / (per + 1) == splits ? per + 1 : per;
 }
 
-// Where the kernel of lq_gemm_few.hip runs, 17 to 128 tokens. A tile of 16 columns for each of more than half of the units, at most all:
-// everywhere up to K = 8192 (1.01 to 1.3 times the speed of what ran there, 260 sizes), and for up to 32 tokens and less than all units
-// beyond (1.05 to 1.26); beyond, whole tiles of the staged kernel and an even number of groups, up to 48 tokens and
-// K = 10752 1.01 to 1.29 (11008 0.95 to 1.08; 64 tokens 0.84 to 1.11; 1.14 to 1.33 at K = 8192 as well, where a test has the staged kernel). More columns, two rounds of
-// workgroups: up to 32 tokens in place of GEMV launches (1.16 to 1.9), beyond 0.86 to 1.28. Half of the units and fewer (1.1 to 2.2
-// times the speed up to 48 tokens, 0.94 to 1.4 beyond K = 4096 and 48 tokens) but for the sizes at which tests have the other
-// kernels: the smallest matrices, the longest rows, half of the units and rows longer than 2048, columns that are no whole tiles of the
-// staged kernel.
-//
-// 65 tokens and more, against the staged kernel's slices and their sum (310 sizes from K = 1024 on, speed: mean and least; every
-// workgroup reads all of X, so a longer K and fewer columns are what ends it; an even number of groups, and whole tiles of the staged
-// kernel on half of the units and fewer, since tests have that kernel beside them):
+// Where the kernel of lq_gemm_few.hip runs, 17 to 128 tokens, by its speed against what runs otherwise (GEMV launches up to 32 tokens,
+// the staged kernel; 16800 sizes for up to 64 tokens and half of the units' columns, 8200 for 65 tokens and more; mean and least):
+//                                17 to 32 tokens                  33 to 48                            49 to 64
+//   up to 8 columns a unit       1.5 to 2.4, 1.2 to K = 8192;     1.3 to 1.9, 1.1 to K = 7168;        1.1 to 1.7, 0.97 to K = 7168;
+//                                1.1 to 1.25, 1.02 beyond         1.1, 0.98 to 9216; 1.02, 0.90       1.01, 0.88 at 8192
+//   up to 16                     1.3 to 1.6 to K = 8064 (all kernels: 260 sizes, 1.01 least)
+//                                1.05 to 1.26 beyond, not with    1.18, 1.12 at K = 8192 on whole tiles of the staged kernel, 1.01 to
+//                                all units                        1.29 to 10752 with an even number of groups; 64 tokens 0.84 to 1.11
+//   up to 32                     1.16 to 1.9 to 4096^2 weights    0.86 to 1.28
+// 65 tokens and more, against the staged kernel's slices and their sum, from K = 1024 on: every workgroup reads all of X, so a longer K
+// and fewer columns are what ends it:
 //                                65 to 96 tokens                          97 to 128
-//   up to 4 columns a unit       1.28, 1.08 to K = 3072; 0.97 at 4096     1.15, 1.07 to K = 1792; 0.99, 0.96 at 2048; 0.94, 0.91 to 3072
-//   up to 8                      1.25, 1.01 to K = 5376; 0.92 beyond      1.18, 1.15 to K = 2048; 1.02, 0.93 to 3072
-//   up to 12                     1.27, 1.09 to K = 5376; 1.02, 0.95       1.19, 1.05 to K = 3072; 1.06, 0.98 to 4096
-//   up to 16                     1.25, 0.99 to K = 7168                   1.15, 1.01 to K = 4096; 1.00, 0.98 to 5376
+//   up to 4 columns a unit       1.32, 1.02 to K = 3072; 0.97 at 4096     1.20, 1.03 to K = 1920; 1.00, 0.92 at 2048; 0.94, 0.91 to 3072
+//   up to 8                      1.26, 1.02 to K = 4480; 1.04, 0.94       1.19, 1.05 to K = 1920; 1.08, 1.00 at 2048; 1.02, 0.93 to 3072
+//   up to 12                     1.32, 1.09 to K = 4480; 1.06, 0.95       1.21, 1.03 to K = 3072; 1.06, 0.98 to 4096
+//   up to 16                     1.28, 0.97 to K = 7168                   1.20, 1.05 to K = 4096; 1.00, 0.98 to 5376
+// On whole tiles of the staged kernel and an even number of groups some lines lie a step further, where both are level: this kernel does
+// not round the weights there.
 static bool few_takes(long long M, long long N, long long K, long long cus) {
     if (K / LQ_GROUP > lq_gemm_few_groups(M)) return false;
     if (M > 64) {
-        if (K < 1024 || K % 256 != 0 || N > 16 * cus || (N <= 8 * cus && N % 128 != 0)) return false;
-        if (M <= 96) return K <= (N <= 4 * cus ? 3072 : N <= 12 * cus ? 5376 : 7168);
-        return K <= (N <= 8 * cus ? 2048 : N <= 12 * cus ? 3072 : 4096);
+        if (K < 1024 || N > 16 * cus) return false;
+        const bool even = K % 256 == 0 && (N > 8 * cus || N % 128 == 0);
+        if (M <= 96) return K <= (N <= 4 * cus ? 3072 : N <= 12 * cus ? (even ? 5376 : 4480) : 7168);
+        return K <= (N <= 8 * cus ? (even ? 2048 : 1920) : N <= 12 * cus ? 3072 : 4096);
     }
     if (N > 16 * cus) return M <= 32 && N <= 32 * cus && K < 8192 && N * K <= 4096ll * 4096;
-    if (2 * N > 16 * cus) return K < 8192 || (M <= 32 && N < 16 * cus) ||
-                                    (M <= 48 && N % 128 == 0 && K % 256 == 0 && K > 8192 && K <= 10752);
-    if (N % 128 != 0 || K >= (M <= 48 ? 8192 : 7168)) return false;
-    return M <= 32 ? N * K > 2048ll * 2048 : N * K >= 1024ll * 2048 && (2 * N < 16 * cus || K <= 2048);
+    if (N <= 8 * cus) return M <= 32 || K <= (M <= 48 ? 9216 : 7168);
+    return K < 8192 || (M <= 32 && N < 16 * cus) || (M <= 48 && N % 128 == 0 && K % 256 == 0 && K <= 10752);
 }
 
 // Forward pass, M > 16. Up to 128 tokens the kernel of lq_gemm_few.hip where few_takes says so. Otherwise, up to 64 tokens the staged kernel on any number of tiles, with weights that are not rounded to bf16
@@ -851,9 +851,8 @@ static bool few_takes(long long M, long long N, long long K, long long cus) {
 //                                      three workgroups on a unit: ~0.55-0.61 alone (the more units are busy, the lower
 //                                      the clock: 0.55 up to three quarters of them, 0.61 with all), ~0.74 as soon as a
 //                                      few units hold two, ~1.23 for two everywhere, ~1.38 for three.
-// Up to 32 tokens two GEMV launches of 16 are a little faster than the staged kernel where a launch does not wait for the matrix' bytes
-// and K is not long (2048 x 2048: 7.4 / 8.1 us at 17 / 32 tokens against 8.6 / 9.0; 1024 x 4096 9.1 / 10.3 against 9.7 / 10.2); at
-// 11008 x 4096 they take 21.0 / 23.4 us against 18.1 / 17.7, at 1536 x 8192 14.4 / 17.0 against 13.1 / 13.7.
+// Up to 32 tokens two GEMV launches of 16 are a little faster than the staged kernel on many short rows (more than 32 columns a unit, K
+// below 2048); at 11008 x 4096 they take 21.0 / 23.4 us at 17 / 32 tokens against 18.1 / 17.7.
 static W4Plan plan_fwd(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
     W4Plan out;
     if (few_takes(M, N, K, cus)) {
@@ -1056,13 +1055,15 @@ struct GateUpPlan {
 //
 // 17 to 64 tokens: the kernel of lq_gate_up_few.hip (few: scales and zeros lie on 4 bytes, as it wants them). 330 sizes, speed
 // against what the rest of this function says, mean and least:
+//   up to 8 columns a unit                    17 to 32: 1.5, 1.08;  33 to 48: 1.4, 0.97 up to K = 6656, 1.00, 0.92 beyond
+//                                             49 to 64: 1.3, 0.98 up to K = 4864; 1.04, 0.87 beyond (7400 sizes)
 //   more than 8, up to 16 columns a unit      up to 48 tokens 1.50, 1.09, from K = 6912 on 1.00, 0.93
 //                                             49 to 64: 1.20, 1.15 up to K = 4352; 1.14 and 1.03 at the next two; 1.00 (0.93 to 1.08) at
 //                                             5120; 1.06, 1.01 and 1.04, 0.97 at 5376 and 5632; 0.94, 0.89 beyond, where K can be cut (2200 sizes)
 //   up to 30 columns, 48 tokens and K = 4096  1.14, 1.00 (31 and 32 columns 0.98 to 1.29; 49 to 64 tokens 0.96; longer K 0.96)
-// With 8 columns a unit and fewer it is 1.02 to 2.1 times as fast, but tests have the staged kernel's slices there.
 static bool gate_up_few_takes(long long M, long long N, long long K, size_t ws_bytes, long long cus) {
-    if (!lq_gate_up_few_fits(M, N, K, cus) || N <= 8 * cus) return false;
+    if (!lq_gate_up_few_fits(M, N, K, cus)) return false;
+    if (N <= 8 * cus) return K <= (M <= 32 ? 7168 : M <= 48 ? 6656 : 4864) || ws_bytes < (size_t)16 * M * N;
     return N <= 16 * cus ? M <= 48 || K <= 5632 || ws_bytes < (size_t)16 * M * N : N <= 30 * cus && K <= 4096;
 }
 static GateUpPlan plan_gate_up(long long M, long long N, long long K, size_t ws_bytes, long long cus, bool few) {

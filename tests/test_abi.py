@@ -160,11 +160,12 @@ def test_dispatch_plan_host_logic(hip_lib):
 
     # decode sizes
     assert plan(1, 11008, 4096) == ("gemv", 1, 0) and plan(16, 4096, 11008) == ("gemv", 1, 0)
-    # beyond them GEMV launches where they are faster: small matrices with short rows
-    assert plan(17, 2048, 2048)[0] == "gemv_chunks" and plan(32, 1024, 4096)[0] == "gemv_chunks"
+    # beyond them GEMV launches where they are faster: many short rows; few columns in one launch
+    assert plan(17, 8208, 1024)[0] == plan(32, 16384, 1024)[0] == "gemv_chunks"
+    assert plan(17, 2048, 2048)[0] == plan(32, 1024, 4096)[0] == "few_x16"
     for M in (17, 18, 32):
-        assert plan(M, 11008, 4096) == ("staged_128x128", 2, 32) and plan(M, 1536, 8192)[0] == "staged_128x128"
-        assert plan(M, 4096, 4096)[0] == "few_x16"
+        assert plan(M, 11008, 4096) == ("staged_128x128", 2, 32) and plan(M, 1536, 11648)[0] == "staged_128x128"
+        assert plan(M, 4096, 4096)[0] == plan(M, 1536, 8192)[0] == "few_x16"
     # 2048 tokens on the 7B MLP matrices: weights-direct forward, large staged tiles backward, no split
     assert plan(2048, 11008, 4096) == ("direct_128x256", 1, 0)
     assert plan(2048, 4096, 11008) == ("direct_128x256", 1, 0)
@@ -188,7 +189,7 @@ def test_dispatch_plan_host_logic(hip_lib):
         assert plan(M, N, K) == ("direct_128x128", 1, 0) and plan(M, N, K + 128) == ("staged_128x128", 1, 0)
     assert plan(700, 4096, 8192) == plan(640, 4096, 11008) == ("staged_128x128", 1, 0)
     # up to 64 tokens: slices of whole pairs of groups, unless they are short, rows are an odd number of groups or it would be a slice less
-    assert plan(61, 4096, 9216) == ("staged_128x128", 8, 20) and plan(64, 4112, 1792)[2] == plan(56, 1280, 1280)[2] == 10
+    assert plan(61, 4096, 9216) == ("staged_128x128", 8, 20) and plan(64, 4112, 1792)[2] == plan(56, 4880, 2560)[2] == 10
     assert plan(61, 4096, 9088) == ("staged_128x128", 8, 18) and plan(65, 4096, 9216)[2] % 4 == 2
     # skinny grids: split reduction, slices of an even number of steps >= 8 that cover the reduction
     for M, N, K, back in [(128, 11008, 4096, True), (512, 11008, 4096, True), (1024, 11008, 4096, True),

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("backward,M,N,K,kernel", [(0, 64, 4096, 1024, "few_x16"), (0, 17, 4096, 4096, "few_x16"), (0, 45, 3088, 640, "few_x16"),
-                                                   (0, 33, 11008, 384, "staged_128x128"), (0, 100, 1040, 1024, "staged_128x128"),
+                                                   (0, 33, 11008, 384, "staged_128x128"), (0, 100, 1040, 896, "staged_128x128"),
                                                    (0, 256, 11008, 1024, "direct_128x128"), (0, 4224, 4096, 384, "staged_256x128"),
                                                    (1, 300, 1024, 2048, "staged_128x128")])
 def test_every_workgroup_records(hip_lib, backward, M, N, K, kernel):

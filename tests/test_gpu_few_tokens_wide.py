@@ -13,7 +13,7 @@ TOL = 2.0 ** -8
 
 SIZES = [(65, 256, 1024), (80, 1536, 1536), (96, 4096, 4096), (81, 2064, 5376), (90, 3088, 7168), (66, 1024, 3072), (97, 2048, 2048), (113, 512, 1024), (128, 3072, 3072),
          (127, 3088, 3328), (100, 4096, 4096), (112, 4080, 2816), (33, 4096, 4352), (48, 2064, 8064), (49, 3072, 4608), (64, 4080, 7680), (33, 2304, 8448), (48, 4096, 10752),
-         (17, 4096, 10752)]
+         (17, 4096, 10752), (80, 1040, 1152), (65, 2064, 1664), (96, 16, 1024), (81, 4080, 6272), (66, 144, 2944), (128, 144, 1920), (100, 2064, 3072), (113, 3088, 3968)]
 
 
 @pytest.mark.parametrize("M,N,K", SIZES)
@@ -51,7 +51,7 @@ def test_forward(hip_lib, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(129, 2048, 2048), (65, 4112, 1024), (97, 2048, 2304), (97, 3072, 3328), (100, 4096, 4352), (65, 3072, 5632), (65, 1024, 3328), (80, 2048, 896),
-                                   (80, 1040, 1024), (80, 4096, 1152), (48, 4096, 11008), (49, 4096, 8448), (40, 4080, 8448), (40, 4096, 8320)])
+                                   (80, 1040, 4608), (80, 4096, 7296), (81, 2064, 4736), (97, 1040, 2048), (97, 1024, 2176), (48, 4096, 11008), (49, 4096, 8448), (40, 4080, 8448), (40, 4096, 8320)])
 def test_lines(hip_lib, M, N, K):
     from latentq_llm_amd import ops
     assert ops.a16w4_plan(M, (N, K), compute_units=256)[0] == "staged_128x128"

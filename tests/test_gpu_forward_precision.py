@@ -17,8 +17,8 @@ FEW, STAGED = "few_x16", "staged_128x128"
 
 
 @pytest.mark.parametrize("M,N,K,kernel", [(17, 4096, 4096, FEW), (32, 2576, 2560, FEW), (33, 4080, 1664, FEW), (48, 4096, 4096, FEW), (64, 3088, 1024, FEW),
-                                          (18, 11008, 4096, STAGED), (32, 4096, 11008, STAGED), (33, 2560, 8192, STAGED), (45, 5504, 2048, STAGED),
-                                          (48, 1040, 1152, STAGED), (64, 2048, 4224, STAGED), (31, 20480, 1024, STAGED), (64, 33040, 384, STAGED)])
+                                          (18, 11008, 4096, STAGED), (32, 4096, 11008, STAGED), (33, 2576, 8192, STAGED), (45, 5504, 2048, STAGED),
+                                          (48, 4112, 1152, STAGED), (64, 2048, 7296, STAGED), (33, 2560, 8192, FEW), (48, 1040, 1152, FEW), (64, 2048, 4224, FEW), (31, 20480, 1024, STAGED), (64, 33040, 384, STAGED)])
 @pytest.mark.parametrize("zeros", ["integer", "eighths", "large"])
 def test_weights_are_not_rounded(M, N, K, kernel, zeros):
     from latentq_llm_amd import ops

@@ -9,7 +9,7 @@ from tests.util import make_w4, rel_l2
 pytestmark = pytest.mark.gpu
 
 SIZES = [(17, 2064, 1024), (32, 4096, 1280), (33, 2080, 7168), (48, 4096, 2304), (49, 4080, 1024), (64, 2064, 5632), (20, 4112, 1024), (31, 7664, 4096),
-         (48, 7680, 1280), (45, 5504, 2048)]
+         (48, 7680, 1280), (45, 5504, 2048), (32, 128, 1280), (33, 2048, 1024), (35, 1376, 3072), (17, 16, 7168), (48, 144, 6656), (64, 1040, 4864)]
 
 
 def matrices(N, K, offset, frac):

@@ -10,9 +10,9 @@ from tests.util import make_w4, randn_bf16, rel_l2
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,N,K,rows,slices", [(17, 16, 256, 32, 1), (31, 144, 512, 32, 1), (32, 128, 1280, 32, 2), (33, 2048, 1024, 32, 1),
+@pytest.mark.parametrize("M,N,K,rows,slices", [(17, 16, 256, 32, 1), (31, 144, 512, 32, 1), (32, 128, 7424, 32, 8), (33, 2048, 768, 32, 1),
                                                (64, 4112, 768, 32, 1), (65, 528, 2048, 32, 4), (127, 256, 4096, 32, 8), (200, 1040, 256, 32, 1),
-                                               (257, 64, 2304, 32, 4), (33, 8896, 256, 64, 1), (45, 11008, 768, 64, 1), (35, 1376, 3072, 64, 6),
+                                               (257, 64, 2304, 32, 4), (33, 8896, 256, 64, 1), (45, 11008, 768, 64, 1), (49, 1376, 5120, 64, 8),
                                                (71, 8432, 512, 128, 1), (129, 5504, 2048, 128, 1), (66, 2832, 2560, 128, 4), (96, 11008, 512, 0, 0)])
 def test_gate_up(M, N, K, rows, slices):
     from latentq_llm_amd import ops

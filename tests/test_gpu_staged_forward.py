@@ -19,8 +19,8 @@ def ops(hip_lib):
     return o
 
 
-@pytest.mark.parametrize("M,N,K", [(18, 4112, 4224), (31, 2032, 8320), (32, 8208, 4096), (33, 1040, 128), (33, 16, 640), (64, 1040, 1152),
-                                   (65, 2064, 1664), (96, 528, 256), (127, 5504, 2048), (128, 2048, 5504), (129, 1040, 1408),
+@pytest.mark.parametrize("M,N,K", [(18, 4112, 4224), (31, 2032, 11648), (32, 8208, 4096), (33, 4112, 128), (33, 16, 9344), (65, 16, 640), (64, 4112, 1152),
+                                   (65, 4112, 1664), (96, 528, 256), (127, 5504, 2048), (128, 2048, 5504), (129, 1040, 1408),
                                    (257, 4112, 384), (385, 2048, 2048), (513, 2064, 8320), (700, 4096, 8192), (1000, 4096, 1152)])
 def test_staged_forward(ops, M, N, K):
     kernel, _, _ = ops.a16w4_plan(M, (N, K))

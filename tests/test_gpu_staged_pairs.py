@@ -28,14 +28,18 @@ def _x(M, K):
     return torch.randn(M, K, device="cuda", generator=torch.Generator(device="cuda").manual_seed(M)).to(torch.bfloat16)
 
 
-SMALL = [(33, 16, 128), (64, 272, 128), (40, 5504, 256), (64, 1040, 384), (17, 4112, 640), (20, 8208, 1152), (64, 6160, 896),
-         (50, 2048, 5504), (128, 144, 3200), (100, 2064, 1408), (300, 528, 1152), (129, 256, 128), (30, 160, 11008), (61, 4112, 3328), (20, 6160, 4352)]
+SMALL = [(65, 16, 128), (64, 4112, 128), (40, 5504, 256), (64, 4112, 384), (33, 4112, 640), (20, 16400, 1152), (64, 6160, 896),
+         (50, 2048, 7552), (128, 144, 3200), (100, 2064, 3456), (300, 528, 1152), (129, 256, 128), (30, 160, 11776), (61, 4112, 3328), (20, 6160, 4352)]
+# what the kernels of fewer tokens have of the same kinds
+FEW = [(33, 16, 128), (64, 272, 128), (64, 1040, 384), (17, 4112, 640), (20, 8208, 1152), (50, 2048, 5504), (100, 2064, 1408), (30, 160, 11008)]
 LARGE = [(500, 1024, 5504), (257, 2048, 11008), (1000, 2064, 8320)]  # (whose alignment the small ones cover)
 
 
-@pytest.mark.parametrize("M,N,K,offset", [size + (offset,) for offset in (0, 1, 2) for size in SMALL] + [size + (0,) for size in LARGE])
+@pytest.mark.parametrize("M,N,K,offset", [size + (offset,) for offset in (0, 1, 2) for size in SMALL + FEW] + [size + (0,) for size in LARGE])
 def test_forward(hip_lib, M, N, K, offset):
     from latentq_llm_amd import ops
+    kernel = ops.a16w4_plan(M, (N, K), compute_units=256)[0]
+    assert kernel == "staged_128x128" if (M, N, K) in SMALL else (M, N, K) in LARGE or kernel in ("few_x16", "gemv_chunks")
     w = _weights(N, K, M + N + K, offset)
     W = ops.a16w4_dequant(w[0], w[1].clone(), w[2].clone(), (N, K)).double()
     x, b = _x(M, K), _x(1, N)[0]
@@ -52,7 +56,7 @@ def test_forward(hip_lib, M, N, K, offset):
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 11008, 256), (32, 5520, 768), (45, 11024, 512), (64, 8208, 1280), (100, 5504, 512), (150, 2064, 256),
-                                   (40, 144, 2048), (45, 1040, 2816), (55, 5392, 2560), (20, 8176, 2816)])
+                                   (40, 144, 7424), (45, 1040, 6912), (55, 5392, 2560), (20, 8176, 2816)])
 def test_gate_up(hip_lib, M, N, K):
     from latentq_llm_amd import ops
     mats = [_weights(N, K, s, 0) for s in (1, 2)]

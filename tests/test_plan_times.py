@@ -53,6 +53,28 @@ def test_gate_up_on_a_long_k(hip_lib, M, shape):
     assert ops.a16w4_gate_up_plan(M, shape, workspace_bytes=0, compute_units=256)[0] == "few_x16"  # K cannot be cut
 
 
+# forward of 17 to 128 tokens, most on half of the units' columns and fewer; us otherwise / in one launch (36 tokens in the place of 33 and so on)
+@pytest.mark.parametrize("M,shape", [(45, (2048, 4096)),   # 10.6 / 6.9
+                                     (33, (2048, 2304)),   # 9.3 / 5.0
+                                     (64, (2048, 7040)),   # 13.5 / 12.0
+                                     (24, (2048, 2048)),   # 6.8 / 4.4
+                                     (17, (1024, 1024)),   # 6.1 / 3.4
+                                     (45, (4096, 8192)),   # 15.6 / 13.3
+                                     (80, (1536, 1920)),   # 8.8 / 6.5
+                                     (100, (1040, 1664))])  # 8.6 / 7.8
+def test_forward_of_few_columns(hip_lib, M, shape):
+    from latentq_llm_amd import ops
+    assert ops.a16w4_plan(M, shape, compute_units=256) == ("few_x16", 1, 0)
+
+
+# gate / up of 17 to 64 tokens on 8 columns a unit and fewer
+@pytest.mark.parametrize("M,shape", [(20, (2048, 1536)),   # 8.7 / 4.9
+                                     (45, (1408, 4096))])  # 14.3 / 9.6
+def test_gate_up_of_few_columns(hip_lib, M, shape):
+    from latentq_llm_amd import ops
+    assert ops.a16w4_gate_up_plan(M, shape, compute_units=256)[0] == "few_x16"
+
+
 def test_weight_gradient_plan_refuses_what_the_product_does(hip_lib):
     from latentq_llm_amd import ops
     from latentq_llm_amd._C import LatentQError
