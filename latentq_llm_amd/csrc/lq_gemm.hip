@@ -798,23 +798,24 @@ static int whole_pairs(int per, int splits, int groups) {
 }
 
 // Where the kernel of lq_gemm_few.hip runs, 17 to 128 tokens, by its speed against what runs otherwise (GEMV launches up to 32 tokens,
-// the staged kernel; 16800 sizes for up to 64 tokens and half of the units' columns, 8200 for 65 tokens and more; mean and least):
+// the staged kernel). Mean and least over 16000 sizes for up to 64 tokens and 8 columns a unit, 260 for more, 9900 for 65 tokens and more:
 //                                17 to 32 tokens                  33 to 48                            49 to 64
-//   up to 8 columns a unit       1.5 to 2.4, 1.2 to K = 8192;     1.3 to 1.9, 1.1 to K = 7168;        1.1 to 1.7, 0.97 to K = 7168;
-//                                1.1 to 1.25, 1.02 beyond         1.1, 0.98 to 9216; 1.02, 0.90       1.01, 0.88 at 8192
-//   up to 16                     1.3 to 1.6 to K = 8064 (all kernels: 260 sizes, 1.01 least)
-//                                1.05 to 1.26 beyond, not with    1.18, 1.12 at K = 8192 on whole tiles of the staged kernel, 1.01 to
-//                                all units                        1.29 to 10752 with an even number of groups; 64 tokens 0.84 to 1.11
-//   up to 32                     1.16 to 1.9 to 4096^2 weights    0.86 to 1.28
+//   up to 8 columns a unit       1.91, 1.41 to K = 7168; 1.57,    1.57, 1.10 to K = 7168; 1.12, 0.98  1.38, 0.97 to K = 7168; 1.01,
+//                                1.19 to 8192; 1.17, 1.02 beyond  to 9216; 1.02, 0.90 beyond          0.88 to 8192
+//   up to 16                     1.01 to 1.3 up to K = 8064 for all three
+//                                1.05 to 1.26 beyond, not with    1.19, 1.12 at 8192 and 1.01 to      0.84 to 1.11 beyond
+//                                all units                        1.29 to 10752, on whole tiles of the staged kernel and an even
+//                                                                 number of groups
+//   up to 32                     1.39, 1.10 to 4096^2 weights     0.86 to 1.28
 // 65 tokens and more, against the staged kernel's slices and their sum, from K = 1024 on: every workgroup reads all of X, so a longer K
 // and fewer columns are what ends it:
 //                                65 to 96 tokens                          97 to 128
-//   up to 4 columns a unit       1.32, 1.02 to K = 3072; 0.97 at 4096     1.20, 1.03 to K = 1920; 1.00, 0.92 at 2048; 0.94, 0.91 to 3072
-//   up to 8                      1.26, 1.02 to K = 4480; 1.04, 0.94       1.19, 1.05 to K = 1920; 1.08, 1.00 at 2048; 1.02, 0.93 to 3072
-//   up to 12                     1.32, 1.09 to K = 4480; 1.06, 0.95       1.21, 1.03 to K = 3072; 1.06, 0.98 to 4096
-//   up to 16                     1.28, 0.97 to K = 7168                   1.20, 1.05 to K = 4096; 1.00, 0.98 to 5376
-// On whole tiles of the staged kernel and an even number of groups some lines lie a step further, where both are level: this kernel does
-// not round the weights there.
+//   up to 4 columns a unit       1.30, 1.01 to K = 3072; 0.97 at 4096     1.18, 1.02 to K = 1920; 0.99, 0.91 at 2048; 0.94, 0.91 to 3072
+//   up to 8                      1.28, 1.07 to K = 4480; 1.04, 0.94       1.19, 1.08 to K = 1920; 1.09, 1.02 at 2048; 1.02, 0.93 to 3072
+//   up to 12                     1.35, 1.09 to K = 4480; 1.09, 0.95       1.20, 1.02 to K = 3072; 1.06, 0.98 to 4096
+//   up to 16                     1.28, 0.97 to K = 7168                   1.20, 1.04 to K = 4096; 1.00, 0.98 to 5376
+// On whole tiles of the staged kernel and an even number of groups some lines lie a step further, where both are level (0.96 at least): this
+// kernel does not round the weights there.
 static bool few_takes(long long M, long long N, long long K, long long cus) {
     if (K / LQ_GROUP > lq_gemm_few_groups(M)) return false;
     if (M > 64) {
