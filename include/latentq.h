@@ -93,7 +93,8 @@ int lq_philox_uniform(float *out, int64_t n, uint64_t philox_seed, uint64_t phil
  * QLinearFunctionW4.backward (utils/quant.py:136-140): dX[M,K] = dY[M,N] * deq(W).
  * x, y, dy, dx, bias: bf16 row-major; accumulation in fp32, output rounded to
  * bf16 (round-to-nearest-even). M <= 16 takes the wavefront GEMV path. Up to M = 64 the weights enter the product as they
- * are (codes exact, scale applied to fp32 sums); beyond they are rounded to bf16 first, as the reference's are.
+ * are (codes exact, scale applied to fp32 sums), and up to 128 where LQ_PLAN_FEW runs; beyond they are rounded to bf16
+ * first, as the reference's are.
  * The bias is added to the fp32 sum before that single rounding; the reference rounds the
  * product to bf16 first and then adds (utils/quant.py:118-120), one bf16 rounding more.
  * Requirements: K % 128 == 0; N % 16 == 0 for lq_a16w4_fwd, N % 64 == 0 for lq_a16w4_dx;
